@@ -289,6 +289,8 @@ extern "C" int cs_gemm(const CsGemmArgs* args, void* stream_) {
        (uintptr_t)a.w_col_sum) & 15)
     return CS_ERR_INVALID_ARG;
 
+  // inline norms: instead of the arrays, never next to them; w_col_sum alone says that the norm is a LayerNorm
+  if (a.a_norm_inline && (a.a_row_sumsq || a.a_row_sum || a.c_row_sumsq || a.c_row_sum || a.conv_patch || a.a_norm_inline != 1)) return CS_ERR_INVALID_ARG;
   if (a.conv_patch) {   // strided-gather form of the activation operand: general kernel only
     if (a.conv_patch < 2 || a.conv_patch % 2 || a.conv_w % 2 || a.conv_c < 1 || a.conv_h < a.conv_patch ||
         a.conv_w < a.conv_patch || a.epilogue != CS_EPI_BIAS || a.w_fp8 || a.a_rows || a.a_row_sumsq || a.c_row_sumsq ||
@@ -307,7 +309,7 @@ extern "C" int cs_gemm(const CsGemmArgs* args, void* stream_) {
     const int st = cs_gemm_fast(a, stream, &handled);
     if (handled) return st;
   }
-  if (a.a_row_sumsq || a.c_row_sumsq || a.a_row_sum || a.c_row_sum) return CS_ERR_UNSUPPORTED;  // the folded norms exist in the fast kernel only
+  if (a.a_row_sumsq || a.c_row_sumsq || a.a_row_sum || a.c_row_sum || a.a_norm_inline) return CS_ERR_UNSUPPORTED;  // the folded norms exist in the fast kernel only
   // Tile choice: 256x256 when that fills the chip's 256 CUs reasonably, else smaller tiles for more workgroups.
   const int64_t t256 = (int64_t)((a.M + 255) / 256) * ((a.N + 255) / 256);
   const bool small = t256 < 192;

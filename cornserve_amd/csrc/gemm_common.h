@@ -27,6 +27,14 @@ CS_DEVICE float quick_gelu(float x) { return x * __builtin_amdgcn_rcpf(1.0f + __
 CS_DEVICE float silu(float x) { return x * __builtin_amdgcn_rcpf(1.0f + __expf(-x)); }
 
 
+// One output of a product with a folded LayerNorm: acc * rstd - mean * rstd * w_col_sum + bias, every rounding at a fixed
+// place (the compiler would fuse one of the two products, which one depends on the surrounding code), so that all kernels
+// give the same bits.
+CS_DEVICE float layernorm_scaled(float acc, float rstd, float nmean_rstd, float col_sum, float bias) {
+#pragma clang fp contract(off)
+  return __builtin_fmaf(nmean_rstd, col_sum, acc * rstd) + bias;
+}
+
 // Fused epilogue for one wave's accumulators.  acc[i][j][4g+q] = C[m][n] with
 //   m = m_base + i*32 + lane%32,   n = n_base + j*32 + 8g + 4*(lane/32) + q
 // (W was the MFMA "A" operand, so a lane owns one output row and groups of 4 consecutive columns).

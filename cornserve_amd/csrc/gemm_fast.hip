@@ -10,6 +10,8 @@ int cs_gemm_fast_tile_256x160(const CsGemmArgs& a, hipStream_t stream);
 int cs_gemm_fast_tile_128x160(const CsGemmArgs& a, hipStream_t stream);
 int cs_gemm_fast_tile_128x192(const CsGemmArgs& a, hipStream_t stream);
 int cs_gemm_fast_tile_256x128(const CsGemmArgs& a, hipStream_t stream);
+// The few-row kernel (gemm_small.hip).
+int cs_gemm_small(const CsGemmArgs& a, hipStream_t stream, bool* handled);
 
 namespace {
 
@@ -36,7 +38,13 @@ int cs_gemm_fast(const CsGemmArgs& a, hipStream_t stream, bool* handled) {
   // per-lane source offsets are 32-bit byte offsets from the matrix bases
   if ((int64_t)a.M * a.lda * 2 >= (int64_t)UINT32_MAX || (int64_t)a.N * a.ldw * (a.w_fp8 ? 1 : 2) >= (int64_t)UINT32_MAX)
     return CS_OK;
+  // Few rows: tiles small enough to give most compute units one.
+  {
+    const int st = cs_gemm_small(a, stream, handled);
+    if (*handled) return st;
+  }
   *handled = true;
+  if (a.a_norm_inline) return CS_ERR_UNSUPPORTED;   // the inline norms exist in the few-row kernel only
   // Tile shape: the one that needs the least chip time (tile quantisation over the 256 CUs).  The narrow
   // 256x160 tile exists for N = 1280 (8 column tiles: 8192 rows give exactly 256 workgroups).
   const double c256 = rounds_cost(a.M, a.N, 256, 256);

@@ -1027,7 +1027,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_fast_kernel(const CsGemmArgs p) 
 #pragma unroll
         for (int i = 0; i < MT; ++i) {
           const float mean = total8(p.a_row_sum, rsrc_asum, clamp_m(mrow[i])) / (float)p.K;
-          const float var = fmaxf(total8(p.a_row_sumsq, rsrc_asumsq, clamp_m(mrow[i])) / (float)p.K - mean * mean, 0.f);
+          const float var = fmaxf(__builtin_fmaf(-mean, mean, total8(p.a_row_sumsq, rsrc_asumsq, clamp_m(mrow[i])) / (float)p.K), 0.f);
           rstd[i] = rsqrtf(var + p.norm_eps);
           nmean_rstd[i] = -mean * rstd[i];
         }
@@ -1142,9 +1142,13 @@ __global__ __launch_bounds__(64 * NW) void gemm_fast_kernel(const CsGemmArgs p) 
           for (int r = 0; r < 4; ++r) {
             float t = racc[j][r];
             if constexpr (W_FP8) t *= scale_v[W_FP8 ? j : 0][r];
-            if constexpr (NORM_A) t *= rstd[NORM_A ? i : 0];
-            if constexpr (FUSE == FUSE_LN_A) t += nmean_rstd[FUSE == FUSE_LN_A ? i : 0] * csum_v[FUSE == FUSE_LN_A ? j : 0][r];
-            v[r] = t + bf2f(bias_v[j][r]);
+            if constexpr (FUSE == FUSE_LN_A) {
+              v[r] = layernorm_scaled(t, rstd[NORM_A ? i : 0], nmean_rstd[FUSE == FUSE_LN_A ? i : 0],
+                                      csum_v[FUSE == FUSE_LN_A ? j : 0][r], bf2f(bias_v[j][r]));
+            } else {
+              if constexpr (NORM_A) t *= rstd[NORM_A ? i : 0];
+              v[r] = t + bf2f(bias_v[j][r]);
+            }
           }
           if (EPI == CS_EPI_SWIGLU) {
             // SiLU(gate) * up on the fp32 sums, one rounding of the product (the reference rounds gate, SiLU(gate)

@@ -4,6 +4,10 @@
 // file's compiler output for stray uses of them).
 #include "gemm_fast_impl.h"
 
+int cs_qkv_window_attn_small(const CsGemmArgs& a, int rows, hipStream_t stream);
+// Whether a launch of `windows` windows takes that form (gemm_small.hip).
+bool cs_qkv_window_attn_few(int64_t windows, int heads, int K);
+
 extern "C" int cs_qkv_window_attn(const CsGemmArgs* gemm, const float* cos_sin, float scale, int32_t heads,
                                   int32_t head_dim, void* stream_) {
   hipStream_t stream = (hipStream_t)stream_;
@@ -32,8 +36,16 @@ extern "C" int cs_qkv_window_attn(const CsGemmArgs* gemm, const float* cos_sin, 
   a.attn_cos_sin = cos_sin;
   a.attn_scale_log2e = scale * 1.4426950408889634f;
   a.epilogue = CS_EPI_BIAS;
+  if (ragged && ((uintptr_t)a.attn_win_start & 3 || (int64_t)a.attn_n_win * 64 > INT32_MAX)) return CS_ERR_INVALID_ARG;
+  if (a.a_norm_inline && (a.a_norm_inline != 1 || a.a_row_sumsq || a.w_fp8 || a.w_col_sum)) return CS_ERR_INVALID_ARG;
+  // few windows: a workgroup per window and head
+  if (cs_qkv_window_attn_few(ragged ? a.attn_n_win : a.M / 64, heads, a.K)) {
+    const int rows = a.M;
+    if (ragged) a.M = a.attn_n_win * 64;   // (tiles_m counts windows; the operand ends with its last real row)
+    return cs_qkv_window_attn_small(a, rows, stream);
+  }
+  if (a.a_norm_inline) return CS_ERR_UNSUPPORTED;
   if (ragged) {
-    if ((uintptr_t)a.attn_win_start & 3 || (int64_t)a.attn_n_win * 64 > INT32_MAX) return CS_ERR_INVALID_ARG;
     a.M = a.attn_n_win * 64;   // virtual rows: one 64-row slot per window
     if (a.w_fp8) return launch<256, 256, 4, 1, CS_EPI_QKV_WATTN_RAGGED, true, 0>(a, stream);
     if (a.a_row_sumsq) return launch<256, 256, 4, 1, CS_EPI_QKV_WATTN_RAGGED, false, FUSE_NORM_A>(a, stream);

@@ -43,7 +43,7 @@ extern "C" int cs_gemm_rmsnorm_noalloc(const CsGemmArgs* args, void* stream) {
   if (!args) return CS_ERR_INVALID_ARG;
   // The library supplies the row sums: the caller must not, and A must be a plain matrix whose K columns are the
   // normalised width (no row gather: the sums are taken over A's own rows 0..M-1).
-  if (args->a_row_sumsq || args->a_row_sum || args->a_rows || args->w_fp8) return CS_ERR_INVALID_ARG;
+  if (args->a_row_sumsq || args->a_row_sum || args->a_rows || args->w_fp8 || args->a_norm_inline) return CS_ERR_INVALID_ARG;
   if (args->M < 0 || args->K <= 0 || args->N <= 0) return CS_ERR_INVALID_ARG;
   if (args->M > CS_NOALLOC_MAX_ROWS) return CS_ERR_TOO_LARGE;
   if (args->K > 160 * CS_SUMSQ_PARTS) return CS_ERR_TOO_LARGE;

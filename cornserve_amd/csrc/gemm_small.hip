@@ -1,0 +1,117 @@
+// Few-row GEMM for gfx950: choice of the tile form, and whether the launch is a few-row one at all.  The kernel is in
+// gemm_small_impl.h; each tile form is built in its own translation unit (gemm_small_t*.hip).
+#include "gemm_common.h"
+
+int cs_gemm_small_tile_32x32(const CsGemmArgs& a, hipStream_t stream);
+int cs_gemm_small_tile_32x64(const CsGemmArgs& a, hipStream_t stream);
+int cs_gemm_small_tile_64x64(const CsGemmArgs& a, hipStream_t stream);
+int cs_gemm_small_tile_64x80(const CsGemmArgs& a, hipStream_t stream);
+int cs_gemm_small_tile_64x128(const CsGemmArgs& a, hipStream_t stream);
+int cs_gemm_small_tile_128x128(const CsGemmArgs& a, hipStream_t stream);
+int cs_gemm_small_tile_32x160(const CsGemmArgs& a, hipStream_t stream);
+int cs_gemm_small_tile_64x160(const CsGemmArgs& a, hipStream_t stream);
+
+namespace {
+
+// Time of a launch in microseconds: per round of 256 tiles, `fixed_us` (first loads, epilogue, and once 2 us of launch)
+// plus `stage_us` per 128 k.  From launches of 1280 columns at K = 1280 and 3456 that are one round: 96 rows (32x32: 6.0
+// and 8.6 us), 250 (32x64: 7.0, 10.6), 512 (64x64: 8.1, 14.6), 1024 (64x80: 10.2, 18.2; 32x160: 11.8, 22.6), 1500 (64x128:
+// 13.1, 22.5), 2048 (64x160: 16.2, 30.5), 2744 (128x128: 20.3, 33.4).
+struct Form {
+  int bm, bn;
+  float fixed_us, stage_us;
+  int (*run)(const CsGemmArgs&, hipStream_t);
+};
+const Form FORMS[] = {
+    {32, 32, 4.5f, 0.153f, cs_gemm_small_tile_32x32},   {32, 64, 4.9f, 0.212f, cs_gemm_small_tile_32x64},
+    {64, 64, 4.3f, 0.382f, cs_gemm_small_tile_64x64},   {64, 80, 5.5f, 0.470f, cs_gemm_small_tile_64x80},
+    {64, 128, 7.6f, 0.553f, cs_gemm_small_tile_64x128}, {128, 128, 12.6f, 0.770f, cs_gemm_small_tile_128x128},
+};
+const Form SUMS_FORMS[] = {   // with row sums of the output
+    {32, 160, 5.5f, 0.635f, cs_gemm_small_tile_32x160}, {64, 160, 7.8f, 0.841f, cs_gemm_small_tile_64x160},
+};
+// The big tiles of gemm_fast.hip, which run on from tile to tile without a gap: the fixed part counts once (same shapes at
+// 1500, 2744, 4096 and 5104 rows, 3840 and 6912 columns at 1024 and 4096).
+struct FastForm {
+  int bm, bn;
+  float fixed_us, stage_us;
+};
+const FastForm F128x160 = {128, 160, 8.0f, 1.03f}, F256x160 = {256, 160, 7.0f, 1.50f}, F256x256 = {256, 256, 10.0f, 2.65f},
+               F256x128 = {256, 128, 8.0f, 1.50f};
+
+double rounds(int64_t M, int64_t N, int bm, int bn) {
+  const int64_t tiles = ((M + bm - 1) / bm) * ((N + bn - 1) / bn);
+  return (double)((tiles + 255) / 256);
+}
+
+double small_us(const Form& f, int M, int N, int K, bool norm) {
+  const double r = rounds(M, N, f.bm, f.bn), stages = K / 128.0;
+  // (an inline norm: 8.8 and 9.2 us at 96 and 250 rows x 3840 columns, K = 1280, where the plain product takes 8.0 and 8.2)
+  return r * (f.fixed_us - 2.0 + stages * f.stage_us * (norm ? 1.15 : 1.0)) + 2.0;
+}
+
+double fast_us(int M, int N, int K, bool sums, int epilogue) {
+  const double stages = K / 128.0;
+  auto us = [&](const FastForm& f) { return f.fixed_us + rounds(M, N, f.bm, f.bn) * stages * f.stage_us; };
+  const bool few = (int64_t)((M + 255) / 256) * ((N + 159) / 160) <= 128;   // (the rule of gemm_fast.hip)
+  double t = us(few ? F128x160 : F256x160) + (!few && epilogue == CS_EPI_RESIDUAL ? 11.0 : 0.0);   // (29 us at 4888 x 1280 x 1280)
+  if (!sums) t = us(F256x256) < t ? us(F256x256) : t;
+  if (!sums && epilogue == CS_EPI_SWIGLU) t = us(F256x128) < t ? us(F256x128) : t;
+  return t;
+}
+
+template <int COUNT>
+const Form* best_form(const Form (&forms)[COUNT], const CsGemmArgs& a, double* us) {
+  const Form* best = nullptr;
+  *us = 0;
+  for (const Form& f : forms) {
+    if (f.bn == 80 && (a.w_fp8 || a.a_norm_inline || a.pos || !(a.epilogue == CS_EPI_BIAS || (a.epilogue == CS_EPI_RESIDUAL && a.c_lo)))) continue;
+    const double t = small_us(f, a.M, a.N, a.K, a.a_norm_inline);
+    if (!best || t < *us) {
+      best = &f;
+      *us = t;
+    }
+  }
+  return best;
+}
+
+bool inline_norm_shape(int K) { return K % 128 == 0 && K <= 160 * CS_SUMSQ_PARTS; }
+
+}  // namespace
+
+// Called by cs_gemm for a shape that the direct-to-LDS kernels take (see cs_gemm_fast).  Sets *handled when the launch goes
+// to the few-row kernel.
+int cs_gemm_small(const CsGemmArgs& a, hipStream_t stream, bool* handled) {
+  *handled = false;
+  if (a.K % 128 || a.a_row_sumsq || a.a_row_sum || a.conv_patch) return CS_OK;
+  double us;
+  const Form* f;
+  if (a.c_row_sumsq) {   // (other producers of row sums: the big tiles' 160-column forms)
+    if (a.w_fp8 || a.epilogue != CS_EPI_RESIDUAL || !a.c_lo || a.N > 160 * CS_SUMSQ_PARTS) return CS_OK;
+    f = best_form(SUMS_FORMS, a, &us);
+    if (us >= fast_us(a.M, a.N, a.K, true, a.epilogue)) return CS_OK;
+  } else {
+    if (a.a_norm_inline && (!inline_norm_shape(a.K) || a.w_fp8 || a.pos)) return CS_OK;
+    f = best_form(FORMS, a, &us);
+    if (!a.a_norm_inline && us >= fast_us(a.M, a.N, a.K, false, a.epilogue)) return CS_OK;
+  }
+  *handled = true;
+  return f->run(a, stream);
+}
+
+// One workgroup per window and head while the chip holds them all at once: 22 to 25 us up to 16 windows of 16 heads, where
+// a big tile (four windows) takes 32 to 35 us whatever the count; with a second round (24 windows: 39 us) it is the slower.
+bool cs_qkv_window_attn_few(int64_t windows, int heads, int K) { return K % 128 == 0 && windows * heads <= 256; }
+
+extern "C" int cs_gemm_norm_inline_pays(int32_t M, int32_t N, int32_t K, int32_t window_attn) {
+  if (M < 1 || N < 8 || N % 8 || K < 192 || !inline_norm_shape(K)) return 0;
+  if (window_attn) return cs_qkv_window_attn_few(M / 64, N / 256, K) ? 1 : 0;
+  CsGemmArgs a = {};
+  a.M = M;
+  a.N = N;
+  a.K = K;
+  a.a_norm_inline = 1;
+  double us;
+  best_form(FORMS, a, &us);
+  return us < fast_us(M, N, K, false, CS_EPI_SWIGLU) ? 1 : 0;
+}

@@ -1,0 +1,4 @@
+// The 32x64 tile form (2x2 waves) of the few-row GEMM, with a ring of 6 K stages (see gemm_small_impl.h).
+#include "gemm_small_impl.h"
+
+int cs_gemm_small_tile_32x64(const CsGemmArgs& a, hipStream_t stream) { return dispatch_small<32, 64, 2, 2, 2, 6>(a, stream); }

@@ -111,69 +111,41 @@ __global__ __launch_bounds__(256) void layernorm_kernel(const bf16_t* __restrict
   }
 }
 
-// Eight per-lane partial sums -> their eight totals over the wave, with 10 lane exchanges instead of 48: each of
-// the first three exchanges (lane ^ 32, ^ 16, ^ 8) hands the partner the half of the values it keeps, so the number
-// of live values halves; three more exchanges finish the one value left.  Lane l returns the total of part l >> 3.
-static_assert(CS_SUMSQ_PARTS == 8, "wave_sum_parts halves eight values three times");
-CS_DEVICE float wave_sum_parts(const float (&part)[8], int lane) {
-  const bool b5 = lane & 32, b4 = lane & 16, b3 = lane & 8;
-  float a[4], b[2];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const float keep = b5 ? part[4 + i] : part[i], give = b5 ? part[i] : part[4 + i];
-    a[i] = keep + __shfl_xor(give, 32, 64);
-  }
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const float keep = b4 ? a[2 + i] : a[i], give = b4 ? a[i] : a[2 + i];
-    b[i] = keep + __shfl_xor(give, 16, 64);
-  }
-  float c = (b3 ? b[1] : b[0]) + __shfl_xor(b3 ? b[0] : b[1], 8, 64);
-  c += __shfl_xor(c, 4, 64);
-  c += __shfl_xor(c, 2, 64);
-  c += __shfl_xor(c, 1, 64);
-  return c;
-}
-
-// Sums of squares of a row in parts of 160 columns (20 chunks): the variance term of RMSNorm in the form
-// that a GEMM with CsGemmArgs.a_row_sumsq consumes.  out is [rows][CS_SUMSQ_PARTS].
+// Sums of squares (and sums) of a row in parts of 160 columns: the statistics of RMSNorm / LayerNorm in the form that a
+// GEMM with CsGemmArgs.a_row_sumsq consumes.  out is [rows][CS_SUMSQ_PARTS].  The values are summed in the order in which
+// the GEMM epilogues and the inline norms of the few-row GEMM sum them (columns 160 p + 32 j + 8 q .. + 7 chained over j
+// by lane q of part p, then the four lanes), so the statistics of a row have the same bits whichever kernel made them.
+// Half a wave owns a row: lane (p, q) reads its five 16-byte chunks directly, and two lane exchanges end a part.
 template <bool WITH_SUM>
 __global__ __launch_bounds__(256) void row_sumsq_kernel(const bf16_t* __restrict__ x, int64_t ldx, int rows, int H,
                                                         float* __restrict__ out, float* __restrict__ sum_out) {
-  constexpr int NC = (160 * CS_SUMSQ_PARTS / 8 + 63) / 64;
-  const int lane = threadIdx.x & 63;
-  const int row = blockIdx.x * ROWS_PER_BLOCK + (threadIdx.x >> 6);
+  static_assert(CS_SUMSQ_PARTS == 8, "32 lanes: 8 parts of 4");
+  const int half = threadIdx.x & 31, part = half >> 2, q = half & 3;
+  const int row = blockIdx.x * 8 + (threadIdx.x >> 5);
   if (row >= rows) return;
-  const int nchunks = H >> 3;
-  float v[NC][8];
-  load_row<NC>(x + (int64_t)row * ldx, nchunks, lane, v);
-  float part[CS_SUMSQ_PARTS], spart[WITH_SUM ? CS_SUMSQ_PARTS : 1];
+  u32x4_t v[5];
 #pragma unroll
-  for (int q = 0; q < CS_SUMSQ_PARTS; ++q) {
-    part[q] = 0.f;
-    if (WITH_SUM) spart[WITH_SUM ? q : 0] = 0.f;
+  for (int j = 0; j < 5; ++j) {
+    const int c = part * 160 + 32 * j + 8 * q;
+    v[j] = c < H ? *(const u32x4_t*)(x + (int64_t)row * ldx + c) : u32x4_t{0, 0, 0, 0};
   }
+  float ss = 0.f, sm = 0.f;
 #pragma unroll
-  for (int j = 0; j < NC; ++j) {
-    float ss = 0.f, sm = 0.f;
+  for (int j = 0; j < 5; ++j)
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      ss += v[j][e] * v[j][e];
-      sm += v[j][e];
+    for (int w = 0; w < 4; ++w) {
+      const uint32_t word = v[j][w];   // (a copy: the bit cast of a vector's element takes the vector's first one)
+      const bf16x2_t pair = __builtin_bit_cast(bf16x2_t, word), ones = __builtin_bit_cast(bf16x2_t, 0x3F803F80u);
+      ss = __builtin_amdgcn_fdot2_f32_bf16(pair, pair, ss, false);
+      if constexpr (WITH_SUM) sm = __builtin_amdgcn_fdot2_f32_bf16(pair, ones, sm, false);
     }
-    const int q_of_chunk = (lane + 64 * j) / 20;
-#pragma unroll
-    for (int q = 0; q < CS_SUMSQ_PARTS; ++q) {
-      part[q] += (q == q_of_chunk) ? ss : 0.f;
-      if (WITH_SUM) spart[WITH_SUM ? q : 0] += (q == q_of_chunk) ? sm : 0.f;
-    }
-  }
-  // lane l ends up with the total of part l / 8: eight lanes each store one value
-  const float tot = wave_sum_parts(part, lane);
-  if ((lane & 7) == 0) out[(int64_t)row * CS_SUMSQ_PARTS + (lane >> 3)] = tot;
+  ss += __shfl_xor(ss, 1);
+  ss += __shfl_xor(ss, 2);
+  if (q == 0) out[(int64_t)row * CS_SUMSQ_PARTS + part] = ss;
   if constexpr (WITH_SUM) {
-    const float stot = wave_sum_parts(spart, lane);
-    if ((lane & 7) == 0) sum_out[(int64_t)row * CS_SUMSQ_PARTS + (lane >> 3)] = stot;
+    sm += __shfl_xor(sm, 1);
+    sm += __shfl_xor(sm, 2);
+    if (q == 0) sum_out[(int64_t)row * CS_SUMSQ_PARTS + part] = sm;
   }
 }
 
@@ -295,7 +267,7 @@ extern "C" int cs_row_stats(const void* x, int64_t ldx, int32_t rows, int32_t H,
     return CS_ERR_INVALID_ARG;
   if (H > 160 * CS_SUMSQ_PARTS) return CS_ERR_UNSUPPORTED;
   if (rows == 0) return CS_OK;
-  const dim3 grid((rows + ROWS_PER_BLOCK - 1) / ROWS_PER_BLOCK), block(256);
+  const dim3 grid((rows + 7) / 8), block(256);
   if (sum_out)
     hipLaunchKernelGGL(row_sumsq_kernel<true>, grid, block, 0, stream, (const bf16_t*)x, ldx, rows, H, out, sum_out);
   else

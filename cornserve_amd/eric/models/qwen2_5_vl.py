@@ -482,13 +482,29 @@ class Qwen2_5_VisionTransformer(QwenVisionBase):
         # the folded-norm GEMMs exist in the fast kernel only, whose per-lane byte offsets are 32-bit
         fold = self.fold_norm
         eps = self.norm_eps
-        if fold:
-            mark("norm")
-            ss = ops.row_sumsq(x, out=torch.zeros((L, ops.SUMSQ_PARTS), dtype=torch.float32, device=dev))
         qkv = torch.empty((L, 3 * H), dtype=torch.bfloat16, device=dev)
         att = torch.empty((L, H), dtype=torch.bfloat16, device=dev)
         hmid = torch.empty((L, pk["Ip"]), dtype=torch.bfloat16, device=dev)
         scale = d**-0.5
+        # Few rows: the consumer of a folded norm takes the row sums itself, which lets the residual GEMMs in front of it use
+        # tiles that do not span a part of the sums.  Same bits either way, so the choice follows speed alone.
+        n_blocks = len(pk["blocks"])
+        n_slots = fused_rows // ops.QKV_WATTN_WINDOW if win_start is None else win_start.numel() - 1
+        inline_wattn = fold and n_slots > 0 and ops.window_attn_norm_inline_pays(n_slots, nh, H)
+        inline_full = fold and ops.norm_inline_pays(L, 3 * H, H)
+        inline_sep = fold and fused_rows < L and ops.norm_inline_pays(L - fused_rows, 3 * H, H)
+        inline_mlp = fold and ops.norm_inline_pays(L, 2 * pk["Ip"], H)
+
+        def attn_reads_sums(i: int) -> bool:
+            if i >= n_blocks:
+                return False
+            if i in self.fullatt_block_indexes:
+                return not inline_full
+            return (n_slots > 0 and not inline_wattn) or (fused_rows < L and not inline_sep)
+
+        def norm(inline: bool, rows: slice) -> dict:
+            return {"norm_inline": True, "norm_eps": eps} if inline else {"a_row_sumsq": ss[rows], "norm_eps": eps}
+
         # rows [0, fused_rows) belong to the items whose window blocks run as one launch, the rest to the others
         xf = x[:fused_rows]
         # A batch of few rows leaves most compute units idle in the N = hidden GEMMs, and what bounds those launches is
@@ -503,6 +519,11 @@ class Qwen2_5_VisionTransformer(QwenVisionBase):
             nb = pk["blocks"][i + 1]
             return nb["qkv"]["w"] if nb["qkv"] is not None else nb["qkv_wattn"][0]
 
+        if fold:
+            ss = torch.empty((L, ops.SUMSQ_PARTS), dtype=torch.float32, device=dev)
+            if not inline_mlp or any(attn_reads_sums(i) for i in range(n_blocks)):
+                mark("norm")
+                ops.row_sumsq(x, out=ss)   # (writes every part, zeros past the hidden size: the GEMMs write those up to it)
         for i, b in enumerate(pk["blocks"]):
             full = i in self.fullatt_block_indexes
             pf_qkv = b["gu"]["w"] if hint else None   # (from the one-launch window block only: the plain QKV GEMM of a
@@ -514,8 +535,8 @@ class Qwen2_5_VisionTransformer(QwenVisionBase):
                 wsc = sp[0] if sp else None
                 if fold:
                     mark("gemm_qkv_attn_window")
-                    ops.qkv_window_attn(xf, wp, bp, ix.cos_sin[:fused_rows], nh, scale, a_row_sumsq=ss[:fused_rows], norm_eps=eps,
-                                        out=att[:fused_rows], win_start=win_start, prefetch=pf_qkv)
+                    ops.qkv_window_attn(xf, wp, bp, ix.cos_sin[:fused_rows], nh, scale, out=att[:fused_rows],
+                                        win_start=win_start, prefetch=pf_qkv, **norm(inline_wattn, slice(0, fused_rows)))
                 else:
                     mark("norm")
                     ops.rmsnorm(xf, b["n1"], eps, out=n[:fused_rows])
@@ -526,7 +547,7 @@ class Qwen2_5_VisionTransformer(QwenVisionBase):
                 lo = 0 if full else fused_rows           # first row the separate kernels work on in this block
                 if fold:
                     mark("gemm_qkv")
-                    self._g(x[lo:], self._plain_qkv(b), out=qkv[lo:], a_row_sumsq=ss[lo:], norm_eps=eps)
+                    self._g(x[lo:], self._plain_qkv(b), out=qkv[lo:], **norm(inline_full if full else inline_sep, slice(lo, L)))
                 else:
                     mark("norm")
                     ops.rmsnorm(x[lo:], b["n1"], eps, out=n[lo:])
@@ -536,11 +557,13 @@ class Qwen2_5_VisionTransformer(QwenVisionBase):
                 ops.attn_varlen_rotary_(qkv, plan_full if full else plan_win, nh, d, scale, ix.cos_sin, out=att)
             mark("gemm_proj")
             if fold:
-                self._g(att, b["proj"], epilogue=ops.EPI_RESIDUAL, residual=x, out=x, c_row_sumsq=ss, prefetch=pf_proj, **res)
+                self._g(att, b["proj"], epilogue=ops.EPI_RESIDUAL, residual=x, out=x, c_row_sumsq=None if inline_mlp else ss,
+                        prefetch=pf_proj, **res)
                 mark("gemm_gate_up")
-                self._g(x, b["gu"], epilogue=ops.EPI_SWIGLU, out=hmid, a_row_sumsq=ss, norm_eps=eps)
+                self._g(x, b["gu"], epilogue=ops.EPI_SWIGLU, out=hmid, **norm(inline_mlp, slice(0, L)))
                 mark("gemm_down")
-                self._g(hmid, b["down"], epilogue=ops.EPI_RESIDUAL, residual=x, out=x, c_row_sumsq=ss, prefetch=pf_down, **res)
+                self._g(hmid, b["down"], epilogue=ops.EPI_RESIDUAL, residual=x, out=x,
+                        c_row_sumsq=ss if attn_reads_sums(i + 1) else None, prefetch=pf_down, **res)
             else:
                 self._g(att, b["proj"], epilogue=ops.EPI_RESIDUAL, residual=x, out=x, prefetch=pf_proj, **res)
                 mark("norm")

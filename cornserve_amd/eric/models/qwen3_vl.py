@@ -221,18 +221,28 @@ class Qwen3_VisionTransformer(QwenVisionBase):
         scale = d**-0.5
         kept: list[torch.Tensor] = []
         fold = self.fold_norm
-        if fold:
+        # few rows: the consumer takes the row sums itself (see Qwen2_5_VisionTransformer.forward_device)
+        inline_qkv = fold and ops.norm_inline_pays(L, 3 * E, E)
+        inline_fc1 = fold and ops.norm_inline_pays(L, self.intermediate_size + self.mlp_pad, E)
+        sums: dict = {}
+        if fold and not (inline_qkv and inline_fc1):
             mark("norm")
-            ss = torch.zeros((L, ops.SUMSQ_PARTS), dtype=torch.float32, device=dev)
-            sm = torch.zeros_like(ss)
-            ops.row_stats(x, ss, sm)
-            stats_in = lambda lin: {"a_row_sumsq": ss, "a_row_sum": sm, "w_col_sum": lin["colsum"], "norm_eps": eps}  # noqa: E731
-            stats_out = {"c_row_sumsq": ss, "c_row_sum": sm}
-        else:
-            stats_out = {}
+            ss = torch.empty((L, ops.SUMSQ_PARTS), dtype=torch.float32, device=dev)
+            sm = torch.empty_like(ss)
+            ops.row_stats(x, ss, sm)   # (every part, zeros past the hidden size: the GEMMs write those up to it)
+            sums = {"c_row_sumsq": ss, "c_row_sum": sm}
+
+        def stats_in(lin: dict, inline: bool) -> dict:
+            if inline:
+                return {"norm_inline": True, "w_col_sum": lin["colsum"], "norm_eps": eps}
+            return {"a_row_sumsq": ss, "a_row_sum": sm, "w_col_sum": lin["colsum"], "norm_eps": eps}
+
+        planes: dict = {}
         if self.split_residual:   # the byte plane of the residual stream; zero = "x is exact".  It is updated in place
             lo = torch.zeros(x.shape, dtype=torch.uint8, device=dev)   # even when the bf16 plane moves to a new buffer
-            stats_out = dict(stats_out, residual_lo=lo, out_lo=lo)
+            planes = {"residual_lo": lo, "out_lo": lo}
+        stats_proj = planes if inline_fc1 else {**planes, **sums}
+        stats_fc2 = planes if inline_qkv else {**planes, **sums}
         # few rows: each launch names the weights of the launch after next for its idle compute units to read
         hint = L <= self.prefetch_rows
         for i, b in enumerate(pk["blocks"]):
@@ -242,7 +252,8 @@ class Qwen3_VisionTransformer(QwenVisionBase):
                                                else (None, None, None, None))
             if fold:
                 mark("gemm_qkv")
-                ops.gemm(x, b["qkv"]["w"], b["qkv"]["b"], out=qkv, prefetch=pf_qkv, **stats_in(b["qkv"]))
+                ops.gemm(x, b["qkv"]["w"], b["qkv"]["b"], out=qkv, prefetch=pf_qkv,
+                         **stats_in(b["qkv"], inline_qkv))
             else:
                 mark("norm")
                 ops.layernorm(x, *b["n1"], eps, out=n)
@@ -255,19 +266,19 @@ class Qwen3_VisionTransformer(QwenVisionBase):
             mark("gemm_proj")
             # a hidden state kept for a deepstack merger must survive: the next update goes to a new buffer
             x_next = torch.empty_like(x) if kept and kept[-1] is x else x
-            self._g(att, b["proj"], epilogue=ops.EPI_RESIDUAL, residual=x, out=x_next, prefetch=pf_proj, **stats_out)
+            self._g(att, b["proj"], epilogue=ops.EPI_RESIDUAL, residual=x, out=x_next, prefetch=pf_proj, **stats_proj)
             x = x_next
             if fold:
                 mark("gemm_fc1")
                 ops.gemm(x, b["fc1"]["w"], b["fc1"]["b"], epilogue=self.act_epilogue, out=hmid, prefetch=pf_fc1,
-                         **stats_in(b["fc1"]))
+                         **stats_in(b["fc1"], inline_fc1))
             else:
                 mark("norm")
                 ops.layernorm(x, *b["n2"], eps, out=n)
                 mark("gemm_fc1")
                 self._g(n, b["fc1"], epilogue=self.act_epilogue, out=hmid, prefetch=pf_fc1)
             mark("gemm_fc2")
-            self._g(hmid, b["fc2"], epilogue=ops.EPI_RESIDUAL, residual=x, out=x, prefetch=pf_fc2, **stats_out)
+            self._g(hmid, b["fc2"], epilogue=ops.EPI_RESIDUAL, residual=x, out=x, prefetch=pf_fc2, **stats_fc2)
             if i in self.deepstack_visual_indexes:
                 kept.append(x)
 

@@ -124,6 +124,7 @@ def gemm(
     out_lo: torch.Tensor | None = None,
     conv_patch: int = 0,
     prefetch: torch.Tensor | None = None,
+    norm_inline: bool = False,
 ) -> torch.Tensor:
     """out[M,N] = epilogue(a[M,K] @ w[N,K]^T).  `w` is bf16, or float8_e4m3fn/uint8 with `w_scale`.
 
@@ -142,13 +143,17 @@ def gemm(
     fp32 [N], the row sums of the folded weight) the fold is a LayerNorm's: rstd * (acc - mean * w_col_sum) + bias;
     `c_row_sum` receives the plain sums of the output rows.
 
+    `norm_inline`: the folded norm without the arrays: the row sums are taken inside the launch (few rows: see
+    `norm_inline_pays`); RMSNorm, or LayerNorm with `w_col_sum`.  Same bits as with the arrays.
+
     `out_lo` (uint8, shaped and strided like `out`; EPI_RESIDUAL only) carries the residual stream with 16
     significant bits: the sum is not rounded to bf16 but split into `out` (the leading 16 bits) and `out_lo` (the
     next 8 as a signed correction); `residual_lo` is the same plane of the addend (None: the addend is `residual`
     exactly).  A zero-filled plane next to any bf16 tensor is a valid pair.
 
     Dispatches to `torch.ops.cornserve_amd.gemm_` (or the functional `gemm` when nothing is written in place)."""
-    if out is None and c_row_sumsq is None and c_row_sum is None and out_lo is None and residual_lo is None and prefetch is None:
+    if (out is None and c_row_sumsq is None and c_row_sum is None and out_lo is None and residual_lo is None
+            and prefetch is None and not norm_inline):
         return torch.ops.cornserve_amd.gemm(a, w, bias, epilogue, residual, w_scale, pos, a_rows, c_rows, k,
                                             a_row_sumsq, norm_eps, a_row_sum, w_col_sum, conv_patch)
     if out is None:  # (with c_rows: a permutation of the M rows; anything else needs the caller's `out`)
@@ -156,8 +161,19 @@ def gemm(
                           dtype=torch.bfloat16, device=a.device)
     torch.ops.cornserve_amd.gemm_(out, a, w, bias, epilogue, residual, w_scale, pos, a_rows, c_rows, k, a_row_sumsq,
                                   c_row_sumsq, norm_eps, a_row_sum, c_row_sum, w_col_sum, residual_lo, out_lo, conv_patch,
-                                  prefetch)
+                                  prefetch, norm_inline)
     return out
+
+
+def norm_inline_pays(rows: int, n: int, k: int) -> bool:
+    """Whether a folded-norm product of `rows` rows with an [n, k] weight is faster with `norm_inline` than with row sums
+    from arrays (then the producer of its input need not emit any)."""
+    return bool(_l.load().cs_gemm_norm_inline_pays(rows, n, k, 0))
+
+
+def window_attn_norm_inline_pays(windows: int, heads: int, k: int) -> bool:
+    """The same question for `qkv_window_attn`."""
+    return bool(_l.load().cs_gemm_norm_inline_pays(windows * QKV_WATTN_WINDOW, heads * QKV_WATTN_TILE_ROWS, k, 1))
 
 
 def _set_prefetch(args, prefetch: torch.Tensor | None, device: torch.device) -> None:
@@ -191,7 +207,8 @@ def _gemm_functional(a, w, bias, epilogue, residual, w_scale, pos, a_rows, c_row
 
 
 def _gemm_impl(out, a, w, bias, epilogue, residual, w_scale, pos, a_rows, c_rows, k, a_row_sumsq, c_row_sumsq, norm_eps,
-               a_row_sum, c_row_sum, w_col_sum, residual_lo, out_lo, conv_patch=0, prefetch=None) -> None:
+               a_row_sum, c_row_sum, w_col_sum, residual_lo, out_lo, conv_patch=0, prefetch=None,
+               norm_inline=False) -> None:
     """Implementation of cornserve_amd::gemm_: argument checks, then cs_gemm on the current stream."""
     lib = _l.load()
     _req(a, torch.bfloat16, "a")
@@ -304,6 +321,7 @@ def _gemm_impl(out, a, w, bias, epilogue, residual, w_scale, pos, a_rows, c_rows
     args.w_col_sum = _ptr(w_col_sum)
     args.residual_lo = _ptr(residual_lo)
     args.c_lo = _ptr(out_lo)
+    args.a_norm_inline = int(norm_inline)
     _set_prefetch(args, prefetch, a.device)
     _l.check(lib.cs_gemm(ctypes.byref(args), _stream()), "cs_gemm")
 
@@ -919,7 +937,8 @@ def unpack_qkv_window_attn(w_packed: torch.Tensor, b_packed: torch.Tensor, heads
 def qkv_window_attn(x: torch.Tensor, w_packed: torch.Tensor, b_packed: torch.Tensor, cos_sin: torch.Tensor, heads: int,
                     scale: float, *, a_row_sumsq: torch.Tensor | None = None, norm_eps: float = 0.0,
                     out: torch.Tensor | None = None, win_start: torch.Tensor | None = None,
-                    w_scale: torch.Tensor | None = None, prefetch: torch.Tensor | None = None) -> torch.Tensor:
+                    w_scale: torch.Tensor | None = None, prefetch: torch.Tensor | None = None,
+                    norm_inline: bool = False) -> torch.Tensor:
     """attention(rotary(x . Wq^T + bq), rotary(x . Wk^T + bk), x . Wv^T + bv) over windows of up to 64 rows, one launch.
 
     Replaces qkv Linear -> split -> rotary -> flash_attn_varlen_func (qwen2_5_vl.py:93-120).  Without `win_start` the
@@ -928,17 +947,17 @@ def qkv_window_attn(x: torch.Tensor, w_packed: torch.Tensor, b_packed: torch.Ten
     4, which the caller guarantees.  `w_packed`, `b_packed` come from `pack_qkv_window_attn`; with `a_row_sumsq` the
     rows of `x` are RMS-normalised on the way (the norm weight folded into the packed weight's columns, as for
     `gemm`).  fp8 weights: `w_packed` uint8 with `w_scale` (both from `pack_qkv_window_attn`), no folded norm.
-    `prefetch` as for `gemm`.
+    `prefetch` and `norm_inline` as for `gemm`.
     Raises ValueError for shapes the kernel does not take."""
     if out is None:
         out = torch.empty((x.shape[0], heads * QKV_WATTN_HEAD_DIM), dtype=torch.bfloat16, device=x.device)
     torch.ops.cornserve_amd.qkv_window_attn_(out, x, w_packed, b_packed, cos_sin, heads, scale, a_row_sumsq, norm_eps,
-                                              win_start, w_scale, prefetch)
+                                              win_start, w_scale, prefetch, norm_inline)
     return out
 
 
 def _qkv_window_attn_impl(out, x, w_packed, b_packed, cos_sin, heads, scale, a_row_sumsq, norm_eps, win_start=None,
-                          w_scale=None, prefetch=None) -> None:
+                          w_scale=None, prefetch=None, norm_inline=False) -> None:
     lib = _l.load()
     _rows_2d(x, torch.bfloat16, "x")
     fp8 = w_scale is not None
@@ -986,6 +1005,7 @@ def _qkv_window_attn_impl(out, x, w_packed, b_packed, cos_sin, heads, scale, a_r
     args.M, args.N, args.K = M, heads * QKV_WATTN_TILE_ROWS, K
     args.a_row_sumsq = _ptr(a_row_sumsq)
     args.norm_eps = norm_eps
+    args.a_norm_inline = int(norm_inline)
     if win_start is not None:
         args.attn_win_start, args.attn_n_win = win_start.data_ptr(), win_start.numel() - 1
     if fp8:
@@ -1007,7 +1027,7 @@ _OPERATORS: dict[str, tuple[str, object]] = {
     "gemm_": ("(Tensor(a!) out, Tensor a, Tensor w, Tensor? bias, int epilogue, Tensor? residual, Tensor? w_scale, "
               "Tensor? pos, Tensor? a_rows, Tensor? c_rows, int? k, Tensor? a_row_sumsq, Tensor(b!)? c_row_sumsq, "
               "float norm_eps, Tensor? a_row_sum, Tensor(c!)? c_row_sum, Tensor? w_col_sum, Tensor? residual_lo, "
-              "Tensor(d!)? out_lo, int conv_patch=0, Tensor? prefetch=None) -> ()", _gemm_impl),
+              "Tensor(d!)? out_lo, int conv_patch=0, Tensor? prefetch=None, bool norm_inline=False) -> ()", _gemm_impl),
     "row_stats_": ("(Tensor(a!) sumsq_out, Tensor(b!)? sum_out, Tensor x) -> ()", _row_stats_impl),
     "rmsnorm_": ("(Tensor(a!) out, Tensor x, Tensor w, float eps, bool gemma) -> ()", _rmsnorm_impl),
     "layernorm_": ("(Tensor(a!) out, Tensor x, Tensor w, Tensor b, float eps) -> ()", _layernorm_impl),
@@ -1030,7 +1050,7 @@ _OPERATORS: dict[str, tuple[str, object]] = {
     "patchify_nchw_": ("(Tensor(a!) out, Tensor pixels, int patch) -> ()", _patchify_nchw_impl),
     "qkv_window_attn_": ("(Tensor(a!) out, Tensor x, Tensor w_packed, Tensor b_packed, Tensor cos_sin, int heads, "
                          "float scale, Tensor? a_row_sumsq, float norm_eps, Tensor? win_start=None, Tensor? w_scale=None, "
-                         "Tensor? prefetch=None) -> ()",
+                         "Tensor? prefetch=None, bool norm_inline=False) -> ()",
                          _qkv_window_attn_impl),
 }
 

@@ -36,7 +36,7 @@ extern "C" {
 #define CS_ERR_TOO_LARGE 4
 
 /* ABI version of this header; cs_abi_version() returns the value the library was built with. */
-#define CS_ABI_VERSION 7
+#define CS_ABI_VERSION 8
 int cs_abi_version(void);
 
 /* ------------------------------------------------------------------------------------------------
@@ -140,11 +140,23 @@ typedef struct CsGemmArgs {
    * of 20 K tiles costs nothing, 18 MB behind a 192-tile one doubles its duration.                                */
   const void* prefetch;
   int64_t prefetch_bytes;
+  /* Folded norm without the row-sum arrays: with a_norm_inline = 1 the sums over the rows of A are taken inside the
+   * launch (K is the normalised width, at most 160 * CS_SUMSQ_PARTS); a_row_sumsq and a_row_sum are NULL, w_col_sum says
+   * which norm (NULL: RMSNorm, set: LayerNorm), and W, bias and norm_eps are those of the array form.  Same bits as the
+   * array form.  Meant for few rows: cs_gemm_norm_inline_pays tells whether this form is the faster one for a shape.
+   * CS_EPI_BIAS and CS_EPI_SWIGLU (RMSNorm), CS_EPI_BIAS, CS_EPI_GELU_TANH and CS_EPI_QUICK_GELU (LayerNorm); bf16 W,
+   * K a multiple of 128; also taken by cs_qkv_window_attn (RMSNorm).  CS_ERR_UNSUPPORTED otherwise.               */
+  int32_t a_norm_inline;
 } CsGemmArgs;
 #define CS_SUMSQ_PARTS 8
 
 /* Constraints: K % 8 == 0 (16 with fp8), lda/ldw % 8 == 0, N % 4 == 0, A and W 16-byte aligned. */
 int cs_gemm(const CsGemmArgs* args, void* stream);
+
+/* Host routine: 1 if a folded-norm launch of M rows, N weight rows and width K is faster with a_norm_inline than with row
+ * sums read from arrays (few rows), 0 if not or if the shape has no inline form.  window_attn = 1: the same question for
+ * cs_qkv_window_attn with M = 64 * windows and N = 256 * heads.                                                      */
+int cs_gemm_norm_inline_pays(int32_t M, int32_t N, int32_t K, int32_t window_attn);
 
 /* The RMSNorm-folded form of cs_gemm without a workspace: cs_row_sumsq on A followed by cs_gemm with a_row_sumsq, the
  * [M][CS_SUMSQ_PARTS] row sums living in a static device array of the library instead of a buffer of the caller's.

@@ -419,6 +419,99 @@ def test_gemm_fast_path_forms(ops, dev, M, N, K):
     assert torch.equal(scat, ref)
 
 
+# The few-row kernel (K a multiple of 128): every tile form at row and column tails, at the shortest K and at one that runs
+# through its steady loop.  An output has the bits it has as a row of a product with many rows (which the big tiles take),
+# with the norms folded inline or from arrays, and the row sums of its output are the big tiles'.
+@pytest.mark.parametrize("M,N,K", [
+    (1, 64, 256),         # one row
+    (33, 1296, 1280),     # 32x32 tiles, row and column tails
+    (200, 1280, 1152),    # 32x64
+    (500, 1280, 1280),    # 64x64
+    (1000, 1280, 1280),   # 64x80, 32x160 with row sums
+    (1450, 1280, 1280),   # 64x128, 64x160 with row sums
+    (2700, 1280, 1280),   # 128x128 (long K: the residual GEMMs of the larger K)
+    (2196, 1152, 4352),   # 128x128
+])
+def test_gemm_few_rows_equal_the_rows_of_a_large_product(ops, dev, M, N, K):
+    many = 8192
+    a, w, b = rnd((many, K), 1.0, 101, dev), rnd((N, K), 0.05, 102, dev), rnd((N,), 0.02, 103, dev)
+    res = rnd((many, N), 1.0, 104, dev)
+    lo = torch.randint(0, 256, (many, N), generator=torch.Generator().manual_seed(105), dtype=torch.uint8).to(dev)
+    close(ops.gemm(a[:M], w, b)[:64], lin_ref(a[:64][:M], w, b), 2**-7, f"{M}x{N}x{K}")
+    for epi in (ops.EPI_BIAS, ops.EPI_GELU_ERF, ops.EPI_GELU_TANH, ops.EPI_QUICK_GELU, ops.EPI_SWIGLU):
+        assert torch.equal(ops.gemm(a[:M], w, b, epilogue=epi), ops.gemm(a, w, b, epilogue=epi)[:M]), epi
+    assert torch.equal(ops.gemm(a[:M], w, None), ops.gemm(a, w, None)[:M])
+    assert torch.equal(ops.gemm(a[:M], w, b, pos=res[:7]), ops.gemm(a, w, b, pos=res[:7])[:M])
+    assert torch.equal(ops.gemm(a[:M], w, b, epilogue=ops.EPI_RESIDUAL, residual=res[:M]),
+                       ops.gemm(a, w, b, epilogue=ops.EPI_RESIDUAL, residual=res)[:M])
+    perm = torch.randperm(M, generator=torch.Generator().manual_seed(106)).int().to(dev)
+    assert torch.equal(ops.gemm(a[:M], w, b, c_rows=perm)[perm.long()], ops.gemm(a[:M], w, b))
+    # the split residual stream, without and with row sums of the output
+    def split(rows, **sums):
+        out, out_lo = torch.empty_like(res[:rows]), torch.empty_like(lo[:rows])
+        ops.gemm(a[:rows], w, b, epilogue=ops.EPI_RESIDUAL, residual=res[:rows], residual_lo=lo[:rows], out=out, out_lo=out_lo, **sums)
+        return out, out_lo
+    want, want_lo = split(many)
+    got, got_lo = split(M)
+    assert torch.equal(got, want[:M]) and torch.equal(got_lo, want_lo[:M])
+    if N <= 1280:
+        for both in (False, True):
+            s_many, s_few = ([torch.zeros((r, 8), device=dev) for _ in range(1 + both)] for r in (many, M))
+            kw = lambda s: {"c_row_sumsq": s[0], **({"c_row_sum": s[1]} if both else {})}  # noqa: E731
+            split(many, **kw(s_many))
+            got, got_lo = split(M, **kw(s_few))
+            assert torch.equal(got, want[:M]) and torch.equal(got_lo, want_lo[:M])
+            assert all(torch.equal(f, m[:M]) for f, m in zip(s_few, s_many))
+    # folded norms: sums taken inside the launch = sums from the arrays
+    if K <= 1280:
+        ss, sm = torch.empty((M, 8), device=dev), torch.empty((M, 8), device=dev)
+        ops.row_stats(a[:M], ss, sm)
+        for epi in (ops.EPI_BIAS, ops.EPI_SWIGLU):
+            assert torch.equal(ops.gemm(a[:M], w, b, epilogue=epi, norm_inline=True, norm_eps=1e-6),
+                               ops.gemm(a[:M], w, b, epilogue=epi, a_row_sumsq=ss, norm_eps=1e-6)), epi
+        cs = w.float().sum(1)
+        for epi in (ops.EPI_BIAS, ops.EPI_GELU_TANH, ops.EPI_QUICK_GELU):
+            assert torch.equal(ops.gemm(a[:M], w, b, epilogue=epi, norm_inline=True, w_col_sum=cs, norm_eps=1e-6),
+                               ops.gemm(a[:M], w, b, epilogue=epi, a_row_sumsq=ss, a_row_sum=sm, w_col_sum=cs, norm_eps=1e-6)), epi
+    # fp8 weights
+    sc = (w.float().abs().amax(1) / 448.0).contiguous()
+    q = (w.float() / sc[:, None]).to(torch.float8_e4m3fn)
+    assert torch.equal(ops.gemm(a[:M], q, b, w_scale=sc), ops.gemm(a, q, b, w_scale=sc)[:M])
+    with pytest.raises(RuntimeError):      # no inline form: K not a multiple of 128
+        ops.gemm(a[:M, :192].contiguous(), w[:, :192].contiguous(), b, norm_inline=True)
+    with pytest.raises(ValueError):        # inline sums instead of the arrays, not next to them
+        ops.gemm(a[:M], w, b, norm_inline=True, a_row_sumsq=torch.zeros((M, 8), device=dev))
+
+
+@pytest.mark.parametrize("windows,heads,ragged,form", [(1, 1, False, "array"), (16, 16, False, "inline"), (5, 16, True, "inline"),
+                                                       (7, 3, True, "plain"), (6, 2, True, "fp8"), (3, 16, False, "fp8")])
+def test_qkv_window_attn_few_windows_equal_many(ops, dev, windows, heads, ragged, form):
+    """Few windows run one workgroup per window and head: the bits of the four-windows-per-workgroup form, which the same
+    windows take as a part of a larger launch."""
+    K, d = 1280, 80
+    many = 256 // heads + 1 + windows                       # more than the few-window form takes
+    g = torch.Generator().manual_seed(windows)
+    counts = torch.randint(1, 17, (many,), generator=g) * 4 if ragged else torch.full((many,), 64)
+    cu = torch.cat([torch.zeros(1, dtype=torch.int64), counts.cumsum(0)]).int().to(dev)
+    M, rows = int(counts.sum()), int(counts[:windows].sum())
+    x, w, b = rnd((M, K), 1.0, 111, dev), rnd((3 * heads * d, K), 0.05, 112, dev), rnd((3 * heads * d,), 0.02, 113, dev)
+    cos = torch.rand((M, d), generator=g).to(dev)
+    kw = {"norm_eps": 1e-6} if form in ("array", "inline") else {}
+    if form == "fp8":
+        sc = (w.float().abs().amax(1) / 448.0).contiguous()
+        wp, bp, sp = ops.pack_qkv_window_attn((w.float() / sc[:, None]).to(torch.float8_e4m3fn), b, heads, w_scale=sc)
+        kw["w_scale"] = sp
+    else:
+        wp, bp = ops.pack_qkv_window_attn(w, b, heads)
+    ss = ops.row_sumsq(x)
+    sums = {"a_row_sumsq": ss} if form in ("array", "inline") else {}
+    want = ops.qkv_window_attn(x, wp, bp, cos, heads, d**-0.5, win_start=cu if ragged else None, **kw, **sums)[:rows]
+    few = {"norm_inline": True} if form == "inline" else {k: v[:rows] for k, v in sums.items()}
+    got = ops.qkv_window_attn(x[:rows], wp, bp, cos[:rows], heads, d**-0.5,
+                              win_start=cu[: windows + 1].contiguous() if ragged else None, **kw, **few)
+    assert torch.equal(got, want)
+
+
 def test_gemm_prefetch_hint_leaves_the_result_alone(ops, dev):
     """A launch with few tiles and a `prefetch` tensor starts extra workgroups that only read that tensor: the product
     has the bits it has without the hint, whatever the hinted size (odd, shorter than one 16-byte piece, many MB), on
