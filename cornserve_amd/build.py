@@ -1,4 +1,5 @@
-"""Build libcornserve_amd.so (the C-ABI kernel library) in-tree with hipcc for gfx950.
+"""Build libcornserve_amd.so (the C-ABI kernel library) in-tree with hipcc for gfx950, and libcornserve_amd_torch.so
+(host code: native implementations of torch operators over that ABI) with g++.
 
 Usage: ``python -m cornserve_amd.build`` or ``cornserve_amd.build.build_library()``.  The library is
 written next to the sources so that it travels with the tree; nothing is JIT-compiled at import.
@@ -11,6 +12,7 @@ import re
 import shutil
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
@@ -18,6 +20,7 @@ PKG_DIR = Path(__file__).resolve().parent
 CSRC = PKG_DIR / "csrc"
 INCLUDE = PKG_DIR.parent / "include"
 LIB_PATH = PKG_DIR / "libcornserve_amd.so"
+TORCH_LIB_PATH = PKG_DIR / "libcornserve_amd_torch.so"
 OBJ_DIR = CSRC / "build"
 
 ARCH = "gfx950"
@@ -106,6 +109,20 @@ def _check_no_missing_kernels(lib: Path) -> None:
         raise RuntimeError(f"{lib.name} has undefined symbols of its own (dropped kernels?):\n  " + "\n  ".join(own))
 
 
+def _build_torch_ops() -> None:
+    import torch
+
+    root = Path(torch.__file__).resolve().parent
+    gxx = shutil.which("g++")
+    if gxx is None:
+        raise RuntimeError("g++ not found; cannot build libcornserve_amd_torch.so")
+    system = [root / "include", root / "include/torch/csrc/api/include", "/opt/rocm/include", sysconfig.get_paths()["include"]]
+    _run([gxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+          f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}", f"-I{INCLUDE}",
+          *(arg for d in system for arg in ("-isystem", str(d))), str(CSRC / "torch_ops.cpp"), "-o", str(TORCH_LIB_PATH),
+          f"-L{PKG_DIR}", f"-l:{LIB_PATH.name}", f"-L{root / 'lib'}", "-ltorch_cpu", "-lc10", "-lc10_hip", "-Wl,-rpath,$ORIGIN"])
+
+
 def build_library(force: bool = True, jobs: int = 8) -> Path:
     """Compile every .hip source under csrc/ and link the shared library. Returns its path."""
     hipcc = _hipcc()
@@ -127,6 +144,7 @@ def build_library(force: bool = True, jobs: int = 8) -> Path:
         list(pool.map(lambda job: job(), todo))
     _run([hipcc, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", str(LIB_PATH), *map(str, objs)])
     _check_no_missing_kernels(LIB_PATH)
+    _build_torch_ops()
     return LIB_PATH
 
 

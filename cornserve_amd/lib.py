@@ -11,6 +11,7 @@ from ctypes import POINTER, c_float, c_int32, c_int64, c_void_p
 from pathlib import Path
 
 LIB_PATH = Path(__file__).resolve().parent / "libcornserve_amd.so"
+TORCH_LIB_PATH = LIB_PATH.with_name("libcornserve_amd_torch.so")   # operators implemented natively, linked to the former
 
 CS_OK = 0
 CS_ERR_INVALID_ARG = 1
@@ -147,6 +148,16 @@ def load() -> ctypes.CDLL:
         raise KernelLibraryError(f"ABI version mismatch: library {got}, binding {ABI_VERSION}; rebuild")
     _lib = lib
     return lib
+
+
+def load_operators() -> None:
+    """Load the native implementations of the operators (csrc/torch_ops.cpp), whose schemas cornserve_amd.ops defines.
+    They may be missing while nothing is built yet; an operator without its implementation raises when it is called."""
+    if LIB_PATH.exists() and TORCH_LIB_PATH.exists():
+        load()
+        import torch
+
+        torch.ops.load_library(str(TORCH_LIB_PATH))
 
 
 def check(status: int, what: str) -> None:

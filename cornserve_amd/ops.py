@@ -3,7 +3,8 @@
 Every kernel entry point of libcornserve_amd.so is registered as an operator of the `cornserve_amd` namespace
 (`torch.ops.cornserve_amd.gemm_`, `.attn_varlen_`, `.rmsnorm_`, ...: schema, a fake implementation for shape
 propagation, and one implementation that validates its arguments and enqueues the HIP kernels on torch's current
-stream through ctypes).  The functions of this module are the keyword-argument front ends the encoders call: they
+stream: in csrc/torch_ops.cpp for the operators of an encoder's blocks, here through ctypes for those that a pass
+issues once).  The functions of this module are the keyword-argument front ends the encoders call: they
 allocate outputs with torch's caching allocator (so outputs stay IPC-exportable for the sidecar, reference:
 sidecar/api.py:198-242) and dispatch through `torch.ops`, so the launches are visible to the dispatcher, the
 profiler's operator records and tracing.  The operators that write into caller-provided tensors end in `_` and
@@ -159,9 +160,8 @@ def gemm(
     if out is None:  # (with c_rows: a permutation of the M rows; anything else needs the caller's `out`)
         out = torch.empty((_gemm_rows(a, a_rows, conv_patch), w.shape[0] // 2 if epilogue == EPI_SWIGLU else w.shape[0]),
                           dtype=torch.bfloat16, device=a.device)
-    torch.ops.cornserve_amd.gemm_(out, a, w, bias, epilogue, residual, w_scale, pos, a_rows, c_rows, k, a_row_sumsq,
-                                  c_row_sumsq, norm_eps, a_row_sum, c_row_sum, w_col_sum, residual_lo, out_lo, conv_patch,
-                                  prefetch, norm_inline)
+    _gemm_op(out, a, w, bias, epilogue, residual, w_scale, pos, a_rows, c_rows, k, a_row_sumsq, c_row_sumsq, norm_eps,
+             a_row_sum, c_row_sum, w_col_sum, residual_lo, out_lo, conv_patch, prefetch, norm_inline)
     return out
 
 
@@ -176,14 +176,6 @@ def window_attn_norm_inline_pays(windows: int, heads: int, k: int) -> bool:
     return bool(_l.load().cs_gemm_norm_inline_pays(windows * QKV_WATTN_WINDOW, heads * QKV_WATTN_TILE_ROWS, k, 1))
 
 
-def _set_prefetch(args, prefetch: torch.Tensor | None, device: torch.device) -> None:
-    if prefetch is None:
-        return
-    if not prefetch.is_cuda or prefetch.device != device or not prefetch.is_contiguous() or prefetch.data_ptr() % 16:
-        raise ValueError("prefetch must be a contiguous, 16-byte aligned tensor on the operands' device")
-    args.prefetch, args.prefetch_bytes = prefetch.data_ptr(), prefetch.numel() * prefetch.element_size()
-
-
 def _gemm_rows(a, a_rows, conv_patch) -> int:
     """Output rows of a product: A's rows, the gathered rows, or the patches of NCHW pixels."""
     if conv_patch:
@@ -193,137 +185,6 @@ def _gemm_rows(a, a_rows, conv_patch) -> int:
     if a.dim() != 2:
         raise ValueError("gemm operands must be 2-D")
     return a.shape[0] if a_rows is None else a_rows.shape[0]
-
-
-def _gemm_functional(a, w, bias, epilogue, residual, w_scale, pos, a_rows, c_rows, k, a_row_sumsq, norm_eps, a_row_sum,
-                     w_col_sum, conv_patch=0):
-    if w.dim() != 2:
-        raise ValueError("gemm operands must be 2-D")
-    M = _gemm_rows(a, a_rows, conv_patch)
-    out = torch.empty((M, w.shape[0] // 2 if epilogue == EPI_SWIGLU else w.shape[0]), dtype=torch.bfloat16, device=a.device)
-    _gemm_impl(out, a, w, bias, epilogue, residual, w_scale, pos, a_rows, c_rows, k, a_row_sumsq, None, norm_eps,
-               a_row_sum, None, w_col_sum, None, None, conv_patch)
-    return out
-
-
-def _gemm_impl(out, a, w, bias, epilogue, residual, w_scale, pos, a_rows, c_rows, k, a_row_sumsq, c_row_sumsq, norm_eps,
-               a_row_sum, c_row_sum, w_col_sum, residual_lo, out_lo, conv_patch=0, prefetch=None,
-               norm_inline=False) -> None:
-    """Implementation of cornserve_amd::gemm_: argument checks, then cs_gemm on the current stream."""
-    lib = _l.load()
-    _req(a, torch.bfloat16, "a")
-    if w.dim() != 2:
-        raise ValueError("gemm operands must be 2-D")
-    conv = None
-    if conv_patch:
-        if a.dim() != 4 or not a.is_contiguous() or conv_patch < 2 or conv_patch % 2 or a.shape[3] % 2:
-            raise ValueError("with conv_patch, `a` must be contiguous NCHW pixels with an even width and patch size")
-        if a_rows is not None or k is not None or epilogue != EPI_BIAS:
-            raise ValueError("the strided-gather product takes no a_rows / k and only the bias epilogue")
-        conv = (a.shape[1], a.shape[2], a.shape[3], conv_patch)
-        kreal = a.shape[1] * conv_patch * conv_patch
-        if w.shape[1] != (kreal + 7) // 8 * 8:
-            raise ValueError(f"w must have {(kreal + 7) // 8 * 8} columns (C*patch*patch = {kreal} rounded up to a multiple of 8)")
-        a2d_rows, a2d_cols = _gemm_rows(a, None, conv_patch), w.shape[1]
-    elif a.dim() != 2:
-        raise ValueError("gemm operands must be 2-D")
-    else:
-        a2d_rows, a2d_cols = a.shape
-    fp8 = w.dtype in (torch.float8_e4m3fn, torch.uint8)
-    if not fp8:
-        _req(w, torch.bfloat16, "w")
-    elif w_scale is None:
-        raise ValueError("fp8 weights need w_scale")
-    for name, t in (("a_rows", a_rows), ("c_rows", c_rows)):
-        if t is not None:
-            _req(t, torch.int32, name)
-            if t.dim() != 1 or not t.is_contiguous():
-                raise ValueError(f"{name} must be a contiguous int32 vector")
-    M = a2d_rows if a_rows is None else a_rows.shape[0]
-    K = a2d_cols if k is None else k
-    N = w.shape[0]
-    if K > a2d_cols or K < 1:
-        raise ValueError(f"k={K} exceeds the {a2d_cols} columns of a")
-    if w.shape[1] < K:
-        raise ValueError(f"w has {w.shape[1]} columns, need at least K={K}")
-    if c_rows is not None and c_rows.shape[0] < M:
-        raise ValueError(f"c_rows has {c_rows.shape[0]} entries for {M} output rows")
-    n_out = N // 2 if epilogue == EPI_SWIGLU else N
-    # Everything below reaches the kernel as a raw pointer: shapes, dtypes and devices are checked here, before
-    # anything is enqueued, because an undersized or mistyped buffer would be an out-of-bounds device access.
-    _req(out, torch.bfloat16, "out")
-    if out.dim() != 2 or out.shape[1] < n_out or (c_rows is None and out.shape[0] < M):
-        raise ValueError(f"out must be bf16 [>={M}, >={n_out}], got {tuple(out.shape)}")
-    if bias is not None:
-        _req(bias, torch.bfloat16, "bias")
-        if bias.dim() != 1 or bias.shape[0] < N:
-            raise ValueError(f"bias must be bf16 [{N}], got {tuple(bias.shape)}")
-    if epilogue == EPI_RESIDUAL and residual is None:
-        raise ValueError("EPI_RESIDUAL needs `residual`")
-    if residual is not None:
-        _req(residual, torch.bfloat16, "residual")
-        if residual.dim() != 2 or residual.shape[0] < M or residual.shape[1] < N:
-            raise ValueError(f"residual must be bf16 [>={M}, >={N}], got {tuple(residual.shape)}")
-    if pos is not None:
-        _req(pos, torch.bfloat16, "pos")
-        if pos.dim() != 2 or pos.shape[0] < 1 or pos.shape[1] < N:
-            raise ValueError(f"pos must be bf16 [period, >={N}], got {tuple(pos.shape)}")
-    if w_scale is not None:
-        _req(w_scale, torch.float32, "w_scale")
-        if w_scale.dim() != 1 or w_scale.shape[0] < N or not w_scale.is_contiguous():
-            raise ValueError(f"w_scale must be a contiguous fp32 [{N}] tensor")
-    if residual_lo is not None or out_lo is not None:
-        if epilogue != EPI_RESIDUAL or out_lo is None:
-            raise ValueError("residual_lo / out_lo belong to EPI_RESIDUAL, and residual_lo needs out_lo")
-        _req(out_lo, torch.uint8, "out_lo")
-        if out_lo.shape != out.shape or out_lo.stride() != out.stride():
-            raise ValueError("out_lo must have the shape and strides of out")
-        if residual_lo is not None:
-            _req(residual_lo, torch.uint8, "residual_lo")
-            if residual_lo.shape != residual.shape or residual_lo.stride() != residual.stride():
-                raise ValueError("residual_lo must have the shape and strides of residual")
-    on = {t.device for t in (a, w, out, bias, residual, pos, w_scale, a_rows, c_rows, residual_lo, out_lo) if t is not None}
-    if len(on) != 1:
-        raise ValueError(f"gemm operands live on different devices: {sorted(map(str, on))}")
-    args = _l.CsGemmArgs()
-    args.A, args.lda = a.data_ptr(), (0 if conv else a.stride(0))
-    if conv:
-        args.conv_c, args.conv_h, args.conv_w, args.conv_patch = conv
-    args.W, args.ldw = w.data_ptr(), w.stride(0)
-    args.w_scale = _ptr(w_scale)
-    args.bias = _ptr(bias)
-    args.residual = _ptr(residual)
-    args.ldr = residual.stride(0) if residual is not None else 0
-    args.pos = _ptr(pos)
-    args.ldpos = pos.stride(0) if pos is not None else 0
-    args.pos_period = pos.shape[0] if pos is not None else 0
-    args.C, args.ldc = out.data_ptr(), out.stride(0)
-    args.a_rows = _ptr(a_rows)
-    args.c_rows = _ptr(c_rows)
-    args.M, args.N, args.K = M, N, K
-    args.epilogue = epilogue
-    args.w_fp8 = 1 if fp8 else 0
-    for name, t in (("a_row_sumsq", a_row_sumsq), ("c_row_sumsq", c_row_sumsq), ("a_row_sum", a_row_sum),
-                    ("c_row_sum", c_row_sum)):
-        if t is not None:
-            _req(t, torch.float32, name)
-            if t.dim() != 2 or t.shape[1] != SUMSQ_PARTS or not t.is_contiguous() or t.shape[0] < M:
-                raise ValueError(f"{name} must be a contiguous fp32 [>=M, {SUMSQ_PARTS}] tensor")
-    args.a_row_sumsq = _ptr(a_row_sumsq)
-    args.c_row_sumsq = _ptr(c_row_sumsq)
-    args.norm_eps = norm_eps
-    if w_col_sum is not None:
-        _req(w_col_sum, torch.float32, "w_col_sum")
-        if tuple(w_col_sum.shape) != (N,) or not w_col_sum.is_contiguous():
-            raise ValueError(f"w_col_sum must be a contiguous fp32 [{N}] tensor")
-    args.a_row_sum = _ptr(a_row_sum)
-    args.c_row_sum = _ptr(c_row_sum)
-    args.w_col_sum = _ptr(w_col_sum)
-    args.residual_lo = _ptr(residual_lo)
-    args.c_lo = _ptr(out_lo)
-    args.a_norm_inline = int(norm_inline)
-    _set_prefetch(args, prefetch, a.device)
-    _l.check(lib.cs_gemm(ctypes.byref(args), _stream()), "cs_gemm")
 
 
 # -------------------------------------------------------------------------------------------- norms
@@ -365,33 +226,6 @@ def row_sumsq(x: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:
         out = torch.empty((x.shape[0], SUMSQ_PARTS), dtype=torch.float32, device=x.device)
     torch.ops.cornserve_amd.row_stats_(out, None, x)
     return out
-
-
-def _norm_args(out, x, w, b) -> None:
-    _rows_2d(x, torch.bfloat16, "x")
-    _rows_2d(out, torch.bfloat16, "out")
-    H = x.shape[1]
-    if out.shape[0] < x.shape[0] or out.shape[1] < H or out.device != x.device:
-        raise ValueError(f"out must be bf16 [>={x.shape[0]}, >={H}] on x's device")
-    for name, t in (("w", w), ("b", b)):
-        if t is not None:
-            _req(t, torch.bfloat16, name)
-            if t.dim() != 1 or t.shape[0] < H or t.device != x.device:
-                raise ValueError(f"{name} must be bf16 [{H}] on x's device")
-
-
-def _rmsnorm_impl(out, x, w, eps, gemma) -> None:
-    lib = _l.load()
-    _norm_args(out, x, w, None)
-    _l.check(lib.cs_rmsnorm(x.data_ptr(), x.stride(0), w.data_ptr(), out.data_ptr(), out.stride(0), x.shape[0],
-                            x.shape[1], eps, int(gemma), _stream()), "cs_rmsnorm")
-
-
-def _layernorm_impl(out, x, w, b, eps) -> None:
-    lib = _l.load()
-    _norm_args(out, x, w, b)
-    _l.check(lib.cs_layernorm(x.data_ptr(), x.stride(0), w.data_ptr(), b.data_ptr(), out.data_ptr(), out.stride(0),
-                              x.shape[0], x.shape[1], eps, _stream()), "cs_layernorm")
 
 
 def rmsnorm(x: torch.Tensor, w: torch.Tensor, eps: float, *, gemma: bool = False,
@@ -632,20 +466,6 @@ def rope_qk_(qkv: torch.Tensor, cos_sin: torch.Tensor, heads: int, head_dim: int
     return qkv
 
 
-def _rope_qk_impl(qkv, cos_sin, heads, head_dim) -> None:
-    lib = _l.load()
-    _rows_2d(qkv, torch.bfloat16, "qkv")
-    _req(cos_sin, torch.float32, "cos_sin")
-    if cos_sin.shape != (qkv.shape[0], head_dim) or not cos_sin.is_contiguous() or cos_sin.device != qkv.device:
-        raise ValueError("cos_sin must be contiguous [L, head_dim] on qkv's device")
-    if heads < 1 or qkv.shape[1] < 2 * heads * head_dim:
-        raise ValueError(f"qkv rows hold {qkv.shape[1]} values, fewer than the q and k blocks of {heads} heads")
-    _l.check(
-        lib.cs_rope_qk(qkv.data_ptr(), qkv.stride(0), cos_sin.data_ptr(), qkv.shape[0], heads, head_dim, _stream()),
-        "cs_rope_qk",
-    )
-
-
 # --------------------------------------------------------------------------------------- attention
 @dataclass
 class AttnPlan:
@@ -686,35 +506,8 @@ def attn_varlen(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, plan: AttnPla
     `keys_rotated`: k already carries the rotary of `cos_sin`; only q is rotated (long segments only)."""
     if out is None:
         out = torch.empty((q.shape[0], heads * head_dim), dtype=torch.bfloat16, device=q.device)
-    torch.ops.cornserve_amd.attn_varlen_(out, q, k, v, plan.work, plan.n_work, plan.max_seqlen, heads, head_dim, scale,
-                                         cos_sin, keys_rotated)
+    _attn_varlen_op(out, q, k, v, plan.work, plan.n_work, plan.max_seqlen, heads, head_dim, scale, cos_sin, keys_rotated)
     return out
-
-
-def _attn_varlen_impl(out, q, k, v, work, n_work, max_seqlen, heads, head_dim, scale, cos_sin, keys_rotated) -> None:
-    lib = _l.load()
-    for name, t in (("q", q), ("k", k), ("v", v), ("out", out)):
-        _rows_2d(t, torch.bfloat16, name)
-        if t.shape[1] < heads * head_dim or t.device != q.device:
-            raise ValueError(f"{name} must hold {heads} heads of {head_dim} values per row on q's device")
-    if not (q.stride(0) == k.stride(0) == v.stride(0)):
-        raise ValueError("q, k, v must share a row stride")
-    L = q.shape[0]
-    if k.shape[0] != L or v.shape[0] != L or out.shape[0] < L:
-        raise ValueError("q, k, v and out must have one row per token")
-    _req(work, torch.int32, "work")
-    if work.dim() != 2 or work.shape[1] != 4 or not work.is_contiguous() or work.shape[0] < n_work or work.device != q.device:
-        raise ValueError("work must be a contiguous int32 [>=n_work, 4] tensor on q's device")
-    if cos_sin is not None:
-        _req(cos_sin, torch.float32, "cos_sin")
-        if cos_sin.shape != (L, head_dim) or not cos_sin.is_contiguous() or cos_sin.device != q.device:
-            raise ValueError("cos_sin must be contiguous [L, head_dim] on q's device")
-    entry = lib.cs_attn_varlen_keys_rotated if keys_rotated else lib.cs_attn_varlen
-    _l.check(
-        entry(q.data_ptr(), k.data_ptr(), v.data_ptr(), q.stride(0), out.data_ptr(), out.stride(0),
-              work.data_ptr(), n_work, heads, head_dim, scale, _ptr(cos_sin), max_seqlen, _stream()),
-        "cs_attn_varlen_keys_rotated" if keys_rotated else "cs_attn_varlen",
-    )
 
 
 def attn_varlen_rotary_(qkv: torch.Tensor, plan: AttnPlan, heads: int, head_dim: int, scale: float,
@@ -951,67 +744,9 @@ def qkv_window_attn(x: torch.Tensor, w_packed: torch.Tensor, b_packed: torch.Ten
     Raises ValueError for shapes the kernel does not take."""
     if out is None:
         out = torch.empty((x.shape[0], heads * QKV_WATTN_HEAD_DIM), dtype=torch.bfloat16, device=x.device)
-    torch.ops.cornserve_amd.qkv_window_attn_(out, x, w_packed, b_packed, cos_sin, heads, scale, a_row_sumsq, norm_eps,
-                                              win_start, w_scale, prefetch, norm_inline)
+    _qkv_window_attn_op(out, x, w_packed, b_packed, cos_sin, heads, scale, a_row_sumsq, norm_eps, win_start, w_scale, prefetch,
+                        norm_inline)
     return out
-
-
-def _qkv_window_attn_impl(out, x, w_packed, b_packed, cos_sin, heads, scale, a_row_sumsq, norm_eps, win_start=None,
-                          w_scale=None, prefetch=None, norm_inline=False) -> None:
-    lib = _l.load()
-    _rows_2d(x, torch.bfloat16, "x")
-    fp8 = w_scale is not None
-    _rows_2d(w_packed, torch.uint8 if fp8 else torch.bfloat16, "w_packed")
-    if fp8:
-        _req(w_scale, torch.float32, "w_scale")
-        if tuple(w_scale.shape) != (heads * QKV_WATTN_TILE_ROWS,) or not w_scale.is_contiguous():
-            raise ValueError(f"w_scale must be a contiguous fp32 [{heads * QKV_WATTN_TILE_ROWS}] tensor")
-        if a_row_sumsq is not None:
-            raise ValueError("the folded norm (a_row_sumsq) does not exist for fp8 weights")
-    _rows_2d(out, torch.bfloat16, "out")
-    _req(b_packed, torch.bfloat16, "b_packed")
-    _req(cos_sin, torch.float32, "cos_sin")
-    M, K = x.shape
-    d = QKV_WATTN_HEAD_DIM
-    if heads < 1 or tuple(w_packed.shape) != (heads * QKV_WATTN_TILE_ROWS, K):
-        raise ValueError(f"w_packed must be [{heads}*{QKV_WATTN_TILE_ROWS}, {K}], got {tuple(w_packed.shape)}")
-    if tuple(b_packed.shape) != (heads * QKV_WATTN_TILE_ROWS,) or not b_packed.is_contiguous():
-        raise ValueError(f"b_packed must be a contiguous [{heads * QKV_WATTN_TILE_ROWS}] tensor")
-    if win_start is None:
-        if M % QKV_WATTN_WINDOW:
-            raise ValueError(f"the rows of x ({M}) must be a whole number of {QKV_WATTN_WINDOW}-row windows")
-    else:
-        _req(win_start, torch.int32, "win_start")
-        n_win = win_start.numel() - 1
-        if win_start.dim() != 1 or not win_start.is_contiguous() or n_win < 1 or not 4 * n_win <= M <= QKV_WATTN_WINDOW * n_win or M % 4:
-            raise ValueError(f"win_start must be a contiguous int32 [windows + 1] tensor whose windows of 4 .. "
-                             f"{QKV_WATTN_WINDOW} rows add up to the {M} rows of x")
-    if tuple(cos_sin.shape) != (M, d) or not cos_sin.is_contiguous():
-        raise ValueError(f"cos_sin must be a contiguous fp32 [{M}, {d}] table")
-    if out.shape[0] < M or out.shape[1] < heads * d:
-        raise ValueError(f"out must be bf16 [>={M}, >={heads * d}], got {tuple(out.shape)}")
-    if a_row_sumsq is not None:
-        _req(a_row_sumsq, torch.float32, "a_row_sumsq")
-        if a_row_sumsq.dim() != 2 or a_row_sumsq.shape[1] != SUMSQ_PARTS or not a_row_sumsq.is_contiguous() or a_row_sumsq.shape[0] < M:
-            raise ValueError(f"a_row_sumsq must be a contiguous fp32 [>=M, {SUMSQ_PARTS}] tensor")
-    on = {t.device for t in (out, x, w_packed, b_packed, cos_sin, a_row_sumsq, win_start, w_scale) if t is not None}
-    if len(on) != 1:
-        raise ValueError(f"qkv_window_attn operands live on different devices: {sorted(map(str, on))}")
-    args = _l.CsGemmArgs()
-    args.A, args.lda = x.data_ptr(), x.stride(0)
-    args.W, args.ldw = w_packed.data_ptr(), w_packed.stride(0)
-    args.bias = b_packed.data_ptr()
-    args.C, args.ldc = out.data_ptr(), out.stride(0)
-    args.M, args.N, args.K = M, heads * QKV_WATTN_TILE_ROWS, K
-    args.a_row_sumsq = _ptr(a_row_sumsq)
-    args.norm_eps = norm_eps
-    args.a_norm_inline = int(norm_inline)
-    if win_start is not None:
-        args.attn_win_start, args.attn_n_win = win_start.data_ptr(), win_start.numel() - 1
-    if fp8:
-        args.w_fp8, args.w_scale = 1, w_scale.data_ptr()
-    _set_prefetch(args, prefetch, x.device)
-    _l.check(lib.cs_qkv_window_attn(ctypes.byref(args), cos_sin.data_ptr(), scale, heads, d, _stream()), "cs_qkv_window_attn")
 
 
 # ------------------------------------------------------------------------------- operator registration
@@ -1020,17 +755,17 @@ def _qkv_window_attn_impl(out, x, w_packed, b_packed, cos_sin, heads, scale, a_r
 # schema, so the dispatcher sees it.  The implementation is registered for every backend key: it validates devices and
 # dtypes itself and raises ValueError, the reference model API's error for bad input.
 _LIBRARY = torch.library.Library("cornserve_amd", "DEF")
-_OPERATORS: dict[str, tuple[str, object]] = {
+_OPERATORS: dict[str, tuple[str, object]] = {   # schema, and the implementation (None: csrc/torch_ops.cpp)
     "gemm": ("(Tensor a, Tensor w, Tensor? bias, int epilogue, Tensor? residual, Tensor? w_scale, Tensor? pos, "
              "Tensor? a_rows, Tensor? c_rows, int? k, Tensor? a_row_sumsq, float norm_eps, Tensor? a_row_sum, "
-             "Tensor? w_col_sum, int conv_patch=0) -> Tensor", _gemm_functional),
+             "Tensor? w_col_sum, int conv_patch=0) -> Tensor", None),
     "gemm_": ("(Tensor(a!) out, Tensor a, Tensor w, Tensor? bias, int epilogue, Tensor? residual, Tensor? w_scale, "
               "Tensor? pos, Tensor? a_rows, Tensor? c_rows, int? k, Tensor? a_row_sumsq, Tensor(b!)? c_row_sumsq, "
               "float norm_eps, Tensor? a_row_sum, Tensor(c!)? c_row_sum, Tensor? w_col_sum, Tensor? residual_lo, "
-              "Tensor(d!)? out_lo, int conv_patch=0, Tensor? prefetch=None, bool norm_inline=False) -> ()", _gemm_impl),
+              "Tensor(d!)? out_lo, int conv_patch=0, Tensor? prefetch=None, bool norm_inline=False) -> ()", None),
     "row_stats_": ("(Tensor(a!) sumsq_out, Tensor(b!)? sum_out, Tensor x) -> ()", _row_stats_impl),
-    "rmsnorm_": ("(Tensor(a!) out, Tensor x, Tensor w, float eps, bool gemma) -> ()", _rmsnorm_impl),
-    "layernorm_": ("(Tensor(a!) out, Tensor x, Tensor w, Tensor b, float eps) -> ()", _layernorm_impl),
+    "rmsnorm_": ("(Tensor(a!) out, Tensor x, Tensor w, float eps, bool gemma) -> ()", None),
+    "layernorm_": ("(Tensor(a!) out, Tensor x, Tensor w, Tensor b, float eps) -> ()", None),
     "avgpool_gemma_rmsnorm_": ("(Tensor(a!) out, Tensor x, Tensor w, int side, int k, float eps) -> ()",
                                _avgpool_gemma_rmsnorm_impl),
     "cast_f32_bf16_": ("(Tensor(a!) out, Tensor x) -> ()", _cast_impl),
@@ -1041,9 +776,9 @@ _OPERATORS: dict[str, tuple[str, object]] = {
                           _pos_embed_interp_impl),
     "rows_bilinear_": ("(Tensor(a!) out, Tensor src, Tensor taps, Tensor frac) -> ()", _rows_bilinear_impl),
     "row_gather_": ("(Tensor(a!) out, Tensor x, Tensor rows) -> ()", _row_gather_impl),
-    "rope_qk_": ("(Tensor(a!) qkv, Tensor cos_sin, int heads, int head_dim) -> ()", _rope_qk_impl),
+    "rope_qk_": ("(Tensor(a!) qkv, Tensor cos_sin, int heads, int head_dim) -> ()", None),
     "attn_varlen_": ("(Tensor(a!) out, Tensor q, Tensor k, Tensor v, Tensor work, int n_work, int max_seqlen, int heads, "
-                     "int head_dim, float scale, Tensor? cos_sin, bool keys_rotated) -> ()", _attn_varlen_impl),
+                     "int head_dim, float scale, Tensor? cos_sin, bool keys_rotated) -> ()", None),
     "qwen_patchify_u8_": ("(Tensor(a!) out, Tensor frames, Tensor table, int patch, int merge, int temporal) -> ()",
                           _qwen_patchify_u8_impl),
     "resize_u8_pass_": ("(Tensor(a!) out, Tensor src, Tensor bounds, Tensor taps, int axis) -> ()", _resize_u8_pass_impl),
@@ -1051,7 +786,7 @@ _OPERATORS: dict[str, tuple[str, object]] = {
     "qkv_window_attn_": ("(Tensor(a!) out, Tensor x, Tensor w_packed, Tensor b_packed, Tensor cos_sin, int heads, "
                          "float scale, Tensor? a_row_sumsq, float norm_eps, Tensor? win_start=None, Tensor? w_scale=None, "
                          "Tensor? prefetch=None, bool norm_inline=False) -> ()",
-                         _qkv_window_attn_impl),
+                         None),
 }
 
 
@@ -1067,5 +802,11 @@ def _fake_nothing(*args, **kwargs) -> None:   # the in-place operators return no
 
 for _name, (_schema, _impl) in _OPERATORS.items():
     _LIBRARY.define(_name + _schema)
-    _LIBRARY.impl(_name, _impl, "CompositeExplicitAutograd")
+    if _impl is not None:
+        _LIBRARY.impl(_name, _impl, "CompositeExplicitAutograd")
     torch.library.register_fake(f"cornserve_amd::{_name}", _fake_gemm if _name == "gemm" else _fake_nothing, lib=_LIBRARY)
+_l.load_operators()
+
+_gemm_op = torch.ops.cornserve_amd.gemm_.default     # (the overloads themselves: a packet looks its overload up per call)
+_qkv_window_attn_op = torch.ops.cornserve_amd.qkv_window_attn_.default
+_attn_varlen_op = torch.ops.cornserve_amd.attn_varlen_.default

@@ -155,3 +155,22 @@ def test_resize_taps_host_matches_the_oracle_bit_for_bit():
     b = np.zeros((5, 2), dtype=np.int32)
     assert dll.cs_resize_bicubic_taps_host(10, 5, b.ctypes.data, small.ctypes.data, 4, ctypes.byref(k)) == lib.CS_ERR_INVALID_ARG
     assert dll.cs_resize_u8_pass(None, 1, 4, 4, 3, None, None, 5, None, None) == lib.CS_ERR_INVALID_ARG
+
+
+def test_native_operators_refuse_what_their_kernels_cannot_take():
+    """The natively implemented operators raise the exception categories of the model API (ValueError for bad input)."""
+    import torch
+
+    a = torch.zeros((4, 8), dtype=torch.bfloat16)
+    f = a.float()
+    work = torch.zeros((1, 4), dtype=torch.int32)
+    plan = ops.AttnPlan(work, 1, 4)
+    for call in (lambda: ops.gemm(a, a), lambda: ops.gemm(a, a, out=a), lambda: ops.gemm(a[0], a), lambda: ops.gemm(a, a[0]),
+                 lambda: ops.gemm(a, a, conv_patch=2), lambda: ops.rmsnorm(a, a[0], 1e-6), lambda: ops.layernorm(a, a[0], a[0], 1e-6),
+                 lambda: ops.rope_qk_(a, f, 1, 4), lambda: ops.attn_varlen(a, a, a, plan, 1, 8, 1.0),
+                 lambda: ops.qkv_window_attn(a, a, a[0], f, 1, 1.0)):
+        with pytest.raises(ValueError, match="device tensor|2-D|NCHW"):
+            call()
+    # every operator has an implementation, here or in the native library
+    for name in ops._OPERATORS:
+        assert torch._C._dispatch_has_kernel_for_dispatch_key(f"cornserve_amd::{name}", "CompositeExplicitAutograd"), name
