@@ -36,21 +36,8 @@ constexpr int WAVES_N = 4;
 
 // 16 fp8-e4m3 (OCP) values -> 16 bf16.  Conversion is exact: every e4m3 value is representable in bf16.
 CS_DEVICE void fp8x16_to_bf16(const i32x4_t& in, bf16x8_t& lo, bf16x8_t& hi) {
-  float f[16];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    auto p0 = __builtin_amdgcn_cvt_pk_f32_fp8(in[i], false);
-    auto p1 = __builtin_amdgcn_cvt_pk_f32_fp8(in[i], true);
-    f[4 * i + 0] = p0[0];
-    f[4 * i + 1] = p0[1];
-    f[4 * i + 2] = p1[0];
-    f[4 * i + 3] = p1[1];
-  }
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    lo[i] = (bf16_t)f[i];
-    hi[i] = (bf16_t)f[8 + i];
-  }
+  lo = fp8x8_to_bf16(i32x2_t{in[0], in[1]});
+  hi = fp8x8_to_bf16(i32x2_t{in[2], in[3]});
 }
 
 // CONV: the activation operand is gathered from NCHW pixels (a convolution with stride = kernel; see CsGemmArgs.conv_patch):

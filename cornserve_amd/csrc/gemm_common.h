@@ -14,6 +14,22 @@ constexpr int BK = 64;  // K step (bf16 elements): 128 bytes per tile row = 8 ch
 CS_DEVICE int swz_key(int row) { return (row ^ (row >> 3)) & 7; }
 CS_DEVICE int swz(int row, int chunk) { return row * 128 + ((chunk ^ swz_key(row)) << 4); }
 
+// 8 e4m3 bytes -> 8 bf16 (exact: every e4m3 value is a bf16 value).  One instruction a pair; by way of fp32 it takes two,
+// and in the tile forms whose waves have few rows the conversion of a weight fragment outlasts the MFMAs that use it.
+CS_DEVICE bf16x8_t fp8x8_to_bf16(i32x2_t raw) {
+  bf16x8_t o;
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const auto lo = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(raw[h], 1.0f, false);
+    const auto hi = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(raw[h], 1.0f, true);
+    o[4 * h + 0] = lo[0];
+    o[4 * h + 1] = lo[1];
+    o[4 * h + 2] = hi[0];
+    o[4 * h + 3] = hi[1];
+  }
+  return o;
+}
+
 CS_DEVICE float gelu_erf(float x) { return 0.5f * x * (1.0f + erff(x * 0.70710678118654752440f)); }
 // 0.5 x (1 + tanh(u)) == x * sigmoid(2u): one exponential and one hardware reciprocal instead of tanhf.
 CS_DEVICE float gelu_tanh(float x) {

@@ -53,7 +53,8 @@ int cs_gemm_fast(const CsGemmArgs& a, hipStream_t stream, bool* handled) {
   // gives 8 column tiles, so 1024 rows are 32 workgroups).  The 128x160 form has the same waves-by-columns layout,
   // so every output element and every row-sum part is computed by the same sequence of operations: results do not
   // depend on which of the two a batch size selects.
-  const bool few_rows = !a.w_fp8 && (int64_t)((a.M + 255) / 256) * ((a.N + 159) / 160) <= 128;
+  // (fp8 weights: for the residual products, which would fill half of the chip otherwise)
+  const bool few_rows = (!a.w_fp8 || a.epilogue == CS_EPI_RESIDUAL) && (int64_t)((a.M + 255) / 256) * ((a.N + 159) / 160) <= 128;
   auto narrow = [&]() { return few_rows ? cs_gemm_fast_tile_128x160(a, stream) : cs_gemm_fast_tile_256x160(a, stream); };
   // Row sums of squares come in CS_SUMSQ_PARTS parts, one per column tile of the 160-column forms.
   if (a.c_row_sumsq) {

@@ -137,7 +137,9 @@ template <int BM, int BN, bool W_FP8>
 struct RingShape {
   static constexpr int A_BYTES = BM * BK * 2, W_BYTES = BN * BK * (W_FP8 ? 1 : 2);
   static constexpr bool FIVE_UNITS = A_BYTES == W_BYTES && 5 * A_BYTES <= LDS_BYTES && 3 * (A_BYTES + W_BYTES) > LDS_BYTES;
-  static constexpr int BYTES = FIVE_UNITS ? 5 * A_BYTES : 3 * (A_BYTES + W_BYTES);
+  // (the 160-column forms keep the room of a bf16 stage with fp8 weights too: the residual piece passes through the slots)
+  static constexpr int STAGE = A_BYTES + (BN == 160 ? BN * BK * 2 : W_BYTES);
+  static constexpr int BYTES = FIVE_UNITS ? 5 * A_BYTES : 3 * STAGE;
   static_assert(BYTES <= LDS_BYTES, "tile does not fit a ring");
 };
 
@@ -154,11 +156,12 @@ struct RingShape {
 // folded into W, its bias into the GEMM bias, and w_col_sum[n] = sum_k W'[n,k] carries the mean term).
 constexpr int FUSE_NORM_A = 1, FUSE_SUMSQ_C = 2, FUSE_LN_A = 3, FUSE_STATS_C = 4;
 // The forms whose epilogue takes its residual piece through the LDS ring (see the kernel): residual epilogue on the split
-// stream, one wave spanning the tile's columns, bf16 weights.  They use 4 KB of LDS behind the ring.
+// stream, one wave spanning the tile's columns.  They use 4 KB of LDS behind the ring.  With fp8 weights as well:
+// 16128 rows x 1280 columns, mean of K = 1280 and 3456, 121.0 -> 110.5 us.
 template <int BM, int BN, int WAVES_M, int WAVES_N, int EPI, bool W_FP8, int FUSE, bool SPLIT_RES>
 constexpr bool residual_piece_through_ring() {
   constexpr int MT = BM / WAVES_M / 16, NT = BN / WAVES_N / 16;
-  return SPLIT_RES && EPI == CS_EPI_RESIDUAL && NT % 2 == 0 && !W_FP8 && !RingShape<BM, BN, W_FP8>::FIVE_UNITS && WAVES_N == 1 &&
+  return SPLIT_RES && EPI == CS_EPI_RESIDUAL && NT % 2 == 0 && !RingShape<BM, BN, W_FP8>::FIVE_UNITS && WAVES_N == 1 &&
          (MT == 2 || MT == 4) && FUSE != FUSE_NORM_A && FUSE != FUSE_LN_A;
 }
 template <int BM, int BN, int WAVES_M, int WAVES_N, int EPI, bool W_FP8, int FUSE, bool SPLIT_RES>
@@ -171,7 +174,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_fast_kernel(const CsGemmArgs p) 
   constexpr bool RING5 = Ring::FIVE_UNITS;
   // Byte offsets of operand tile slots.  Three-stage ring: slot s holds A at s*STAGE and W behind it.
   // Five-unit ring: every unit is one operand tile.
-  constexpr int STAGE = A_BYTES + W_BYTES;
+  constexpr int STAGE = Ring::STAGE;
   constexpr int WTM = BM / WAVES_M, WTN = BN / WAVES_N;
   static_assert(WTM % 16 == 0 && WTN % 16 == 0 && BM % 8 == 0 && BN % 8 == 0, "tile shape");
   constexpr int MT = WTM / 16, NT = WTN / 16;
@@ -298,6 +301,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_fast_kernel(const CsGemmArgs p) 
   const __amdgpu_buffer_rsrc_t rsrc_clo = __builtin_amdgcn_make_buffer_rsrc((void*)p.c_lo, 0, -1, 0x00020000);
   const __amdgpu_buffer_rsrc_t rsrc_res = __builtin_amdgcn_make_buffer_rsrc((void*)p.residual, 0, -1, 0x00020000);
   const __amdgpu_buffer_rsrc_t rsrc_reslo = __builtin_amdgcn_make_buffer_rsrc((void*)p.residual_lo, 0, -1, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rsrc_scale = __builtin_amdgcn_make_buffer_rsrc((void*)p.w_scale, 0, -1, 0x00020000);
   const __amdgpu_buffer_rsrc_t rsrc_bias = __builtin_amdgcn_make_buffer_rsrc((void*)p.bias, 0, -1, 0x00020000);
   const __amdgpu_buffer_rsrc_t rsrc_asumsq = __builtin_amdgcn_make_buffer_rsrc((void*)p.a_row_sumsq, 0, -1, 0x00020000);
   const __amdgpu_buffer_rsrc_t rsrc_asum = __builtin_amdgcn_make_buffer_rsrc((void*)p.a_row_sum, 0, -1, 0x00020000);
@@ -360,17 +364,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_fast_kernel(const CsGemmArgs p) 
   };
   auto convert_w = [&](int b, auto j_c) {  // 8 e4m3 bytes -> 8 bf16 (exact)
     constexpr int J = decltype(j_c)::value;
-    bf16x8_t o;
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const auto p0 = __builtin_amdgcn_cvt_pk_f32_fp8(wraw[b][W_FP8 ? J : 0][h], false);
-      const auto p1 = __builtin_amdgcn_cvt_pk_f32_fp8(wraw[b][W_FP8 ? J : 0][h], true);
-      o[4 * h + 0] = (bf16_t)p0[0];
-      o[4 * h + 1] = (bf16_t)p0[1];
-      o[4 * h + 2] = (bf16_t)p1[0];
-      o[4 * h + 3] = (bf16_t)p1[1];
-    }
-    wcv[J & 1] = o;
+    wcv[J & 1] = fp8x8_to_bf16(wraw[b][W_FP8 ? J : 0]);
   };
   // The MFMAs of one k-step on fragment set B, in program order (asm volatile statements keep it), with a
   // hook call after each: that is where LDS reads and direct loads are placed.  ZERO: the first k-step of an
@@ -386,21 +380,24 @@ __global__ __launch_bounds__(64 * NW) void gemm_fast_kernel(const CsGemmArgs p) 
       const bf16x8_t& w = W_FP8 ? wcv[J & 1] : wf[B][W_FP8 ? 0 : J];
       // A register written by a vector instruction must not be read by an MFMA in the next few cycles; the
       // compiler pads that for its own MFMAs but cannot see into these.  Only the first MFMA after a
-      // conversion can be that close.
-      if constexpr (W_FP8 && I == 0) asm volatile("s_nop 3");
+      // conversion can be that close; its wait is part of the statement, so that nothing is scheduled in between.
+#define CS_MFMA(OPERANDS, ADDEND)                                                                                                      \
+  do {                                                                                                                                 \
+    if constexpr (W_FP8 && I == 0)                                                                                                     \
+      asm volatile("s_nop 3\n\tv_mfma_f32_16x16x32_bf16 a[%2:%3], " OPERANDS ", " ADDEND ::"v"(w), "v"(xf[B][I]), "n"(R), "n"(R + 3)); \
+    else                                                                                                                               \
+      asm volatile("v_mfma_f32_16x16x32_bf16 a[%2:%3], " OPERANDS ", " ADDEND ::"v"(w), "v"(xf[B][I]), "n"(R), "n"(R + 3));            \
+  } while (0)
       if constexpr (WATTN && J >= 10) {
         // The V fragments are computed TRANSPOSED (activation rows as the first operand): a lane then owns one
         // head dim and four consecutive keys, the operand layout of the P.V product.  Fragment 15 is padding.
         if constexpr (J < 15) {
-          if constexpr (ZERO)
-            asm volatile("v_mfma_f32_16x16x32_bf16 a[%2:%3], %1, %0, 0" ::"v"(w), "v"(xf[B][I]), "n"(R), "n"(R + 3));
-          else
-            asm volatile("v_mfma_f32_16x16x32_bf16 a[%2:%3], %1, %0, a[%2:%3]" ::"v"(w), "v"(xf[B][I]), "n"(R), "n"(R + 3));
+          if constexpr (ZERO) CS_MFMA("%1, %0", "0");
+          else CS_MFMA("%1, %0", "a[%2:%3]");
         }
-      } else if constexpr (ZERO)
-        asm volatile("v_mfma_f32_16x16x32_bf16 a[%2:%3], %0, %1, 0" ::"v"(w), "v"(xf[B][I]), "n"(R), "n"(R + 3));
-      else
-        asm volatile("v_mfma_f32_16x16x32_bf16 a[%2:%3], %0, %1, a[%2:%3]" ::"v"(w), "v"(xf[B][I]), "n"(R), "n"(R + 3));
+      } else if constexpr (ZERO) CS_MFMA("%0, %1", "0");
+      else CS_MFMA("%0, %1", "a[%2:%3]");
+#undef CS_MFMA
       if constexpr (W_FP8 && I == 0 && J + 1 < NT) convert_w(B, ic<J + 1>{});
       hook(n);
     });
@@ -469,12 +466,15 @@ __global__ __launch_bounds__(64 * NW) void gemm_fast_kernel(const CsGemmArgs p) 
     constexpr int ROW_LD = NP + LO_LD;                  // direct loads per wave and row block
     constexpr int ROW_HI_BYTES = NW * NP * 1024, ROW_LO_BYTES = NW * LO_LD * 1024, ROW_BYTES = ROW_HI_BYTES + ROW_LO_BYTES;
     static_assert(!PRE || ((MT <= 2 ? ROW_BYTES : ROW_BYTES + ROW_HI_BYTES) <= STAGE && Ring::BYTES + NW * 1024 <= LDS_BYTES && BN * 2 <= 1024 &&
-                           2 * (ROW_LD + 1) <= NMFMA && MT <= 4),
+                           2 * (ROW_LD + 2) <= NMFMA && MT <= 4),
                   "two row blocks' bf16 planes and one byte plane fit a ring slot, the bias the room behind the ring");
+    // fp8 weights: the columns' scales, in row block 0's slot behind everything that passes through it
+    constexpr int SCALE_OFF = MT <= 2 ? ROW_BYTES : ROW_BYTES + ROW_LO_BYTES;
+    static_assert(!PRE || !W_FP8 || (SCALE_OFF + NW * 1024 <= STAGE && BN * 4 <= 1024), "the scales fit row block 0's slot");
     const bool fast_tile = p.fast_epilogue && m0 + BM <= p.M && n0 + BN <= p.N;
     const bool pre_on = PRE && fast_tile && !has_next;
     // lane-only byte offsets of the direct loads (the tile and the row block go into the scalar offset)
-    uint32_t pre_hi_v = 0, pre_lo_v[PRE ? LO_LD : 1] = {}, pre_bias_v = 0;
+    uint32_t pre_hi_v = 0, pre_lo_v[PRE ? LO_LD : 1] = {}, pre_bias_v = 0, pre_scale_v = 0;
     int pre_sbase = 0;   // element offset of the wave's first row and the tile's first column in the residual matrix
     if constexpr (PRE) {
       if (pre_on) {
@@ -487,10 +487,12 @@ __global__ __launch_bounds__(64 * NW) void gemm_fast_kernel(const CsGemmArgs p) 
           pre_lo_v[k] = r * (uint32_t)p.ldr + c * 16;
         }
         pre_bias_v = (uint32_t)min(lane_p, BN * 2 / 16 - 1) * 16;
+        if constexpr (W_FP8) pre_scale_v = (uint32_t)min(lane_p, BN * 4 / 16 - 1) * 16;
         pre_sbase = (m0 + wm * WTM) * (int)p.ldr + n0;
       }
     }
-    // Direct load IDX (bf16 plane of pair IDX, then the byte plane's chunks, then -- IDX == ROW_LD -- the bias) of row
+    // Direct load IDX (bf16 plane of pair IDX, then the byte plane's chunks, then -- IDX == ROW_LD -- the bias, then the
+    // scales) of row
     // block I; hi_base / lo_base are the LDS byte offsets of the row block's two regions.  A missing byte plane or
     // bias is replaced by loads of the same size from the bf16 plane (never read back): the waits count loads, so every
     // wave always issues the same number.  (Row block and piece go into the scalar offset: an immediate offset of a
@@ -508,13 +510,15 @@ __global__ __launch_bounds__(64 * NW) void gemm_fast_kernel(const CsGemmArgs p) 
         constexpr int Kk = IDX - NP;
         dma16(p.residual_lo ? rsrc_reslo : rsrc_res, smem + lo_base + (wave * LO_LD + Kk) * 1024, pre_lo_v[PRE ? Kk : 0],
               pre_sbase + I * 16 * (int)p.ldr);
+      } else if constexpr (IDX > ROW_LD) {
+        dma16(rsrc_scale, smem + hi_base + SCALE_OFF + wave * 1024, pre_scale_v, n0 * 4);
       } else {
         dma16(p.bias ? rsrc_bias : rsrc_res, smem + Ring::BYTES + wave * 1024, pre_bias_v, p.bias ? n0 * 2 : 0);
       }
     };
-    // loads of row block 0 (+ bias) issued in the second half of the third-last iteration; the rest follows in the
+    // loads of row block 0 (+ bias, scales) issued in the second half of the third-last iteration; the rest follows in the
     // first half of the second-last.  Row block 1 likewise, one half-iteration later.
-    constexpr int PRE_N0 = ROW_LD + 1, PRE_N0A = (PRE_N0 + 1) / 2, PRE_N1 = ROW_LD, PRE_N1A = (PRE_N1 + 1) / 2;
+    constexpr int PRE_N0 = ROW_LD + 1 + (W_FP8 ? 1 : 0), PRE_N0A = (PRE_N0 + 1) / 2, PRE_N1 = ROW_LD, PRE_N1A = (PRE_N1 + 1) / 2;
     // K tile 0 has landed once at most the loads issued after it are outstanding.  (Loads complete in
     // order; stores of the previous epilogue that are still in flight only make this wait longer.)
     __builtin_amdgcn_s_waitcnt(waitcnt_vm(PENDING_AT_TILE_START));
@@ -923,6 +927,12 @@ __global__ __launch_bounds__(64 * NW) void gemm_fast_kernel(const CsGemmArgs p) 
           }
         }
       }
+      f32x4_t scale_f[W_FP8 ? NT : 1];
+      if constexpr (W_FP8) {
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+          scale_f[W_FP8 ? j : 0] = *(const f32x4_t*)(smem + slot0 + SCALE_OFF + wave * 1024 + (kq * (4 * G) + piece_col(j)) * 4);
+      }
       static_for<MT>([&](auto i_c) {
         constexpr int i = decltype(i_c)::value;
         if constexpr (i > 0) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * NP + (i + 1 < MT ? ROW_LD : 0)) : "memory");
@@ -955,7 +965,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_fast_kernel(const CsGemmArgs p) 
               constexpr int Rr = decltype(r_c)::value;
               float t;
               asm volatile("v_accvgpr_read_b32 %0, a[%1]" : "=v"(t) : "n"((i * NT + J) * 4 + Rr));
-              v[Rr] = t + bias_f[J][Rr];
+              v[Rr] = W_FP8 ? __builtin_fmaf(t, scale_f[W_FP8 ? J : 0][Rr], bias_f[J][Rr]) : t + bias_f[J][Rr];
             });
             add_split24(v, u32x2_t{hi_in[2 * Hh], hi_in[2 * Hh + 1]}, lo_in[Hh], hi_o[Hh], lo_o[Hh]);
             if constexpr (FUSE == FUSE_SUMSQ_C || FUSE == FUSE_STATS_C) {
@@ -1333,7 +1343,7 @@ int launch(const CsGemmArgs& a, hipStream_t stream) {
   // The epilogue's fast form addresses C, the residual and their byte planes with 32-bit byte offsets from the
   // matrix bases, and takes output row m for accumulator row m.
   const int64_t lim = (int64_t)UINT32_MAX - 64;
-  p.fast_epilogue = !p.c_rows && (int64_t)p.M * p.ldc * 2 < lim && (!p.residual || (int64_t)p.M * p.ldr * 2 < lim);
+  p.fast_epilogue = !p.c_rows && !((uintptr_t)p.w_scale & 15) && (int64_t)p.M * p.ldc * 2 < lim && (!p.residual || (int64_t)p.M * p.ldr * 2 < lim);
   constexpr int lds = RingShape<BM, BN, W_FP8>::BYTES +
                       (residual_piece_through_ring<BM, BN, WAVES_M, WAVES_N, EPI, W_FP8, FUSE, SPLIT_RES>() ? NW * 1024 : 0);
   static bool attr_set = false;
@@ -1417,9 +1427,13 @@ int dispatch_epi_w(const CsGemmArgs& a, hipStream_t s) {
 template <int BM, int BN, int WAVES_M, int WAVES_N>
 int dispatch_epi(const CsGemmArgs& a, hipStream_t s) {
   if (a.w_fp8) {
-    // (the few-rows form is only dispatched for bf16 weights: its fp8 kernels are not built)
-    if constexpr (BM == 128 && BN == 160) return CS_ERR_UNSUPPORTED;
-    else return dispatch_epi_w<BM, BN, WAVES_M, WAVES_N, true>(a, s);
+    // (the few-rows form is dispatched to the residual products only: its other fp8 kernels are not built.  3996 rows x
+    // 1280 columns, mean of K = 1280 and 3456: 57.3 us in 128 tiles of 256x160, 36.2 us in 256 of 128x160)
+    if constexpr (BM == 128 && BN == 160) {
+      if (a.epilogue != CS_EPI_RESIDUAL || a.a_row_sumsq || a.c_row_sumsq || a.a_row_sum || a.c_row_sum) return CS_ERR_UNSUPPORTED;
+      return a.c_lo ? launch<BM, BN, WAVES_M, WAVES_N, CS_EPI_RESIDUAL, true, 0, true>(a, s)
+                    : launch<BM, BN, WAVES_M, WAVES_N, CS_EPI_RESIDUAL, true>(a, s);
+    } else return dispatch_epi_w<BM, BN, WAVES_M, WAVES_N, true>(a, s);
   }
   return dispatch_epi_w<BM, BN, WAVES_M, WAVES_N, false>(a, s);
 }

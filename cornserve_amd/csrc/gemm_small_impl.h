@@ -48,18 +48,6 @@ typedef __attribute__((__vector_size__(4 * sizeof(short)))) short sm_short4_t;
 CS_DEVICE f32x4_t sm_mfma16(bf16x4_t w, bf16x4_t x, f32x4_t c) {
   return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(sm_short4_t, w), __builtin_bit_cast(sm_short4_t, x), c, 0, 0, 0);
 }
-CS_DEVICE bf16x8_t sm_fp8x8_to_bf16(i32x2_t raw) {   // 8 e4m3 bytes -> 8 bf16 (exact)
-  bf16x8_t o;
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const auto p0 = __builtin_amdgcn_cvt_pk_f32_fp8(raw[h], false), p1 = __builtin_amdgcn_cvt_pk_f32_fp8(raw[h], true);
-    o[4 * h + 0] = (bf16_t)p0[0];
-    o[4 * h + 1] = (bf16_t)p0[1];
-    o[4 * h + 2] = (bf16_t)p1[0];
-    o[4 * h + 3] = (bf16_t)p1[1];
-  }
-  return o;
-}
 constexpr uint32_t SM_ONE_PAIR = 0x3F803F80u;   // {1.0, 1.0}
 
 // Wait until at most N of this wave's vector memory operations are outstanding and its LDS reads have returned, then
@@ -517,7 +505,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, EPI == SM_EPI_QKV_WATTN ? 1
 #pragma unroll
       for (int j = 0; j < NT; ++j) {
         bf16x8_t w;
-        if constexpr (W_FP8) w = sm_fp8x8_to_bf16(wraw[SET][W_FP8 ? s : 0][W_FP8 ? j : 0]);
+        if constexpr (W_FP8) w = fp8x8_to_bf16(wraw[SET][W_FP8 ? s : 0][W_FP8 ? j : 0]);
         else w = wf[SET][W_FP8 ? 0 : s][W_FP8 ? 0 : j];
 #pragma unroll
         for (int i = 0; i < MT; ++i) acc[i][j] = sm_mfma(w, xf[SET][s][i], acc[i][j]);

@@ -328,6 +328,29 @@ def test_both_gemm_kernels_round_their_epilogues_alike(ops, dev):
     assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
 
 
+@pytest.mark.parametrize("M,N,K", [(96, 1280, 192), (1500, 1280, 1280), (2743, 1280, 192), (2744, 1152, 320), (4096, 1280, 192),
+                                   (4100, 1280, 448), (8192, 1280, 192), (16500, 320, 192)])
+def test_fp8_residual_products_equal_bf16_weights_bit_for_bit(ops, dev, M, N, K):
+    """e4m3 weights are bf16 values, and with powers of two as scales so are the scaled ones: the same sums in the same
+    order, so the residual product on the split stream must give the bits of the product with the bf16 weights, in every
+    tile form (128 and 256 rows, edge tiles, several tiles a workgroup, with and without bias and byte plane)."""
+    g = torch.Generator().manual_seed(M + K)
+    q = torch.randint(0, 256, (N, K), generator=g, dtype=torch.uint8)
+    q[(q & 0x7F) == 0x7F] = 0x01                                          # (NaN codes; the least subnormal instead)
+    scale = 2.0 ** torch.randint(-6, 1, (N,), generator=g).float()
+    w = (q.view(torch.float8_e4m3fn).float() * scale[:, None]).bfloat16()
+    a, b, res = rnd((M, K), 1.0, 2, dev), rnd((N,), 1.0, 3, dev), rnd((M, N), 4.0, 4, dev)
+    lo = torch.randint(0, 256, (M, N), generator=g, dtype=torch.uint8).to(dev)
+    q, scale, w = q.to(dev), scale.to(dev), w.to(dev)
+    for bias, plane in ((b, lo), (None, None)):
+        outs = []
+        for kw in (dict(w=w), dict(w=q, w_scale=scale)):
+            o, ol = torch.empty_like(res), torch.empty_like(lo)
+            ops.gemm(a, bias=bias, epilogue=ops.EPI_RESIDUAL, residual=res, residual_lo=plane, out=o, out_lo=ol, **kw)
+            outs.append((o, ol))
+        assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
+
+
 def test_kernels_are_registered_torch_operators(ops, dev):
     """Every kernel entry point is an operator of the `cornserve_amd` namespace with a schema that names what it
     mutates and a fake implementation (shape propagation without running a kernel); `torch.library.opcheck` checks both
