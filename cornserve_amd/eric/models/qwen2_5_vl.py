@@ -220,6 +220,26 @@ class QwenVisionBase(EricModel):
             row += gt * gh * gw
         return px, grid
 
+    # Row count of the per-block buffers: a whole number of 256-row tiles (the tallest form; 128-row tiles divide it) for
+    # batches that the big tiles run.  A tile with rows past the end cannot take the guard-free epilogue with its residual
+    # piece through the LDS ring, and a launch lasts as long as its slowest tile: 1280 columns at K = 1280 and 3456, 7900
+    # rows 39 and 68 us, 7936 rows 32 and 60; 20400 rows 97 and 182 us, 20480 rows 90 and 174.  The matrix cores work on
+    # the rows past the end either way; rows are independent of each other, so nothing else changes.  Whole passes: 5076
+    # rows 9.19 -> 8.65 ms, 8068 rows 10.5 -> 10.1, 3996 rows (fp8 weights) 7.08 -> 6.98.  Batches of fewer rows partly run
+    # in the few-row kernel's smaller tiles, where whole tiles are more work: 2196 rows (Qwen2-VL) 5.90 -> 6.09 ms.
+    row_tile, row_tile_min = 256, 3585
+
+    def _whole_tile_rows(self, rows: int, max_rows: int) -> int:
+        whole = -(-rows // self.row_tile) * self.row_tile
+        return whole if rows >= self.row_tile_min and whole <= max_rows else rows
+
+    def _row_buffer(self, rows: int, used: int, cols: int) -> torch.Tensor:
+        """bf16 [rows, cols] whose rows from `used` on are zero."""
+        t = torch.empty((rows, cols), dtype=torch.bfloat16, device=self.device)
+        if used < rows:
+            t[used:].zero_()
+        return t
+
     @staticmethod
     def _addressable_groups(grid_thw: np.ndarray, max_rows: int) -> list[tuple[int, int]]:
         """Consecutive item ranges [first, last) of at most `max_rows` patches each (items are independent, so a batch
@@ -463,9 +483,10 @@ class Qwen2_5_VisionTransformer(QwenVisionBase):
         win = self.window_size // merge // self.patch_size
         dev = self.device
 
+        max_rows = (2**32 - 1) // (2 * max(3 * H, pk["Ip"]))
         # the folded-norm GEMMs address their operands with 32-bit byte offsets: a batch beyond that runs as several
         if self.fold_norm:
-            groups = self._addressable_groups(grid_thw, (2**32 - 1) // (2 * max(3 * H, pk["Ip"])))
+            groups = self._addressable_groups(grid_thw, max_rows)
             if len(groups) > 1:
                 return self._forward_in_groups(pixel_values, grid_thw, groups, mark)
         mark("index")
@@ -475,25 +496,27 @@ class Qwen2_5_VisionTransformer(QwenVisionBase):
 
         # patch embed; rows come out already in window order
         mark("patch_embed")
-        x = ops.gemm(pixel_values, pk["pe_w"], None, a_rows=ix.src_rows)
+        R = self._whole_tile_rows(L, max_rows)
+        x = self._row_buffer(R, L, H)
+        ops.gemm(pixel_values, pk["pe_w"], None, a_rows=ix.src_rows, out=x)
         # the low-order plane of the residual stream; zero = "x is exact"
         res = {"residual_lo": (lo := torch.zeros(x.shape, dtype=torch.uint8, device=dev)), "out_lo": lo} if self.split_residual else {}
         n = torch.empty_like(x)
         # the folded-norm GEMMs exist in the fast kernel only, whose per-lane byte offsets are 32-bit
         fold = self.fold_norm
         eps = self.norm_eps
-        qkv = torch.empty((L, 3 * H), dtype=torch.bfloat16, device=dev)
-        att = torch.empty((L, H), dtype=torch.bfloat16, device=dev)
-        hmid = torch.empty((L, pk["Ip"]), dtype=torch.bfloat16, device=dev)
+        qkv = torch.empty((R, 3 * H), dtype=torch.bfloat16, device=dev)
+        att = self._row_buffer(R, L, H)
+        hmid = torch.empty((R, pk["Ip"]), dtype=torch.bfloat16, device=dev)
         scale = d**-0.5
         # Few rows: the consumer of a folded norm takes the row sums itself, which lets the residual GEMMs in front of it use
         # tiles that do not span a part of the sums.  Same bits either way, so the choice follows speed alone.
         n_blocks = len(pk["blocks"])
         n_slots = fused_rows // ops.QKV_WATTN_WINDOW if win_start is None else win_start.numel() - 1
         inline_wattn = fold and n_slots > 0 and ops.window_attn_norm_inline_pays(n_slots, nh, H)
-        inline_full = fold and ops.norm_inline_pays(L, 3 * H, H)
-        inline_sep = fold and fused_rows < L and ops.norm_inline_pays(L - fused_rows, 3 * H, H)
-        inline_mlp = fold and ops.norm_inline_pays(L, 2 * pk["Ip"], H)
+        inline_full = fold and ops.norm_inline_pays(R, 3 * H, H)
+        inline_sep = fold and fused_rows < L and ops.norm_inline_pays(R - fused_rows, 3 * H, H)
+        inline_mlp = fold and ops.norm_inline_pays(R, 2 * pk["Ip"], H)
 
         def attn_reads_sums(i: int) -> bool:
             if i >= n_blocks:
@@ -520,7 +543,7 @@ class Qwen2_5_VisionTransformer(QwenVisionBase):
             return nb["qkv"]["w"] if nb["qkv"] is not None else nb["qkv_wattn"][0]
 
         if fold:
-            ss = torch.empty((L, ops.SUMSQ_PARTS), dtype=torch.float32, device=dev)
+            ss = torch.empty((R, ops.SUMSQ_PARTS), dtype=torch.float32, device=dev)
             if not inline_mlp or any(attn_reads_sums(i) for i in range(n_blocks)):
                 mark("norm")
                 ops.row_sumsq(x, out=ss)   # (writes every part, zeros past the hidden size: the GEMMs write those up to it)
@@ -547,20 +570,20 @@ class Qwen2_5_VisionTransformer(QwenVisionBase):
                 lo = 0 if full else fused_rows           # first row the separate kernels work on in this block
                 if fold:
                     mark("gemm_qkv")
-                    self._g(x[lo:], self._plain_qkv(b), out=qkv[lo:], **norm(inline_full if full else inline_sep, slice(lo, L)))
+                    self._g(x[lo:], self._plain_qkv(b), out=qkv[lo:], **norm(inline_full if full else inline_sep, slice(lo, R)))
                 else:
                     mark("norm")
                     ops.rmsnorm(x[lo:], b["n1"], eps, out=n[lo:])
                     mark("gemm_qkv")
                     self._g(n[lo:], self._plain_qkv(b), out=qkv[lo:])
                 mark("attn_full" if full else "attn_window")
-                ops.attn_varlen_rotary_(qkv, plan_full if full else plan_win, nh, d, scale, ix.cos_sin, out=att)
+                ops.attn_varlen_rotary_(qkv[:L], plan_full if full else plan_win, nh, d, scale, ix.cos_sin, out=att)
             mark("gemm_proj")
             if fold:
                 self._g(att, b["proj"], epilogue=ops.EPI_RESIDUAL, residual=x, out=x, c_row_sumsq=None if inline_mlp else ss,
                         prefetch=pf_proj, **res)
                 mark("gemm_gate_up")
-                self._g(x, b["gu"], epilogue=ops.EPI_SWIGLU, out=hmid, **norm(inline_mlp, slice(0, L)))
+                self._g(x, b["gu"], epilogue=ops.EPI_SWIGLU, out=hmid, **norm(inline_mlp, slice(0, R)))
                 mark("gemm_down")
                 self._g(hmid, b["down"], epilogue=ops.EPI_RESIDUAL, residual=x, out=x,
                         c_row_sumsq=ss if attn_reads_sums(i + 1) else None, prefetch=pf_down, **res)
@@ -576,7 +599,7 @@ class Qwen2_5_VisionTransformer(QwenVisionBase):
         mark("norm")
         ops.rmsnorm(x, pk["ln_q"], self.norm_eps, out=n)
         mark("gemm_merger")
-        y = self._g(n.view(L // unit, H * unit), pk["fc1"], epilogue=ops.EPI_GELU_ERF)
+        y = self._g(n[:L].view(L // unit, H * unit), pk["fc1"], epilogue=ops.EPI_GELU_ERF)
         out = torch.empty((L // unit, self.out_hidden_size), dtype=torch.bfloat16, device=dev)
         # merged row m sits at window-order position m; it belongs at row window_index[m]
         self._g(y, pk["fc2"], c_rows=ix.window_index32, out=out)

@@ -138,8 +138,9 @@ class Qwen2VisionTransformer(QwenVisionBase):
         pk = self._ensure_packed()
         E, nh, d, unit, dev = self.embed_dim, self.num_heads, self.head_dim, self.spatial_merge_unit, self.device
         eps = self.norm_eps
+        max_rows = (2**32 - 1) // (2 * max(3 * E, self.mlp_hidden))
         if self.fold_norm:   # 32-bit operand offsets in the folded-norm GEMMs: a batch beyond them runs as several
-            groups = self._addressable_groups(grid_thw, (2**32 - 1) // (2 * max(3 * E, self.mlp_hidden)))
+            groups = self._addressable_groups(grid_thw, max_rows)
             if len(groups) > 1:
                 return self._forward_in_groups(pixel_values, grid_thw, groups, mark)
 
@@ -157,11 +158,13 @@ class Qwen2VisionTransformer(QwenVisionBase):
             raise ValueError(f"pixel_values has {pixel_values.shape[0]} rows but grid_thw describes {L} patches")
 
         mark("patch_embed")
-        x = ops.gemm(pixel_values, pk["pe_w"], None)
+        R = self._whole_tile_rows(L, max_rows)
+        x = self._row_buffer(R, L, E)
+        ops.gemm(pixel_values, pk["pe_w"], None, out=x)
         n = torch.empty_like(x)
-        qkv = torch.empty((L, 3 * E), dtype=torch.bfloat16, device=dev)
-        att = torch.empty((L, E), dtype=torch.bfloat16, device=dev)
-        hmid = torch.empty((L, self.mlp_hidden), dtype=torch.bfloat16, device=dev)
+        qkv = torch.empty((R, 3 * E), dtype=torch.bfloat16, device=dev)
+        att = self._row_buffer(R, L, E)
+        hmid = torch.empty((R, self.mlp_hidden), dtype=torch.bfloat16, device=dev)
         scale = d**-0.5
         fold = self.fold_norm
         res = {}
@@ -170,7 +173,7 @@ class Qwen2VisionTransformer(QwenVisionBase):
             res = {"residual_lo": lo, "out_lo": lo}
         if fold:
             mark("norm")
-            ss = torch.zeros((L, ops.SUMSQ_PARTS), dtype=torch.float32, device=dev)
+            ss = torch.zeros((R, ops.SUMSQ_PARTS), dtype=torch.float32, device=dev)
             sm = torch.zeros_like(ss)
             ops.row_stats(x, ss, sm)
             stats_in = lambda lin: {"a_row_sumsq": ss, "a_row_sum": sm, "w_col_sum": lin["colsum"], "norm_eps": eps}  # noqa: E731
@@ -191,7 +194,7 @@ class Qwen2VisionTransformer(QwenVisionBase):
                 mark("gemm_qkv")
                 self._g(n, b["qkv"], out=qkv, prefetch=pf_qkv)
             mark("attn_full")
-            ops.attn_varlen_rotary_(qkv, plan, nh, d, scale, ix.cos_sin, out=att)
+            ops.attn_varlen_rotary_(qkv[:L], plan, nh, d, scale, ix.cos_sin, out=att)
             mark("gemm_proj")
             self._g(att, b["proj"], epilogue=ops.EPI_RESIDUAL, residual=x, out=x, prefetch=pf_proj, **res,
                     **(stats_out if fold else {}))
@@ -210,7 +213,7 @@ class Qwen2VisionTransformer(QwenVisionBase):
         mark("norm")
         ops.layernorm(x, *pk["ln_q"], eps, out=n)
         mark("gemm_merger")
-        y = self._g(n.view(L // unit, E * unit), pk["m1"], epilogue=ops.EPI_GELU_ERF)
+        y = self._g(n[:L].view(L // unit, E * unit), pk["m1"], epilogue=ops.EPI_GELU_ERF)
         out = self._g(y, pk["m2"])
         mark("end")
         g = grid_thw.reshape(-1, 3)

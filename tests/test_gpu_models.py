@@ -296,6 +296,24 @@ def test_qwen_batch_items_are_independent(dev):
         assert all(torch.equal(a, b) for a, b in zip(hinted, plain)), kw
 
 
+@pytest.mark.parametrize("family,kw", [("2.5", {}), ("2.5", {"fuse_window_attn": False}), ("2.5", {"fold_norm": False}),
+                                       ("2.5", {"weight_format": "fp8_e4m3"}), ("2", {})])
+def test_rows_filled_up_to_whole_tiles_change_no_bit(dev, family, kw):
+    """From `row_tile_min` patches on the per-block products run over whole 256-row tiles.  Rows are independent, so the
+    embeddings are those of the exact row count, bit for bit: just below and above a tile, items with short windows and
+    whole ones, and a count that needs no filling."""
+    model = build_qwen(dev, 2, (1,), seed=7, **kw)[0] if family == "2.5" else build_qwen2(dev, 2, seed=7, **kw)[0]
+    for grids in ([(1, 32, 32), (1, 32, 32)], [(1, 32, 32), (1, 32, 34)], [(1, 48, 64), (1, 26, 38)], [(1, 2, 2), (1, 64, 64)]):
+        px, grid = synth.qwen_inputs(grids, seed=7)
+        batch = {"pixel_values": px, "image_grid_thw": grid}
+        model.row_tile_min = 2048
+        filled = model(Modality.IMAGE, "", batch)
+        model.row_tile_min = 1 << 30
+        exact = model(Modality.IMAGE, "", batch)
+        assert all(torch.isfinite(o).all() for o in exact)
+        assert all(torch.equal(a, b) for a, b in zip(filled, exact, strict=True)), grids
+
+
 def test_qwen_fp8_weights(dev):
     """Config-5 style: fp8-e4m3 weights with per-output-channel scales vs the de-quantised oracle."""
     model, sd, ocfg = build_qwen(dev, 3, (2,), seed=5, weight_format="fp8_e4m3")
