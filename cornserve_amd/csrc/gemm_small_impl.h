@@ -9,7 +9,7 @@
 // unit (128 bytes a clock) in every tile form; the rest of a launch is 4 to 5 us of launch, first loads and epilogue.
 // Measured on an MI355X with weights that no cache holds: 1280 columns, K = 3456: 96 rows 34.3 -> 8.7 us (32x32 tiles),
 // 1024 rows 38 -> 20 us (64x80); K = 1280: 96 rows 19 -> 6 us, 1024 rows 19 -> 11 us.  From about 2048 rows on the big
-// tiles are the faster ones (the choice is in gemm_fast.hip).
+// tiles are the faster ones (the choice is in gemm_small.hip).
 //
 // The arithmetic of an output element is the same sequence of operations as in gemm_fast_impl.h (v_mfma_f32_16x16x32_bf16
 // over ascending K from a zero accumulator, W as the first operand, the same epilogue functions in the same order), so an
