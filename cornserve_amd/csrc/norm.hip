@@ -149,6 +149,75 @@ __global__ __launch_bounds__(256) void row_sumsq_kernel(const bf16_t* __restrict
   }
 }
 
+// Eight per-lane partial sums -> their eight totals over the wave, with 10 lane exchanges instead of 48: each of
+// the first three exchanges (lane ^ 32, ^ 16, ^ 8) hands the partner the half of the values it keeps, so the number
+// of live values halves; three more exchanges finish the one value left.  Lane l returns the total of part l >> 3.
+static_assert(CS_SUMSQ_PARTS == 8, "wave_sum_parts halves eight values three times");
+CS_DEVICE float wave_sum_parts(const float (&part)[8], int lane) {
+  const bool b5 = lane & 32, b4 = lane & 16, b3 = lane & 8;
+  float a[4], b[2];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float keep = b5 ? part[4 + i] : part[i], give = b5 ? part[i] : part[4 + i];
+    a[i] = keep + __shfl_xor(give, 32, 64);
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const float keep = b4 ? a[2 + i] : a[i], give = b4 ? a[i] : a[2 + i];
+    b[i] = keep + __shfl_xor(give, 16, 64);
+  }
+  float c = (b3 ? b[1] : b[0]) + __shfl_xor(b3 ? b[0] : b[1], 8, 64);
+  c += __shfl_xor(c, 4, 64);
+  c += __shfl_xor(c, 2, 64);
+  c += __shfl_xor(c, 1, 64);
+  return c;
+}
+
+// The same statistics in another order of summation: one wave owns a row, lane l sums chunks l, l + 64, l + 128 of 8 values
+// one after the other, and the lanes of a part meet in a tree.  An encoder takes the statistics of its patch embedding in
+// this order (every later row's come from the GEMM epilogues), and the last bit of a row's scale reaches every bf16
+// rounding behind it: both orders are as near to the exact sums, but only this one keeps an embedding's bits.
+template <bool WITH_SUM>
+__global__ __launch_bounds__(256) void row_stats_chunk_order_kernel(const bf16_t* __restrict__ x, int64_t ldx, int rows,
+                                                                    int H, float* __restrict__ out,
+                                                                    float* __restrict__ sum_out) {
+  constexpr int NC = (160 * CS_SUMSQ_PARTS / 8 + 63) / 64;
+  const int lane = threadIdx.x & 63;
+  const int row = blockIdx.x * ROWS_PER_BLOCK + (threadIdx.x >> 6);
+  if (row >= rows) return;
+  const int nchunks = H >> 3;
+  float v[NC][8];
+  load_row<NC>(x + (int64_t)row * ldx, nchunks, lane, v);
+  float part[CS_SUMSQ_PARTS], spart[WITH_SUM ? CS_SUMSQ_PARTS : 1];
+#pragma unroll
+  for (int q = 0; q < CS_SUMSQ_PARTS; ++q) {
+    part[q] = 0.f;
+    if (WITH_SUM) spart[WITH_SUM ? q : 0] = 0.f;
+  }
+#pragma unroll
+  for (int j = 0; j < NC; ++j) {
+    float ss = 0.f, sm = 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      ss += v[j][e] * v[j][e];
+      sm += v[j][e];
+    }
+    const int q_of_chunk = (lane + 64 * j) / 20;
+#pragma unroll
+    for (int q = 0; q < CS_SUMSQ_PARTS; ++q) {
+      part[q] += (q == q_of_chunk) ? ss : 0.f;
+      if (WITH_SUM) spart[WITH_SUM ? q : 0] += (q == q_of_chunk) ? sm : 0.f;
+    }
+  }
+  // lane l ends up with the total of part l / 8: eight lanes each store one value
+  const float tot = wave_sum_parts(part, lane);
+  if ((lane & 7) == 0) out[(int64_t)row * CS_SUMSQ_PARTS + (lane >> 3)] = tot;
+  if constexpr (WITH_SUM) {
+    const float stot = wave_sum_parts(spart, lane);
+    if ((lane & 7) == 0) sum_out[(int64_t)row * CS_SUMSQ_PARTS + (lane >> 3)] = stot;
+  }
+}
+
 // One wave per pooled token: mean over a k x k neighbourhood of the side x side token grid, rounded to
 // bf16 (AvgPool2d output dtype), then GemmaRMSNorm over the channel axis.
 template <int NC>
@@ -260,18 +329,35 @@ extern "C" int cs_rmsnorm(const void* x, int64_t ldx, const void* w, void* y, in
   return cs_launch_status();
 }
 
-extern "C" int cs_row_stats(const void* x, int64_t ldx, int32_t rows, int32_t H, float* out, float* sum_out, void* stream_) {
-  hipStream_t stream = (hipStream_t)stream_;
+static int row_stats_status(const void* x, int64_t ldx, int32_t rows, int32_t H, const float* out, const float* sum_out) {
   if (!x || !out || rows < 0 || H <= 0 || H % 8 || ldx % 8 || ldx < H ||
       (((uintptr_t)x | (uintptr_t)out | (uintptr_t)sum_out) & 15))
     return CS_ERR_INVALID_ARG;
-  if (H > 160 * CS_SUMSQ_PARTS) return CS_ERR_UNSUPPORTED;
-  if (rows == 0) return CS_OK;
+  return H > 160 * CS_SUMSQ_PARTS ? CS_ERR_UNSUPPORTED : CS_OK;
+}
+
+extern "C" int cs_row_stats(const void* x, int64_t ldx, int32_t rows, int32_t H, float* out, float* sum_out, void* stream_) {
+  hipStream_t stream = (hipStream_t)stream_;
+  const int st = row_stats_status(x, ldx, rows, H, out, sum_out);
+  if (st != CS_OK || rows == 0) return st;
   const dim3 grid((rows + 7) / 8), block(256);
   if (sum_out)
     hipLaunchKernelGGL(row_sumsq_kernel<true>, grid, block, 0, stream, (const bf16_t*)x, ldx, rows, H, out, sum_out);
   else
     hipLaunchKernelGGL(row_sumsq_kernel<false>, grid, block, 0, stream, (const bf16_t*)x, ldx, rows, H, out, sum_out);
+  return cs_launch_status();
+}
+
+extern "C" int cs_row_stats_chunk_order(const void* x, int64_t ldx, int32_t rows, int32_t H, float* out, float* sum_out,
+                                        void* stream_) {
+  hipStream_t stream = (hipStream_t)stream_;
+  const int st = row_stats_status(x, ldx, rows, H, out, sum_out);
+  if (st != CS_OK || rows == 0) return st;
+  const dim3 grid((rows + ROWS_PER_BLOCK - 1) / ROWS_PER_BLOCK), block(256);
+  if (sum_out)
+    hipLaunchKernelGGL(row_stats_chunk_order_kernel<true>, grid, block, 0, stream, (const bf16_t*)x, ldx, rows, H, out, sum_out);
+  else
+    hipLaunchKernelGGL(row_stats_chunk_order_kernel<false>, grid, block, 0, stream, (const bf16_t*)x, ldx, rows, H, out, sum_out);
   return cs_launch_status();
 }
 

@@ -272,7 +272,7 @@ class SiglipEncoderBase(EricModel):
         if fold:
             ss = torch.zeros((M, ops.SUMSQ_PARTS), dtype=torch.float32, device=x.device)
             sm = torch.zeros_like(ss)
-            ops.row_stats(x, ss, sm)
+            ops.row_stats(x, ss, sm, chunk_order=True)
             stats_out.update(c_row_sumsq=ss, c_row_sum=sm)
         for lyr in pk["layers"]:
             if fold:

@@ -510,7 +510,8 @@ class Qwen2_5_VisionTransformer(QwenVisionBase):
         hmid = torch.empty((R, pk["Ip"]), dtype=torch.bfloat16, device=dev)
         scale = d**-0.5
         # Few rows: the consumer of a folded norm takes the row sums itself, which lets the residual GEMMs in front of it use
-        # tiles that do not span a part of the sums.  Same bits either way, so the choice follows speed alone.
+        # tiles that do not span a part of the sums.  Same bits either way, so the choice follows speed alone.  (The first
+        # block's are summed in an order of their own, see cs_row_stats_chunk_order: always from the arrays.)
         n_blocks = len(pk["blocks"])
         n_slots = fused_rows // ops.QKV_WATTN_WINDOW if win_start is None else win_start.numel() - 1
         inline_wattn = fold and n_slots > 0 and ops.window_attn_norm_inline_pays(n_slots, nh, H)
@@ -543,10 +544,8 @@ class Qwen2_5_VisionTransformer(QwenVisionBase):
             return nb["qkv"]["w"] if nb["qkv"] is not None else nb["qkv_wattn"][0]
 
         if fold:
-            ss = torch.empty((R, ops.SUMSQ_PARTS), dtype=torch.float32, device=dev)
-            if not inline_mlp or any(attn_reads_sums(i) for i in range(n_blocks)):
-                mark("norm")
-                ops.row_sumsq(x, out=ss)   # (writes every part, zeros past the hidden size: the GEMMs write those up to it)
+            mark("norm")   # (writes every part, zeros past the hidden size: the GEMMs write those up to it)
+            ss = ops.row_sumsq(x, out=torch.empty((R, ops.SUMSQ_PARTS), dtype=torch.float32, device=dev), chunk_order=True)
         for i, b in enumerate(pk["blocks"]):
             full = i in self.fullatt_block_indexes
             pf_qkv = b["gu"]["w"] if hint else None   # (from the one-launch window block only: the plain QKV GEMM of a
@@ -559,7 +558,7 @@ class Qwen2_5_VisionTransformer(QwenVisionBase):
                 if fold:
                     mark("gemm_qkv_attn_window")
                     ops.qkv_window_attn(xf, wp, bp, ix.cos_sin[:fused_rows], nh, scale, out=att[:fused_rows],
-                                        win_start=win_start, prefetch=pf_qkv, **norm(inline_wattn, slice(0, fused_rows)))
+                                        win_start=win_start, prefetch=pf_qkv, **norm(inline_wattn and i > 0, slice(0, fused_rows)))
                 else:
                     mark("norm")
                     ops.rmsnorm(xf, b["n1"], eps, out=n[:fused_rows])
@@ -570,7 +569,8 @@ class Qwen2_5_VisionTransformer(QwenVisionBase):
                 lo = 0 if full else fused_rows           # first row the separate kernels work on in this block
                 if fold:
                     mark("gemm_qkv")
-                    self._g(x[lo:], self._plain_qkv(b), out=qkv[lo:], **norm(inline_full if full else inline_sep, slice(lo, R)))
+                    self._g(x[lo:], self._plain_qkv(b), out=qkv[lo:],
+                            **norm((inline_full if full else inline_sep) and i > 0, slice(lo, R)))
                 else:
                     mark("norm")
                     ops.rmsnorm(x[lo:], b["n1"], eps, out=n[lo:])

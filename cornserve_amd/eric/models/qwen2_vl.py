@@ -175,7 +175,7 @@ class Qwen2VisionTransformer(QwenVisionBase):
             mark("norm")
             ss = torch.zeros((R, ops.SUMSQ_PARTS), dtype=torch.float32, device=dev)
             sm = torch.zeros_like(ss)
-            ops.row_stats(x, ss, sm)
+            ops.row_stats(x, ss, sm, chunk_order=True)
             stats_in = lambda lin: {"a_row_sumsq": ss, "a_row_sum": sm, "w_col_sum": lin["colsum"], "norm_eps": eps}  # noqa: E731
             stats_out = {"c_row_sumsq": ss, "c_row_sum": sm}
         # few rows: each launch names the weights of the launch after next for its idle compute units to read

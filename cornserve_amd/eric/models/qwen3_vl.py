@@ -225,11 +225,12 @@ class Qwen3_VisionTransformer(QwenVisionBase):
         inline_qkv = fold and ops.norm_inline_pays(L, 3 * E, E)
         inline_fc1 = fold and ops.norm_inline_pays(L, self.intermediate_size + self.mlp_pad, E)
         sums: dict = {}
-        if fold and not (inline_qkv and inline_fc1):
+        if fold:
             mark("norm")
             ss = torch.empty((L, ops.SUMSQ_PARTS), dtype=torch.float32, device=dev)
             sm = torch.empty_like(ss)
-            ops.row_stats(x, ss, sm)   # (every part, zeros past the hidden size: the GEMMs write those up to it)
+            # (every part, zeros past the hidden size: the GEMMs write those up to it)
+            ops.row_stats(x, ss, sm, chunk_order=True)
             sums = {"c_row_sumsq": ss, "c_row_sum": sm}
 
         def stats_in(lin: dict, inline: bool) -> dict:
@@ -253,7 +254,7 @@ class Qwen3_VisionTransformer(QwenVisionBase):
             if fold:
                 mark("gemm_qkv")
                 ops.gemm(x, b["qkv"]["w"], b["qkv"]["b"], out=qkv, prefetch=pf_qkv,
-                         **stats_in(b["qkv"], inline_qkv))
+                         **stats_in(b["qkv"], inline_qkv and i > 0))
             else:
                 mark("norm")
                 ops.layernorm(x, *b["n1"], eps, out=n)

@@ -145,7 +145,7 @@ def gemm(
     `c_row_sum` receives the plain sums of the output rows.
 
     `norm_inline`: the folded norm without the arrays: the row sums are taken inside the launch (few rows: see
-    `norm_inline_pays`); RMSNorm, or LayerNorm with `w_col_sum`.  Same bits as with the arrays.
+    `norm_inline_pays`); RMSNorm, or LayerNorm with `w_col_sum`.  Same bits as with arrays from a GEMM or from `row_stats`.
 
     `out_lo` (uint8, shaped and strided like `out`; EPI_RESIDUAL only) carries the residual stream with 16
     significant bits: the sum is not rounded to bf16 but split into `out` (the leading 16 bits) and `out_lo` (the
@@ -197,7 +197,7 @@ def _rows_2d(t: torch.Tensor, dtype: torch.dtype, name: str) -> None:
         raise ValueError(f"{name} must be 2-D")
 
 
-def _row_stats_impl(sumsq_out, sum_out, x) -> None:
+def _row_stats_impl(sumsq_out, sum_out, x, chunk_order=False) -> None:
     lib = _l.load()
     _rows_2d(x, torch.bfloat16, "x")
     for name, t in (("sumsq_out", sumsq_out), ("sum_out", sum_out)):
@@ -205,7 +205,10 @@ def _row_stats_impl(sumsq_out, sum_out, x) -> None:
             _req(t, torch.float32, name)
             if tuple(t.shape) != (x.shape[0], SUMSQ_PARTS) or not t.is_contiguous() or t.device != x.device:
                 raise ValueError(f"{name} must be a contiguous fp32 [rows, {SUMSQ_PARTS}] tensor on x's device")
-    if sum_out is None:
+    if chunk_order:
+        _l.check(lib.cs_row_stats_chunk_order(x.data_ptr(), x.stride(0), x.shape[0], x.shape[1], sumsq_out.data_ptr(),
+                                              _ptr(sum_out), _stream()), "cs_row_stats_chunk_order")
+    elif sum_out is None:
         _l.check(lib.cs_row_sumsq(x.data_ptr(), x.stride(0), x.shape[0], x.shape[1], sumsq_out.data_ptr(), _stream()),
                  "cs_row_sumsq")
     else:
@@ -213,18 +216,21 @@ def _row_stats_impl(sumsq_out, sum_out, x) -> None:
                                   sum_out.data_ptr(), _stream()), "cs_row_stats")
 
 
-def row_stats(x: torch.Tensor, sumsq_out: torch.Tensor, sum_out: torch.Tensor) -> None:
-    """Sums of squares and sums of the rows of `x`, each fp32 [rows, SUMSQ_PARTS] in parts of 160 columns."""
-    torch.ops.cornserve_amd.row_stats_(sumsq_out, sum_out, x)
+def row_stats(x: torch.Tensor, sumsq_out: torch.Tensor, sum_out: torch.Tensor, *, chunk_order: bool = False) -> None:
+    """Sums of squares and sums of the rows of `x`, each fp32 [rows, SUMSQ_PARTS] in parts of 160 columns.
+
+    Summed in the order of the GEMM epilogues and of `norm_inline`, so a row's statistics have the same bits whichever
+    kernel made them.  `chunk_order`: the order of the encoders' first statistics (see cs_row_stats_chunk_order)."""
+    torch.ops.cornserve_amd.row_stats_(sumsq_out, sum_out, x, chunk_order)
 
 
-def row_sumsq(x: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:
-    """fp32 [rows, SUMSQ_PARTS]: sums of squares of the rows of `x` in parts of 160 columns."""
+def row_sumsq(x: torch.Tensor, out: torch.Tensor | None = None, *, chunk_order: bool = False) -> torch.Tensor:
+    """fp32 [rows, SUMSQ_PARTS]: sums of squares of the rows of `x` in parts of 160 columns (`chunk_order`: see row_stats)."""
     if out is None:
         if x.dim() != 2:
             raise ValueError("row_sumsq takes a 2-D tensor")
         out = torch.empty((x.shape[0], SUMSQ_PARTS), dtype=torch.float32, device=x.device)
-    torch.ops.cornserve_amd.row_stats_(out, None, x)
+    torch.ops.cornserve_amd.row_stats_(out, None, x, chunk_order)
     return out
 
 
@@ -763,7 +769,7 @@ _OPERATORS: dict[str, tuple[str, object]] = {   # schema, and the implementation
               "Tensor? pos, Tensor? a_rows, Tensor? c_rows, int? k, Tensor? a_row_sumsq, Tensor(b!)? c_row_sumsq, "
               "float norm_eps, Tensor? a_row_sum, Tensor(c!)? c_row_sum, Tensor? w_col_sum, Tensor? residual_lo, "
               "Tensor(d!)? out_lo, int conv_patch=0, Tensor? prefetch=None, bool norm_inline=False) -> ()", None),
-    "row_stats_": ("(Tensor(a!) sumsq_out, Tensor(b!)? sum_out, Tensor x) -> ()", _row_stats_impl),
+    "row_stats_": ("(Tensor(a!) sumsq_out, Tensor(b!)? sum_out, Tensor x, bool chunk_order=False) -> ()", _row_stats_impl),
     "rmsnorm_": ("(Tensor(a!) out, Tensor x, Tensor w, float eps, bool gemma) -> ()", None),
     "layernorm_": ("(Tensor(a!) out, Tensor x, Tensor w, Tensor b, float eps) -> ()", None),
     "avgpool_gemma_rmsnorm_": ("(Tensor(a!) out, Tensor x, Tensor w, int side, int k, float eps) -> ()",

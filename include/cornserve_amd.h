@@ -36,7 +36,7 @@ extern "C" {
 #define CS_ERR_TOO_LARGE 4
 
 /* ABI version of this header; cs_abi_version() returns the value the library was built with. */
-#define CS_ABI_VERSION 8
+#define CS_ABI_VERSION 9
 int cs_abi_version(void);
 
 /* ------------------------------------------------------------------------------------------------
@@ -143,7 +143,7 @@ typedef struct CsGemmArgs {
   /* Folded norm without the row-sum arrays: with a_norm_inline = 1 the sums over the rows of A are taken inside the
    * launch (K is the normalised width, at most 160 * CS_SUMSQ_PARTS); a_row_sumsq and a_row_sum are NULL, w_col_sum says
    * which norm (NULL: RMSNorm, set: LayerNorm), and W, bias and norm_eps are those of the array form.  Same bits as the
-   * array form.  Meant for few rows: cs_gemm_norm_inline_pays tells whether this form is the faster one for a shape.
+   * array form with sums from a GEMM's c_row_sumsq / c_row_sum or from cs_row_sumsq / cs_row_stats.  Meant for few rows: cs_gemm_norm_inline_pays tells whether this form is the faster one for a shape.
    * CS_EPI_BIAS and CS_EPI_SWIGLU (RMSNorm), CS_EPI_BIAS, CS_EPI_GELU_TANH and CS_EPI_QUICK_GELU (LayerNorm); bf16 W,
    * K a multiple of 128; also taken by cs_qkv_window_attn (RMSNorm).  CS_ERR_UNSUPPORTED otherwise.               */
   int32_t a_norm_inline;
@@ -191,6 +191,11 @@ int cs_row_sumsq(const void* x, int64_t ldx, int32_t rows, int32_t H, float* out
 /* The same with the plain row sums next to them (sum_out in the same layout): the statistics of LayerNorm for a
  * GEMM launched with a_row_sum.                                                                     */
 int cs_row_stats(const void* x, int64_t ldx, int32_t rows, int32_t H, float* sumsq_out, float* sum_out, void* stream);
+/* The same statistics (sum_out may be NULL) summed in another order: chunks of 8 columns, 64 apart, then a tree over the
+ * chunks of a part, where the two above sum in the order of the GEMM epilogues.  Both are as near to the exact sums; the
+ * results differ in the last bit of some rows.  The encoders take their first statistics with this one.             */
+int cs_row_stats_chunk_order(const void* x, int64_t ldx, int32_t rows, int32_t H, float* sumsq_out, float* sum_out,
+                             void* stream);
 /* nn.LayerNorm with affine, siglip.py:173-175,333.                                                */
 int cs_layernorm(const void* x, int64_t ldx, const void* w, const void* b, void* y, int64_t ldy,
                  int32_t rows, int32_t H, float eps, void* stream);

@@ -296,6 +296,46 @@ def test_qwen_batch_items_are_independent(dev):
         assert all(torch.equal(a, b) for a, b in zip(hinted, plain)), kw
 
 
+@pytest.mark.parametrize("family", ["2.5", "2.5, unfused windows", "2.5, full attention first", "2, folded", "3", "gemma, folded"])
+@pytest.mark.parametrize("few", [True, False])
+def test_the_first_statistics_are_summed_in_chunk_order(dev, monkeypatch, family, few):
+    """An embedding's bits hang on the last bit of every row's scale.  The statistics of the patch embedding are summed in
+    one stated order at every batch size: with sums computed outside of the library in that order, no bit changes."""
+    from cornserve_amd import ops
+    from oracle.row_stats import in_chunk_order
+
+    items = 1 if few else 4
+    if family.startswith("gemma"):
+        model = build_gemma(dev, 2, 224, 640, 16, seed=9, fold_norm=True)[0]
+        px, crops = synth.gemma3_inputs(items, 224, seed=9)
+        name, batch = "a", {"pixel_values": px, "num_crops": crops}
+    else:
+        if family == "3":
+            model = build_qwen3(dev, 2, (0,), 1024, seed=9)[0]
+        elif family.startswith("2,"):
+            model = build_qwen2(dev, 2, seed=9, fold_norm=True)[0]
+        else:
+            model = build_qwen(dev, 2, (0,) if "first" in family else (1,), seed=9, fuse_window_attn="unfused" not in family)[0]
+        grids = [(1, 16, 20)] if few else [(1, 32, 32), (1, 10, 26), (1, 16, 20), (1, 48, 32)]
+        px, grid = (synth.qwen3_inputs if family == "3" else synth.qwen_inputs)(grids, seed=9)
+        name, batch = "", {"pixel_values": px, "image_grid_thw": grid}
+    got = model(Modality.IMAGE, name, batch)
+    calls = []
+
+    def row_stats(x, sumsq_out, sum_out, **kw):
+        ss, sm = in_chunk_order(x.cpu())
+        sumsq_out.copy_(ss)
+        if sum_out is not None:
+            sum_out.copy_(sm)
+        calls.append(x.shape[0])
+
+    monkeypatch.setattr(ops, "row_stats", row_stats)
+    monkeypatch.setattr(ops, "row_sumsq", lambda x, out, **kw: (row_stats(x, out, None), out)[1])
+    want = model(Modality.IMAGE, name, batch)
+    assert len(calls) == 1
+    assert all(torch.equal(a, b) for a, b in zip(got, want, strict=True))
+
+
 @pytest.mark.parametrize("family,kw", [("2.5", {}), ("2.5", {"fuse_window_attn": False}), ("2.5", {"fold_norm": False}),
                                        ("2.5", {"weight_format": "fp8_e4m3"}), ("2", {})])
 def test_rows_filled_up_to_whole_tiles_change_no_bit(dev, family, kw):

@@ -611,6 +611,21 @@ def test_row_sumsq(ops, dev, rows, H):
         ops.row_sumsq(rnd((4, 1288), 1.0, 1, dev))
 
 
+@pytest.mark.parametrize("rows,H", [(1, 1280), (1001, 1280), (77, 1152), (5, 64), (3, 8)])
+def test_row_stats_in_chunk_order_bit_for_bit(ops, dev, rows, H):
+    """The statistics an encoder's first block starts from: every fp32 addition in the order that the oracle states."""
+    from oracle import row_stats
+
+    x = rnd((rows, H), 2.0, 33, dev)
+    want_ss, want_sm = row_stats.in_chunk_order(x.cpu())
+    ss, sm = torch.full((rows, 8), 7.0, device=dev), torch.full((rows, 8), 7.0, device=dev)
+    ops.row_stats(x, ss, sm, chunk_order=True)
+    assert torch.equal(ss.cpu(), want_ss) and torch.equal(sm.cpu(), want_sm)
+    assert torch.equal(ops.row_sumsq(x, chunk_order=True).cpu(), want_ss)
+    with pytest.raises(RuntimeError):
+        ops.row_sumsq(rnd((4, 1288), 1.0, 1, dev), chunk_order=True)
+
+
 # RMSNorm folded into the GEMMs on both sides of it: the producer (residual epilogue) emits the sums of squares
 # of the rows it writes, the consumer scales its accumulators by rsqrt(mean square + eps).
 @pytest.mark.parametrize("M,N,K", [(8192, 1280, 192), (1000, 1280, 320), (300, 1152, 448), (257, 168, 192)])
