@@ -4,6 +4,10 @@
 
 namespace csgemm {
 
+// Widths whose norm can be taken inline (CsGemmArgs.a_norm_inline): the row sums are kept as CS_SUMSQ_PARTS parts of 160
+// columns in LDS, and K is walked in steps of 128.
+inline bool inline_norm_width(int K) { return K % 128 == 0 && K <= 160 * CS_SUMSQ_PARTS; }
+
 constexpr int BK = 64;  // K step (bf16 elements): 128 bytes per tile row = 8 chunks of 16 B
 
 // Byte offset of 16-byte chunk `chunk` of row `row` in a [rows][64] bf16 LDS tile (128-byte rows).

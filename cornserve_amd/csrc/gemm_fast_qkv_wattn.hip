@@ -38,6 +38,7 @@ extern "C" int cs_qkv_window_attn(const CsGemmArgs* gemm, const float* cos_sin, 
   a.epilogue = CS_EPI_BIAS;
   if (ragged && ((uintptr_t)a.attn_win_start & 3 || (int64_t)a.attn_n_win * 64 > INT32_MAX)) return CS_ERR_INVALID_ARG;
   if (a.a_norm_inline && (a.a_norm_inline != 1 || a.a_row_sumsq || a.w_fp8 || a.w_col_sum)) return CS_ERR_INVALID_ARG;
+  if (a.a_norm_inline && !csgemm::inline_norm_width(a.K)) return CS_ERR_UNSUPPORTED;
   // few windows: a workgroup per window and head
   if (cs_qkv_window_attn_few(ragged ? a.attn_n_win : a.M / 64, heads, a.K)) {
     const int rows = a.M;

@@ -75,8 +75,6 @@ const Form* best_form(const Form (&forms)[COUNT], const CsGemmArgs& a, double* u
   return best;
 }
 
-bool inline_norm_shape(int K) { return K % 128 == 0 && K <= 160 * CS_SUMSQ_PARTS; }
-
 }  // namespace
 
 // Called by cs_gemm for a shape that the direct-to-LDS kernels take (see cs_gemm_fast).  Sets *handled when the launch goes
@@ -91,7 +89,7 @@ int cs_gemm_small(const CsGemmArgs& a, hipStream_t stream, bool* handled) {
     f = best_form(SUMS_FORMS, a, &us);
     if (us >= fast_us(a.M, a.N, a.K, true, a.epilogue)) return CS_OK;
   } else {
-    if (a.a_norm_inline && (!inline_norm_shape(a.K) || a.w_fp8 || a.pos)) return CS_OK;
+    if (a.a_norm_inline && (!csgemm::inline_norm_width(a.K) || a.w_fp8 || a.pos)) return CS_OK;
     f = best_form(FORMS, a, &us);
     if (!a.a_norm_inline && us >= fast_us(a.M, a.N, a.K, false, a.epilogue)) return CS_OK;
   }
@@ -104,7 +102,7 @@ int cs_gemm_small(const CsGemmArgs& a, hipStream_t stream, bool* handled) {
 bool cs_qkv_window_attn_few(int64_t windows, int heads, int K) { return K % 128 == 0 && windows * heads <= 256; }
 
 extern "C" int cs_gemm_norm_inline_pays(int32_t M, int32_t N, int32_t K, int32_t window_attn) {
-  if (M < 1 || N < 8 || N % 8 || K < 192 || !inline_norm_shape(K)) return 0;
+  if (M < 1 || N < 8 || N % 8 || K < 192 || !csgemm::inline_norm_width(K)) return 0;
   if (window_attn) return cs_qkv_window_attn_few(M / 64, N / 256, K) ? 1 : 0;
   CsGemmArgs a = {};
   a.M = M;

@@ -137,6 +137,28 @@ def test_attention_work_list_host():
     assert l.cs_attn_work_host(cu.ctypes.data, 3, 128, work.ctypes.data, 2, ctypes.byref(n)) == lib.CS_ERR_TOO_LARGE
 
 
+def _window_attn_args(K: int, windows: int = 2, heads: int = 16) -> lib.CsGemmArgs:
+    """A cs_qkv_window_attn call that is valid but for what the test changes (pointers that nothing follows on the host)."""
+    a = lib.CsGemmArgs()
+    a.A = a.W = a.C = a.bias = 1 << 20
+    a.M, a.N, a.K = 64 * windows, 256 * heads, K
+    a.lda = a.ldw = K
+    a.ldc = 80 * heads
+    return a
+
+
+@pytest.mark.parametrize("K", [1408, 2048, 3456, 1280 + 64, 192])
+def test_window_attn_refuses_inline_norms_of_a_width_they_do_not_have(K):
+    """Inline norms keep eight parts of 160 columns in LDS and exist for K a multiple of 128: any other width is refused
+    before a launch (a ninth part would lie behind the launch's LDS)."""
+    a = _window_attn_args(K)
+    a.a_norm_inline = 1
+    for windows in (2, 64):
+        a.M = 64 * windows
+        assert lib.load().cs_qkv_window_attn(ctypes.byref(a), 1 << 20, 0.1, 16, 80, None) == lib.CS_ERR_UNSUPPORTED
+    assert lib.load().cs_gemm_norm_inline_pays(64, 4096, K, 1) == 0
+
+
 def test_resize_taps_host_matches_the_oracle_bit_for_bit():
     """cs_resize_bicubic_taps_host is host arithmetic (doubles, then 22-bit fixed point): no GPU needed."""
     from oracle import qwen_preprocess as qp
