@@ -290,6 +290,7 @@ extern "C" int cs_gemm(const CsGemmArgs* args, void* stream_) {
     const int64_t t256 = (int64_t)((a.M + 255) / 256) * ((a.N + 255) / 256);
     return t256 < 192 ? launch<128, 128, CS_EPI_BIAS, false, true>(a, stream) : launch<256, 256, CS_EPI_BIAS, false, true>(a, stream);
   }
+  if (a.c_row_sum && !a.c_row_sumsq) return CS_ERR_UNSUPPORTED;   // (no kernel emits the sums alone)
   // Fast path (direct-to-LDS pipeline) when the shape allows it; otherwise the general kernel below.
   {
     bool handled = false;

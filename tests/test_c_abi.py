@@ -159,6 +159,22 @@ def test_window_attn_refuses_inline_norms_of_a_width_they_do_not_have(K):
     assert lib.load().cs_gemm_norm_inline_pays(64, 4096, K, 1) == 0
 
 
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("M", [1, 200, 1450, 8192])
+def test_gemm_refuses_row_sums_it_would_not_write(M, fp8):
+    """c_row_sum needs c_row_sumsq: whatever the row count, a call with the sums alone is refused before a launch."""
+    a = lib.CsGemmArgs()
+    a.A = a.W = a.C = a.residual = a.c_row_sum = 1 << 20
+    a.M, a.N, a.K = M, 1280, 1280
+    a.lda = a.ldw = a.ldc = a.ldr = 1280
+    if fp8:
+        a.w_fp8, a.w_scale = 1, 1 << 20
+    for epilogue in range(6):
+        for byte_plane in (None, 1 << 20) if epilogue == lib.EPI_RESIDUAL else (None,):
+            a.epilogue, a.c_lo = epilogue, byte_plane
+            assert lib.load().cs_gemm(ctypes.byref(a), None) == lib.CS_ERR_UNSUPPORTED, epilogue
+
+
 def test_resize_taps_host_matches_the_oracle_bit_for_bit():
     """cs_resize_bicubic_taps_host is host arithmetic (doubles, then 22-bit fixed point): no GPU needed."""
     from oracle import qwen_preprocess as qp
