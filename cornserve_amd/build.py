@@ -142,6 +142,7 @@ def build_library(force: bool = True, jobs: int = 8) -> Path:
                 todo.append(lambda src=src: _check_source(hipcc, src))
     with ThreadPoolExecutor(max_workers=max(1, min(jobs, len(todo) or 1))) as pool:
         list(pool.map(lambda job: job(), todo))
+    TORCH_LIB_PATH.unlink(missing_ok=True)   # (an older one must not stay beside the new kernel library if its own step fails)
     _run([hipcc, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", str(LIB_PATH), *map(str, objs)])
     _check_no_missing_kernels(LIB_PATH)
     _build_torch_ops()

@@ -12,6 +12,7 @@
 #include <ATen/core/Tensor.h>
 #include <ATen/ops/empty.h>
 #include <c10/hip/HIPStream.h>
+#include <c10/util/Exception.h>
 #include <pybind11/pybind11.h>
 #include <torch/library.h>
 
@@ -356,13 +357,28 @@ void layernorm_(const Tensor& out, const Tensor& x, const Tensor& w, const Tenso
 
 }  // namespace
 
-// (For every backend key, as the operators that cornserve_amd/ops.py implements: the checks above turn host tensors away.)
-TORCH_LIBRARY_IMPL(cornserve_amd, CompositeExplicitAutograd, m) {
-  m.impl("gemm", gemm);
-  m.impl("gemm_", gemm_);
-  m.impl("qkv_window_attn_", qkv_window_attn_);
-  m.impl("attn_varlen_", attn_varlen_);
-  m.impl("rope_qk_", rope_qk_);
-  m.impl("rmsnorm_", rmsnorm_);
-  m.impl("layernorm_", layernorm_);
+// The layout of CsGemmArgs is compiled in here as well as in the kernel library: lib.py compares the versions before it has
+// the operators registered.
+extern "C" int cs_torch_ops_abi_version(void) { return CS_ABI_VERSION; }
+
+// Registers the implementations, once.  (For every backend key, as the operators that cornserve_amd/ops.py implements: the
+// checks above turn host tensors away.)  While nothing was built yet, ops.py has put implementations in their place that
+// come here at their first call; the dispatcher's remark that these are now overridden is no news.
+extern "C" void cs_torch_ops_register(void) {
+  struct : c10::WarningHandler {
+    void process(const c10::Warning&) override {}
+  } quiet;
+  c10::WarningUtils::WarningHandlerGuard guard(&quiet);
+  static torch::Library* const library = [] {
+    auto* m = new torch::Library(torch::Library::IMPL, "cornserve_amd", c10::DispatchKey::CompositeExplicitAutograd, __FILE__, __LINE__);
+    m->impl("gemm", gemm);
+    m->impl("gemm_", gemm_);
+    m->impl("qkv_window_attn_", qkv_window_attn_);
+    m->impl("attn_varlen_", attn_varlen_);
+    m->impl("rope_qk_", rope_qk_);
+    m->impl("rmsnorm_", rmsnorm_);
+    m->impl("layernorm_", layernorm_);
+    return m;
+  }();
+  (void)library;   // (for the life of the process)
 }

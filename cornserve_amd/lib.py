@@ -152,13 +152,18 @@ def load() -> ctypes.CDLL:
 
 
 def load_operators() -> None:
-    """Load the native implementations of the operators (csrc/torch_ops.cpp), whose schemas cornserve_amd.ops defines.
-    They may be missing while nothing is built yet; an operator without its implementation raises when it is called."""
-    if LIB_PATH.exists() and TORCH_LIB_PATH.exists():
-        load()
-        import torch
-
-        torch.ops.load_library(str(TORCH_LIB_PATH))
+    """Register the native implementations of the operators (csrc/torch_ops.cpp), whose schemas cornserve_amd.ops defines."""
+    load()
+    if not TORCH_LIB_PATH.exists():
+        raise KernelLibraryError(f"{TORCH_LIB_PATH} not found: build it with `python -m cornserve_amd.build` (hipcc, g++)")
+    try:
+        native = ctypes.CDLL(str(TORCH_LIB_PATH))
+        got = native.cs_torch_ops_abi_version()
+    except (OSError, AttributeError) as e:
+        raise KernelLibraryError(f"{TORCH_LIB_PATH} does not load; rebuild it (`python -m cornserve_amd.build`): {e}") from e
+    if got != ABI_VERSION:   # it hands CsGemmArgs of its own version to the kernel library
+        raise KernelLibraryError(f"ABI version mismatch: operator library {got}, binding {ABI_VERSION}; rebuild")
+    native.cs_torch_ops_register()
 
 
 def check(status: int, what: str) -> None:

@@ -811,7 +811,25 @@ for _name, (_schema, _impl) in _OPERATORS.items():
     if _impl is not None:
         _LIBRARY.impl(_name, _impl, "CompositeExplicitAutograd")
     torch.library.register_fake(f"cornserve_amd::{_name}", _fake_gemm if _name == "gemm" else _fake_nothing, lib=_LIBRARY)
-_l.load_operators()
+
+
+def _load_and_call(name: str):
+    """Stands in for a native implementation: the call loads the libraries (KernelLibraryError while they are missing or
+    stale) and goes to the implementation that is then registered."""
+
+    def call(*args, **kwargs):
+        _l.load_operators()
+        return getattr(torch.ops.cornserve_amd, name).default(*args, **kwargs)
+
+    return call
+
+
+try:
+    _l.load_operators()
+except _l.KernelLibraryError:   # (a package that is not built can be imported, and built by the importing process)
+    for _name, (_schema, _impl) in _OPERATORS.items():
+        if _impl is None:
+            _LIBRARY.impl(_name, _load_and_call(_name), "CompositeExplicitAutograd")
 
 _gemm_op = torch.ops.cornserve_amd.gemm_.default     # (the overloads themselves: a packet looks its overload up per call)
 _qkv_window_attn_op = torch.ops.cornserve_amd.qkv_window_attn_.default

@@ -3,6 +3,8 @@
 import ctypes
 import json
 import re
+import subprocess
+import sys
 from pathlib import Path
 
 import numpy as np
@@ -193,6 +195,51 @@ def test_resize_taps_host_matches_the_oracle_bit_for_bit():
     b = np.zeros((5, 2), dtype=np.int32)
     assert dll.cs_resize_bicubic_taps_host(10, 5, b.ctypes.data, small.ctypes.data, 4, ctypes.byref(k)) == lib.CS_ERR_INVALID_ARG
     assert dll.cs_resize_u8_pass(None, 1, 4, 4, 3, None, None, 5, None, None) == lib.CS_ERR_INVALID_ARG
+
+
+_LATE_BUILD = """
+import sys
+from pathlib import Path
+import torch
+from cornserve_amd import lib
+built, built_torch, version = lib.LIB_PATH, lib.TORCH_LIB_PATH, lib.ABI_VERSION
+lib.LIB_PATH, lib.TORCH_LIB_PATH = Path("/nonexistent/k.so"), Path("/nonexistent/t.so")
+from cornserve_amd import ops
+a = torch.zeros((4, 8), dtype=torch.bfloat16)
+f, work = a.float(), torch.zeros((1, 4), dtype=torch.int32)
+calls = [lambda: ops.gemm(a, a), lambda: ops.gemm(a, a, out=a), lambda: ops.rmsnorm(a, a[0], 1e-6),
+         lambda: ops.layernorm(a, a[0], a[0], 1e-6), lambda: ops.rope_qk_(a, f, 1, 4),
+         lambda: ops.attn_varlen(a, a, a, ops.AttnPlan(work, 1, 4), 1, 8, 1.0), lambda: ops.qkv_window_attn(a, a, a[0], f, 1, 1.0),
+         lambda: torch.ops.cornserve_amd.rmsnorm_(a, a, a[0], 1e-6, False)]
+
+def all_raise(kind, words):
+    for n, call in enumerate(calls):
+        try:
+            call()
+        except kind as e:
+            assert any(w in str(e) for w in words), (n, str(e))
+        else:
+            sys.exit(f"call {n} did not raise {kind}")
+
+all_raise(lib.KernelLibraryError, ["python -m cornserve_amd.build"])        # nothing built
+lib.LIB_PATH = built
+all_raise(lib.KernelLibraryError, ["python -m cornserve_amd.build"])        # the kernel library alone
+lib.TORCH_LIB_PATH = Path(__import__("os").devnull)
+all_raise(lib.KernelLibraryError, ["rebuild"])                              # not a library
+lib.TORCH_LIB_PATH, lib.ABI_VERSION = built_torch, version + 1
+all_raise(lib.KernelLibraryError, ["mismatch"])                             # of another version
+lib.ABI_VERSION = version
+all_raise(ValueError, ["device tensor", "2-D"])                             # built after the import: loaded by the call
+print("late build ok")
+"""
+
+
+def test_a_missing_or_late_library_is_reported_and_loaded_by_the_call():
+    """Importing the operators needs no library; a call names the build command while one is missing, refuses one of another
+    version, and loads what was built after the import."""
+    run = subprocess.run([sys.executable, "-c", _LATE_BUILD], cwd=ROOT, capture_output=True, text=True, timeout=100)
+    assert run.returncode == 0 and "late build ok" in run.stdout, run.stdout + run.stderr
+    assert "verrid" not in run.stderr, run.stderr
 
 
 def test_native_operators_refuse_what_their_kernels_cannot_take():
