@@ -16,7 +16,9 @@
 #include <pybind11/pybind11.h>
 #include <torch/library.h>
 
+#include <set>
 #include <sstream>
+#include <string>
 
 #include "cornserve_amd.h"
 
@@ -46,13 +48,26 @@ void check_status(int status, const char* what) {
   throw pybind11::error_already_set();
 }
 
-const char* dtype_name(at::ScalarType dt) {
-  return dt == at::kBFloat16 ? "torch.bfloat16" : dt == at::kFloat ? "torch.float32" : dt == at::kInt ? "torch.int32" : "torch.uint8";
+// What Python prints for a dtype, a shape and a set of devices
+std::string py(at::ScalarType dt) { return "torch." + c10::getDtypeNames(dt).first; }
+
+std::string py(at::IntArrayRef sizes) {
+  std::ostringstream s;
+  s << "(";
+  for (size_t i = 0; i < sizes.size(); ++i) s << (i ? ", " : "") << sizes[i];
+  s << (sizes.size() == 1 ? ",)" : ")");
+  return s.str();
+}
+
+std::string py(const std::set<std::string>& devices) {
+  std::string s;
+  for (const std::string& d : devices) s += (s.empty() ? "['" : ", '") + d + "'";
+  return s + "]";
 }
 
 void require(const Tensor& t, at::ScalarType dt, const char* name) {
   TORCH_CHECK_VALUE(t.is_cuda(), name, " must be a device tensor");
-  TORCH_CHECK_VALUE(t.scalar_type() == dt, name, " must be ", dtype_name(dt), ", got ", t.scalar_type());
+  TORCH_CHECK_VALUE(t.scalar_type() == dt, name, " must be ", py(dt), ", got ", py(t.scalar_type()));
   TORCH_CHECK_VALUE(t.dim() < 1 || t.stride(-1) == 1, name, " must be contiguous in its last dimension");
 }
 
@@ -71,10 +86,14 @@ void require_sums(const Tensor* t, int64_t rows, const char* name) {
 // A contiguous vector of exactly n elements
 bool is_vector(const Tensor& t, int64_t n) { return t.dim() == 1 && t.size(0) == n && t.is_contiguous(); }
 
-void one_device(const Tensor& first, std::initializer_list<const Tensor*> others, const char* op) {
-  for (const Tensor* t : others) {
-    TORCH_CHECK_VALUE(!t || t->device() == first.device(), op, " operands live on different devices: ", first.device(), ", ",
-                      t ? t->device() : first.device());
+void one_device(std::initializer_list<const Tensor*> operands, const char* op) {
+  const Tensor& first = **operands.begin();
+  for (const Tensor* t : operands) {
+    if (!t || t->device() == first.device()) continue;
+    std::set<std::string> on;
+    for (const Tensor* o : operands)
+      if (o) on.insert(o->device().str());
+    TORCH_CHECK_VALUE(false, op, " operands live on different devices: ", py(on));
   }
 }
 
@@ -146,20 +165,20 @@ void gemm_(const Tensor& out, const Tensor& a, const Tensor& w, const OptTensor&
   const int64_t n_out = epilogue == CS_EPI_SWIGLU ? N / 2 : N;
   require(out, at::kBFloat16, "out");
   TORCH_CHECK_VALUE(out.dim() == 2 && out.size(1) >= n_out && (c_rows || out.size(0) >= M), "out must be bf16 [>=", M, ", >=", n_out,
-                    "], got ", out.sizes());
+                    "], got ", py(out.sizes()));
   if (bias) {
     require(*bias, at::kBFloat16, "bias");
-    TORCH_CHECK_VALUE(bias->dim() == 1 && bias->size(0) >= N, "bias must be bf16 [", N, "], got ", bias->sizes());
+    TORCH_CHECK_VALUE(bias->dim() == 1 && bias->size(0) >= N, "bias must be bf16 [", N, "], got ", py(bias->sizes()));
   }
   TORCH_CHECK_VALUE(epilogue != CS_EPI_RESIDUAL || residual, "EPI_RESIDUAL needs `residual`");
   if (residual) {
     require(*residual, at::kBFloat16, "residual");
     TORCH_CHECK_VALUE(residual->dim() == 2 && residual->size(0) >= M && residual->size(1) >= N, "residual must be bf16 [>=", M, ", >=", N,
-                      "], got ", residual->sizes());
+                      "], got ", py(residual->sizes()));
   }
   if (pos) {
     require(*pos, at::kBFloat16, "pos");
-    TORCH_CHECK_VALUE(pos->dim() == 2 && pos->size(0) >= 1 && pos->size(1) >= N, "pos must be bf16 [period, >=", N, "], got ", pos->sizes());
+    TORCH_CHECK_VALUE(pos->dim() == 2 && pos->size(0) >= 1 && pos->size(1) >= N, "pos must be bf16 [period, >=", N, "], got ", py(pos->sizes()));
   }
   if (w_scale) {
     require(*w_scale, at::kFloat, "w_scale");
@@ -176,7 +195,7 @@ void gemm_(const Tensor& out, const Tensor& a, const Tensor& w, const OptTensor&
                         "residual_lo must have the shape and strides of residual");
     }
   }
-  one_device(a, {&w, &out, bias, residual, pos, w_scale, a_rows, c_rows, residual_lo, out_lo}, "gemm");
+  one_device({&a, &w, &out, bias, residual, pos, w_scale, a_rows, c_rows, residual_lo, out_lo}, "gemm");
   require_sums(a_row_sumsq, M, "a_row_sumsq");
   require_sums(c_row_sumsq, M, "c_row_sumsq");
   require_sums(a_row_sum, M, "a_row_sum");
@@ -244,7 +263,7 @@ void qkv_window_attn_(const Tensor& out, const Tensor& x, const Tensor& w_packed
   require(b_packed, at::kBFloat16, "b_packed");
   require(cos_sin, at::kFloat, "cos_sin");
   TORCH_CHECK_VALUE(heads >= 1 && w_packed.size(0) == w_rows && w_packed.size(1) == K, "w_packed must be [", heads, "*", WATTN_TILE_ROWS,
-                    ", ", K, "], got ", w_packed.sizes());
+                    ", ", K, "], got ", py(w_packed.sizes()));
   TORCH_CHECK_VALUE(is_vector(b_packed, w_rows), "b_packed must be a contiguous [", w_rows, "] tensor");
   CsGemmArgs args = {};
   if (!win_start) {
@@ -261,9 +280,9 @@ void qkv_window_attn_(const Tensor& out, const Tensor& x, const Tensor& w_packed
   }
   TORCH_CHECK_VALUE(cos_sin.dim() == 2 && cos_sin.size(0) == M && cos_sin.size(1) == d && cos_sin.is_contiguous(),
                     "cos_sin must be a contiguous fp32 [", M, ", ", d, "] table");
-  TORCH_CHECK_VALUE(out.size(0) >= M && out.size(1) >= heads * d, "out must be bf16 [>=", M, ", >=", heads * d, "], got ", out.sizes());
+  TORCH_CHECK_VALUE(out.size(0) >= M && out.size(1) >= heads * d, "out must be bf16 [>=", M, ", >=", heads * d, "], got ", py(out.sizes()));
   require_sums(a_row_sumsq, M, "a_row_sumsq");
-  one_device(x, {&out, &w_packed, &b_packed, &cos_sin, a_row_sumsq, win_start, w_scale}, "qkv_window_attn");
+  one_device({&x, &out, &w_packed, &b_packed, &cos_sin, a_row_sumsq, win_start, w_scale}, "qkv_window_attn");
   args.A = x.data_ptr();
   args.lda = x.stride(0);
   args.W = w_packed.data_ptr();

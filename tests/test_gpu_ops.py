@@ -389,6 +389,40 @@ def test_kernels_are_registered_torch_operators(ops, dev):
         assert hasattr(torch.ops.cornserve_amd, name), name
 
 
+def test_native_operators_name_dtypes_shapes_and_devices_as_python_does(ops, dev):
+    """The operators of the blocks are implemented in C++; what they refuse, they refuse with the words of the others."""
+    bf = lambda *s: torch.zeros(s, dtype=torch.bfloat16, device=dev)  # noqa: E731
+    f32 = lambda *s: torch.zeros(s, dtype=torch.float32, device=dev)  # noqa: E731
+    a, w, h = bf(8, 64), bf(16, 64), torch.zeros((8, 64), dtype=torch.float16, device=dev)
+    q = torch.zeros((16, 64), dtype=torch.uint8)
+    wp, bp, cos = bf(256, 192), bf(256), f32(64, 80)
+    for call, message in (
+        (lambda: ops.gemm(f32(8, 64), w), "a must be torch.bfloat16, got torch.float32"),
+        (lambda: ops.gemm(a, w, a_rows=torch.zeros(4, dtype=torch.int64, device=dev)), "a_rows must be torch.int32, got torch.int64"),
+        (lambda: ops.gemm(a, q, w_scale=f32(16)), "gemm operands live on different devices: ['cpu', 'cuda:0']"),
+        (lambda: ops.gemm(a, w, out=bf(8, 8)), "out must be bf16 [>=8, >=16], got (8, 8)"),
+        (lambda: ops.gemm(a, w, bf(8)), "bias must be bf16 [16], got (8,)"),
+        (lambda: ops.gemm(a, w, epilogue=ops.EPI_RESIDUAL, residual=bf(4, 16)), "residual must be bf16 [>=8, >=16], got (4, 16)"),
+        (lambda: ops.gemm(a, w, pos=bf(16)), "pos must be bf16 [period, >=16], got (16,)"),
+        (lambda: ops.gemm(a, w, epilogue=ops.EPI_RESIDUAL, residual=bf(8, 16), out=bf(8, 16), out_lo=bf(8, 16)),
+         "out_lo must be torch.uint8, got torch.bfloat16"),
+        (lambda: ops.gemm(a, bf(16, 32)), "w has 32 columns, need at least K=64"),
+        (lambda: ops.qkv_window_attn(bf(64, 192), bf(128, 192), bp, cos, 1, 0.1), "w_packed must be [1*256, 192], got (128, 192)"),
+        (lambda: ops.qkv_window_attn(bf(64, 192), wp, bp, cos, 1, 0.1, out=bf(64, 72)), "out must be bf16 [>=64, >=80], got (64, 72)"),
+        (lambda: ops.qkv_window_attn(bf(64, 192), wp.cpu().to(torch.uint8).to(dev), bp, cos, 1, 0.1),
+         "w_packed must be torch.bfloat16, got torch.uint8"),
+        (lambda: ops.attn_varlen(h, h, h, ops.AttnPlan(torch.zeros((1, 4), dtype=torch.int32, device=dev), 1, 8), 1, 64, 1.0),
+         "q must be torch.bfloat16, got torch.float16"),
+        (lambda: ops.rope_qk_(bf(8, 64), torch.zeros((8, 64), dtype=torch.float64, device=dev), 1, 64),
+         "cos_sin must be torch.float32, got torch.float64"),
+        (lambda: ops.rmsnorm(a, f32(64), 1e-6), "w must be torch.bfloat16, got torch.float32"),
+        (lambda: ops.layernorm(a, bf(64), bf(32), 1e-6), "b must be bf16 [64] on x's device"),
+    ):
+        with pytest.raises(ValueError) as e:
+            call()
+        assert str(e.value) == message
+
+
 def _epilogue_ref(ops, epi, base, res):
     """fp32 reference of one fused epilogue on `base` = A.W^T + bias in fp32.  The residual epilogue rounds the linear
     layer's output before the addition (the reference's two bf16 operations); an activation takes the fp32 sum."""
