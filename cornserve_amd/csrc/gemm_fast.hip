@@ -12,6 +12,7 @@ int cs_gemm_fast_tile_128x192(const CsGemmArgs& a, hipStream_t stream);
 int cs_gemm_fast_tile_256x128(const CsGemmArgs& a, hipStream_t stream);
 // The few-row kernel (gemm_small.hip).
 int cs_gemm_small(const CsGemmArgs& a, hipStream_t stream, bool* handled);
+int cs_gemm_small_workgroups(const CsGemmArgs& a);
 
 namespace {
 
@@ -24,20 +25,28 @@ double rounds_cost(int M, int N, int bm, int bn) {
   return (double)rounds * bm * bn / (256.0 * 256.0);
 }
 
+// Whether the direct-to-LDS kernels (the big tiles and the few-row kernel) take a problem.
+bool direct_shape(const CsGemmArgs& a) {
+  if (a.M < 1 || a.N < 8) return false;
+  if (a.w_fp8 ? (!a.w_scale || a.pos) : (a.w_scale != nullptr)) return false;
+  if (a.K % BK || a.K < 3 * BK) return false;  // the ring pipeline is written for at least three K tiles
+  if (a.N % 8 || a.ldc % 8 || ((uintptr_t)a.C & 15)) return false;  // 16-byte output stores
+  if (a.pos && a.epilogue != CS_EPI_BIAS) return false;  // the position addend only pairs with the plain epilogue here
+  if (a.a_rows) return false;  // gathered A rows can lie anywhere: the general kernel keeps 64-bit pointers
+  // per-lane source offsets are 32-bit byte offsets from the matrix bases
+  return (int64_t)a.M * a.lda * 2 < (int64_t)UINT32_MAX && (int64_t)a.N * a.ldw * (a.w_fp8 ? 1 : 2) < (int64_t)UINT32_MAX;
+}
+
 }  // namespace
+
+extern "C" int cs_gemm_few_row_workgroups(const CsGemmArgs* args) {
+  return args && !args->conv_patch && direct_shape(*args) ? cs_gemm_small_workgroups(*args) : 0;
+}
 
 // Called by cs_gemm after argument validation.  Sets *handled when this path took the problem.
 int cs_gemm_fast(const CsGemmArgs& a, hipStream_t stream, bool* handled) {
   *handled = false;
-  if (a.M < 1 || a.N < 8) return CS_OK;
-  if (a.w_fp8 ? (!a.w_scale || a.pos) : (a.w_scale != nullptr)) return CS_OK;
-  if (a.K % BK || a.K < 3 * BK) return CS_OK;  // the ring pipeline is written for at least three K tiles
-  if (a.N % 8 || a.ldc % 8 || ((uintptr_t)a.C & 15)) return CS_OK;  // 16-byte output stores
-  if (a.pos && a.epilogue != CS_EPI_BIAS) return CS_OK;  // the position addend only pairs with the plain epilogue here
-  if (a.a_rows) return CS_OK;  // gathered A rows can lie anywhere: the general kernel keeps 64-bit pointers
-  // per-lane source offsets are 32-bit byte offsets from the matrix bases
-  if ((int64_t)a.M * a.lda * 2 >= (int64_t)UINT32_MAX || (int64_t)a.N * a.ldw * (a.w_fp8 ? 1 : 2) >= (int64_t)UINT32_MAX)
-    return CS_OK;
+  if (!direct_shape(a)) return CS_OK;
   // Few rows: tiles small enough to give most compute units one.
   {
     const int st = cs_gemm_small(a, stream, handled);

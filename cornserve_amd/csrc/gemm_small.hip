@@ -50,15 +50,22 @@ double small_us(const Form& f, int M, int N, int K, bool norm) {
   return r * (f.fixed_us - 2.0 + stages * f.stage_us * (norm ? 1.15 : 1.0)) + 2.0;
 }
 
-double fast_us(int M, int N, int K, bool sums, int epilogue) {
+double fast_us(int M, int N, int K, bool sums, int epilogue, bool split) {
   const double stages = K / 128.0;
   auto us = [&](const FastForm& f) { return f.fixed_us + rounds(M, N, f.bm, f.bn) * stages * f.stage_us; };
   const bool few = (int64_t)((M + 255) / 256) * ((N + 159) / 160) <= 128;   // (the rule of gemm_fast.hip)
-  double t = us(few ? F128x160 : F256x160) + (!few && epilogue == CS_EPI_RESIDUAL ? 11.0 : 0.0);   // (29 us at 4888 x 1280 x 1280)
+  // (a tail tile of the split residual stream: 29 us at 4888 x 1280 x 1280; a bf16 one: 22 us at 4160 .. 5376 x 1152 x 1152)
+  double t = us(few ? F128x160 : F256x160) + (!few && epilogue == CS_EPI_RESIDUAL && split ? 11.0 : 0.0);
   if (!sums) t = us(F256x256) < t ? us(F256x256) : t;
   if (!sums && epilogue == CS_EPI_SWIGLU) t = us(F256x128) < t ? us(F256x128) : t;
   return t;
 }
+
+// A launch of more than two rounds is no few-row launch: the times above are of one round, and five rounds of 64x64 take 33 us
+// (28 without the byte planes) where they promise 30.7 and 256x160 takes 30 (22): 4160 and 4374 rows x 1152 x 1152.  Two rounds
+// of 32x64 hold: 200 rows x 4352 x 1152 12.6 us against 16.0, 288 fp8 rows x 3584 x 5120 31.7 against 93.  (Inline norms have
+// no other kernel.)
+constexpr double MAX_ROUNDS = 2.0;
 
 template <int COUNT>
 const Form* best_form(const Form (&forms)[COUNT], const CsGemmArgs& a, double* us) {
@@ -66,6 +73,7 @@ const Form* best_form(const Form (&forms)[COUNT], const CsGemmArgs& a, double* u
   *us = 0;
   for (const Form& f : forms) {
     if (f.bn == 80 && (a.w_fp8 || a.a_norm_inline || a.pos || !(a.epilogue == CS_EPI_BIAS || (a.epilogue == CS_EPI_RESIDUAL && a.c_lo)))) continue;
+    if (!a.a_norm_inline && rounds(a.M, a.N, f.bm, f.bn) > MAX_ROUNDS) continue;
     const double t = small_us(f, a.M, a.N, a.K, a.a_norm_inline);
     if (!best || t < *us) {
       best = &f;
@@ -75,26 +83,36 @@ const Form* best_form(const Form (&forms)[COUNT], const CsGemmArgs& a, double* u
   return best;
 }
 
+// The form of a launch, nullptr if it is not a few-row one.
+const Form* few_row_form(const CsGemmArgs& a) {
+  if (a.K % 128 || a.a_row_sumsq || a.a_row_sum || a.conv_patch) return nullptr;
+  double us;
+  const Form* f;
+  if (a.c_row_sumsq) {   // (other producers of row sums: the big tiles' 160-column forms)
+    if (a.w_fp8 || a.epilogue != CS_EPI_RESIDUAL || !a.c_lo || a.N > 160 * CS_SUMSQ_PARTS) return nullptr;
+    f = best_form(SUMS_FORMS, a, &us);
+  } else {
+    if (a.a_norm_inline && (!csgemm::inline_norm_width(a.K) || a.w_fp8 || a.pos)) return nullptr;
+    f = best_form(FORMS, a, &us);
+    if (a.a_norm_inline) return f;
+  }
+  return f && us < fast_us(a.M, a.N, a.K, a.c_row_sumsq != nullptr, a.epilogue, a.c_lo != nullptr) ? f : nullptr;
+}
+
 }  // namespace
 
 // Called by cs_gemm for a shape that the direct-to-LDS kernels take (see cs_gemm_fast).  Sets *handled when the launch goes
 // to the few-row kernel.
 int cs_gemm_small(const CsGemmArgs& a, hipStream_t stream, bool* handled) {
-  *handled = false;
-  if (a.K % 128 || a.a_row_sumsq || a.a_row_sum || a.conv_patch) return CS_OK;
-  double us;
-  const Form* f;
-  if (a.c_row_sumsq) {   // (other producers of row sums: the big tiles' 160-column forms)
-    if (a.w_fp8 || a.epilogue != CS_EPI_RESIDUAL || !a.c_lo || a.N > 160 * CS_SUMSQ_PARTS) return CS_OK;
-    f = best_form(SUMS_FORMS, a, &us);
-    if (us >= fast_us(a.M, a.N, a.K, true, a.epilogue)) return CS_OK;
-  } else {
-    if (a.a_norm_inline && (!csgemm::inline_norm_width(a.K) || a.w_fp8 || a.pos)) return CS_OK;
-    f = best_form(FORMS, a, &us);
-    if (!a.a_norm_inline && us >= fast_us(a.M, a.N, a.K, false, a.epilogue)) return CS_OK;
-  }
-  *handled = true;
-  return f->run(a, stream);
+  const Form* f = few_row_form(a);
+  *handled = f != nullptr;
+  return f ? f->run(a, stream) : CS_OK;
+}
+
+// Workgroups of such a launch, 0 if the big tiles take it.
+int cs_gemm_small_workgroups(const CsGemmArgs& a) {
+  const Form* f = few_row_form(a);
+  return f ? ((a.M + f->bm - 1) / f->bm) * ((a.N + f->bn - 1) / f->bn) : 0;
 }
 
 // One workgroup per window and head while the chip holds them all at once: 22 to 25 us up to 16 windows of 16 heads, where
@@ -111,5 +129,5 @@ extern "C" int cs_gemm_norm_inline_pays(int32_t M, int32_t N, int32_t K, int32_t
   a.a_norm_inline = 1;
   double us;
   best_form(FORMS, a, &us);
-  return us < fast_us(M, N, K, false, CS_EPI_SWIGLU) ? 1 : 0;
+  return us < fast_us(M, N, K, false, CS_EPI_SWIGLU, false) ? 1 : 0;
 }

@@ -18,7 +18,7 @@ CS_ERR_INVALID_ARG = 1
 CS_ERR_UNSUPPORTED = 2
 CS_ERR_LAUNCH = 3
 CS_ERR_TOO_LARGE = 4
-ABI_VERSION = 9
+ABI_VERSION = 10
 
 EPI_BIAS, EPI_RESIDUAL, EPI_SWIGLU, EPI_GELU_ERF, EPI_GELU_TANH, EPI_QUICK_GELU = range(6)
 
@@ -76,6 +76,7 @@ class CsGemmArgs(ctypes.Structure):
 _SIGNATURES: dict[str, list] = {
     "cs_abi_version": [],
     "cs_gemm": [POINTER(CsGemmArgs), c_void_p],
+    "cs_gemm_few_row_workgroups": [POINTER(CsGemmArgs)],
     "cs_gemm_norm_inline_pays": [c_int32, c_int32, c_int32, c_int32],
     "cs_gemm_rmsnorm_noalloc": [POINTER(CsGemmArgs), c_void_p],
     "cs_qkv_window_attn": [POINTER(CsGemmArgs), c_void_p, c_float, c_int32, c_int32, c_void_p],

@@ -36,7 +36,7 @@ extern "C" {
 #define CS_ERR_TOO_LARGE 4
 
 /* ABI version of this header; cs_abi_version() returns the value the library was built with. */
-#define CS_ABI_VERSION 9
+#define CS_ABI_VERSION 10
 int cs_abi_version(void);
 
 /* ------------------------------------------------------------------------------------------------
@@ -152,6 +152,10 @@ typedef struct CsGemmArgs {
 
 /* Constraints: K % 8 == 0 (16 with fp8), lda/ldw % 8 == 0, N % 4 == 0, A and W 16-byte aligned. */
 int cs_gemm(const CsGemmArgs* args, void* stream);
+
+/* Host routine: how many workgroups cs_gemm starts for these arguments if the few-row kernel takes them, 0 if another kernel
+ * does.  Nothing is read through the pointers.                                                                       */
+int cs_gemm_few_row_workgroups(const CsGemmArgs* args);
 
 /* Host routine: 1 if a folded-norm launch of M rows, N weight rows and width K is faster with a_norm_inline than with row
  * sums read from arrays (few rows), 0 if not or if the shape has no inline form.  window_attn = 1: the same question for

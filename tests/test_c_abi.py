@@ -149,6 +149,38 @@ def _window_attn_args(K: int, windows: int = 2, heads: int = 16) -> lib.CsGemmAr
     return a
 
 
+def _gemm_args(M: int, N: int, K: int, *, epilogue: int = lib.EPI_BIAS, split: bool = False) -> lib.CsGemmArgs:
+    a = lib.CsGemmArgs()
+    a.A = a.W = a.C = 1 << 20
+    a.M, a.N, a.K = M, N, K
+    a.lda = a.ldw = K
+    a.ldc = N
+    a.epilogue = epilogue
+    if epilogue == lib.EPI_RESIDUAL:
+        a.residual, a.ldr = 1 << 20, N
+    if split:
+        a.residual_lo = a.c_lo = 1 << 20
+    return a
+
+
+def test_few_row_kernel_takes_launches_of_at_most_two_rounds():
+    """The few-row kernel's times hold for launches of one or two rounds of 256 workgroups: 4097 to 4480 rows x 1152 x 1152,
+    which it would run in five, belong to the 256-row tiles."""
+    groups = lambda *a, **kw: lib.load().cs_gemm_few_row_workgroups(ctypes.byref(_gemm_args(*a, **kw)))  # noqa: E731
+    for M in (4100, 4160, 4374, 4480):
+        for split in (False, True):
+            assert groups(M, 1152, 1152, epilogue=lib.EPI_RESIDUAL, split=split) == 0
+    for N in (1152, 1280, 3456, 3840, 4352, 5120, 6912):
+        for K in (256, 1152, 1280, 3456, 4352, 5120):
+            for epilogue, split in ((lib.EPI_BIAS, False), (lib.EPI_RESIDUAL, False), (lib.EPI_RESIDUAL, True)):
+                for M in (1, 96, 250, 500, 1000, 1450, 2196, 3000, 4200, 6000, 9000, 20000):
+                    assert groups(M, N, K, epilogue=epilogue, split=split) <= 512
+    assert groups(96, 1280, 1280) == 3 * 40                                          # 32x32 tiles
+    assert groups(1000, 1280, 1280, epilogue=lib.EPI_RESIDUAL, split=True) == 16 * 16    # 64x80
+    assert groups(200, 4352, 1152, epilogue=lib.EPI_GELU_TANH) == 7 * 68             # 32x64, two rounds
+    assert groups(96, 1280, 1216) == groups(8192, 1280, 1280) == 0                   # K % 128; many rows
+
+
 @pytest.mark.parametrize("K", [1408, 2048, 3456, 1280 + 64, 192])
 def test_window_attn_refuses_inline_norms_of_a_width_they_do_not_have(K):
     """Inline norms keep eight parts of 160 columns in LDS and exist for K a multiple of 128: any other width is refused
