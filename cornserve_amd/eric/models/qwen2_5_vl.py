@@ -223,15 +223,22 @@ class QwenVisionBase(EricModel):
     # Row count of the per-block buffers: a whole number of 256-row tiles (the tallest form; 128-row tiles divide it) for
     # batches that the big tiles run.  A tile with rows past the end cannot take the guard-free epilogue with its residual
     # piece through the LDS ring, and a launch lasts as long as its slowest tile: 1280 columns at K = 1280 and 3456, 7900
-    # rows 39 and 68 us, 7936 rows 32 and 60; 20400 rows 97 and 182 us, 20480 rows 90 and 174.  The matrix cores work on
-    # the rows past the end either way; rows are independent of each other, so nothing else changes.  Whole passes: 5076
-    # rows 9.19 -> 8.65 ms, 8068 rows 10.5 -> 10.1, 3996 rows (fp8 weights) 7.08 -> 6.98.  Batches of fewer rows partly run
-    # in the few-row kernel's smaller tiles, where whole tiles are more work: 2196 rows (Qwen2-VL) 5.90 -> 6.09 ms.
-    row_tile, row_tile_min = 256, 3585
+    # rows 39 and 68 us, 7936 rows 32 and 60; 20400 rows 97 and 182 us, 20480 rows 90 and 174.  Rows are independent of
+    # each other, so nothing else changes.  From 3841 patches on, because from there on the filled launches of 1280 columns
+    # are whole rounds of 256 workgroups (4096 rows) or 256-row tiles (more); and for at most 192 rows of filling: those
+    # rows are worked on as well, and read and written, where the rows past the end of a ragged tile repeat its last one.
+    # Whole passes, exact -> filled, one process alternating, Qwen2.5-VL bf16 | fp8 | Qwen2-VL in ms: 4092 patches 7.34 ->
+    # 7.04 | 7.31 -> 7.01 | 10.18 -> 9.99; 4488 8.57 -> 8.26 | 9.16 -> 8.87 | 14.40 -> 14.27; 5776 9.82 -> 9.46 | 11.03 ->
+    # 10.71 | 17.54 -> 17.22; 7396 11.47 -> 10.84 | 12.63 -> 12.11 | 21.86 -> 21.35; 3968, 8280 and 9800 within 0.5 % or
+    # 1 % faster.  On the other side of the two lines: 3596 patches 5.98 -> 6.14 | 6.78 -> 6.82 | 9.27 -> 9.52; 3720 6.07 ->
+    # 6.16 | 6.83 -> 6.84 | 9.39 -> 9.66; 3844 (252 rows of filling) 6.06 -> 6.22 | 6.65 -> 6.72 | 9.90 -> 9.79; 4624 (240)
+    # 8.70 -> 8.83 | 9.90 -> 9.95 | 14.58 -> 14.70.  (2400 to 3072 patches gain up to 4 % with Qwen2.5-VL where the filling is
+    # short, and lose 2 % with Qwen2-VL.)
+    row_tile, row_tile_min, row_tile_fill = 256, 3841, 192
 
     def _whole_tile_rows(self, rows: int, max_rows: int) -> int:
         whole = -(-rows // self.row_tile) * self.row_tile
-        return whole if rows >= self.row_tile_min and whole <= max_rows else rows
+        return whole if rows >= self.row_tile_min and whole - rows <= self.row_tile_fill and whole <= max_rows else rows
 
     def _row_buffer(self, rows: int, used: int, cols: int) -> torch.Tensor:
         """bf16 [rows, cols] whose rows from `used` on are zero."""

@@ -492,3 +492,17 @@ def test_qkv_window_attn_pack_and_unpack_are_inverse():
     assert torch.equal(q2, q) and torch.equal(b2, b) and torch.equal(s2, sc)
     with pytest.raises(ValueError):
         ops.unpack_qkv_window_attn(wp[:-1], bp, heads)
+
+
+def test_rows_are_filled_to_whole_tiles_only_where_that_pays():
+    """Per-block buffers of whole 256-row tiles: from 3841 patches on, with at most 192 rows of filling, within the row
+    limit of the operand offsets; any other batch keeps its count (filling 3600 to 3840 patches cost Qwen2.5-VL and
+    Qwen2-VL 1.5 to 3 % of a pass, 3844 and 4624 patches up to 2.6 %)."""
+    from cornserve_amd.eric.models.qwen2_5_vl import QwenVisionBase
+
+    rows = lambda n, limit=1 << 20: QwenVisionBase._whole_tile_rows(QwenVisionBase, n, limit)  # noqa: E731
+    for n in (1, 96, 1024, 2304, 3024, 3596, 3600, 3720, 3840, 3844, 3903, 4096, 4100, 4624, 8192, 20480):
+        assert rows(n) == n
+    for n, whole in ((3904, 4096), (3996, 4096), (4092, 4096), (4224, 4352), (5076, 5120), (7396, 7424), (27600, 27648)):
+        assert rows(n) == whole and rows(n, whole) == whole
+        assert rows(n, whole - 1) == n
