@@ -8,6 +8,24 @@ namespace csgemm {
 // columns in LDS, and K is walked in steps of 128.
 inline bool inline_norm_width(int K) { return K % 128 == 0 && K <= 160 * CS_SUMSQ_PARTS; }
 
+// Weight-prefetch hints (CsGemmArgs.prefetch) of few-row launches: up to 128 workgroups, on compute units without a tile, read
+// 8 KB a microsecond each from about 4 us after the launch begins.  A launch ends with its last workgroup, so what is read is
+// what fits the launch's own time.  Whole passes without hint -> with this rule (without the 4 us): Qwen2.5-VL 96 patches 1.81 ->
+// 1.80 (1.83) ms, 1280 3.88 -> 3.69 (3.68); Qwen2-VL 64 patches 1.74 -> 1.72 (1.89), 1936 6.06 -> 5.99 (5.99); Qwen3-VL 1280 4.09 ->
+// 3.96 (3.77).  Beyond 192 tiles the few idle compute units cost more than they bring (200 tiles, Qwen2.5-VL 1600 patches: 4.19
+// -> 4.26), as in the big tiles' launches.
+constexpr int HINT_MAX_TILES = 192;
+inline int hint_workgroups(int tiles) { return tiles > HINT_MAX_TILES ? 0 : 256 - tiles < 128 ? 256 - tiles : 128; }
+inline void fit_hint(CsGemmArgs& a, int tiles, double us) {
+  const int64_t room = us > 4.0 ? (int64_t)(hint_workgroups(tiles) * 8192.0 * (us - 4.0)) : 0;
+  if (!a.prefetch || a.prefetch_bytes < 16 || room < 16) {
+    a.prefetch = nullptr;
+    a.prefetch_bytes = 0;
+  } else if (a.prefetch_bytes > room) {
+    a.prefetch_bytes = room;
+  }
+}
+
 constexpr int BK = 64;  // K step (bf16 elements): 128 bytes per tile row = 8 chunks of 16 B
 
 // Byte offset of 16-byte chunk `chunk` of row `row` in a [rows][64] bf16 LDS tile (128-byte rows).

@@ -83,20 +83,39 @@ const Form* best_form(const Form (&forms)[COUNT], const CsGemmArgs& a, double* u
   return best;
 }
 
-// The form of a launch, nullptr if it is not a few-row one.
-const Form* few_row_form(const CsGemmArgs& a) {
+int tiles_of(const Form& f, const CsGemmArgs& a) { return ((a.M + f.bm - 1) / f.bm) * ((a.N + f.bn - 1) / f.bn); }
+
+// Whether a launch has too many tiles to read its hint where the big form would read it.  The launch that the hint is for then
+// finds its weights cold (2700 rows of Qwen2-VL: projection 24 us instead of 17), so such a launch goes to the few-row kernel only
+// if it is 15 % faster there.  Passes with few-row tiles and the hint unread -> with the big form: Qwen2-VL 2700 patches (fc2: 220
+// tiles of 128x128 or 176 of 128x160; 43 and 49 us by the table) 7.51 -> 7.31 ms, 3024 8.17 -> 7.93.  One image of 1024 rows has
+// 256 small tiles that are 30 to 50 % faster, and keeps them.  Not so with row sums, where it goes either way (Qwen2.5-VL 1600
+// patches 4.17 -> 4.14, 1764 4.22 -> 4.34, 1936 4.27 -> 4.13) and the few-row forms stay; nor with fp8 weights, where the big form
+// is slower by more than that (2700 patches 5.78 -> 6.06).  A hint that the big form has no time for either, as that for the
+// merger's 52 MB, would only make its launch longer.
+constexpr double HINT_WORTH = 0.15;
+bool loses_hint(const Form& f, const CsGemmArgs& a, double big_us) {
+  if (!a.prefetch || a.prefetch_bytes < 16 || a.w_fp8 || a.c_row_sumsq || tiles_of(f, a) <= csgemm::HINT_MAX_TILES) return false;
+  const int big_rows = (int64_t)((a.M + 255) / 256) * ((a.N + 159) / 160) <= 128 ? 128 : 256;
+  const int64_t big_tiles = (int64_t)((a.M + big_rows - 1) / big_rows) * ((a.N + 159) / 160);
+  return big_tiles <= csgemm::HINT_MAX_TILES && a.prefetch_bytes <= csgemm::hint_workgroups((int)big_tiles) * 8192.0 * big_us;
+}
+
+// The form of a launch and its time, nullptr if it is not a few-row one.
+const Form* few_row_form(const CsGemmArgs& a, double* us) {
   if (a.K % 128 || a.a_row_sumsq || a.a_row_sum || a.conv_patch) return nullptr;
-  double us;
   const Form* f;
   if (a.c_row_sumsq) {   // (other producers of row sums: the big tiles' 160-column forms)
     if (a.w_fp8 || a.epilogue != CS_EPI_RESIDUAL || !a.c_lo || a.N > 160 * CS_SUMSQ_PARTS) return nullptr;
-    f = best_form(SUMS_FORMS, a, &us);
+    f = best_form(SUMS_FORMS, a, us);
   } else {
     if (a.a_norm_inline && (!csgemm::inline_norm_width(a.K) || a.w_fp8 || a.pos)) return nullptr;
-    f = best_form(FORMS, a, &us);
+    f = best_form(FORMS, a, us);
     if (a.a_norm_inline) return f;
   }
-  return f && us < fast_us(a.M, a.N, a.K, a.c_row_sumsq != nullptr, a.epilogue, a.c_lo != nullptr) ? f : nullptr;
+  if (!f) return nullptr;
+  const double big_us = fast_us(a.M, a.N, a.K, a.c_row_sumsq != nullptr, a.epilogue, a.c_lo != nullptr);
+  return *us < big_us * (loses_hint(*f, a, big_us) ? 1.0 - HINT_WORTH : 1.0) ? f : nullptr;
 }
 
 }  // namespace
@@ -104,15 +123,24 @@ const Form* few_row_form(const CsGemmArgs& a) {
 // Called by cs_gemm for a shape that the direct-to-LDS kernels take (see cs_gemm_fast).  Sets *handled when the launch goes
 // to the few-row kernel.
 int cs_gemm_small(const CsGemmArgs& a, hipStream_t stream, bool* handled) {
-  const Form* f = few_row_form(a);
+  double us;
+  const Form* f = few_row_form(a, &us);
   *handled = f != nullptr;
-  return f ? f->run(a, stream) : CS_OK;
+  if (!f) return CS_OK;
+  CsGemmArgs p = a;
+  csgemm::fit_hint(p, tiles_of(*f, a), us);
+  return f->run(p, stream);
 }
 
 // Workgroups of such a launch, 0 if the big tiles take it.
 int cs_gemm_small_workgroups(const CsGemmArgs& a) {
-  const Form* f = few_row_form(a);
-  return f ? ((a.M + f->bm - 1) / f->bm) * ((a.N + f->bn - 1) / f->bn) : 0;
+  double us;
+  const Form* f = few_row_form(a, &us);
+  if (!f) return 0;
+  const int tiles = tiles_of(*f, a);
+  CsGemmArgs p = a;
+  csgemm::fit_hint(p, tiles, us);
+  return tiles + (p.prefetch ? csgemm::hint_workgroups(tiles) : 0);
 }
 
 // One workgroup per window and head while the chip holds them all at once: 22 to 25 us up to 16 windows of 16 heads, where

@@ -129,15 +129,16 @@ typedef struct CsGemmArgs {
   /* cs_qkv_window_attn only, set by the caller: windows of fewer than 64 rows (see there); NULL / 0 otherwise         */
   const int32_t* attn_win_start;
   int32_t attn_n_win;
-  /* Optional hint for launches that leave compute units idle (at most 192 workgroups of the fast path's tile forms and
-   * of cs_qkv_window_attn): prefetch_bytes bytes at prefetch (16-byte aligned) -- typically the weights of the NEXT
+  /* Optional hint for launches that leave compute units idle (at most 192 tiles of the direct-to-LDS kernels, cs_gemm and
+   * cs_qkv_window_attn alike): prefetch_bytes bytes at prefetch (16-byte aligned) -- typically the weights of the NEXT
    * launch, which no kernel has touched since the previous forward pass -- are read once by up to 128 workgroups
    * started next to the computing ones, so that they sit in the last-level cache when the next launch asks for them
-   * (a few-row launch is bound by operand latency, not by arithmetic).  Results are not affected; the hint is ignored
+   * (such a launch is bound by operand latency, not by arithmetic).  Results are not affected; the hint is ignored
    * by launches that fill the chip and by the general kernel.  NULL / 0: no hint.  A prefetching workgroup moves
-   * about 8 KB per microsecond and the launch ends when its last workgroup does: hint what the idle compute units
-   * (256 minus the launch's tiles, at most 128) can read in the launch's own time -- 9 MB behind a 64-tile launch
-   * of 20 K tiles costs nothing, 18 MB behind a 192-tile one doubles its duration.                                */
+   * about 8 KB per microsecond and the launch ends when its last workgroup does.  The few-row kernel reads of the hint,
+   * from its start, what fits the launch's own time.  The big tiles read all of it: hint what the idle compute units
+   * (256 minus the launch's tiles, at most 128) can read in that time -- 9 MB behind a 64-tile launch of 20 K tiles costs
+   * nothing, 18 MB behind a 192-tile one doubles its duration.                                                        */
   const void* prefetch;
   int64_t prefetch_bytes;
   /* Folded norm without the row-sum arrays: with a_norm_inline = 1 the sums over the rows of A are taken inside the
@@ -153,8 +154,8 @@ typedef struct CsGemmArgs {
 /* Constraints: K % 8 == 0 (16 with fp8), lda/ldw % 8 == 0, N % 4 == 0, A and W 16-byte aligned. */
 int cs_gemm(const CsGemmArgs* args, void* stream);
 
-/* Host routine: how many workgroups cs_gemm starts for these arguments if the few-row kernel takes them, 0 if another kernel
- * does.  Nothing is read through the pointers.                                                                       */
+/* Host routine: how many workgroups cs_gemm starts for these arguments if the few-row kernel takes them (one a tile, and those
+ * that read the prefetch hint), 0 if another kernel does.  Nothing is read through the pointers.                        */
 int cs_gemm_few_row_workgroups(const CsGemmArgs* args);
 
 /* Host routine: 1 if a folded-norm launch of M rows, N weight rows and width K is faster with a_norm_inline than with row

@@ -181,6 +181,30 @@ def test_few_row_kernel_takes_launches_of_at_most_two_rounds():
     assert groups(96, 1280, 1216) == groups(8192, 1280, 1280) == 0                   # K % 128; many rows
 
 
+def test_few_row_launches_read_their_prefetch_hint():
+    """A launch of at most 192 tiles starts workgroups on idle compute units that read the hint: up to 128, none without a
+    hint or time.  Where a few-row form of nearly the big form's time is too full for that and the big form is not, the big
+    form gets the launch."""
+    def groups(M, N, K, nbytes, **kw):
+        a = _gemm_args(M, N, K, **kw)
+        plain = lib.load().cs_gemm_few_row_workgroups(ctypes.byref(a))
+        a.prefetch, a.prefetch_bytes = (1 << 20, nbytes) if nbytes else (None, 0)
+        return plain, lib.load().cs_gemm_few_row_workgroups(ctypes.byref(a)) - plain
+
+    split = {"epilogue": lib.EPI_RESIDUAL, "split": True}
+    assert groups(96, 1280, 1280, 8 << 20, **split) == (120, 128)
+    assert groups(500, 1280, 3456, 10 << 20, **split) == (160, 96)
+    assert groups(1000, 1280, 1280, 8 << 20, **split) == (256, 0)      # one tile for every compute unit
+    assert groups(200, 4352, 1152, 8 << 20, epilogue=lib.EPI_GELU_TANH) == (476, 0)
+    assert groups(40, 320, 256, 8 << 20, **split)[1] == 128 and groups(2400, 1280, 5120, 3 << 20, **split) == (190, 66)
+    for M in (2700, 3024):                                             # 128x128 tiles without a hint, 128x160 with one
+        assert groups(M, 1280, 5120, 3 << 20, **split) == ((M + 127) // 128 * 10, -((M + 127) // 128 * 10))
+    assert groups(3248, 1280, 5120, 3 << 20, **split) == (0, 0)
+    for nbytes in (0, 8):                                              # no hint, none of a whole piece
+        assert groups(96, 1280, 1280, nbytes, **split) == (120, 0)
+        assert groups(2700, 1280, 5120, nbytes, **split) == (220, 0)
+
+
 @pytest.mark.parametrize("K", [1408, 2048, 3456, 1280 + 64, 192])
 def test_window_attn_refuses_inline_norms_of_a_width_they_do_not_have(K):
     """Inline norms keep eight parts of 160 columns in LDS and exist for K a multiple of 128: any other width is refused

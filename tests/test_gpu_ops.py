@@ -602,6 +602,37 @@ def test_gemm_prefetch_hint_leaves_the_result_alone(ops, dev):
         ops.gemm(a, q, b, w_scale=sc, prefetch=torch.zeros(64))
 
 
+def test_few_row_launches_with_a_prefetch_hint_keep_their_bits(ops, dev):
+    """The few-row kernel's extra workgroups only read: every tile form, with row sums, inline norms and fp8 weights, and the
+    few-window attention launch, with hints from none of a whole piece to more than the launch has time for."""
+    hints = [torch.zeros(n, dtype=torch.uint8, device=dev) for n in (8, 16, 1000003, 40 << 20)]
+    for M, N, K in [(33, 1280, 1280), (200, 1280, 1152), (500, 1280, 1280), (1450, 1152, 1280), (2196, 1152, 4352), (90, 320, 256)]:
+        a, w, b = rnd((M, K), 1.0, 121, dev), rnd((N, K), 0.05, 122, dev), rnd((N,), 0.02, 123, dev)
+        res, lo = rnd((M, N), 1.0, 124, dev), torch.zeros((M, N), dtype=torch.uint8, device=dev)
+        sc = (w.float().abs().amax(1) / 448.0).contiguous()
+        q = (w.float() / sc[:, None]).to(torch.float8_e4m3fn)
+
+        def forms(hint):
+            ss, out_lo = torch.zeros((M, ops.SUMSQ_PARTS), device=dev), torch.empty_like(lo)
+            kw = {"epilogue": ops.EPI_RESIDUAL, "residual": res, "residual_lo": lo, "out_lo": out_lo, "prefetch": hint}
+            got = [ops.gemm(a, w, b, **kw), out_lo.clone(), ops.gemm(a, w, b, c_row_sumsq=ss, **kw), ss]
+            got += [ops.gemm(a, w, b, epilogue=ops.EPI_GELU_TANH, prefetch=hint), ops.gemm(a, q, b, w_scale=sc, prefetch=hint)]
+            return got + ([ops.gemm(a, w, b, norm_inline=True, norm_eps=1e-6, prefetch=hint)] if K <= 1280 else [])
+
+        plain = forms(None)
+        for h in hints:
+            assert all(torch.equal(x, y) for x, y in zip(forms(h), plain, strict=True)), (M, N, K, h.numel())
+    heads, d, K = 16, 80, 1280
+    w, b = rnd((3 * heads * d, K), 0.05, 126, dev), rnd((3 * heads * d,), 0.02, 127, dev)
+    wp, bp = ops.pack_qkv_window_attn(w, b, heads)
+    for M, win_start in ((64, None), (15 * 64, None), (100, torch.tensor([0, 64, 100], dtype=torch.int32, device=dev))):
+        x, cos = rnd((M, K), 1.0, 125, dev), torch.rand((M, d), generator=torch.Generator().manual_seed(1)).to(dev)
+        run = lambda h: ops.qkv_window_attn(x, wp, bp, cos, heads, d**-0.5, win_start=win_start, norm_inline=True,  # noqa: E731
+                                            norm_eps=1e-6, prefetch=h)
+        plain = run(None)
+        assert all(torch.equal(run(h), plain) for h in hints), M
+
+
 @pytest.mark.parametrize("M,N,K", [
     (8192, 3072, 192),    # 256x256 (three-stage ring with byte-wide W tiles) + 256x128 remainder, 3 K tiles
     (8192, 2304, 256),    # 256x256 + 128x192 remainder
