@@ -90,8 +90,6 @@ def _check_source(hipcc: str, src: Path) -> None:
     offenders = check_hand_managed_acc_registers(asm.read_text())
     asm.unlink()
     if offenders:
-        # the object of a source that fails this check must not survive for a later incremental build to link
-        (OBJ_DIR / (src.stem + ".o")).unlink(missing_ok=True)
         raise RuntimeError(f"{src.name}: the compiler used accumulation registers that inline assembly owns:\n  "
                            + "\n  ".join(offenders))
 
@@ -130,18 +128,24 @@ def build_library(force: bool = True, jobs: int = 8) -> Path:
     sources = sorted(CSRC.glob("*.hip"))
     headers = list(CSRC.glob("*.h")) + list(INCLUDE.glob("*.h"))
     newest_hdr = max(h.stat().st_mtime for h in headers)
-    objs = []
+    objs, stale_objs = [], []
     todo = []
     for src in sources:
         obj = OBJ_DIR / (src.stem + ".o")
         objs.append(obj)
         stale = force or not obj.exists() or obj.stat().st_mtime < max(src.stat().st_mtime, newest_hdr)
         if stale:
+            stale_objs.append(obj)
             todo.append(lambda cmd=[hipcc, *HIPCC_FLAGS, "-c", str(src), "-o", str(obj)]: _run(cmd))
             if HAND_MANAGED_ACC_MARKER in src.read_text():
                 todo.append(lambda src=src: _check_source(hipcc, src))
-    with ThreadPoolExecutor(max_workers=max(1, min(jobs, len(todo) or 1))) as pool:
-        list(pool.map(lambda job: job(), todo))
+    try:
+        with ThreadPoolExecutor(max_workers=max(1, min(jobs, len(todo) or 1))) as pool:
+            list(pool.map(lambda job: job(), todo))
+    except BaseException:   # (here every job has ended) no later incremental build may link what was not checked
+        for obj in stale_objs:
+            obj.unlink(missing_ok=True)
+        raise
     TORCH_LIB_PATH.unlink(missing_ok=True)   # (an older one must not stay beside the new kernel library if its own step fails)
     _run([hipcc, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", str(LIB_PATH), *map(str, objs)])
     _check_no_missing_kernels(LIB_PATH)

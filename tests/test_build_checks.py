@@ -1,5 +1,11 @@
 """Host-side checks of the build helpers (no GPU, no compiler run)."""
 
+import time
+from pathlib import Path
+
+import pytest
+
+from cornserve_amd import build
 from cornserve_amd.build import check_hand_managed_acc_registers
 
 _CLEAN = """
@@ -42,3 +48,32 @@ def test_kernels_without_inline_accumulators_are_not_checked():
     # a kernel whose accumulators the compiler manages itself may use the registers freely
     assert check_hand_managed_acc_registers(_COMPILER_ONLY) == []
     assert len(check_hand_managed_acc_registers(_COMPILER_ONLY + _SPILL)) == 1
+
+
+def test_an_object_whose_source_fails_the_check_does_not_survive(tmp_path, monkeypatch):
+    """Compilation and check of a source run side by side: whichever ends first, an incremental build that follows a failed
+    check must compile and check the source again instead of linking its object."""
+    csrc, out = tmp_path / "csrc", tmp_path / "build"
+    csrc.mkdir()
+    (csrc / "a.hip").write_text(f"// {build.HAND_MANAGED_ACC_MARKER}\n")
+    (csrc / "a.h").write_text("")
+    linked = []
+
+    def run(cmd):
+        target = Path(cmd[cmd.index("-o") + 1])
+        if "-shared" in cmd:
+            linked.append(target)
+        elif "-S" in cmd:
+            target.write_text(_SPILL)
+        else:
+            time.sleep(0.3)        # the compilation outlasts the check
+            target.write_text("object")
+
+    monkeypatch.setattr(build, "CSRC", csrc)
+    monkeypatch.setattr(build, "OBJ_DIR", out)
+    monkeypatch.setattr(build, "_hipcc", lambda: "hipcc")
+    monkeypatch.setattr(build, "_run", run)
+    for force in (True, False):
+        with pytest.raises(RuntimeError, match="accumulation registers"):
+            build.build_library(force=force)
+        assert not (out / "a.o").exists() and not linked
