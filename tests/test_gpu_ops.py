@@ -476,9 +476,10 @@ def test_gemm_fast_path_forms(ops, dev, M, N, K):
     assert torch.equal(scat, ref)
 
 
-# The few-row kernel (K a multiple of 128): every tile form at row and column tails, at the shortest K and at one that runs
-# through its steady loop.  An output has the bits it has as a row of a product with many rows (which the big tiles take),
-# with the norms folded inline or from arrays, and the row sums of its output are the big tiles'.
+# The few-row kernel (K a multiple of 128) at shapes of the encoders: an output has the bits it has as a row of a product with
+# many rows, with the norms folded inline or from arrays, and the row sums of its output are the big tiles'.  (Inline norms
+# always run here; of the rest, (1, 64, 256) compares the few-row kernel with itself and (2700, 1280, 1280) the big tiles.
+# Every form against the big tiles, at its tails and both ends of its K loop: the test after this one.)
 @pytest.mark.parametrize("M,N,K", [
     (1, 64, 256),         # one row
     (33, 1296, 1280),     # 32x32 tiles, row and column tails
@@ -538,6 +539,90 @@ def test_gemm_few_rows_equal_the_rows_of_a_large_product(ops, dev, M, N, K):
         ops.gemm(a[:M, :192].contiguous(), w[:, :192].contiguous(), b, norm_inline=True)
     with pytest.raises(ValueError):        # inline sums instead of the arrays, not next to them
         ops.gemm(a[:M], w, b, norm_inline=True, a_row_sumsq=torch.zeros((M, 8), device=dev))
+
+
+# Every tile form with a row and a column tail, at the shortest K that it is chosen for and at one where the loop over its ring
+# is entered (32x32: from 17 stages of 128 k, 32x64: 13, 64x64 and 64x80: 9, the others earlier), against the same rows of a
+# product that the big tiles take; which kernel and form a call gets is asserted.
+@pytest.mark.parametrize("tile,M,N,K,many", [
+    ((32, 32), 1, 64, 256, 65600),
+    ((32, 32), 33, 1288, 256, 8192),
+    ((32, 32), 33, 1288, 3456, 8192),
+    ((32, 64), 200, 1288, 512, 8192),
+    ((32, 64), 200, 1288, 3456, 8192),
+    ((64, 64), 500, 1304, 256, 8192),
+    ((64, 64), 500, 1304, 1280, 8192),
+    ((64, 80), 1000, 1272, 256, 8192),
+    ((64, 80), 1000, 1272, 1280, 8192),
+    ((64, 128), 1450, 1272, 640, 8192),
+    ((64, 128), 1450, 1272, 1280, 8192),
+    ((128, 128), 2196, 1144, 2304, 8192),
+    ((128, 128), 2196, 1144, 4352, 8192),
+    ((32, 160), 500, 1152, 256, 8192),
+    ((32, 160), 500, 1152, 1152, 8192),
+    ((32, 160), 1000, 1272, 1280, 8192),
+    ((64, 160), 1450, 1152, 256, 8192),
+    ((64, 160), 1450, 1152, 1152, 8192),
+    ((64, 160), 1450, 1272, 1280, 8192),
+])
+def test_every_few_row_form_gives_the_bits_of_the_big_tiles(ops, dev, tile, M, N, K, many):
+    import ctypes
+
+    from cornserve_amd import lib
+
+    a, w, b = rnd((many, K), 1.0, 131, dev), rnd((N, K), 0.05, 132, dev), rnd((N,), 0.02, 133, dev)
+    res = rnd((many, N), 1.0, 134, dev)
+    lo = torch.randint(0, 256, (many, N), generator=torch.Generator().manual_seed(135), dtype=torch.uint8).to(dev)
+    sc = (w.float().abs().amax(1) / 448.0).contiguous()
+    q = (w.float() / sc[:, None]).to(torch.float8_e4m3fn)
+    residual_form = tile[1] == 160
+
+    def groups(rows, epilogue, sums=False, fp8=False):
+        g = lib.CsGemmArgs()
+        g.A, g.W, g.C = a.data_ptr(), w.data_ptr(), res.data_ptr()
+        g.M, g.N, g.K, g.lda, g.ldw, g.ldc, g.epilogue = rows, N, K, K, K, N, epilogue
+        if epilogue == ops.EPI_RESIDUAL:
+            g.residual, g.ldr, g.residual_lo, g.c_lo = res.data_ptr(), N, lo.data_ptr(), lo.data_ptr()
+        if sums:
+            g.c_row_sumsq = res.data_ptr()
+        if fp8:
+            g.w_fp8, g.w_scale = 1, sc.data_ptr()
+        return lib.load().cs_gemm_few_row_workgroups(ctypes.byref(g))
+
+    tiles = -(-M // tile[0]) * -(-N // tile[1])
+    assert groups(M, ops.EPI_RESIDUAL, sums=residual_form) == tiles
+    assert residual_form or groups(M, ops.EPI_BIAS) == tiles
+
+    def split(rows, **sums):
+        out, out_lo = torch.empty_like(res[:rows]), torch.empty_like(lo[:rows])
+        ops.gemm(a[:rows], w, b, epilogue=ops.EPI_RESIDUAL, residual=res[:rows], residual_lo=lo[:rows], out=out, out_lo=out_lo, **sums)
+        return out, out_lo
+
+    want = split(many)
+    if residual_form:
+        for both in (False, True):
+            s_many, s_few = ([torch.zeros((r, ops.SUMSQ_PARTS), device=dev) for _ in range(1 + both)] for r in (many, M))
+            kw = lambda s: {"c_row_sumsq": s[0], **({"c_row_sum": s[1]} if both else {})}  # noqa: E731
+            assert groups(many, ops.EPI_RESIDUAL, sums=True) == 0
+            split(many, **kw(s_many))
+            got = split(M, **kw(s_few))
+            assert all(torch.equal(g, x[:M]) for g, x in zip((*got, *s_few), (*want, *s_many), strict=True))
+        return
+    got = split(M)
+    assert groups(many, ops.EPI_RESIDUAL) == 0 and all(torch.equal(g, x[:M]) for g, x in zip(got, want, strict=True))
+    close(ops.gemm(a[:M], w, b)[:64], lin_ref(a[:64][:M], w, b), 2**-7, f"{M}x{N}x{K}")
+    for epi in (ops.EPI_BIAS, ops.EPI_GELU_ERF, ops.EPI_GELU_TANH, ops.EPI_QUICK_GELU, ops.EPI_SWIGLU):
+        assert groups(M, epi) and not groups(many, epi)
+        assert torch.equal(ops.gemm(a[:M], w, b, epilogue=epi), ops.gemm(a, w, b, epilogue=epi)[:M]), epi
+        assert groups(M, epi, fp8=True) and not groups(many, epi, fp8=True)
+        assert torch.equal(ops.gemm(a[:M], q, b, epilogue=epi, w_scale=sc), ops.gemm(a, q, b, epilogue=epi, w_scale=sc)[:M]), epi
+    if K <= 1280:
+        ss, sm = torch.empty((M, ops.SUMSQ_PARTS), device=dev), torch.empty((M, ops.SUMSQ_PARTS), device=dev)
+        ops.row_stats(a[:M], ss, sm)
+        assert torch.equal(ops.gemm(a[:M], w, b, norm_inline=True, norm_eps=1e-6), ops.gemm(a[:M], w, b, a_row_sumsq=ss, norm_eps=1e-6))
+        cs = w.float().sum(1)
+        assert torch.equal(ops.gemm(a[:M], w, b, norm_inline=True, w_col_sum=cs, norm_eps=1e-6),
+                           ops.gemm(a[:M], w, b, a_row_sumsq=ss, a_row_sum=sm, w_col_sum=cs, norm_eps=1e-6))
 
 
 @pytest.mark.parametrize("windows,heads,ragged,form", [(1, 1, False, "array"), (16, 16, False, "inline"), (5, 16, True, "inline"),
