@@ -16,7 +16,10 @@ namespace {
 // Time of a launch in microseconds: per round of 256 tiles, `fixed_us` (first loads, epilogue, and once 2 us of launch)
 // plus `stage_us` per 128 k.  From launches of 1280 columns at K = 1280 and 3456 that are one round: 96 rows (32x32: 6.0
 // and 8.6 us), 250 (32x64: 7.0, 10.6), 512 (64x64: 8.1, 14.6), 1024 (64x80: 10.2, 18.2; 32x160: 11.8, 22.6), 1500 (64x128:
-// 13.1, 22.5), 2048 (64x160: 16.2, 30.5), 2744 (128x128: 20.3, 33.4).
+// 13.1, 22.5), 2048 (64x160: 16.2, 30.5), 2744 (128x128: 20.3, 33.4).  With weights from HBM and longer K both kernels take up
+// to a third longer than this says, and fp8 weights cost the big forms more than the small ones; the comparison holds all the
+// same: of 29 products of the encoders at 44 row counts each, 581 launches come here, and the one that loses most against the big
+// tiles takes 38.7 us instead of 38.2 (2048 rows x 1280 x 3456).
 struct Form {
   int bm, bn;
   float fixed_us, stage_us;
@@ -143,10 +146,15 @@ int cs_gemm_small_workgroups(const CsGemmArgs& a) {
   return tiles + (p.prefetch ? csgemm::hint_workgroups(tiles) : 0);
 }
 
-// One workgroup per window and head while the chip holds them all at once: 22 to 25 us up to 16 windows of 16 heads, where
-// a big tile (four windows) takes 32 to 35 us whatever the count; with a second round (24 windows: 39 us) it is the slower.
+// One workgroup per window and head while the chip holds them all at once: 24 to 26 us up to 16 windows of 16 heads (inline norm,
+// weights from HBM; 21 to 23 without norm), where a big tile (four windows) takes 32 to 35 us whatever the count; with a second
+// round (24 windows: 39 us) it is the slower.
 bool cs_qkv_window_attn_few(int64_t windows, int heads, int K) { return K % 128 == 0 && windows * heads <= 256; }
 
+// (Compared with the big forms of any epilogue, also where a folded LayerNorm has the 160-column ones alone, so it says no too
+// early rather than too late: passes with the rule | both | neither inline, Qwen3-VL 256 patches 1.95 | 1.94 | 2.68 ms, 576 2.62 |
+// 2.54 | 2.87, 896 3.17 | 2.94 | 3.17, 1280 4.03 | 4.59 | 4.03; Qwen2.5-VL 256 2.12 | 2.12 | 2.59, 432 2.57 | 2.42 | 2.61, 576 2.78 |
+// 2.74 | 2.76, 896 2.95 | 3.24 | 2.93, 1280 3.89 | 4.60 | 3.88.)
 extern "C" int cs_gemm_norm_inline_pays(int32_t M, int32_t N, int32_t K, int32_t window_attn) {
   if (M < 1 || N < 8 || N % 8 || K < 192 || !csgemm::inline_norm_width(K)) return 0;
   if (window_attn) return cs_qkv_window_attn_few(M / 64, N / 256, K) ? 1 : 0;

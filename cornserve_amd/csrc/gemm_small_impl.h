@@ -6,10 +6,12 @@
 // or eight waves per tile, and as deep a ring of K stages in LDS as fits, so that most of a tile's operands are in
 // flight at once.  What bounds it is the LDS: per stage of 128 k it takes in (BM + BN) x 256 bytes and hands out
 // waves x (MT + NT) x 4 KB of fragments, and time per stage follows that sum at about 270 KB a microsecond and compute
-// unit (128 bytes a clock) in every tile form; the rest of a launch is 4 to 5 us of launch, first loads and epilogue.
+// unit (128 bytes a clock) in the GEMM's tile forms; the rest of a launch is 4 to 5 us of launch, first loads and epilogue.
+// (That gives the window attention form, one wave a SIMD, 13 us.  It takes 14.6 with weights in the caches, 19.7 with the inline
+// norm, and 4 to 8 more with its 10 MB of weights from HBM.)
 // Measured on an MI355X with weights that no cache holds: 1280 columns, K = 3456: 96 rows 34.3 -> 8.7 us (32x32 tiles),
-// 1024 rows 38 -> 20 us (64x80); K = 1280: 96 rows 19 -> 6 us, 1024 rows 19 -> 11 us.  From about 2048 rows on the big
-// tiles are the faster ones (the choice is in gemm_small.hip).
+// 1024 rows 38 -> 20 us (64x80); K = 1280: 96 rows 19 -> 6 us, 1024 rows 19 -> 11 us.  The big tiles are the faster ones from
+// about 2000 rows on at K = 1280, from 3100 (128x128 tiles until then) at K = 3456 to 5120: the choice is in gemm_small.hip.
 //
 // The arithmetic of an output element is the same sequence of operations as in gemm_fast_impl.h (v_mfma_f32_16x16x32_bf16
 // over ascending K from a zero accumulator, W as the first operand, the same epilogue functions in the same order), so an

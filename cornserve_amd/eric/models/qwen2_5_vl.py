@@ -316,8 +316,9 @@ class Qwen2_5_VisionTransformer(QwenVisionBase):
         routes agree within the parity tolerance, not bit for bit; since the route depends on the item alone, an item's
         embedding is the same bits whatever it is batched with (setting the attribute to False afterwards selects the
         separate kernels for every item).  `fuse_min_rows` > 0 is a deployment knob that gives this up for latency: a
-        batch with fewer one-launch rows than that takes the separate kernels throughout, whose GEMM has narrower tiles
-        for few rows (one 1024-patch image alone: 3.99 against 4.28 ms; 3072 is where the one launch starts to pay).
+        batch with fewer one-launch rows than that takes the separate kernels throughout, whose GEMM spreads over more
+        compute units than a workgroup per window and head (96 patches 1.52 against 1.80 ms; 1024 3.08 against 2.95, 2048 4.23
+        against 4.25, 3072 5.40 against 5.00: only the smallest batches gain).
 
         `split_residual`: carry the residual stream (:175,177) with 16 significant bits -- the bf16 tensor every
         kernel reads plus a byte plane with the next 8 mantissa bits, joined and re-split inside the two residual GEMMs
@@ -538,10 +539,12 @@ class Qwen2_5_VisionTransformer(QwenVisionBase):
 
         # rows [0, fused_rows) belong to the items whose window blocks run as one launch, the rest to the others
         xf = x[:fused_rows]
-        # A batch of few rows leaves most compute units idle in the N = hidden GEMMs, and what bounds those launches is
+        # A batch of few rows leaves compute units idle in the N = hidden GEMMs, and what bounds those launches is
         # the latency of weights that nothing has touched since the previous forward pass: the one-launch window block
         # has its idle units read the gate|up weights, the attention-output projection the down-projection's, the
-        # down-projection the next block's qkv weights.
+        # down-projection the next block's qkv weights.  (A launch of more than 192 tiles reads none: those of 1024 rows have
+        # 224 to 256 small ones; one of the few-row kernel reads what fits its own time.  3072 patches 5.39 -> 5.02 ms, 1280
+        # 3.87 -> 3.57, 96 1.82 -> 1.80, 1024 the same.)
         hint = L <= self.prefetch_rows
 
         def next_qkv(i: int) -> torch.Tensor | None:

@@ -144,7 +144,8 @@ typedef struct CsGemmArgs {
   /* Folded norm without the row-sum arrays: with a_norm_inline = 1 the sums over the rows of A are taken inside the
    * launch (K is the normalised width, at most 160 * CS_SUMSQ_PARTS); a_row_sumsq and a_row_sum are NULL, w_col_sum says
    * which norm (NULL: RMSNorm, set: LayerNorm), and W, bias and norm_eps are those of the array form.  Same bits as the
-   * array form with sums from a GEMM's c_row_sumsq / c_row_sum or from cs_row_sumsq / cs_row_stats.  Meant for few rows: cs_gemm_norm_inline_pays tells whether this form is the faster one for a shape.
+   * array form with sums from a GEMM's c_row_sumsq / c_row_sum or from cs_row_sumsq / cs_row_stats.  Meant for few rows:
+   * cs_gemm_norm_inline_pays tells whether this form is the faster one for a shape.
    * CS_EPI_BIAS and CS_EPI_SWIGLU (RMSNorm), CS_EPI_BIAS, CS_EPI_GELU_TANH and CS_EPI_QUICK_GELU (LayerNorm); bf16 W,
    * K a multiple of 128; also taken by cs_qkv_window_attn (RMSNorm).  CS_ERR_UNSUPPORTED otherwise.               */
   int32_t a_norm_inline;
