@@ -163,6 +163,78 @@ CS_DEVICE void write_output(const f32x16_t (&oacc)[DT], float l_run, bf16_t* oro
     }
 }
 
+// ---- softmax of the long-segment kernels, half a key tile (32 keys) at a time, and per query.  The reference maximum m of a query
+//      is that of its segment's first tile, and P = exp2((s - m) * scale - shift).  With the shift, a score has to exceed m by
+//      2^(shift + 1) before P reaches 2; until then m stays.  Whether it happened shows in the packed words themselves -- P >= 2
+//      is the top exponent bit of a bf16 -- so the usual half tile needs no maximum, no exchange between lanes and no
+//      comparison in front of its exponentials: 4 word-wise ORs instead of 9 instructions and an LDS round trip (a NaN has
+//      the bit set as well and takes the slow way, where fmaxf leaves m alone).  The slow way raises m for exactly the
+//      queries that exceeded it, so that a query's bits depend on its own scores only, whichever queries share its wave.
+//      The shift cancels in the division by the denominator; segments of one tile cannot exceed their maximum and use none,
+//      which gives them the bits of attn_kernel.
+constexpr float P_SHIFT_LOG2 = 8.0f;
+constexpr uint32_t P_TWO_BIT = 0x40004000u;   // set in a bf16 pair iff one of two non-negative values is >= 2 (or NaN)
+
+CS_DEVICE float row_max(const f32x16_t& s) {
+  float mx = s[0];
+#pragma unroll
+  for (int r = 1; r < 16; ++r) mx = fmaxf(mx, s[r]);
+  return mx;
+}
+// over the two lanes that hold a query's scores (lane, lane ^ 32)
+CS_DEVICE float pair_max(float v) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, v), __builtin_bit_cast(uint32_t, v), false, false);
+  const uint32_t lower = r[0], upper = r[1];   // (named: a bit cast of a vector element takes the vector's first)
+  return fmaxf(__builtin_bit_cast(float, lower), __builtin_bit_cast(float, upper));
+}
+// P of one half tile as operands of the second product (two bf16 per word); the OR of their words.  SUM: adds P to the lane's
+// running sum.
+template <bool SUM>
+CS_DEVICE uint32_t exp_half(const f32x16_t& s, i32x4_t (&p)[2], float sl2, float mb, float& l_run) {
+  uint32_t any = 0;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const float a = __builtin_amdgcn_exp2f(__builtin_fmaf(s[2 * i], sl2, -mb));
+    const float b = __builtin_amdgcn_exp2f(__builtin_fmaf(s[2 * i + 1], sl2, -mb));
+    if constexpr (SUM) {
+      l_run += a;
+      l_run += b;
+    }
+    bf16x2_t w;
+    w[0] = f2bf(a);
+    w[1] = f2bf(b);
+    const uint32_t word = __builtin_bit_cast(uint32_t, w);
+    p[i >> 2][i & 3] = (int)word;
+    any |= word;
+  }
+  return any;
+}
+// The slow way: m raised where a query exceeded it, O and the sum rescaled, P computed again.
+template <int DT, bool SUM>
+CS_DEVICE void raise_reference(const f32x16_t& s, i32x4_t (&p)[2], f32x16_t (&oacc)[DT], float& m_run, float& mb, float& l_run, float sl2,
+                               float shift) {
+  const float mx = pair_max(row_max(s));
+  const bool up = __builtin_fmaf(mx, sl2, -mb) >= 1.0f;
+  const float alpha = up ? __builtin_amdgcn_exp2f((m_run - mx) * sl2) : 1.0f;
+#pragma unroll
+  for (int t = 0; t < DT; ++t)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) oacc[t][r] *= alpha;
+  if constexpr (SUM) l_run *= alpha;
+  m_run = up ? mx : m_run;
+  mb = __builtin_fmaf(m_run, sl2, shift);
+  exp_half<SUM>(s, p, sl2, mb, l_run);
+}
+// exp_half, and raise_reference if any lane of the wave asks for it (l_run of before the half tile is what is rescaled)
+template <int DT, bool SUM>
+CS_DEVICE void softmax_half(const f32x16_t& s, i32x4_t (&p)[2], f32x16_t (&oacc)[DT], float& m_run, float& mb, float& l_run, float sl2,
+                            float shift) {
+  float l_new = l_run;
+  const uint32_t any = exp_half<SUM>(s, p, sl2, mb, l_new);
+  if (__any((any & P_TWO_BIT) != 0)) raise_reference<DT, SUM>(s, p, oacc, m_run, mb, l_run, sl2, shift);
+  else l_run = l_new;
+}
+
 template <int D, int NWAVES, bool ROPE, int HPW>
 __global__ __launch_bounds__(NWAVES * 64, 2) void attn_kernel(const AttnArgs a) {
   constexpr int NT = NWAVES * 64;
@@ -433,10 +505,13 @@ __global__ __launch_bounds__(256, 2) void attn_full_kernel(const AttnArgs a) {
   // chunks of `chunk` consecutive work items of one head (a segment's query blocks are consecutive work
   // items), chunk c goes to XCD c % 8, and an XCD walks its chunks in order.
   const int xcd = blockIdx.x & 7, j = blockIdx.x >> 3;
+  // The chunks of all heads come first item by item: with the longest segments in front of the work list (ops.attn_plan), the
+  // long workgroups start first, and every XCD gets its share of them (with heads outermost and two chunks, one long and one
+  // short, all long ones met on four of the eight XCDs: segments of 3300, 1196, 1024 and 720 rows, d = 72, 131 -> 105 us).
   const int cid = (j / a.chunk) * 8 + xcd;           // chunk id in [0, n_chunks_x * heads)
-  const int item = (cid % a.n_chunks_x) * a.chunk + j % a.chunk;
-  const int head = cid / a.n_chunks_x;
-  if (item >= a.n_work || head >= a.heads) return;   // padding of the last chunks (uniform per workgroup)
+  const int item = (cid / a.heads) * a.chunk + j % a.chunk;
+  const int head = cid % a.heads;
+  if (item >= a.n_work) return;                      // padding of the last chunks (uniform per workgroup)
   const int seg_start = a.work[item * 4 + 0];
   const int seg_end = a.work[item * 4 + 1];
   const int q0 = a.work[item * 4 + 2];
@@ -584,9 +659,9 @@ __global__ __launch_bounds__(256, 2) void attn_full_kernel(const AttnArgs a) {
   for (int t = 0; t < DT; ++t)
 #pragma unroll
     for (int r = 0; r < 16; ++r) oacc[t][r] = 0.f;
-  float m_run = -INFINITY, l_run = 0.f;
+  float m_run = 0.f, mb = 0.f, l_run = 0.f;
   const bool wave_active = wave * 32 < nq;
-  const float sl2 = a.scale_log2e;
+  const float sl2 = a.scale_log2e, shift = seg_len > BKV ? P_SHIFT_LOG2 : 0.0f;
 
   int buf = 0;
   for (int kv0 = 0; kv0 < seg_len; kv0 += BKV, buf ^= 1) {
@@ -597,17 +672,21 @@ __global__ __launch_bounds__(256, 2) void attn_full_kernel(const AttnArgs a) {
       const char* kd = k_buf(buf);
       const char* vd = v_buf(buf);
       f32x16_t sacc[2];
-      bf16x8_t pf[2][2];
       score_tile<KS, RS>(sacc, kd, qf, nvalid, fr, hf);
-      softmax_tile<DT, L_FROM_MFMA>(sacc, pf, oacc, m_run, l_run, sl2);
+      if (kv0 == 0) {
+        m_run = pair_max(fmaxf(row_max(sacc[0]), row_max(sacc[1])));
+        mb = __builtin_fmaf(m_run, sl2, shift);
+      }
 #pragma unroll
-      for (int t = 0; t < DT; ++t) {
+      for (int kt = 0; kt < 2; ++kt) {
+        i32x4_t pf[2];
+        softmax_half<DT, !L_FROM_MFMA>(sacc[kt], pf, oacc, m_run, mb, l_run, sl2, shift);
 #pragma unroll
-        for (int kt = 0; kt < 2; ++kt)
+        for (int t = 0; t < DT; ++t)
 #pragma unroll
           for (int kk = 0; kk < 2; ++kk) {
             const bf16x8_t vf = read_vt_frag(vd, t, kt * 2 + kk, lane);
-            oacc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, pf[kt][kk], oacc[t], 0, 0, 0);
+            oacc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, __builtin_bit_cast(bf16x8_t, pf[kk]), oacc[t], 0, 0, 0);
           }
       }
     }
@@ -615,48 +694,43 @@ __global__ __launch_bounds__(256, 2) void attn_full_kernel(const AttnArgs a) {
     __syncthreads();
   }
 
+  if constexpr (!L_FROM_MFMA) l_run += __shfl_xor(l_run, 32, 64);
   const int qi = wave * 32 + fr;
   write_output<D, DT, L_FROM_MFMA>(oacc, l_run, a.out + (int64_t)(q0 + min(qi, nq - 1)) * a.ldo + hoff, qi < nq, hf);
 }
 
-// Full attention without rotary (SigLIP): K and V tiles go global -> LDS directly (buffer_load ... lds: no
-// staging registers, no LDS store instructions, no address arithmetic per tile) into a ring of NB tile buffers:
-// three buffers requested two tiles ahead with two workgroups per CU, or two buffers requested one tile ahead with
-// three workgroups per CU (what launch_attn selects).  A direct load fixes the LDS side -- the 64 lanes of a wave fill 1 KB of
-// consecutive LDS -- so the padded row layout is produced on the global side: a tile is the flat sequence of
-// 16-byte chunk slots (row, slot), lane l of load j owns slot j*64 + l and fetches chunk `slot % slots_per_row`
-// of row `slot / slots_per_row`; lanes that own padding slots are switched off for the load, which leaves the
-// padding as initialised once per buffer (zeros behind the K rows that the last k-step reads, the ones
-// column of V that yields the softmax denominator).
+// Full attention without rotary on the keys (SigLIP; the Qwen families after cs_rope_qk): a software pipeline over half tiles of
+// 32 keys.  One step issues the matrix instructions of two different half tiles -- P.V of the previous one and the scores of the
+// next one -- while the vector unit works on the softmax of the one between them.  Nothing in a step waits for a result of the
+// same step, so the matrix cores run under the softmax of the SAME wave: with the three phases one after the other, three waves
+// per SIMD took 1,370 clocks of a SIMD per wave and 64-key tile (704 of them matrix instructions), two waves of this kernel take
+// 960 to 1,080.  How the instructions of a step interleave is laid down with scheduling groups; two waves per SIMD (two
+// workgroups per CU) use what a wave leaves free.  V fragments live in two register sets, the next step's being read during
+// this one; K fragments are read at the start of their own step, whose first matrix instructions are those of P.V (two
+// register sets for K as well: the same time, and head dim 96 spills).
+//   16 heads, back to back, before -> after, d = 72: 4 x 4096 rows 411 -> 365 us, 4096 rows 124 -> 102, 3300 + 1196 + 1024 + 720 rows
+//   125 -> 100, 7 x 729 rows 38.0 -> 36.4, 2 x 729 rows 19.8 -> 15.4; d = 80: 8 x 1024 rows 75 -> 68, 1024 rows 24.0 -> 17.8, 1380 + 816
+//   rows 43 -> 29, 4888 rows 230 -> 172, 16 segments of 432 to 9000 rows 2918 -> 2025, 16 x 1008 rows 138 -> 131; d = 64: 2 x 1500 rows 43.1 ->
+//   40.4; d = 96: 55.4 -> 52.0 us.
+// What bounds it now is power: under it the shader clock falls from 1.9 to 1.4 .. 1.7 GHz, and a build without the LDS reads runs as many
+// clocks at a higher clock rate.  Also measured: 64 query rows per wave and one wave per SIMD (half the LDS reads, but a lone wave
+// issues an instruction every five clocks: 2,630 clocks per 64 rows and tile against 1,930), eight waves around one K/V stream
+// (the same time within 3 %; 7 x 729 rows 41 us), and dims 64 .. 79 of O^T in 16x16 blocks (a sixth less V read and multiplied,
+// eight lane swaps more: no faster).
+//
+// K and V tiles go global -> LDS directly (buffer_load ... lds: no staging registers, no LDS store instructions, no
+// address arithmetic per tile) into a ring of three tile buffers, requested two tiles ahead.  A direct load fixes the LDS
+// side -- the 64 lanes of a wave fill 1 KB of consecutive LDS -- so the padded row layout is produced on the global side: a
+// tile is the flat sequence of 16-byte chunk slots (row, slot), lane l of load j owns slot j*64 + l and fetches chunk
+// `slot % slots_per_row` of row `slot / slots_per_row`; lanes that own padding slots are switched off for the load, which
+// leaves the padding as initialised once per buffer (zeros behind the K rows that the last k-step reads, the ones
+// column of V that yields the softmax denominator).  The loads are written in assembly, which writes LDS only: behind the
+// builtin, the compiler takes every transposing LDS read for a possible reader of the bytes in flight and waits for
+// ALL outstanding loads in front of it.  The kernel's own waits are explicit (one per tile, in front of its barrier).
 typedef __attribute__((address_space(3))) void lds_void_t;
+typedef int i32x4_sgpr_t __attribute__((ext_vector_type(4)));
 
-// Transposing LDS reads of the four V^T fragments (keys 16g .. 16g+15, g = 0..3) of dims 32*TT .. 32*TT+31, written in
-// assembly (see the kernel for why); the caller waits for them with an explicit s_waitcnt.
-template <int TT, int G>
-CS_DEVICE void read_vt_pair_asm(i32x2_t& lo, i32x2_t& hi, uint32_t vbase) {
-  asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(lo) : "v"(vbase), "n"(G * 16 * V_RS + TT * 64));
-  asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(hi) : "v"(vbase), "n"(G * 16 * V_RS + TT * 64 + 8 * V_RS));
-}
-template <int TT>
-CS_DEVICE void read_vt_block_asm(i32x2_t (&raw)[8], uint32_t vbase) {
-  read_vt_pair_asm<TT, 0>(raw[0], raw[1], vbase);
-  read_vt_pair_asm<TT, 1>(raw[2], raw[3], vbase);
-  read_vt_pair_asm<TT, 2>(raw[4], raw[5], vbase);
-  read_vt_pair_asm<TT, 3>(raw[6], raw[7], vbase);
-}
-template <bool LAST>
-CS_DEVICE void pv_block(f32x16_t& o, i32x2_t (&raw)[8], const bf16x8_t (&pf)[2][2]) {
-  if constexpr (LAST) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-  else asm volatile("s_waitcnt lgkmcnt(8)" ::: "memory");
-#pragma unroll
-  for (int g = 0; g < 4; ++g) {
-    i32x4_t both = {raw[2 * g][0], raw[2 * g][1], raw[2 * g + 1][0], raw[2 * g + 1][1]};
-    asm volatile("" : "+v"(both));  // the registers hold the data only after the wait above
-    o = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, both), pf[g >> 1][g & 1], o, 0, 0, 0);
-  }
-}
-
-template <int D, int NB = 3>
+template <int D>
 struct AttnDirectShape {
   static constexpr int KS = (D + 15) / 16, DKC = KS * 2, DC = D / 8;
   static constexpr int K_SLOTS = DKC | 1, V_SLOTS = V_RS / 16;      // 16-byte slots per tile row
@@ -664,19 +738,18 @@ struct AttnDirectShape {
   static constexpr int K_BYTES = BKV * RS, V_BYTES = BKV * V_RS, TILE_BYTES = K_BYTES + V_BYTES;
   static constexpr int K_LOADS = BKV * K_SLOTS / 64, V_LOADS = BKV * V_SLOTS / 64;   // BKV == 64: one load per slot column
   static constexpr int LOADS = K_LOADS + V_LOADS, PER_WAVE = (LOADS + 3) / 4;
-  static constexpr int NBUF = NB, LDS = NBUF * TILE_BYTES;
-  static constexpr int WGS_PER_CU = NB == 2 ? 3 : 2;
-  static_assert(128 * RS <= (NBUF - 1) * TILE_BYTES, "the Q tile aliases the buffers behind the first");
-  static_assert(WGS_PER_CU * LDS <= 160 * 1024, "workgroups per CU");
+  static constexpr int Q_BYTES = 128 * RS;                          // the Q tile starts out in the third buffer
+  static constexpr int LDS = 2 * TILE_BYTES + (Q_BYTES > TILE_BYTES ? Q_BYTES : TILE_BYTES);
+  static_assert(2 * LDS <= 160 * 1024, "two workgroups per CU");
 };
 
 // ROPE_Q: the keys were rotated in place beforehand; the query rows are rotated here while they are staged (a
 // query block is staged once, whereas every query block of a segment would rotate the segment's keys again).
-template <int D, bool ROPE_Q = false, int NB = 3>
-__global__ __launch_bounds__(256, (NB == 2 ? 3 : 2)) void attn_full_direct_kernel(const AttnArgs a) {
+template <int D, bool ROPE_Q = false>
+__global__ __launch_bounds__(256, 2) void attn_full_direct_kernel(const AttnArgs a) {
   constexpr int NT = 256, BQ = 128;
   static_assert(!ROPE_Q || D % 16 == 0, "rotary needs an even number of 16-byte chunks per half");
-  using Shape = AttnDirectShape<D, NB>;
+  using Shape = AttnDirectShape<D>;
   constexpr int KS = Shape::KS, DT = (D + 31) / 32, DC = Shape::DC, DKC = Shape::DKC;
   constexpr int RS = Shape::RS, K_SLOTS = Shape::K_SLOTS, V_SLOTS = Shape::V_SLOTS;
   constexpr int K_BYTES = Shape::K_BYTES, TILE_BYTES = Shape::TILE_BYTES;
@@ -686,16 +759,16 @@ __global__ __launch_bounds__(256, (NB == 2 ? 3 : 2)) void attn_full_direct_kerne
   extern __shared__ __attribute__((aligned(1024))) char lds[];
   auto k_buf = [&](int b) -> char* { return lds + b * TILE_BYTES; };
   auto v_buf = [&](int b) -> char* { return lds + b * TILE_BYTES + K_BYTES; };
-  char* const q_lds = lds + TILE_BYTES;
+  char* const q_lds = lds + 2 * TILE_BYTES;
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int fr = lane & 31, hf = lane >> 5;
   const int xcd = blockIdx.x & 7, j = blockIdx.x >> 3;   // workgroup mapping: see attn_full_kernel
   const int cid = (j / a.chunk) * 8 + xcd;
-  const int item = (cid % a.n_chunks_x) * a.chunk + j % a.chunk;
-  const int head = cid / a.n_chunks_x;
-  if (item >= a.n_work || head >= a.heads) return;
+  const int item = (cid / a.heads) * a.chunk + j % a.chunk;
+  const int head = cid % a.heads;
+  if (item >= a.n_work) return;
   const int seg_start = a.work[item * 4 + 0];
   const int seg_end = a.work[item * 4 + 1];
   const int q0 = a.work[item * 4 + 2];
@@ -708,41 +781,51 @@ __global__ __launch_bounds__(256, (NB == 2 ? 3 : 2)) void attn_full_direct_kerne
   // ---- the wave's direct loads of a tile.  Load u of this wave is load number jl = min(4u + wave, LOADS-1) of the
   //      tile (the clamp makes a wave without a load of its own repeat the last one: every wave must issue the
   //      same number, because the waits count loads).  Byte offsets are relative to the segment's first row.
-  const __amdgpu_buffer_rsrc_t rsrc_k =
-      __builtin_amdgcn_make_buffer_rsrc((void*)(a.k + (int64_t)seg_start * a.ld + hoff), 0, -1, 0x00020000);
-  const __amdgpu_buffer_rsrc_t rsrc_v =
-      __builtin_amdgcn_make_buffer_rsrc((void*)(a.v + (int64_t)seg_start * a.ld + hoff), 0, -1, 0x00020000);
   const uint32_t row_bytes = (uint32_t)a.ld * 2u;
-  int l_row[PER], l_chunk[PER];
+  const uint64_t k_base = (uint64_t)(a.k + (int64_t)seg_start * a.ld + hoff), v_base = (uint64_t)(a.v + (int64_t)seg_start * a.ld + hoff);
+  uint32_t l_off[PER], l_dst[PER];   // offset in a whole tile, LDS address in buffer 0
+  uint64_t l_mask[PER];              // the lanes that own data slots
+  i32x4_sgpr_t l_rsrc[PER];
+  // row and 16-byte column of this lane's slot of load u
+  auto slot_of = [&](int u, int ln, int& row, int& chunk) {
+    const int jl = min(4 * u + wave, LOADS - 1);
+    const bool is_k = jl < K_LOADS;
+    const int slot = (is_k ? jl : jl - K_LOADS) * 64 + ln;
+    const int per_row = is_k ? K_SLOTS : V_SLOTS;
+    row = slot / per_row;
+    chunk = slot - row * per_row;
+  };
 #pragma unroll
   for (int u = 0; u < PER; ++u) {
     const int jl = min(4 * u + wave, LOADS - 1);
     const bool is_k = jl < K_LOADS;
-    const int slot = (is_k ? jl : jl - K_LOADS) * 64 + lane;
-    const int per_row = is_k ? K_SLOTS : V_SLOTS;
-    l_row[u] = slot / per_row;
-    l_chunk[u] = slot - l_row[u] * per_row;   // >= DC: a padding slot, the lane sits the load out
+    int row, chunk;
+    slot_of(u, lane, row, chunk);
+    l_mask[u] = __ballot(chunk < DC);
+    l_off[u] = (uint32_t)row * row_bytes + (uint32_t)chunk * 16u;
+    const uint64_t base = is_k ? k_base : v_base;
+    l_rsrc[u] = i32x4_sgpr_t{__builtin_amdgcn_readfirstlane((int)(uint32_t)base), __builtin_amdgcn_readfirstlane((int)((base >> 32) & 0xFFFFu)), -1, 0x00020000};
+    l_dst[u] = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_void_t*)lds + (uint32_t)(is_k ? jl * 1024 : K_BYTES + (jl - K_LOADS) * 1024));
   }
-  auto issue_k = [&](char* dst, uint32_t off, uint32_t soff) {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_k, (lds_void_t*)dst, 16, off, soff, 0, 0);
-  };
-  auto issue_v = [&](char* dst, uint32_t off, uint32_t soff) {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_v, (lds_void_t*)dst, 16, off, soff, 0, 0);
+  auto issue_load = [&](uint32_t dst, uint64_t mask, uint32_t off, i32x4_sgpr_t rsrc, uint32_t soff) {
+    uint64_t exec_was;   // (m0, the LDS address, is nobody else's in this kernel: no builtin that uses it is called)
+    asm volatile("s_mov_b32 m0, %1\n\ts_and_saveexec_b64 %0, %2\n\tbuffer_load_dwordx4 %3, %4, %5 offen lds\n\ts_mov_b64 exec, %0"
+                 : "=&s"(exec_was) : "s"(dst), "s"(mask), "v"(off), "s"(rsrc), "s"(soff) : "scc", "memory");
   };
   auto issue_tile = [&](int t, int b) {
     const int nvalid = min(BKV, seg_len - t * BKV);
-    const uint32_t soff = (uint32_t)(t * BKV) * row_bytes;
+    const uint32_t soff = (uint32_t)(t * BKV) * row_bytes, to = (uint32_t)(b * TILE_BYTES);
+    if (nvalid == BKV) {
 #pragma unroll
-    for (int u = 0; u < PER; ++u) {
-      const int jl = min(4 * u + wave, LOADS - 1);
-      // rows past the segment end repeat the last valid row: as keys they are masked, and P = 0 times a finite V row is 0
-      const uint32_t off = (uint32_t)min(l_row[u], nvalid - 1) * row_bytes + (uint32_t)l_chunk[u] * 16u;
-      if (jl < K_LOADS) {   // uniform
-        char* dst = k_buf(b) + jl * 1024;
-        if (l_chunk[u] < DC) issue_k(dst, off, soff);
-      } else {
-        char* dst = v_buf(b) + (jl - K_LOADS) * 1024;
-        if (l_chunk[u] < DC) issue_v(dst, off, soff);
+      for (int u = 0; u < PER; ++u) issue_load(l_dst[u] + to, l_mask[u], l_off[u], l_rsrc[u], soff);
+    } else {   // rows past the segment end repeat the last valid row: as keys they are masked, and P = 0 times a finite V row is 0
+      int lane_p = lane;
+      asm volatile("" : "+v"(lane_p));   // (once a segment: its offsets are not kept in registers across the loop)
+#pragma unroll
+      for (int u = 0; u < PER; ++u) {
+        int row, chunk;
+        slot_of(u, lane_p, row, chunk);
+        issue_load(l_dst[u] + to, l_mask[u], (uint32_t)min(row, nvalid - 1) * row_bytes + (uint32_t)chunk * 16u, l_rsrc[u], soff);
       }
     }
   };
@@ -753,140 +836,202 @@ __global__ __launch_bounds__(256, (NB == 2 ? 3 : 2)) void attn_full_direct_kerne
         *(bf16x8_t*)(k_buf(b) + r * RS + c * 16) = zero8;
       }
     }
-    if constexpr (L_FROM_MFMA) {
-      bf16x8_t one = zero8;
-      one[0] = f2bf(1.0f);
-      for (int r = tid; r < BKV; r += NT) *(bf16x8_t*)(v_buf(b) + r * V_RS + DC * 16) = one;
+    // (V columns past the head dim: the column of ones, then zeros -- rows of O^T that nobody reads, but random bytes there would
+    // cost the multipliers power)
+    constexpr int VPAD = L_FROM_MFMA ? V_SLOTS - DC : 0;
+    for (int i = tid; i < BKV * VPAD; i += NT) {
+      const int r = i / (VPAD ? VPAD : 1), c = i - r * VPAD;
+      bf16x8_t x = zero8;
+      if (c == 0) x[0] = f2bf(1.0f);
+      *(bf16x8_t*)(v_buf(b) + r * V_RS + (DC + c) * 16) = x;
     }
   };
-  auto wait_loads = [&](auto pending_c) {   // at most `pending` of this wave's direct loads still in flight
-    constexpr int N = decltype(pending_c)::value;
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-  };
-  auto barrier = [&]() {
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  // every load of this wave has landed and every LDS access is done, in every wave
+  auto sync_all = [&]() {
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
   };
 
-  // ---- prologue: tile 0 requested, Q -> LDS -> fragments, then the Q region becomes buffers 1 and 2
+  // ---- prologue: tiles 0 and 1 requested; Q, all of its loads in flight together, -> LDS (third buffer) -> fragments
   issue_tile(0, 0);
-  init_padding(0);
+  if (n_tiles > 1) issue_tile(1, 1);
   if constexpr (ROPE_Q) {
-    constexpr int HC = DC / 2;   // chunks per half; D % 16 == 0, so there are no padding chunks (DKC == DC)
-    for (int i = tid; i < BQ * HC; i += NT) {
-      const int r = i / HC, jc = i - r * HC;
-      bf16x8_t o1 = zero8, o2 = zero8;
-      if (r < nq) {
-        const int64_t g = q0 + r;
-        const bf16_t* p = a.q + g * a.ld + hoff + jc * 8;
-        const bf16x8_t x1 = *(const bf16x8_t*)p;
-        const bf16x8_t x2 = *(const bf16x8_t*)(p + D / 2);
-        const float* cs = a.cos_sin + g * D + jc * 8;
-        const f32x4_t c0 = *(const f32x4_t*)cs, c1 = *(const f32x4_t*)(cs + 4);
-        const f32x4_t s0 = *(const f32x4_t*)(cs + D / 2), s1 = *(const f32x4_t*)(cs + D / 2 + 4);
+    constexpr int HC = DC / 2, ITEMS = BQ * HC, N = (ITEMS + NT - 1) / NT;   // D % 16 == 0: no padding chunks (DKC == DC)
+    bf16x8_t x1[N], x2[N];
+    f32x4_t c0[N], c1[N], s0[N], s1[N];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const float co = e < 4 ? c0[e] : c1[e - 4];
-          const float si = e < 4 ? s0[e] : s1[e - 4];
-          const float xa = bf2f(x1[e]), xb = bf2f(x2[e]);
-          o1[e] = f2bf(rot_first(xa, xb, co, si));
-          o2[e] = f2bf(rot_second(xa, xb, co, si));
-        }
+    for (int it = 0; it < N; ++it) {
+      const int i = min(tid + it * NT, ITEMS - 1), r = i / HC, jc = i - r * HC;
+      const int64_t g = q0 + min(r, nq - 1);
+      const bf16_t* p = a.q + g * a.ld + hoff + jc * 8;
+      x1[it] = *(const bf16x8_t*)p;
+      x2[it] = *(const bf16x8_t*)(p + D / 2);
+      const float* cs = a.cos_sin + g * D + jc * 8;
+      c0[it] = *(const f32x4_t*)cs;
+      c1[it] = *(const f32x4_t*)(cs + 4);
+      s0[it] = *(const f32x4_t*)(cs + D / 2);
+      s1[it] = *(const f32x4_t*)(cs + D / 2 + 4);
+    }
+    init_padding(0);
+    init_padding(1);
+#pragma unroll
+    for (int it = 0; it < N; ++it) {
+      const int i = min(tid + it * NT, ITEMS - 1), r = i / HC, jc = i - r * HC;
+      bf16x8_t o1, o2;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float co = e < 4 ? c0[it][e] : c1[it][e - 4];
+        const float si = e < 4 ? s0[it][e] : s1[it][e - 4];
+        const float xa = bf2f(x1[it][e]), xb = bf2f(x2[it][e]);
+        o1[e] = f2bf(rot_first(xa, xb, co, si));
+        o2[e] = f2bf(rot_second(xa, xb, co, si));
       }
       *(bf16x8_t*)(q_lds + r * RS + jc * 16) = o1;
       *(bf16x8_t*)(q_lds + r * RS + (jc + HC) * 16) = o2;
     }
   } else {
-    for (int i = tid; i < BQ * DKC; i += NT) {
-      const int r = i / DKC, c = i - r * DKC;
-      bf16x8_t x = zero8;
-      if (r < nq && c < DC) x = *(const bf16x8_t*)(a.q + (int64_t)(q0 + r) * a.ld + hoff + c * 8);
-      *(bf16x8_t*)(q_lds + r * RS + c * 16) = x;
+    constexpr int N = BQ * DKC / NT;
+    static_assert(BQ * DKC % NT == 0, "whole batches");
+    bf16x8_t x[N];
+#pragma unroll
+    for (int it = 0; it < N; ++it) {
+      const int i = tid + it * NT, r = i / DKC, c = i - r * DKC;
+      x[it] = *(const bf16x8_t*)(a.q + (int64_t)(q0 + min(r, nq - 1)) * a.ld + hoff + min(c, DC - 1) * 8);
+    }
+    init_padding(0);
+    init_padding(1);
+#pragma unroll
+    for (int it = 0; it < N; ++it) {
+      const int i = tid + it * NT, r = i / DKC, c = i - r * DKC;
+      *(bf16x8_t*)(q_lds + r * RS + c * 16) = c < DC ? x[it] : zero8;
     }
   }
-  __syncthreads();
+  sync_all();   // (tiles 0 and 1 have landed with the Q rows)
   bf16x8_t qf[KS];
 #pragma unroll
   for (int ks = 0; ks < KS; ++ks) qf[ks] = *(const bf16x8_t*)(q_lds + (wave * 32 + fr) * RS + (2 * ks + hf) * 16);
-  __syncthreads();
-  init_padding(1);
-  if constexpr (NB == 3) {
-    init_padding(2);
-    if (n_tiles > 1) issue_tile(1, 1);
-  }
 
   f32x16_t oacc[DT];
 #pragma unroll
   for (int t = 0; t < DT; ++t)
 #pragma unroll
     for (int r = 0; r < 16; ++r) oacc[t][r] = 0.f;
-  float m_run = -INFINITY, l_run = 0.f;
+  float m_run = 0.f, mb = 0.f, l_run = 0.f;
   const bool wave_active = wave * 32 < nq;
-  const float sl2 = a.scale_log2e;
+  const float sl2 = a.scale_log2e, shift = n_tiles > 1 ? P_SHIFT_LOG2 : 0.0f;
+  const int sg = lane & 15;
+  const int k_lane = fr * RS + hf * 16;
+  const int v_lane = (4 * hf + (sg >> 2)) * V_RS + (16 * ((lane >> 4) & 1) + 4 * (sg & 3)) * 2;   // see read_vt_frag
 
-  int buf = 0, buf2 = 2;   // buffers of tile t and of tile t+2
-  for (int t = 0; t < n_tiles; ++t) {
-    // Tile t has landed when only the loads requested after it (tile t+1's) are in flight; the barrier then also
-    // says that every wave is done with tile t-1, whose buffer the request for tile t+2 reuses.
-    if constexpr (NB == 3) {
-      if (t + 1 < n_tiles) wait_loads(std::integral_constant<int, PER>{});
-      else wait_loads(std::integral_constant<int, 0>{});
-      barrier();
-      if (t + 2 < n_tiles) issue_tile(t + 2, buf2);
-    } else {   // two buffers: tile t+1 travels while tile t is worked on (three workgroups per CU hide the rest)
-      wait_loads(std::integral_constant<int, 0>{});
-      barrier();
-      if (t + 1 < n_tiles) issue_tile(t + 1, buf ^ 1);
-    }
-    const int nvalid = min(BKV, seg_len - t * BKV);
-    if (wave_active) {
-      const char* kd = k_buf(buf);
-      const char* vd = v_buf(buf);
-      f32x16_t sacc[2];
-      bf16x8_t pf[2][2];
-      score_tile<KS, RS>(sacc, kd, qf, nvalid, fr, hf);
-      softmax_tile<DT, L_FROM_MFMA>(sacc, pf, oacc, m_run, l_run, sl2);
-      // V^T fragments (see read_vt_frag for the addressing).  The transposing reads are written in assembly: as
-      // an intrinsic, the compiler takes them for possible readers of the LDS bytes that the direct loads in
-      // flight will write and puts a wait for ALL outstanding loads in front of them -- the tiles requested
-      // ahead included.  The waits on the reads themselves are therefore explicit too: the reads of block
-      // tt+1 are issued before the MFMAs of block tt, which wait until only those 8 are outstanding.
-      {
-        const int sg = lane & 15;
-        const uint32_t vbase = (uint32_t)(uintptr_t)(lds_void_t*)vd + (uint32_t)((4 * hf + (sg >> 2)) * V_RS + (16 * ((lane >> 4) & 1) + 4 * (sg & 3)) * 2);
-        i32x2_t vraw[2][8];   // [block parity][2 * fragment + half]
-        read_vt_block_asm<0>(vraw[0], vbase);
-        read_vt_block_asm<1>(vraw[1], vbase);
-        pv_block<false>(oacc[0], vraw[0], pf);
-        if constexpr (DT == 2) {
-          pv_block<true>(oacc[1], vraw[1], pf);
-        } else {
-          static_assert(DT == 3, "head dims up to 96");
-          read_vt_block_asm<2>(vraw[0], vbase);
-          pv_block<false>(oacc[1], vraw[1], pf);
-          pv_block<true>(oacc[DT - 1], vraw[0], pf);
-        }
+  auto read_k = [&](bf16x8_t (&kf)[KS], int b, int half) {
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) kf[ks] = *(const bf16x8_t*)(k_buf(b) + k_lane + half * 32 * RS + ks * 32);
+  };
+  auto read_v = [&](bf16x8_t (&vf)[DT][2], int b, int half) {
+#pragma unroll
+    for (int t = 0; t < DT; ++t)
+#pragma unroll
+      for (int kk = 0; kk < 2; ++kk) {
+        const char* p = v_buf(b) + v_lane + (32 * half + 16 * kk) * V_RS + t * 64;
+        const s16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t*)p);
+        const s16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t*)(p + 8 * V_RS));
+        vf[t][kk] = __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
       }
+  };
+  auto scores = [&](f32x16_t& s, const bf16x8_t (&kf)[KS]) {
+    const f32x16_t z = {};
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[ks], qf[ks], ks == 0 ? z : s, 0, 0, 0);
+  };
+  auto pv = [&](const i32x4_t (&p)[2], const bf16x8_t (&vf)[DT][2]) {
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+      for (int t = 0; t < DT; ++t) oacc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[t][kk], __builtin_bit_cast(bf16x8_t, p[kk]), oacc[t], 0, 0, 0);
+  };
+  // keys past `nvalid` of the tile (the last tile of a segment only)
+  auto mask = [&](f32x16_t& s, int nvalid, int half) {
+    int left = nvalid - half * 32 - 4 * hf;
+    asm volatile("" : "+v"(left));   // one register compared with constants, not 32 loop-invariant comparisons kept in registers
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+      if (8 * (r >> 2) + (r & 3) >= left) s[r] = -INFINITY;
+  };
+  // One step: O += V^T.P of p_in and vf, s_out = scores of half k_half of the tile in buffer k_b, p_out = softmax of s_in; meanwhile
+  // the V fragments of the next step are read (half v_half of the tile in buffer v_b).
+  auto step = [&](const f32x16_t& s_in, i32x4_t (&p_out)[2], f32x16_t& s_out, const i32x4_t (&p_in)[2],
+                  const bf16x8_t (&vf)[DT][2], int k_b, int k_half, bf16x8_t (&vf_next)[DT][2], int v_b, int v_half) {
+    bf16x8_t kf[KS];
+    read_k(kf, k_b, k_half);
+    read_v(vf_next, v_b, v_half);
+    pv(p_in, vf);
+    scores(s_out, kf);
+    float l_new = l_run;
+    const uint32_t any = exp_half<!L_FROM_MFMA>(s_in, p_out, sl2, mb, l_new);
+    // per matrix instruction two LDS reads, its share of the plain vector instructions (16 multiply-adds, 8 conversions, 4 ORs, the
+    // sums, a few addresses) and two exponentials
+    constexpr int N_MFMA = KS + 2 * DT, N_VALU = (L_FROM_MFMA ? 32 : 48) / N_MFMA + (L_FROM_MFMA ? 1 : 0);
+#pragma unroll
+    for (int i = 0; i < N_MFMA; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+      __builtin_amdgcn_sched_group_barrier(0x002, N_VALU, 0);
+      __builtin_amdgcn_sched_group_barrier(0x400, 2, 0);
     }
-    if constexpr (NB == 3) {
-      buf2 = buf;   // tile t+3 will reuse this iteration's buffer
-      buf = buf == 2 ? 0 : buf + 1;
-    } else {
-      buf ^= 1;
-    }
-  }
+    if (__any((any & P_TWO_BIT) != 0)) raise_reference<DT, !L_FROM_MFMA>(s_in, p_out, oacc, m_run, mb, l_run, sl2, shift);
+    else l_run = l_new;
+  };
 
+  f32x16_t s0, s1;
+  bf16x8_t vfa[DT][2], vfb[DT][2];
+  i32x4_t p0[2], p1[2];
+#pragma unroll
+  for (int t = 0; t < DT; ++t) vfa[t][0] = vfa[t][1] = zero8;
+  p1[0] = p1[1] = i32x4_t{0, 0, 0, 0};   // the first step multiplies zeros
+  if (wave_active) {
+    bf16x8_t kfa[KS], kfb[KS];
+    read_k(kfa, 0, 0);
+    read_k(kfb, 0, 1);
+    scores(s0, kfa);
+    scores(s1, kfb);
+    if (seg_len < BKV) {
+      mask(s0, seg_len, 0);
+      mask(s1, seg_len, 1);
+    }
+    m_run = pair_max(fmaxf(row_max(s0), row_max(s1)));
+    mb = __builtin_fmaf(m_run, sl2, shift);
+  }
+  int b0 = 0, b1 = 1, b2 = 2;   // buffers of tiles t, t+1, t+2
+  for (int t = 0; t < n_tiles; ++t) {
+    sync_all();   // tile t+1 has landed; every wave has read what it needs of tile t-1 (t == 0: of the Q tile), whose buffer is free
+    if (t == 0) init_padding(2);   // (read two barriers from here at the earliest)
+    if (t + 2 < n_tiles) issue_tile(t + 2, b2);
+    if (wave_active) {
+      const int left = seg_len - t * BKV;
+      step(s0, p0, s1, p1, vfa, b0, 1, vfb, b0, 0);   // scores: second half of t; P.V: second half of t-1; softmax: first half of t
+      if (left < BKV) mask(s1, left, 1);
+      // (behind the last tile, the scores of whatever the next buffer holds are computed and not used)
+      step(s1, p1, s0, p0, vfb, b1, 0, vfa, b0, 1);   // scores: first half of t+1; P.V: first half of t; softmax: second half of t
+      if (left > BKV && left < 2 * BKV) mask(s0, left - BKV, 0);
+    }
+    const int bt = b0;
+    b0 = b1;
+    b1 = b2;
+    b2 = bt;
+  }
+  if (wave_active) pv(p1, vfa);
+
+  if constexpr (!L_FROM_MFMA) l_run += __shfl_xor(l_run, 32, 64);
   const int qi = wave * 32 + fr;
   write_output<D, DT, L_FROM_MFMA>(oacc, l_run, a.out + (int64_t)(q0 + min(qi, nq - 1)) * a.ldo + hoff, qi < nq, hf);
 }
 
-
-template <int D, bool ROPE_Q = false, int NB = 3>
+template <int D, bool ROPE_Q = false>
 int launch_attn_full_direct(const AttnArgs& a, dim3 grid, hipStream_t stream) {
-  constexpr int lds = AttnDirectShape<D, NB>::LDS;
+  constexpr int lds = AttnDirectShape<D>::LDS;
   static bool attr_set = false;
-  auto kern = attn_full_direct_kernel<D, ROPE_Q, NB>;
+  auto kern = attn_full_direct_kernel<D, ROPE_Q>;
   if (!attr_set) {
     if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
       return CS_ERR_LAUNCH;
@@ -906,15 +1051,11 @@ int launch_attn(AttnArgs a, int n_work, int heads, int block_q, int max_seqlen, 
   a.n_chunks_x = (n_work + a.chunk - 1) / a.chunk;
   const int n_chunks = a.n_chunks_x * heads;
   const dim3 grid_full(((n_chunks + 7) / 8) * 8 * a.chunk);
-  // The direct-to-LDS kernel with two tile buffers and three workgroups per CU where its LDS allows (head dims up to
-  // 80): the softmax keeps the vector unit as busy as the matrix cores, so a third wave per SIMD buys more overlap
-  // than a third buffer of prefetch (measured: 4096 keys at d = 72 513 -> 444 us, 1024 keys at d = 80 87 -> 80 us).
-  constexpr int RING_DEPTH = D <= 80 ? 2 : 3;
   if (keys_rotated) {
     // only the long-segment kernel has this form (short segments rotate q and k while staging, one workgroup each)
     if constexpr (D % 16 == 0) {
       if (block_q != 64 && rope && (int64_t)max_seqlen * a.ld * 2 < (int64_t)1 << 31)
-        return launch_attn_full_direct<D, true, RING_DEPTH>(a, grid_full, stream);
+        return launch_attn_full_direct<D, true>(a, grid_full, stream);
     }
     return CS_ERR_UNSUPPORTED;
   }
@@ -938,7 +1079,7 @@ int launch_attn(AttnArgs a, int n_work, int heads, int block_q, int max_seqlen, 
     } else {
       // the direct-to-LDS kernel addresses a segment's K/V rows with 32-bit byte offsets
       if ((int64_t)max_seqlen * a.ld * 2 < (int64_t)1 << 31)
-        return launch_attn_full_direct<D, false, RING_DEPTH>(a, grid_full, stream);
+        return launch_attn_full_direct<D, false>(a, grid_full, stream);
       hipLaunchKernelGGL((attn_full_kernel<D, false>), grid_full, dim3(256), 0, stream, a);
     }
   }

@@ -483,7 +483,8 @@ class AttnPlan:
 
 
 def attn_work_host(cu_seqlens_host: np.ndarray) -> tuple[np.ndarray, int]:
-    """Host half of attn_plan: the work list int32 [n_work, 4] (still on the host) and the longest segment."""
+    """Host half of attn_plan: the work list int32 [n_work, 4] (still on the host) and the longest segment.  Query blocks of the
+    longest segments come first: workgroups start in list order, and one that streams the most keys must not start last."""
     lib = _l.load()
     cu = np.ascontiguousarray(cu_seqlens_host, dtype=np.int32)
     n_seg = cu.shape[0] - 1
@@ -497,7 +498,10 @@ def attn_work_host(cu_seqlens_host: np.ndarray) -> tuple[np.ndarray, int]:
     n_work = ctypes.c_int32(0)
     _l.check(lib.cs_attn_work_host(cu.ctypes.data, n_seg, bq, work.ctypes.data, cap, ctypes.byref(n_work)),
              "cs_attn_work_host")
-    return work[: n_work.value], max_seqlen
+    work = work[: n_work.value]
+    if max_seqlen > 64 and int(lens.min()) < max_seqlen:
+        work = np.ascontiguousarray(work[np.argsort(work[:, 0] - work[:, 1], kind="stable")])
+    return work, max_seqlen
 
 
 def attn_plan(cu_seqlens_host: np.ndarray, device: torch.device) -> AttnPlan:

@@ -1125,6 +1125,55 @@ def test_attention_short_segment_same_bits_in_either_kernel(ops, dev, d, rotary)
     assert torch.equal(both[:104], short)
 
 
+@pytest.mark.parametrize("d,rotary", [(64, False), (64, True), (72, False), (80, False), (80, True), (96, False), (96, True)])
+def test_attention_segment_lengths_around_tiles_and_query_blocks(ops, dev, d, rotary):
+    """The long-segment kernels at the edges of half tiles (32 keys), tiles (64) and query blocks (128), in one batch and in
+    mixed order: against fp32 (bar: bf16 inputs and weights of P, as in the tests above), and every segment alone equals the
+    segment in the batch bit for bit."""
+    nh, lens = 4, [65, 1, 96, 97, 127, 128, 129, 31, 192, 193, 255, 257, 64, 320, 450]
+    cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    L, H = int(cu[-1]), nh * d
+    g = torch.Generator().manual_seed(31)
+    qkv = torch.randn((L, 3 * H), generator=g).bfloat16().to(dev)
+    ang = torch.rand((L, d // 2), generator=g) * 6.0 if rotary else None
+    cs = torch.cat([ang.cos(), ang.sin()], dim=1).float().contiguous().to(dev) if rotary else None
+
+    def run(lo, hi, seg):
+        x = qkv[lo:hi].clone()
+        plan = ops.attn_plan(np.asarray(seg, np.int32), dev)
+        if rotary:
+            return ops.attn_varlen_rotary_(x, plan, nh, d, d**-0.5, cs[lo:hi].contiguous())
+        return ops.attn_varlen(x[:, :H], x[:, H:2 * H], x[:, 2 * H:], plan, nh, d, d**-0.5)
+
+    got = run(0, L, cu)
+    close(got, attn_ref(qkv, cu.tolist(), nh, d, ang), 2**-6, f"d={d} rotary={rotary}")
+    for i, n in enumerate(lens):
+        assert torch.equal(run(int(cu[i]), int(cu[i + 1]), [0, n]), got[cu[i]:cu[i + 1]]), f"segment of {n} rows"
+
+
+@pytest.mark.parametrize("d", [72, 80, 96])
+def test_attention_query_is_independent_of_its_neighbours(ops, dev, d):
+    """Raising the reference maximum of one query (its largest scores sit in the last tile and exceed the first tile's by far
+    more than 2^9) must not touch the bits of the queries that share its wave; infinite and NaN queries stay their own."""
+    nh, L = 2, 300
+    H = nh * d
+    g = torch.Generator().manual_seed(33)
+    qkv = torch.randn((L, 3 * H), generator=g)
+    qkv[256:, H:2 * H] *= 8.0
+    qkv = qkv.bfloat16().to(dev)
+    plan = ops.attn_plan(np.array([0, L], np.int32), dev)
+    run = lambda x: ops.attn_varlen(x[:, :H], x[:, H:2 * H], x[:, 2 * H:], plan, nh, d, d**-0.5)   # noqa: E731
+    base = run(qkv)
+    close(base, attn_ref(qkv, [0, L], nh, d), 2**-6, f"raised late d={d}")
+    for value in (40.0, float("inf"), float("nan")):
+        x = qkv.clone()
+        x[37, :H] = x[37, :H] * value
+        out = run(x)
+        keep = torch.arange(L, device=dev) != 37
+        assert torch.equal(out[keep], base[keep]), value
+        assert bool(torch.isfinite(out[37].float()).all()) == (value == 40.0)
+
+
 def test_rotary_head_dim_72(ops, dev):
     """Qwen3-VL: head dim 72, rotary halves of 36 (the 8-byte-vector path of the in-place kernel)."""
     nh, d, L = 16, 72, 333
