@@ -7,9 +7,12 @@
 // Epilogue / folded-norm dispatch of one tile form each (gemm_fast_t<rows>x<cols>.hip).
 int cs_gemm_fast_tile_256x256(const CsGemmArgs& a, hipStream_t stream);
 int cs_gemm_fast_tile_256x160(const CsGemmArgs& a, hipStream_t stream);
-int cs_gemm_fast_tile_128x160(const CsGemmArgs& a, hipStream_t stream);
-int cs_gemm_fast_tile_128x192(const CsGemmArgs& a, hipStream_t stream);
 int cs_gemm_fast_tile_256x128(const CsGemmArgs& a, hipStream_t stream);
+int cs_gemm_fast_tile_224x192(const CsGemmArgs& a, hipStream_t stream);
+int cs_gemm_fast_tile_192x192(const CsGemmArgs& a, hipStream_t stream);
+int cs_gemm_fast_tile_192x160(const CsGemmArgs& a, hipStream_t stream);
+int cs_gemm_fast_tile_128x192(const CsGemmArgs& a, hipStream_t stream);
+int cs_gemm_fast_tile_128x160(const CsGemmArgs& a, hipStream_t stream);
 // The few-row kernel (gemm_small.hip).
 int cs_gemm_small(const CsGemmArgs& a, hipStream_t stream, bool* handled);
 int cs_gemm_small_workgroups(const CsGemmArgs& a);
@@ -18,11 +21,92 @@ namespace {
 
 using csgemm::BK;
 
-// Time of a launch in units of "one 256x256 tile on every CU": rounds of 256 workgroups times tile area.
-double rounds_cost(int M, int N, int bm, int bn) {
-  const int64_t tiles = (int64_t)((M + bm - 1) / bm) * ((N + bn - 1) / bn);
-  const int64_t rounds = (tiles + 255) / 256;
-  return (double)rounds * bm * bn / (256.0 * 256.0);
+// Time of a launch in microseconds: LAUNCH_US; per round of 256 tiles, and per K tile of 64, `stage` plus `flow` times the share of the
+// compute units that have a tile (full launches draw more power and more bandwidth); and what the epilogues add -- per round: bias
+// alone, SwiGLU, another activation, a folded LayerNorm; residual products: the workgroup's last tile, whose residual piece came
+// through the ring, and the tiles before it.  Fitted to 27 products of the encoders at up to 34 row counts from 1100 to 20000, every
+// form that takes them, weights from HBM (about 3,700 launches; root mean square error 2 to 3 % with fp8 weights, 8 to 10 % with
+// bf16 ones, most of it common to all forms of a product).  A launch is as long as its rounds, and a round as long as a tile of
+// its form however few of the 256 compute units have one, so what counts is a form whose tiles fill whole rounds: 6240 rows x 3456
+// (folded LayerNorm) are 550 tiles of 256x160 in three rounds, 58.6 us, and 504 of 224x192 in two, 45.2 us.  Chosen by this table,
+// launches take 1.010 of the time of the best form on average (residual products from 2500 rows on, the others from 1000); with
+// five forms (256x256, 256x160 and its 128-row half, 256x128 and 128x192 behind whole rounds of 256x256) and tile area as the
+// cost they took 1.062.
+struct FormUs {
+  float bias, swiglu, act, ln, res, res_more, stage, flow;
+};
+struct BigForm {
+  int bm, bn;
+  FormUs bf16, fp8;
+  int (*run)(const CsGemmArgs&, hipStream_t);
+};
+constexpr float LAUNCH_US = 3.0f;
+const BigForm FORMS[] = {
+    {256, 256, {5.7f, 6.1f, 11.8f, 0.f, 18.9f, 21.3f, 0.99f, 0.38f}, {6.5f, 6.0f, 28.8f, 0.f, 20.2f, 18.9f, 1.08f, 0.29f}, cs_gemm_fast_tile_256x256},
+    {256, 160, {4.2f, 4.4f, 8.4f, 6.5f, 12.1f, 12.9f, 0.61f, 0.30f}, {5.0f, 4.6f, 18.2f, 0.f, 11.9f, 12.3f, 0.85f, 0.19f}, cs_gemm_fast_tile_256x160},
+    {256, 128, {2.9f, 3.6f, 6.3f, 5.4f, 9.1f, 8.6f, 0.55f, 0.25f}, {3.7f, 3.3f, 14.4f, 0.f, 10.5f, 8.9f, 0.59f, 0.20f}, cs_gemm_fast_tile_256x128},
+    {224, 192, {4.4f, 4.7f, 8.6f, 7.0f, 14.5f, 13.9f, 0.67f, 0.28f}, {4.7f, 4.4f, 18.7f, 0.f, 17.4f, 13.5f, 0.75f, 0.22f}, cs_gemm_fast_tile_224x192},
+    {192, 192, {3.7f, 4.2f, 7.5f, 6.1f, 11.1f, 10.1f, 0.62f, 0.23f}, {4.1f, 3.8f, 15.0f, 0.f, 14.1f, 10.0f, 0.68f, 0.19f}, cs_gemm_fast_tile_192x192},
+    {192, 160, {3.1f, 3.5f, 6.5f, 4.9f, 9.1f, 9.7f, 0.52f, 0.22f}, {3.6f, 3.0f, 11.2f, 0.f, 9.3f, 9.4f, 0.73f, 0.14f}, cs_gemm_fast_tile_192x160},
+    {128, 192, {1.5f, 2.3f, 4.3f, 3.1f, 6.7f, 5.7f, 0.48f, 0.19f}, {3.1f, 2.8f, 9.1f, 0.f, 9.9f, 6.5f, 0.56f, 0.12f}, cs_gemm_fast_tile_128x192},
+    {128, 160, {1.3f, 2.0f, 3.9f, 2.7f, 6.1f, 5.9f, 0.41f, 0.20f}, {0.f, 0.f, 0.f, 0.f, 7.3f, 7.2f, 0.57f, 0.09f}, cs_gemm_fast_tile_128x160},
+};
+
+int64_t tiles_of(const BigForm& f, int M, int N) { return (int64_t)(((uint32_t)M + f.bm - 1) / (uint32_t)f.bm) * (((uint32_t)N + f.bn - 1) / (uint32_t)f.bn); }
+
+double form_us(const BigForm& f, const CsGemmArgs& a, int N) {
+  const FormUs& u = a.w_fp8 ? f.fp8 : f.bf16;
+  const int64_t tiles = tiles_of(f, a.M, N);
+  const double rounds = (double)((tiles + 255) / 256);
+  const double k = (a.K / BK) * (rounds * u.stage + tiles / 256.0 * u.flow);
+  if (a.epilogue == CS_EPI_RESIDUAL) return LAUNCH_US + k + u.res + (rounds - 1) * u.res_more;
+  return LAUNCH_US + k + rounds * (a.a_row_sum ? u.ln : a.epilogue == CS_EPI_BIAS ? u.bias : a.epilogue == CS_EPI_SWIGLU ? u.swiglu : u.act);
+}
+
+// Row sums come in CS_SUMSQ_PARTS parts, one per column tile of the 160-column forms.  A folded LayerNorm's per-column sums do not fit
+// the registers of 256x256, and of 128x160 with fp8 weights only the residual products are built (see dispatch_epi_w, dispatch_epi).
+// The accumulation order of an output element, and of a row-sum part, is the same in every form: the choice changes no bit.
+bool takes(const BigForm& f, const CsGemmArgs& a) {
+  if (a.c_row_sumsq && f.bn != 160) return false;
+  if (a.a_row_sum && f.bm == 256 && f.bn == 256) return false;
+  return !(a.w_fp8 && f.bm == 128 && f.bn == 160 && a.epilogue != CS_EPI_RESIDUAL);
+}
+
+// The form for the first N columns, and its time.
+const BigForm* best_form(const CsGemmArgs& a, int N, double* us) {
+  const BigForm* best = nullptr;
+  for (const BigForm& f : FORMS) {
+    if (!takes(f, a)) continue;
+    const double t = form_us(f, a, N);
+    if (!best || t < 0.98 * *us) {   // (largest tiles first; what is closer than this is a tie, and theirs)
+      best = &f;
+      *us = t;
+    }
+  }
+  return best;
+}
+
+// How a launch is made: `form` alone (lead_cols == 0), or 256x256 tiles over the first lead_cols columns, which fill whole rounds or
+// nearly, and `form` over the rest in a launch of its own.
+struct Plan {
+  const BigForm* form;
+  int lead_cols;
+  double us;
+};
+Plan plan_of(const CsGemmArgs& a) {
+  Plan p = {nullptr, 0, 0};
+  p.form = best_form(a, a.N, &p.us);
+  if (tiles_of(*p.form, a.M, a.N) <= 256 || !takes(FORMS[0], a) || a.c_row_sumsq) return p;   // (one round: nothing to split)
+  Plan split = p;
+  const int tn = (a.N + 255) / 256;
+  for (int c = tn - 1; c >= 1 && c >= tn - 12; --c) {
+    double tail_us = 0;
+    const BigForm* tail = best_form(a, a.N - c * 256, &tail_us);
+    const double t = form_us(FORMS[0], a, c * 256) + tail_us;
+    if (tail != &FORMS[0] && t < split.us) split = {tail, c * 256, t};
+  }
+  // (for a clear gain only: 4096 rows x 6912 x 1280 take 65 us as 256x256 in two rounds, and 72 in two launches of the same estimate)
+  return split.us < 0.96 * p.us ? split : p;
 }
 
 // Whether the direct-to-LDS kernels (the big tiles and the few-row kernel) take a problem.
@@ -54,79 +138,38 @@ int cs_gemm_fast(const CsGemmArgs& a, hipStream_t stream, bool* handled) {
   }
   *handled = true;
   if (a.a_norm_inline) return CS_ERR_UNSUPPORTED;   // the inline norms exist in the few-row kernel only
-  // Tile shape: the one that needs the least chip time (tile quantisation over the 256 CUs).  The narrow
-  // 256x160 tile exists for N = 1280 (8 column tiles: 8192 rows give exactly 256 workgroups).
-  const double c256 = rounds_cost(a.M, a.N, 256, 256);
-  const double c160 = rounds_cost(a.M, a.N, 256, 160) * 1.15;  // narrower tiles: more LDS and L2 traffic per FLOP
-  // Few rows: 160-column tiles of 256 rows would leave half of the compute units or more without a tile (N = 1280
-  // gives 8 column tiles, so 1024 rows are 32 workgroups).  The 128x160 form has the same waves-by-columns layout,
-  // so every output element and every row-sum part is computed by the same sequence of operations: results do not
-  // depend on which of the two a batch size selects.
-  // (fp8 weights: for the residual products, which would fill half of the chip otherwise)
-  const bool few_rows = (!a.w_fp8 || a.epilogue == CS_EPI_RESIDUAL) && (int64_t)((a.M + 255) / 256) * ((a.N + 159) / 160) <= 128;
-  auto narrow = [&]() { return few_rows ? cs_gemm_fast_tile_128x160(a, stream) : cs_gemm_fast_tile_256x160(a, stream); };
-  // Row sums of squares come in CS_SUMSQ_PARTS parts, one per column tile of the 160-column forms.
-  if (a.c_row_sumsq) {
-    if (a.N > CS_SUMSQ_PARTS * 160 || a.w_fp8) return CS_ERR_UNSUPPORTED;
-    return narrow();
+  if (a.c_row_sumsq && (a.N > CS_SUMSQ_PARTS * 160 || a.w_fp8)) return CS_ERR_UNSUPPORTED;
+  const Plan plan = plan_of(a);
+  if (plan.lead_cols == 0) return plan.form->run(a, stream);
+  // two launches that write disjoint column ranges of C
+  const int n1 = plan.lead_cols;
+  CsGemmArgs lo = a, hi = a;
+  lo.N = n1;
+  lo.prefetch = nullptr;  // the tail launch is the one with idle compute units
+  hi.N = a.N - n1;
+  hi.W = (const char*)a.W + (int64_t)n1 * a.ldw * (a.w_fp8 ? 1 : 2);
+  if (a.w_scale) hi.w_scale = a.w_scale + n1;
+  if (a.bias) hi.bias = (const char*)a.bias + (int64_t)n1 * 2;
+  if (a.residual) hi.residual = (const char*)a.residual + (int64_t)n1 * 2;
+  if (a.residual_lo) hi.residual_lo = a.residual_lo + n1;
+  if (a.c_lo) hi.c_lo = a.c_lo + n1;
+  if (a.pos) hi.pos = (const char*)a.pos + (int64_t)n1 * 2;
+  hi.C = (char*)a.C + (int64_t)(a.epilogue == CS_EPI_SWIGLU ? n1 / 2 : n1) * 2;
+  const int st = FORMS[0].run(lo, stream);
+  return st != CS_OK ? st : plan.form->run(hi, stream);
+}
+
+// For the few-row kernel's choice: the time of a launch as a share of what the best of 256x256, 256x128 (SwiGLU), and 256x160 or, for at
+// most 128 tiles of it, 128x160 would take; and the tiles of its (last) launch.
+double cs_gemm_fast_saves(const CsGemmArgs& a, int64_t* tiles) {
+  const Plan p = plan_of(a);
+  *tiles = tiles_of(*p.form, a.M, a.N - p.lead_cols);
+  double of = 0;
+  for (const BigForm& f : FORMS) {
+    const bool narrow = f.bn == 160 && f.bm == ((int64_t)((a.M + 255) / 256) * ((a.N + 159) / 160) <= 128 ? 128 : 256);
+    const bool one = narrow || (!a.c_row_sumsq && f.bm == 256 && (f.bn == 256 || (f.bn == 128 && a.epilogue == CS_EPI_SWIGLU)));
+    const double t = form_us(f, a, a.N);
+    if (one && (of == 0 || t < of)) of = t;
   }
-  if (a.a_row_sum) return narrow();   // see dispatch_epi_w
-  // Few rows and many columns: when 256x128 tiles fit in one round they put more compute units to work than the
-  // forms above (1024 rows x 6912 columns: 216 workgroups against 176 of 256x160 or 108 of 256x256), and a launch
-  // of one round is bound by what a single compute unit pulls in per K tile, not by the chip's throughput.  The
-  // accumulation order of an output element is the same in every tile form, so the choice changes no bit.  Taken
-  // for the SwiGLU epilogue only, where it measures faster inside the model (gate|up of one image); the QKV
-  // projection of two images (240 workgroups against 192) is faster alone and slower in the model.
-  if (a.epilogue == CS_EPI_SWIGLU) {
-    const int64_t t128 = (int64_t)((a.M + 255) / 256) * ((a.N + 127) / 128);
-    const double c128 = rounds_cost(a.M, a.N, 256, 128) * 1.10;
-    if (t128 <= 256 && !few_rows && c128 < c160 - 0.05 && c128 < c256 - 0.05) return cs_gemm_fast_tile_256x128(a, stream);
-  }
-  if (c160 < c256) return narrow();
-  // Column split.  When the last round of 256x256 tiles would leave most CUs idle, the leading columns
-  // that fill whole rounds go to one launch and the remaining columns to a second launch with smaller
-  // tiles (256x128 or 128x192: more workgroups, each shorter).  The two launches write disjoint column
-  // ranges of C.
-  {
-    const int tn = (a.N + 255) / 256;
-    double best = c256;
-    int best_cols = 0;
-    bool best_192 = false;
-    for (int c = tn - 1; c >= 1 && c >= tn - 12; --c) {
-      const int rest = a.N - c * 256;
-      const double lead = rounds_cost(a.M, c * 256, 256, 256);
-      const double c128 = lead + rounds_cost(a.M, rest, 256, 128) * 1.10 + 0.15;  // + per-tile fixed cost of a round
-      const double c192 = lead + rounds_cost(a.M, rest, 128, 192) * 1.20 + 0.15;
-      if (c128 < best - 0.05) {
-        best = c128;
-        best_cols = c;
-        best_192 = false;
-      }
-      if (c192 < best - 0.02) {
-        best = c192;
-        best_cols = c;
-        best_192 = true;
-      }
-    }
-    if (best_cols > 0) {
-      const int n1 = best_cols * 256;
-      CsGemmArgs lo = a, hi = a;
-      lo.N = n1;
-      lo.prefetch = nullptr;  // the tail launch is the one with idle compute units
-      hi.N = a.N - n1;
-      hi.W = (const char*)a.W + (int64_t)n1 * a.ldw * (a.w_fp8 ? 1 : 2);
-      if (a.w_scale) hi.w_scale = a.w_scale + n1;
-      if (a.bias) hi.bias = (const char*)a.bias + (int64_t)n1 * 2;
-      if (a.residual) hi.residual = (const char*)a.residual + (int64_t)n1 * 2;
-      if (a.residual_lo) hi.residual_lo = a.residual_lo + n1;
-      if (a.c_lo) hi.c_lo = a.c_lo + n1;
-      if (a.pos) hi.pos = (const char*)a.pos + (int64_t)n1 * 2;
-      hi.C = (char*)a.C + (int64_t)(a.epilogue == CS_EPI_SWIGLU ? n1 / 2 : n1) * 2;
-      const int st = cs_gemm_fast_tile_256x256(lo, stream);
-      if (st != CS_OK) return st;
-      if (best_192) return cs_gemm_fast_tile_128x192(hi, stream);
-      return cs_gemm_fast_tile_256x128(hi, stream);
-    }
-  }
-  return cs_gemm_fast_tile_256x256(a, stream);
+  return p.us < of ? p.us / of : 1.0;
 }

@@ -137,8 +137,9 @@ template <int BM, int BN, bool W_FP8>
 struct RingShape {
   static constexpr int A_BYTES = BM * BK * 2, W_BYTES = BN * BK * (W_FP8 ? 1 : 2);
   static constexpr bool FIVE_UNITS = A_BYTES == W_BYTES && 5 * A_BYTES <= LDS_BYTES && 3 * (A_BYTES + W_BYTES) > LDS_BYTES;
-  // (the 160-column forms keep the room of a bf16 stage with fp8 weights too: the residual piece passes through the slots)
-  static constexpr int STAGE = A_BYTES + (BN == 160 ? BN * BK * 2 : W_BYTES);
+  // (the forms that are dispatched to residual products keep the room of a bf16 stage with fp8 weights too: the residual piece
+  // passes through the slots)
+  static constexpr int STAGE = A_BYTES + (BN == 160 || (BM == 128 && BN == 192) ? BN * BK * 2 : W_BYTES);
   static constexpr int BYTES = FIVE_UNITS ? 5 * A_BYTES : 3 * STAGE;
   static_assert(BYTES <= LDS_BYTES, "tile does not fit a ring");
 };
@@ -161,8 +162,8 @@ constexpr int FUSE_NORM_A = 1, FUSE_SUMSQ_C = 2, FUSE_LN_A = 3, FUSE_STATS_C = 4
 template <int BM, int BN, int WAVES_M, int WAVES_N, int EPI, bool W_FP8, int FUSE, bool SPLIT_RES>
 constexpr bool residual_piece_through_ring() {
   constexpr int MT = BM / WAVES_M / 16, NT = BN / WAVES_N / 16;
-  return SPLIT_RES && EPI == CS_EPI_RESIDUAL && NT % 2 == 0 && !RingShape<BM, BN, W_FP8>::FIVE_UNITS && WAVES_N == 1 &&
-         (MT == 2 || MT == 4) && FUSE != FUSE_NORM_A && FUSE != FUSE_LN_A;
+  return SPLIT_RES && EPI == CS_EPI_RESIDUAL && NT % 2 == 0 && !RingShape<BM, BN, W_FP8>::FIVE_UNITS &&
+         (WAVES_N == 1 || FUSE == 0) && MT >= 2 && MT <= 4 && FUSE != FUSE_NORM_A && FUSE != FUSE_LN_A;
 }
 template <int BM, int BN, int WAVES_M, int WAVES_N, int EPI, bool W_FP8, int FUSE, bool SPLIT_RES>
 __global__ __launch_bounds__(64 * NW) void gemm_fast_kernel(const CsGemmArgs p) {
@@ -461,15 +462,15 @@ __global__ __launch_bounds__(64 * NW) void gemm_fast_kernel(const CsGemmArgs p) 
     //      worked on.
     constexpr bool PRE = residual_piece_through_ring<BM, BN, WAVES_M, WAVES_N, EPI, W_FP8, FUSE, SPLIT_RES>();
     constexpr int NP = NT / 2;                          // pairs of pieces: 16 bytes of the bf16 plane per lane
-    constexpr int LO_CHUNKS = 16 * BN / 16;             // 16-byte chunks of a row block's byte plane
+    constexpr int LO_CHUNKS = 16 * WTN / 16;            // 16-byte chunks of a row block's byte plane (the wave's columns)
     constexpr int LO_LD = (LO_CHUNKS + 63) / 64;        // ... and the loads that move them
     constexpr int ROW_LD = NP + LO_LD;                  // direct loads per wave and row block
     constexpr int ROW_HI_BYTES = NW * NP * 1024, ROW_LO_BYTES = NW * LO_LD * 1024, ROW_BYTES = ROW_HI_BYTES + ROW_LO_BYTES;
-    static_assert(!PRE || ((MT <= 2 ? ROW_BYTES : ROW_BYTES + ROW_HI_BYTES) <= STAGE && Ring::BYTES + NW * 1024 <= LDS_BYTES && BN * 2 <= 1024 &&
+    static_assert(!PRE || ((MT <= 3 ? ROW_BYTES : ROW_BYTES + ROW_HI_BYTES) <= STAGE && Ring::BYTES + NW * 1024 <= LDS_BYTES && BN * 2 <= 1024 &&
                            2 * (ROW_LD + 2) <= NMFMA && MT <= 4),
                   "two row blocks' bf16 planes and one byte plane fit a ring slot, the bias the room behind the ring");
     // fp8 weights: the columns' scales, in row block 0's slot behind everything that passes through it
-    constexpr int SCALE_OFF = MT <= 2 ? ROW_BYTES : ROW_BYTES + ROW_LO_BYTES;
+    constexpr int SCALE_OFF = MT <= 3 ? ROW_BYTES : ROW_BYTES + ROW_LO_BYTES;
     static_assert(!PRE || !W_FP8 || (SCALE_OFF + NW * 1024 <= STAGE && BN * 4 <= 1024), "the scales fit row block 0's slot");
     const bool fast_tile = p.fast_epilogue && m0 + BM <= p.M && n0 + BN <= p.N;
     const bool pre_on = PRE && fast_tile && !has_next;
@@ -483,12 +484,12 @@ __global__ __launch_bounds__(64 * NW) void gemm_fast_kernel(const CsGemmArgs p) 
         pre_hi_v = ((uint32_t)(lane_p & 15) * (uint32_t)p.ldr + (uint32_t)(lane_p >> 4) * (4 * G)) * 2;
 #pragma unroll
         for (int k = 0; k < LO_LD; ++k) {
-          const uint32_t g = (uint32_t)min(k * 64 + lane_p, LO_CHUNKS - 1), r = g / (BN / 16), c = g - r * (BN / 16);
+          const uint32_t g = (uint32_t)min(k * 64 + lane_p, LO_CHUNKS - 1), r = g / (WTN / 16), c = g - r * (WTN / 16);
           pre_lo_v[k] = r * (uint32_t)p.ldr + c * 16;
         }
         pre_bias_v = (uint32_t)min(lane_p, BN * 2 / 16 - 1) * 16;
         if constexpr (W_FP8) pre_scale_v = (uint32_t)min(lane_p, BN * 4 / 16 - 1) * 16;
-        pre_sbase = (m0 + wm * WTM) * (int)p.ldr + n0;
+        pre_sbase = (m0 + wm * WTM) * (int)p.ldr + n0 + wn * WTN;
       }
     }
     // Direct load IDX (bf16 plane of pair IDX, then the byte plane's chunks, then -- IDX == ROW_LD -- the bias, then the
@@ -916,7 +917,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_fast_kernel(const CsGemmArgs p) 
       const uint32_t lo_mask = p.residual_lo ? 0xFFFFFFFFu : 0u, bias_mask = p.bias ? 0xFFFFFFFFu : 0u;
       float bias_f[NT][4];
       {
-        const char* const bsrc = smem + Ring::BYTES + wave * 1024 + kq * (4 * G) * 2;
+        const char* const bsrc = smem + Ring::BYTES + wave * 1024 + (wn * WTN + kq * (4 * G)) * 2;
 #pragma unroll
         for (int jp = 0; jp < NP; ++jp) {
           const u32x4_t bw = *(const u32x4_t*)(bsrc + piece_col(2 * jp) * 2);
@@ -931,7 +932,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_fast_kernel(const CsGemmArgs p) 
       if constexpr (W_FP8) {
 #pragma unroll
         for (int j = 0; j < NT; ++j)
-          scale_f[W_FP8 ? j : 0] = *(const f32x4_t*)(smem + slot0 + SCALE_OFF + wave * 1024 + (kq * (4 * G) + piece_col(j)) * 4);
+          scale_f[W_FP8 ? j : 0] = *(const f32x4_t*)(smem + slot0 + SCALE_OFF + wave * 1024 + (wn * WTN + kq * (4 * G) + piece_col(j)) * 4);
       }
       static_for<MT>([&](auto i_c) {
         constexpr int i = decltype(i_c)::value;
@@ -939,7 +940,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_fast_kernel(const CsGemmArgs p) 
         // (a wave's chunk of a direct load is 64 lanes x 16 bytes; the bf16 plane: every lane reads back what it
         // requested; the byte plane: rows of BN bytes, one after the other)
         const char* const hi_src = smem + hi_base_of(i) + (wave * NP) * 1024 + lane_e * 16;
-        const char* const lo_src = smem + lo_base_of(i) + (wave * LO_LD) * 1024 + fa * BN + kq * (4 * G);
+        const char* const lo_src = smem + lo_base_of(i) + (wave * LO_LD) * 1024 + fa * WTN + kq * (4 * G);
         const uint32_t off = (row0 + 16 * i) * (uint32_t)p.ldc + n_lane;   // in elements
         float ss = 0.f, sm = 0.f;
         static_for<NP>([&](auto jp_c) {
@@ -1127,7 +1128,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_fast_kernel(const CsGemmArgs p) 
       // compiler's to use), so the addend rows are fetched in batches, the first ahead of the accumulator reads, every
       // later one right before its rows: two batches normally, row by row where the split stream's three registers
       // per piece meet the fp8 scales.
-      constexpr int ADD_BATCH = (SPLIT && W_FP8 && MT >= 8) ? 1 : MT / 2;
+      constexpr int ADD_BATCH = (SPLIT && W_FP8 && MT >= 8) || MT % 2 ? 1 : MT / 2;
       auto load_addend_batch = [&](auto b_c) {
         static_for<ADD_BATCH>([&](auto k_c) { load_addend(ic<decltype(b_c)::value * ADD_BATCH + decltype(k_c)::value>{}); });
       };

@@ -2,6 +2,7 @@
 // gemm_small_impl.h; each tile form is built in its own translation unit (gemm_small_t*.hip).
 #include "gemm_common.h"
 
+double cs_gemm_fast_saves(const CsGemmArgs& a, int64_t* tiles);   // gemm_fast.hip
 int cs_gemm_small_tile_32x32(const CsGemmArgs& a, hipStream_t stream);
 int cs_gemm_small_tile_32x64(const CsGemmArgs& a, hipStream_t stream);
 int cs_gemm_small_tile_64x64(const CsGemmArgs& a, hipStream_t stream);
@@ -34,7 +35,9 @@ const Form SUMS_FORMS[] = {   // with row sums of the output
     {32, 160, 5.5f, 0.635f, cs_gemm_small_tile_32x160}, {64, 160, 7.8f, 0.841f, cs_gemm_small_tile_64x160},
 };
 // The big tiles of gemm_fast.hip, which run on from tile to tile without a gap: the fixed part counts once (same shapes at
-// 1500, 2744, 4096 and 5104 rows, 3840 and 6912 columns at 1024 and 4096).
+// 1500, 2744, 4096 and 5104 rows, 3840 and 6912 columns at 1024 and 4096).  These four, timed where few rows have to choose; the
+// table of gemm_fast.hip, fitted up to 20000 rows, is 15 % off at either end of these (2048 rows x 1280 x 1280, 640 x 3584 x 3584) and
+// says here only what its other forms save over them.
 struct FastForm {
   int bm, bn;
   float fixed_us, stage_us;
@@ -53,15 +56,17 @@ double small_us(const Form& f, int M, int N, int K, bool norm) {
   return r * (f.fixed_us - 2.0 + stages * f.stage_us * (norm ? 1.15 : 1.0)) + 2.0;
 }
 
-double fast_us(int M, int N, int K, bool sums, int epilogue, bool split) {
-  const double stages = K / 128.0;
+double fast_us(const CsGemmArgs& a, int64_t* tiles) {
+  const int M = a.M, N = a.N;
+  const bool sums = a.c_row_sumsq != nullptr;
+  const double stages = a.K / 128.0;
   auto us = [&](const FastForm& f) { return f.fixed_us + rounds(M, N, f.bm, f.bn) * stages * f.stage_us; };
-  const bool few = (int64_t)((M + 255) / 256) * ((N + 159) / 160) <= 128;   // (the rule of gemm_fast.hip)
+  const bool few = (int64_t)((M + 255) / 256) * ((N + 159) / 160) <= 128;   
   // (a tail tile of the split residual stream: 29 us at 4888 x 1280 x 1280; a bf16 one: 22 us at 4160 .. 5376 x 1152 x 1152)
-  double t = us(few ? F128x160 : F256x160) + (!few && epilogue == CS_EPI_RESIDUAL && split ? 11.0 : 0.0);
+  double t = us(few ? F128x160 : F256x160) + (!few && a.epilogue == CS_EPI_RESIDUAL && a.c_lo ? 11.0 : 0.0);
   if (!sums) t = us(F256x256) < t ? us(F256x256) : t;
-  if (!sums && epilogue == CS_EPI_SWIGLU) t = us(F256x128) < t ? us(F256x128) : t;
-  return t;
+  if (!sums && a.epilogue == CS_EPI_SWIGLU) t = us(F256x128) < t ? us(F256x128) : t;
+  return t * cs_gemm_fast_saves(a, tiles);
 }
 
 // A launch of more than two rounds is no few-row launch: the times above are of one round, and five rounds of 64x64 take 33 us
@@ -97,10 +102,8 @@ int tiles_of(const Form& f, const CsGemmArgs& a) { return ((a.M + f.bm - 1) / f.
 // is slower by more than that (2700 patches 5.78 -> 6.06).  A hint that the big form has no time for either, as that for the
 // merger's 52 MB, would only make its launch longer.
 constexpr double HINT_WORTH = 0.15;
-bool loses_hint(const Form& f, const CsGemmArgs& a, double big_us) {
+bool loses_hint(const Form& f, const CsGemmArgs& a, double big_us, int64_t big_tiles) {
   if (!a.prefetch || a.prefetch_bytes < 16 || a.w_fp8 || a.c_row_sumsq || tiles_of(f, a) <= csgemm::HINT_MAX_TILES) return false;
-  const int big_rows = (int64_t)((a.M + 255) / 256) * ((a.N + 159) / 160) <= 128 ? 128 : 256;
-  const int64_t big_tiles = (int64_t)((a.M + big_rows - 1) / big_rows) * ((a.N + 159) / 160);
   return big_tiles <= csgemm::HINT_MAX_TILES && a.prefetch_bytes <= csgemm::hint_workgroups((int)big_tiles) * 8192.0 * big_us;
 }
 
@@ -117,8 +120,9 @@ const Form* few_row_form(const CsGemmArgs& a, double* us) {
     if (a.a_norm_inline) return f;
   }
   if (!f) return nullptr;
-  const double big_us = fast_us(a.M, a.N, a.K, a.c_row_sumsq != nullptr, a.epilogue, a.c_lo != nullptr);
-  return *us < big_us * (loses_hint(*f, a, big_us) ? 1.0 - HINT_WORTH : 1.0) ? f : nullptr;
+  int64_t big_tiles;
+  const double big_us = fast_us(a, &big_tiles);
+  return *us < big_us * (loses_hint(*f, a, big_us, big_tiles) ? 1.0 - HINT_WORTH : 1.0) ? f : nullptr;
 }
 
 }  // namespace
@@ -165,5 +169,8 @@ extern "C" int cs_gemm_norm_inline_pays(int32_t M, int32_t N, int32_t K, int32_t
   a.a_norm_inline = 1;
   double us;
   best_form(FORMS, a, &us);
-  return us < fast_us(M, N, K, false, CS_EPI_SWIGLU, false) ? 1 : 0;
+  a.a_norm_inline = 0;
+  a.epilogue = CS_EPI_SWIGLU;
+  int64_t big_tiles;
+  return us < fast_us(a, &big_tiles) ? 1 : 0;
 }

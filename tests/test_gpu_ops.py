@@ -440,9 +440,9 @@ def _epilogue_ref(ops, epi, base, res):
     return F.silu(gate) * up
 
 
-# Shapes that reach every tile form and every schedule of the fast kernel: the 256x256 five-unit ring, the
-# 256x160 / 256x128 / 128x192 three-stage rings (N = 1280; remainders of a column split), the shortest K the
-# fast path takes (3 K tiles: the ring's tail iterations only) and 4, 5, 7 K tiles, row and column tails.
+# Shapes of every schedule of the fast kernel: the 256x256 five-unit ring and the three-stage rings of the narrower forms, one launch
+# and a column split, the shortest K the fast path takes (3 K tiles: the ring's tail iterations only) and 4, 5, 7 K tiles, row
+# and column tails (the form that a launch takes follows a table of times; every form by itself: the test after this one).
 @pytest.mark.parametrize("M,N,K", [
     (8192, 3072, 192),    # 8 columns of 256x256 + 1024 columns of 256x128, 3 K tiles
     (8192, 2304, 256),    # 8 columns of 256x256 + 256 columns of 128x192, 4 K tiles
@@ -474,6 +474,86 @@ def test_gemm_fast_path_forms(ops, dev, M, N, K):
     ref = torch.empty_like(first)
     ref[perm.long()] = first
     assert torch.equal(scat, ref)
+
+
+BIG_FORMS = ("256x256", "256x160", "256x128", "224x192", "192x192", "192x160", "128x192", "128x160")
+
+
+# Every big tile form, called by itself, on the same products: which form a launch takes must change no bit.  Whole tiles of no
+# form, of some and of most; one tile, one round and several tiles a workgroup; 3, 4, 6 and 18 K tiles; row tails of 1 row and of
+# one less than a tile; column tails of 8, 32 and 96 columns.
+@pytest.mark.parametrize("M,N,K", [(1, 200, 192), (447, 1152, 256), (449, 1288, 192), (1344, 960, 384), (5103, 1152, 1152), (6145, 1280, 192),
+                                   (16500, 320, 192)])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_every_big_tile_form_gives_the_same_bits(ops, dev, M, N, K, fp8):
+    import ctypes
+
+    from cornserve_amd import lib
+
+    dll = ctypes.CDLL(str(lib.LIB_PATH))
+    run = {}
+    for name in BIG_FORMS:
+        base = f"cs_gemm_fast_tile_{name}"
+        run[name] = getattr(dll, f"_Z{len(base)}{base}RK10CsGemmArgsP12ihipStream_t")
+        run[name].argtypes, run[name].restype = [ctypes.POINTER(lib.CsGemmArgs), ctypes.c_void_p], ctypes.c_int
+    a, w, b = rnd((M, K), 1.0, 201, dev), rnd((N, K), 0.05, 202, dev), rnd((N,), 0.02, 203, dev)
+    res, pos = rnd((M, N), 1.0, 204, dev), rnd((7, N), 1.0, 205, dev)
+    lo = torch.randint(0, 256, (M, N), generator=torch.Generator().manual_seed(206), dtype=torch.uint8).to(dev)
+    sc = (w.float().abs().amax(1) / 448.0).contiguous()
+    wq = (w.float() / sc[:, None]).to(torch.float8_e4m3fn).view(torch.uint8) if fp8 else w
+    ss, sm = torch.empty((M, ops.SUMSQ_PARTS), device=dev), torch.empty((M, ops.SUMSQ_PARTS), device=dev)
+    if K <= 160 * ops.SUMSQ_PARTS:
+        ops.row_stats(a, ss, sm)
+    csum = w.float().sum(1)
+    rows = torch.randperm(M, generator=torch.Generator().manual_seed(207)).int().to(dev)
+    cases = [(e, {}) for e in (ops.EPI_BIAS, ops.EPI_SWIGLU, ops.EPI_GELU_ERF, ops.EPI_GELU_TANH, ops.EPI_QUICK_GELU)]
+    cases += [(ops.EPI_RESIDUAL, {}), (ops.EPI_RESIDUAL, {"split": 1}), (ops.EPI_RESIDUAL, {"split": 1, "plane": 0, "bias": 0}), (ops.EPI_BIAS, {"rows": 1})]
+    if not fp8:
+        cases += [(ops.EPI_RESIDUAL, {"split": 1, "sums": 1}), (ops.EPI_RESIDUAL, {"split": 1, "sums": 2}), (ops.EPI_BIAS, {"pos": 1}),
+                  (ops.EPI_BIAS, {"norm": 1}), (ops.EPI_SWIGLU, {"norm": 1}), (ops.EPI_BIAS, {"norm": 2}), (ops.EPI_GELU_TANH, {"norm": 2})]
+    for epi, kw in cases:
+        if kw.get("sums") and N > 160 * ops.SUMSQ_PARTS:
+            continue
+        want, took = None, []
+        for name in BIG_FORMS:
+            # (guard rows and columns around the output: every form has to leave them alone)
+            width = N // 2 if epi == ops.EPI_SWIGLU else N
+            out = torch.full((M + 2, width + 16), 7.0, dtype=torch.bfloat16, device=dev)
+            out_lo = torch.full((M + 2, width + 16), 9, dtype=torch.uint8, device=dev)
+            osum = torch.full((2, M + 1, ops.SUMSQ_PARTS), 5.0, device=dev)
+            g = lib.CsGemmArgs()
+            g.A, g.W, g.C, g.M, g.N, g.K, g.lda, g.ldw, g.ldc, g.epilogue = a.data_ptr(), wq.data_ptr(), out.data_ptr(), M, N, K, K, K, width + 16, epi
+            g.bias = b.data_ptr() if kw.get("bias", 1) else None
+            if fp8:
+                g.w_fp8, g.w_scale = 1, sc.data_ptr()
+            if epi == ops.EPI_RESIDUAL:
+                g.residual, g.ldr = res.data_ptr(), N
+            if kw.get("split"):
+                g.c_lo, g.residual_lo = out_lo.data_ptr(), lo.data_ptr() if kw.get("plane", 1) else None
+            if kw.get("sums"):
+                g.c_row_sumsq = osum[0].data_ptr()
+            if kw.get("sums") == 2:
+                g.c_row_sum = osum[1].data_ptr()
+            if kw.get("pos"):
+                g.pos, g.ldpos, g.pos_period = pos.data_ptr(), N, 7
+            if kw.get("rows"):
+                g.c_rows = rows.data_ptr()
+            if kw.get("norm"):
+                g.a_row_sumsq, g.norm_eps = ss.data_ptr(), 1e-6
+            if kw.get("norm") == 2:
+                g.a_row_sum, g.w_col_sum = sm.data_ptr(), csum.data_ptr()
+            if run[name](ctypes.byref(g), torch.cuda.current_stream().cuda_stream) != 0:
+                continue
+            took.append(name)
+            got = (out, out_lo, osum)
+            assert bool((out[M:] == 7).all()) and bool((out[:, width:] == 7).all()) and bool((osum[:, M:] == 5).all()), (name, epi, kw)
+            assert bool((out_lo[M:] == 9).all()) and bool((out_lo[:, width:] == 9).all()), (name, epi, kw)
+            if want is None:
+                want = got
+            assert all(torch.equal(x, y) for x, y in zip(got, want)), (name, epi, kw)
+        assert len(took) >= (3 if kw.get("sums") else 6), (epi, kw, took)
+        if not kw and not fp8 and epi == ops.EPI_BIAS:
+            close(want[0][:M, :N][:64], lin_ref(a[:64], w, b), 2**-7, f"{M}x{N}x{K}")
 
 
 # The few-row kernel (K a multiple of 128) at shapes of the encoders: an output has the bits it has as a row of a product with
