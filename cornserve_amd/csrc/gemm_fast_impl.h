@@ -297,15 +297,19 @@ __global__ __launch_bounds__(64 * NW) void gemm_fast_kernel(const CsGemmArgs p) 
   };
   const __amdgpu_buffer_rsrc_t rsrc_a = __builtin_amdgcn_make_buffer_rsrc((void*)p.A, 0, -1, 0x00020000);
   const __amdgpu_buffer_rsrc_t rsrc_w = __builtin_amdgcn_make_buffer_rsrc((void*)p.W, 0, -1, 0x00020000);
-  // descriptors of what the epilogue's fast form reads and writes
-  const __amdgpu_buffer_rsrc_t rsrc_c = __builtin_amdgcn_make_buffer_rsrc((void*)p.C, 0, -1, 0x00020000);
-  const __amdgpu_buffer_rsrc_t rsrc_clo = __builtin_amdgcn_make_buffer_rsrc((void*)p.c_lo, 0, -1, 0x00020000);
-  const __amdgpu_buffer_rsrc_t rsrc_res = __builtin_amdgcn_make_buffer_rsrc((void*)p.residual, 0, -1, 0x00020000);
-  const __amdgpu_buffer_rsrc_t rsrc_reslo = __builtin_amdgcn_make_buffer_rsrc((void*)p.residual_lo, 0, -1, 0x00020000);
-  const __amdgpu_buffer_rsrc_t rsrc_scale = __builtin_amdgcn_make_buffer_rsrc((void*)p.w_scale, 0, -1, 0x00020000);
-  const __amdgpu_buffer_rsrc_t rsrc_bias = __builtin_amdgcn_make_buffer_rsrc((void*)p.bias, 0, -1, 0x00020000);
-  const __amdgpu_buffer_rsrc_t rsrc_asumsq = __builtin_amdgcn_make_buffer_rsrc((void*)p.a_row_sumsq, 0, -1, 0x00020000);
-  const __amdgpu_buffer_rsrc_t rsrc_asum = __builtin_amdgcn_make_buffer_rsrc((void*)p.a_row_sum, 0, -1, 0x00020000);
+  // Descriptors of what the epilogue's fast form reads and writes, each as long as its matrix: what a lane past the last row would
+  // load is zero and what it would store is dropped, so row tails need no guards (a row past the last one starts at or behind
+  // the end whatever its column).  A lane past the last column of its row takes an offset behind every end instead (OUTSIDE).
+  constexpr uint32_t OUTSIDE = 0xFFFF0000u;   // (with room for an immediate; p.fast_epilogue: every matrix ends below it)
+  auto rsrc_of = [&](const void* base, int64_t bytes) { return __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, (int)(uint32_t)bytes, 0x00020000); };
+  const __amdgpu_buffer_rsrc_t rsrc_c = rsrc_of(p.C, (int64_t)p.M * p.ldc * 2);
+  const __amdgpu_buffer_rsrc_t rsrc_clo = rsrc_of(p.c_lo, (int64_t)p.M * p.ldc);
+  const __amdgpu_buffer_rsrc_t rsrc_res = rsrc_of(p.residual, (int64_t)p.M * p.ldr * 2);
+  const __amdgpu_buffer_rsrc_t rsrc_reslo = rsrc_of(p.residual_lo, (int64_t)p.M * p.ldr);
+  const __amdgpu_buffer_rsrc_t rsrc_scale = rsrc_of(p.w_scale, (int64_t)p.N * 4);
+  const __amdgpu_buffer_rsrc_t rsrc_bias = rsrc_of(p.bias, (int64_t)p.N * 2);
+  const __amdgpu_buffer_rsrc_t rsrc_asumsq = rsrc_of(p.a_row_sumsq, (int64_t)p.M * (CS_SUMSQ_PARTS * 4));
+  const __amdgpu_buffer_rsrc_t rsrc_asum = rsrc_of(p.a_row_sum, (int64_t)p.M * (CS_SUMSQ_PARTS * 4));
   // (The builtin is called from non-generic lambdas on purpose: inside a generic lambda the host pass of the
   // compiler rejects the device-only builtin, silently drops the kernel and leaves its launch stub undefined.)
   auto load_a = [&](int kt, char* lds_dst, uint32_t off) {
@@ -472,8 +476,11 @@ __global__ __launch_bounds__(64 * NW) void gemm_fast_kernel(const CsGemmArgs p) 
     // fp8 weights: the columns' scales, in row block 0's slot behind everything that passes through it
     constexpr int SCALE_OFF = MT <= 3 ? ROW_BYTES : ROW_BYTES + ROW_LO_BYTES;
     static_assert(!PRE || !W_FP8 || (SCALE_OFF + NW * 1024 <= STAGE && BN * 4 <= 1024), "the scales fit row block 0's slot");
-    const bool fast_tile = p.fast_epilogue && m0 + BM <= p.M && n0 + BN <= p.N;
-    const bool pre_on = PRE && fast_tile && !has_next;
+    const bool m_edge = m0 + BM > p.M, n_edge = n0 + BN > p.N;
+    // (a 16-byte chunk of the byte plane that straddles the last column is left to the other form; so are the edge tiles of the
+    // form whose scales leave no registers for them)
+    constexpr bool PRE_EDGE = PRE && !(W_FP8 && MT * NT >= 40);
+    const bool pre_on = PRE && p.fast_epilogue && !has_next && !(n_edge && p.N % 16) && (PRE_EDGE || !(m_edge || n_edge));
     // lane-only byte offsets of the direct loads (the tile and the row block go into the scalar offset)
     uint32_t pre_hi_v = 0, pre_lo_v[PRE ? LO_LD : 1] = {}, pre_bias_v = 0, pre_scale_v = 0;
     int pre_sbase = 0;   // element offset of the wave's first row and the tile's first column in the residual matrix
@@ -487,8 +494,9 @@ __global__ __launch_bounds__(64 * NW) void gemm_fast_kernel(const CsGemmArgs p) 
           const uint32_t g = (uint32_t)min(k * 64 + lane_p, LO_CHUNKS - 1), r = g / (WTN / 16), c = g - r * (WTN / 16);
           pre_lo_v[k] = r * (uint32_t)p.ldr + c * 16;
         }
-        pre_bias_v = (uint32_t)min(lane_p, BN * 2 / 16 - 1) * 16;
-        if constexpr (W_FP8) pre_scale_v = (uint32_t)min(lane_p, BN * 4 / 16 - 1) * 16;
+        const int cols = min(BN, p.N - n0);
+        pre_bias_v = (uint32_t)min(lane_p, cols * 2 / 16 - 1) * 16;
+        if constexpr (W_FP8) pre_scale_v = (uint32_t)min(lane_p, cols * 4 / 16 - 1) * 16;
         pre_sbase = (m0 + wm * WTM) * (int)p.ldr + n0 + wn * WTN;
       }
     }
@@ -504,13 +512,34 @@ __global__ __launch_bounds__(64 * NW) void gemm_fast_kernel(const CsGemmArgs p) 
     };
     auto residual_to_lds = [&](auto i_c, auto idx_c, int hi_base, int lo_base) {
       constexpr int I = decltype(i_c)::value, IDX = decltype(idx_c)::value;
+      // Tiles at an edge: rows past the last one repeat it and columns past the last piece (chunk) repeat that, in offsets made
+      // here (the loads go past their descriptors' ends otherwise: what a scalar offset adds is not relied on to be checked).
+      auto edge_row = [&]() { return min(m0 + wm * WTM + I * 16, p.M - 1); };
       if constexpr (IDX < NP) {
         constexpr int COL = (2 * IDX / G) * 16 * G + (2 * IDX % G) * 4;
-        dma16(rsrc_res, smem + hi_base + (wave * NP + IDX) * 1024, pre_hi_v, (pre_sbase + I * 16 * (int)p.ldr + COL) * 2);
+        uint32_t voff = pre_hi_v;
+        int soff = (pre_sbase + I * 16 * (int)p.ldr + COL) * 2;
+        if (PRE_EDGE && (m_edge || n_edge)) {
+          const int row = edge_row();
+          int lane_x = lane;
+          asm volatile("" : "+v"(lane_x));
+          voff = ((uint32_t)min(lane_x & 15, p.M - 1 - row) * (uint32_t)p.ldr + (uint32_t)min(n0 + wn * WTN + COL + (lane_x >> 4) * (4 * G), p.N - 4 * G)) * 2;
+          soff = row * (int)p.ldr * 2;
+        }
+        dma16(rsrc_res, smem + hi_base + (wave * NP + IDX) * 1024, voff, soff);
       } else if constexpr (IDX < ROW_LD) {
         constexpr int Kk = IDX - NP;
-        dma16(p.residual_lo ? rsrc_reslo : rsrc_res, smem + lo_base + (wave * LO_LD + Kk) * 1024, pre_lo_v[PRE ? Kk : 0],
-              pre_sbase + I * 16 * (int)p.ldr);
+        uint32_t voff = pre_lo_v[PRE ? Kk : 0];
+        int soff = pre_sbase + I * 16 * (int)p.ldr;
+        if (PRE_EDGE && (m_edge || n_edge)) {
+          const int row = edge_row();
+          int lane_x = lane;
+          asm volatile("" : "+v"(lane_x));
+          const int g = min(Kk * 64 + lane_x, LO_CHUNKS - 1), r = g / (WTN / 16), c = g - r * (WTN / 16);
+          voff = (uint32_t)min(r, p.M - 1 - row) * (uint32_t)p.ldr + (uint32_t)min(n0 + wn * WTN + c * 16, p.N - 16);
+          soff = row * (int)p.ldr;
+        }
+        dma16(p.residual_lo ? rsrc_reslo : rsrc_res, smem + lo_base + (wave * LO_LD + Kk) * 1024, voff, soff);
       } else if constexpr (IDX > ROW_LD) {
         dma16(rsrc_scale, smem + hi_base + SCALE_OFF + wave * 1024, pre_scale_v, n0 * 4);
       } else {
@@ -889,10 +918,13 @@ __global__ __launch_bounds__(64 * NW) void gemm_fast_kernel(const CsGemmArgs p) 
     // ---- epilogue.  Accumulator (i, j), element r = C[m][n], m = m0 + wm*WTM + 16i + lane%16,
     //      n = n0 + wn*WTN + (j/G)*16G + (lane/16)*4G + (j%G)*4 + r : 4G consecutive columns per lane, row and group.
     //      With one wave per SIMD nothing overlaps the epilogue and it is bound by instruction issue (a vector
-    //      instruction every four to five clocks), so it comes in two forms.  FAST: the tile lies inside the matrix
-    //      and rows are not scattered -- no guards, no clamps, and every access is a buffer instruction (scalar
-    //      descriptor + one 32-bit lane offset + an immediate), so an address costs no vector arithmetic.  General:
-    //      edge tiles and scattered rows, with guards and 64-bit addresses.  In both, the loads the epilogue needs
+    //      instruction every four to five clocks), so it comes in three forms.  FAST: rows are not scattered -- every
+    //      access is a buffer instruction (scalar descriptor + one 32-bit lane offset + an immediate), so an address
+    //      costs no vector arithmetic, and the tile lies inside the matrix: no guards, no clamps.  FAST with EDGE: the
+    //      descriptors' ends guard the rows, one select per store the columns.  (Edge tiles took the general form before:
+    //      a launch lasts as long as its slowest tile, and 4888 rows x 1280 x 1280 went from 26.7 to 23.9 us, 6240 x 1152 x
+    //      1152, whose last column tile of 160 is an edge too, from 30.6 to 24.)  General:
+    //      scattered rows and matrices past 32-bit offsets, with guards and 64-bit addresses.  In all, the loads the epilogue needs
     //      (row map, bias, residual / position rows) are issued ahead of the stores that follow them: a load inside the
     //      store loop would make the compiler wait for ALL outstanding memory operations (vmcnt counts stores too),
     //      i.e. for every store issued so far and for the next tile's prefetch, once per row block.
@@ -901,7 +933,8 @@ __global__ __launch_bounds__(64 * NW) void gemm_fast_kernel(const CsGemmArgs p) 
     //      over the packed output words.  `ring` has moved on three slots since row block 0 was requested, so row block 0
     //      sits in slot ring, row block 1 in slot ring + 1; row block 2 goes to slot ring + 2 and row block 3 behind it
     //      (bf16 plane) and behind row block 0 (byte plane), requested while row blocks 0 and 1 are worked on.
-    auto epilogue_from_lds = [&](auto) {
+    auto epilogue_from_lds = [&](auto edge_c) {   // (EDGE: the tile reaches past the last row or column)
+      constexpr bool EDGE = decltype(edge_c)::value;
       int lane_e = lane;
       asm volatile("" : "+v"(lane_e));
       const int kq = lane_e >> 4, fa = lane_e & 15;
@@ -970,31 +1003,43 @@ __global__ __launch_bounds__(64 * NW) void gemm_fast_kernel(const CsGemmArgs p) 
             });
             add_split24(v, u32x2_t{hi_in[2 * Hh], hi_in[2 * Hh + 1]}, lo_in[Hh], hi_o[Hh], lo_o[Hh]);
             if constexpr (FUSE == FUSE_SUMSQ_C || FUSE == FUSE_STATS_C) {
-              ss = dot2_bf16(hi_o[Hh][0], hi_o[Hh][0], ss);
-              ss = dot2_bf16(hi_o[Hh][1], hi_o[Hh][1], ss);
-            }
-            if constexpr (FUSE == FUSE_STATS_C) {
-              sm = dot2_bf16(hi_o[Hh][0], BF16_ONE_PAIR, sm);
-              sm = dot2_bf16(hi_o[Hh][1], BF16_ONE_PAIR, sm);
+              u32x2_t in_row = hi_o[Hh];
+              if (EDGE && n_edge) {   // (uniform: a piece outside the matrix adds exact zeros)
+                const bool nok = (int)n_lane + piece_col(2 * JP) < p.N;
+                in_row = u32x2_t{nok ? in_row[0] : 0u, nok ? in_row[1] : 0u};
+              }
+              ss = dot2_bf16(in_row[0], in_row[0], ss);
+              ss = dot2_bf16(in_row[1], in_row[1], ss);
+              if constexpr (FUSE == FUSE_STATS_C) {
+                sm = dot2_bf16(in_row[0], BF16_ONE_PAIR, sm);
+                sm = dot2_bf16(in_row[1], BF16_ONE_PAIR, sm);
+              }
             }
           });
-          buf_st_u32x4(rsrc_c, (off + piece_col(2 * JP)) * 2, u32x4_t{hi_o[0][0], hi_o[0][1], hi_o[1][0], hi_o[1][1]});
-          buf_st_u32x2(rsrc_clo, off + piece_col(2 * JP), u32x2_t{lo_o[0], lo_o[1]});
+          // (every lane stores, in or outside the matrix: the waits count stores)
+          uint32_t off_hi = (off + piece_col(2 * JP)) * 2, off_lo = off + piece_col(2 * JP);
+          if (EDGE && n_edge) {
+            const bool nok = (int)n_lane + piece_col(2 * JP) < p.N;
+            off_hi = nok ? off_hi : OUTSIDE;
+            off_lo = nok ? off_lo : OUTSIDE;
+          }
+          buf_st_u32x4(rsrc_c, off_hi, u32x4_t{hi_o[0][0], hi_o[0][1], hi_o[1][0], hi_o[1][1]});
+          buf_st_u32x2(rsrc_clo, off_lo, u32x2_t{lo_o[0], lo_o[1]});
         });
         if constexpr (FUSE == FUSE_SUMSQ_C || FUSE == FUSE_STATS_C) {
           ss += __shfl_xor(ss, 16);
           ss += __shfl_xor(ss, 32);
-          if (kq == 0) p.c_row_sumsq[(int64_t)(row0 + 16 * i) * CS_SUMSQ_PARTS + n0 / BN] = ss;
+          if (kq == 0 && (!EDGE || (int)row0 + 16 * i < p.M)) p.c_row_sumsq[(int64_t)(row0 + 16 * i) * CS_SUMSQ_PARTS + n0 / BN] = ss;
         }
         if constexpr (FUSE == FUSE_STATS_C) {
           sm += __shfl_xor(sm, 16);
           sm += __shfl_xor(sm, 32);
-          if (kq == 0) p.c_row_sum[(int64_t)(row0 + 16 * i) * CS_SUMSQ_PARTS + n0 / BN] = sm;
+          if (kq == 0 && (!EDGE || (int)row0 + 16 * i < p.M)) p.c_row_sum[(int64_t)(row0 + 16 * i) * CS_SUMSQ_PARTS + n0 / BN] = sm;
         }
       });
     };
-    auto epilogue = [&](auto fast_c) {
-      constexpr bool FAST = decltype(fast_c)::value;
+    auto epilogue = [&](auto fast_c, auto edge_c) {
+      constexpr bool FAST = decltype(fast_c)::value, EDGE = decltype(edge_c)::value;
       const bf16_t* const pBias = (const bf16_t*)p.bias;
       bf16_t* const pC = (bf16_t*)p.C;
       // The lane's column and row are re-derived behind an opaque copy of the lane number: otherwise the compiler
@@ -1018,7 +1063,9 @@ __global__ __launch_bounds__(64 * NW) void gemm_fast_kernel(const CsGemmArgs p) 
         }
       }
       auto clamp_m = [&](int m) { return FAST ? m : min(m, p.M - 1); };
-      auto clamp_n = [&](int n) { return FAST ? n : min(n, p.N - 4); };
+      auto clamp_n = [&](int n) { return EDGE ? min(n, p.N - 4) : n; };
+      // FAST: where the lane's piece j starts, or OUTSIDE (a piece is inside its row as a whole: N is a multiple of 8)
+      auto piece_at = [&](uint32_t off, int j) { return !EDGE || n_lane + piece_col(j) < p.N ? off : OUTSIDE; };
       constexpr bool NORM_A = FUSE == FUSE_NORM_A || FUSE == FUSE_LN_A;
       float rstd[NORM_A ? MT : 1];
       float nmean_rstd[FUSE == FUSE_LN_A ? MT : 1];   // -mean * rstd
@@ -1136,7 +1183,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_fast_kernel(const CsGemmArgs p) 
       static_for<MT>([&](auto i_c) {
         constexpr int i = decltype(i_c)::value;
         if constexpr (ADDEND && i % ADD_BATCH == 0 && i > 0) load_addend_batch(ic<i / ADD_BATCH>{});
-        const bool mok = FAST || mrow[i] < p.M;
+        const bool mok = !EDGE || mrow[i] < p.M;
         f32x4_t racc[NT];
         static_for<NT * 4>([&](auto e_c) {
           constexpr int E = decltype(e_c)::value;
@@ -1200,7 +1247,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_fast_kernel(const CsGemmArgs p) 
           float ss = 0.f, sm = 0.f;
 #pragma unroll
           for (int j = 0; j < NT; ++j) {
-            const bool nok = FAST || n_lane + piece_col(j) < p.N;
+            const bool nok = !EDGE || n_lane + piece_col(j) < p.N;
             const u32x2_t ow = nok ? __builtin_bit_cast(u32x2_t, out[j]) : u32x2_t{0u, 0u};
             ss = dot2_bf16(ow[0], ow[0], ss);
             ss = dot2_bf16(ow[1], ow[1], ss);
@@ -1227,13 +1274,13 @@ __global__ __launch_bounds__(64 * NW) void gemm_fast_kernel(const CsGemmArgs p) 
 #pragma unroll
               for (int j = 0; j < NT; j += 2) {
                 const bf16x4_t o = {out[j][0], out[j][1], out[j + 1][0], out[j + 1][1]};
-                buf_st_u32x2(rsrc_c, off + (piece_col(j) >> 1) * 2, __builtin_bit_cast(u32x2_t, o));
+                buf_st_u32x2(rsrc_c, piece_at(off + (piece_col(j) >> 1) * 2, j), __builtin_bit_cast(u32x2_t, o));
               }
             } else {
 #pragma unroll
               for (int j = 0; j < NT; ++j) {
                 const bf16x2_t o = {out[j][0], out[j][1]};
-                buf_st_u32(rsrc_c, off + (piece_col(j) >> 1) * 2, __builtin_bit_cast(uint32_t, o));
+                buf_st_u32(rsrc_c, piece_at(off + (piece_col(j) >> 1) * 2, j), __builtin_bit_cast(uint32_t, o));
               }
             }
           } else {
@@ -1242,20 +1289,20 @@ __global__ __launch_bounds__(64 * NW) void gemm_fast_kernel(const CsGemmArgs p) 
 #pragma unroll
               for (int j = 0; j < NT; j += 2) {
                 const u32x2_t a0 = __builtin_bit_cast(u32x2_t, out[j]), a1 = __builtin_bit_cast(u32x2_t, out[j + 1]);
-                buf_st_u32x4(rsrc_c, (off + piece_col(j)) * 2, u32x4_t{a0[0], a0[1], a1[0], a1[1]});
+                buf_st_u32x4(rsrc_c, piece_at((off + piece_col(j)) * 2, j), u32x4_t{a0[0], a0[1], a1[0], a1[1]});
               }
             } else {
 #pragma unroll
-              for (int j = 0; j < NT; ++j) buf_st_u32x2(rsrc_c, (off + piece_col(j)) * 2, __builtin_bit_cast(u32x2_t, out[j]));
+              for (int j = 0; j < NT; ++j) buf_st_u32x2(rsrc_c, piece_at((off + piece_col(j)) * 2, j), __builtin_bit_cast(u32x2_t, out[j]));
             }
             if constexpr (SPLIT) {
               if constexpr (G == 2) {
 #pragma unroll
                 for (int j = 0; j < NT; j += 2)
-                  buf_st_u32x2(rsrc_clo, off + piece_col(j), u32x2_t{out_lo[SPLIT ? j : 0], out_lo[SPLIT ? j + 1 : 0]});
+                  buf_st_u32x2(rsrc_clo, piece_at(off + piece_col(j), j), u32x2_t{out_lo[SPLIT ? j : 0], out_lo[SPLIT ? j + 1 : 0]});
               } else {
 #pragma unroll
-                for (int j = 0; j < NT; ++j) buf_st_u32(rsrc_clo, off + piece_col(j), out_lo[SPLIT ? j : 0]);
+                for (int j = 0; j < NT; ++j) buf_st_u32(rsrc_clo, piece_at(off + piece_col(j), j), out_lo[SPLIT ? j : 0]);
               }
             }
           }
@@ -1326,9 +1373,14 @@ __global__ __launch_bounds__(64 * NW) void gemm_fast_kernel(const CsGemmArgs p) 
       setup_frag_offsets(lane_again);
     }
     else if (PRE && pre_on) {
-      if constexpr (PRE) epilogue_from_lds(0);
-    } else if (fast_tile) epilogue(std::true_type{});
-    else epilogue(std::false_type{});
+      if constexpr (PRE) {
+        if (PRE_EDGE && (m_edge || n_edge)) {
+          if constexpr (PRE_EDGE) epilogue_from_lds(std::true_type{});
+        } else epilogue_from_lds(std::false_type{});
+      }
+    } else if (!p.fast_epilogue) epilogue(std::false_type{}, std::true_type{});
+    else if (m_edge || n_edge) epilogue(std::true_type{}, std::true_type{});
+    else epilogue(std::true_type{}, std::false_type{});
     if (!has_next) break;
     vb = vb_next;
     m0 = m0_next;
@@ -1343,8 +1395,8 @@ int launch(const CsGemmArgs& a, hipStream_t stream) {
   p.tiles_n = (p.N + BN - 1) / BN;
   // The epilogue's fast form addresses C, the residual and their byte planes with 32-bit byte offsets from the
   // matrix bases, and takes output row m for accumulator row m.
-  const int64_t lim = (int64_t)UINT32_MAX - 64;
-  p.fast_epilogue = !p.c_rows && !((uintptr_t)p.w_scale & 15) && (int64_t)p.M * p.ldc * 2 < lim && (!p.residual || (int64_t)p.M * p.ldr * 2 < lim);
+  const int64_t lim = 0xFFFF0000ll, rows = (int64_t)p.tiles_m * BM;   // (rows past the last one have offsets too)
+  p.fast_epilogue = !p.c_rows && !((uintptr_t)p.w_scale & 15) && (rows + 1) * p.ldc * 2 < lim && (!p.residual || (rows + 1) * p.ldr * 2 < lim);
   constexpr int lds = RingShape<BM, BN, W_FP8>::BYTES +
                       (residual_piece_through_ring<BM, BN, WAVES_M, WAVES_N, EPI, W_FP8, FUSE, SPLIT_RES>() ? NW * 1024 : 0);
   static bool attr_set = false;
