@@ -7,9 +7,22 @@
 int cs_qkv_window_attn_small(const CsGemmArgs& a, int rows, hipStream_t stream);
 // Whether a launch of `windows` windows takes that form (gemm_small.hip).
 bool cs_qkv_window_attn_few(int64_t windows, int heads, int K);
+// The two-launch form, and whether it is the faster one.
+int cs_qkv_window_attn_two(const CsGemmArgs& a, int rows, int windows, float* x, hipStream_t stream);
+bool cs_qkv_window_attn_two_pays(int64_t rows, int64_t windows, int heads, int K, bool w_fp8);
+
+extern "C" int cs_qkv_window_attn_workspace(int32_t rows, int32_t windows, int32_t heads, int32_t K, int32_t w_fp8) {
+  if (rows < 1 || windows < 1 || heads < 1 || K < 1 || !cs_qkv_window_attn_two_pays(rows, windows, heads, K, w_fp8 != 0)) return 0;
+  return rows * heads * 256 * (int32_t)sizeof(float);   // (at most 8 MB)
+}
 
 extern "C" int cs_qkv_window_attn(const CsGemmArgs* gemm, const float* cos_sin, float scale, int32_t heads,
-                                  int32_t head_dim, void* stream_) {
+                                  int32_t head_dim, void* stream) {
+  return cs_qkv_window_attn_ws(gemm, cos_sin, scale, heads, head_dim, nullptr, 0, stream);
+}
+
+extern "C" int cs_qkv_window_attn_ws(const CsGemmArgs* gemm, const float* cos_sin, float scale, int32_t heads, int32_t head_dim,
+                                     void* workspace, int64_t workspace_bytes, void* stream_) {
   hipStream_t stream = (hipStream_t)stream_;
   if (!gemm || !cos_sin || heads <= 0) return CS_ERR_INVALID_ARG;
   CsGemmArgs a = *gemm;
@@ -32,6 +45,9 @@ extern "C" int cs_qkv_window_attn(const CsGemmArgs* gemm, const float* cos_sin, 
   // per-lane source offsets of the direct loads are 32-bit byte offsets from the matrix bases
   if ((int64_t)a.M * a.lda * 2 >= (int64_t)UINT32_MAX || (int64_t)a.N * a.ldw * (a.w_fp8 ? 1 : 2) >= (int64_t)UINT32_MAX)
     return CS_ERR_UNSUPPORTED;
+  if (workspace && (((uintptr_t)workspace & 15) ||
+                    workspace_bytes < cs_qkv_window_attn_workspace(a.M, ragged ? a.attn_n_win : a.M / 64, heads, a.K, a.w_fp8)))
+    return CS_ERR_INVALID_ARG;
   if (a.M == 0) return CS_OK;
   a.attn_cos_sin = cos_sin;
   a.attn_scale_log2e = scale * 1.4426950408889634f;
@@ -41,8 +57,10 @@ extern "C" int cs_qkv_window_attn(const CsGemmArgs* gemm, const float* cos_sin, 
   if (a.a_norm_inline && !csgemm::inline_norm_width(a.K)) return CS_ERR_UNSUPPORTED;
   // few windows: a workgroup per window and head
   if (cs_qkv_window_attn_few(ragged ? a.attn_n_win : a.M / 64, heads, a.K)) {
-    const int rows = a.M;
+    const int rows = a.M, windows = ragged ? a.attn_n_win : a.M / 64;
+    const int32_t need = workspace ? cs_qkv_window_attn_workspace(rows, windows, heads, a.K, a.w_fp8) : 0;
     if (ragged) a.M = a.attn_n_win * 64;   // (tiles_m counts windows; the operand ends with its last real row)
+    if (need) return cs_qkv_window_attn_two(a, rows, windows, (float*)workspace, stream);
     return cs_qkv_window_attn_small(a, rows, stream);
   }
   if (a.a_norm_inline) return CS_ERR_UNSUPPORTED;

@@ -155,6 +155,15 @@ int cs_gemm_small_workgroups(const CsGemmArgs& a) {
 // round (24 windows: 39 us) it is the slower.
 bool cs_qkv_window_attn_few(int64_t windows, int heads, int K) { return K % 128 == 0 && windows * heads <= 256; }
 
+// Of these the ones that two launches over a workspace serve better (gemm_small_qkv_wattn.hip): while the projection's tiles are
+// one round.  One launch | two, 16 heads, K = 1280, weights from HBM, inline norm: 96 rows 25.4 | 15.7 us, 256 25.4 | 17.7, 320
+// 25.3 | 21.1, 512 25.1 | 22.6 (64x128 tiles from 257 rows on); whole passes of Qwen2.5-VL, 256 patches 2.10 | 1.86 ms, 576 2.71 |
+// 2.66.  Not with fp8 weights, half the bytes: 96 rows 14.8 | 12.9 us, 192 14.8 | 14.8, and at up to 128 rows, where it would be
+// faster, a pass lasts as long as the host takes to launch it (1.87 | 1.90 ms).
+bool cs_qkv_window_attn_two_pays(int64_t rows, int64_t windows, int heads, int K, bool w_fp8) {
+  return !w_fp8 && cs_qkv_window_attn_few(windows, heads, K) && (rows + 63) / 64 * (heads * 2) <= 256;
+}
+
 // (Compared with the big forms of any epilogue, also where a folded LayerNorm has the 160-column ones alone, so it says no too
 // early rather than too late: passes with the rule | both | neither inline, Qwen3-VL 256 patches 1.95 | 1.94 | 2.68 ms, 576 2.62 |
 // 2.54 | 2.87, 896 3.17 | 2.94 | 3.17, 1280 4.03 | 4.59 | 4.03; Qwen2.5-VL 256 2.12 | 2.12 | 2.59, 432 2.57 | 2.42 | 2.61, 576 2.78 |

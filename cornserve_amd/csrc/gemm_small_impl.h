@@ -36,6 +36,7 @@ using namespace csgemm;
 
 constexpr int SM_EPI_BIAS_POS = 100;  // internal: CS_EPI_BIAS plus the (row % pos_period) position addend
 constexpr int SM_EPI_QKV_WATTN = 101; // internal: QKV projection + rotary + window attention of one head and one window
+constexpr int SM_EPI_QKV_F32 = 103;   // internal: the QKV projection of such a launch alone, fp32 output (see gemm_small_qkv_wattn.hip)
 enum { NORM_NONE = 0, NORM_RMS = 1, NORM_LN = 2 };   // inline norm of A's rows
 enum { SUMS_NONE = 0, SUMS_SQ = 1, SUMS_BOTH = 2 };  // row sums of the output
 
@@ -143,73 +144,13 @@ struct SmallShape {
   static_assert(LDS <= 160 * 1024, "the ring fits the LDS");
 };
 
-// QKV projection + rotary + window attention: the epilogue of a tile of one window (64 rows, `cnt` of them real) and one
-// head (15 fragments: q 0..4, k 5..9, v 10..14; see cs_qkv_window_attn for the packed row order).  In the main loop wave w
-// has computed fragments 4w .. 4w+3 of all rows; from here on wave w owns the window's rows 16w .. 16w+15 as queries.
-// What changes hands goes through LDS (the ring is free by now): q and k in fp32 with norm and bias applied (a rotary
-// pair's halves sit in different fragments), v rounded and transposed, then the rotated keys.  Every operation on a value
-// is the one of the big tile's epilogue (gemm_fast_impl.h), in its order.
-template <int MT, int NT, bool W_FP8, int NORM>
-CS_DEVICE void small_wattn_epilogue(const CsGemmArgs& p, char* smem, const f32x4_t (&acc)[MT][NT],
-                                    const float (&rstd_in)[NORM != NORM_NONE ? MT : 1], const int (&mrow)[MT], int m0, int n0, int cnt, int wave, int lane) {
-  static_assert(MT == 4 && NT == 4, "all four row blocks, four fragments per wave");
-  constexpr int HD = 80, HALF = 40, X_BYTES = 4 * 10 * 1024, VT_ROW = 144, VT_BYTES = HD * VT_ROW;
+// What follows the projection in a window (see small_wattn_epilogue), 16 queries a wave: `qk(f)` is fragment f (0 .. 4 q, 5 .. 9
+// k) of the window's row 16 wave + lane % 16, `vt` holds the transposed values, `ks` takes the keys (both the workgroup's).
+template <class Fragment>
+CS_DEVICE void window_attention(const CsGemmArgs& p, const char* vt, char* ks, Fragment qk, const float (&co)[10], const float (&si)[10],
+                                int m0, int n0, int cnt, int wave, int lane) {
+  constexpr int HD = 80, VT_ROW = 144;
   const int lr = lane & 15, kq = lane >> 4;
-  char* const xs = smem;                              // [row block][fragment 0..9][lane]: 4 fp32
-  char* const vt = smem + X_BYTES;                    // [head dim][key]: bf16, 144-byte rows
-  char* const ks = smem + X_BYTES + VT_BYTES;         // [row block][part 0, 1: 16 bytes, part 2: 8 bytes][lane]
-  // per-row scale of the folded RMSNorm: rows 16 i + lr of the window
-  float rstd[MT];
-#pragma unroll
-  for (int i = 0; i < MT; ++i) {
-    rstd[i] = 1.0f;
-    if constexpr (NORM != NORM_NONE) {
-      rstd[i] = rstd_in[NORM != NORM_NONE ? i : 0];
-    } else if (p.a_row_sumsq) {
-      const float* parts = p.a_row_sumsq + (int64_t)mrow[i] * CS_SUMSQ_PARTS;
-      const f32x4_t s0 = *(const f32x4_t*)parts, s1 = *(const f32x4_t*)(parts + 4);
-      const float ss = ((s0[0] + s0[1]) + (s0[2] + s0[3])) + ((s1[0] + s1[1]) + (s1[2] + s1[3]));
-      rstd[i] = rsqrtf(ss / (float)p.K + p.norm_eps);
-    }
-  }
-  // the rotary table's rows of this wave's queries
-  float co[10], si[10];
-  {
-    const float* cs = p.attn_cos_sin + (int64_t)(m0 + min(16 * wave + lr, cnt - 1)) * HD + 10 * kq;
-#pragma unroll
-    for (int t = 0; t < 10; t += 2) {
-      const f32x2_t c2 = *(const f32x2_t*)(cs + t), s2 = *(const f32x2_t*)(cs + HALF + t);
-      co[t] = c2[0];
-      co[t + 1] = c2[1];
-      si[t] = s2[0];
-      si[t + 1] = s2[1];
-    }
-  }
-  __syncthreads();   // (nobody reads operands from the ring any more)
-#pragma unroll
-  for (int j = 0; j < NT; ++j) {
-    const int J = 4 * wave + j;
-    if (J >= 15) break;
-    const int ch = n0 + (J / 2) * 32 + 8 * kq + (J % 2) * 4;
-    const bf16x4_t bias_b = *(const bf16x4_t*)((const bf16_t*)p.bias + ch);
-    f32x4_t wsc = {1.f, 1.f, 1.f, 1.f};
-    if constexpr (W_FP8) wsc = *(const f32x4_t*)(p.w_scale + ch);
-#pragma unroll
-    for (int i = 0; i < MT; ++i) {
-      f32x4_t x;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        x[r] = __builtin_fmaf(acc[i][j][r], W_FP8 ? wsc[r] : rstd[i], bf2f(bias_b[r]));   // (no folded norm with fp8 weights)
-      }
-      if (J < 10) {
-        *(f32x4_t*)(xs + ((i * 10 + J) * 64 + lane) * 16) = x;
-      } else {   // head dims 16 (J - 10) + 4 kq + r of key 16 i + lr
-#pragma unroll
-        for (int r = 0; r < 4; ++r) *(bf16_t*)(vt + (16 * (J - 10) + 4 * kq + r) * VT_ROW + (16 * i + lr) * 2) = f2bf(x[r]);
-      }
-    }
-  }
-  __syncthreads();
   // ---- rotary of this wave's q and k rows; the keys go back to LDS as operand fragments
   bf16x8_t q8[2];
   bf16x4_t q4;
@@ -218,7 +159,7 @@ CS_DEVICE void small_wattn_epilogue(const CsGemmArgs& p, char* smem, const f32x4
     float x[20], o[20];
 #pragma unroll
     for (int f = 0; f < 5; ++f) {
-      const f32x4_t v = *(const f32x4_t*)(xs + ((wave * 10 + which * 5 + f) * 64 + lane) * 16);
+      const f32x4_t v = qk(which * 5 + f);
 #pragma unroll
       for (int r = 0; r < 4; ++r) x[4 * f + r] = v[r];
     }
@@ -299,6 +240,76 @@ CS_DEVICE void small_wattn_epilogue(const CsGemmArgs& p, char* smem, const f32x4
       *(bf16x4_t*)(out + 16 * d) = o;
     }
   }
+}
+
+// QKV projection + rotary + window attention: the epilogue of a tile of one window (64 rows, `cnt` of them real) and one
+// head (15 fragments: q 0..4, k 5..9, v 10..14; see cs_qkv_window_attn for the packed row order).  In the main loop wave w
+// has computed fragments 4w .. 4w+3 of all rows; from here on wave w owns the window's rows 16w .. 16w+15 as queries.
+// What changes hands goes through LDS (the ring is free by now): q and k in fp32 with norm and bias applied (a rotary
+// pair's halves sit in different fragments), v rounded and transposed, then the rotated keys.  Every operation on a value
+// is the one of the big tile's epilogue (gemm_fast_impl.h), in its order.
+template <int MT, int NT, bool W_FP8, int NORM>
+CS_DEVICE void small_wattn_epilogue(const CsGemmArgs& p, char* smem, const f32x4_t (&acc)[MT][NT],
+                                    const float (&rstd_in)[NORM != NORM_NONE ? MT : 1], const int (&mrow)[MT], int m0, int n0, int cnt, int wave, int lane) {
+  static_assert(MT == 4 && NT == 4, "all four row blocks, four fragments per wave");
+  constexpr int HD = 80, HALF = 40, X_BYTES = 4 * 10 * 1024, VT_ROW = 144, VT_BYTES = HD * VT_ROW;
+  const int lr = lane & 15, kq = lane >> 4;
+  char* const xs = smem;                              // [row block][fragment 0..9][lane]: 4 fp32
+  char* const vt = smem + X_BYTES;                    // [head dim][key]: bf16, 144-byte rows
+  char* const ks = smem + X_BYTES + VT_BYTES;         // [row block][part 0, 1: 16 bytes, part 2: 8 bytes][lane]
+  // per-row scale of the folded RMSNorm: rows 16 i + lr of the window
+  float rstd[MT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i) {
+    rstd[i] = 1.0f;
+    if constexpr (NORM != NORM_NONE) {
+      rstd[i] = rstd_in[NORM != NORM_NONE ? i : 0];
+    } else if (p.a_row_sumsq) {
+      const float* parts = p.a_row_sumsq + (int64_t)mrow[i] * CS_SUMSQ_PARTS;
+      const f32x4_t s0 = *(const f32x4_t*)parts, s1 = *(const f32x4_t*)(parts + 4);
+      const float ss = ((s0[0] + s0[1]) + (s0[2] + s0[3])) + ((s1[0] + s1[1]) + (s1[2] + s1[3]));
+      rstd[i] = rsqrtf(ss / (float)p.K + p.norm_eps);
+    }
+  }
+  // the rotary table's rows of this wave's queries
+  float co[10], si[10];
+  {
+    const float* cs = p.attn_cos_sin + (int64_t)(m0 + min(16 * wave + lr, cnt - 1)) * HD + 10 * kq;
+#pragma unroll
+    for (int t = 0; t < 10; t += 2) {
+      const f32x2_t c2 = *(const f32x2_t*)(cs + t), s2 = *(const f32x2_t*)(cs + HALF + t);
+      co[t] = c2[0];
+      co[t + 1] = c2[1];
+      si[t] = s2[0];
+      si[t + 1] = s2[1];
+    }
+  }
+  __syncthreads();   // (nobody reads operands from the ring any more)
+#pragma unroll
+  for (int j = 0; j < NT; ++j) {
+    const int J = 4 * wave + j;
+    if (J >= 15) break;
+    const int ch = n0 + (J / 2) * 32 + 8 * kq + (J % 2) * 4;
+    const bf16x4_t bias_b = *(const bf16x4_t*)((const bf16_t*)p.bias + ch);
+    f32x4_t wsc = {1.f, 1.f, 1.f, 1.f};
+    if constexpr (W_FP8) wsc = *(const f32x4_t*)(p.w_scale + ch);
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      f32x4_t x;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        x[r] = __builtin_fmaf(acc[i][j][r], W_FP8 ? wsc[r] : rstd[i], bf2f(bias_b[r]));   // (no folded norm with fp8 weights)
+      }
+      if (J < 10) {
+        *(f32x4_t*)(xs + ((i * 10 + J) * 64 + lane) * 16) = x;
+      } else {   // head dims 16 (J - 10) + 4 kq + r of key 16 i + lr
+#pragma unroll
+        for (int r = 0; r < 4; ++r) *(bf16_t*)(vt + (16 * (J - 10) + 4 * kq + r) * VT_ROW + (16 * i + lr) * 2) = f2bf(x[r]);
+      }
+    }
+  }
+  __syncthreads();
+  window_attention(p, vt, ks, [&](int f) { return *(const f32x4_t*)(xs + ((wave * 10 + f) * 64 + lane) * 16); }, co, si, m0, n0, cnt, wave, lane);
 }
 
 template <int BM, int BN, int WAVES_M, int WAVES_N, int KS, int STAGES, int EPI, bool W_FP8, int NORM, bool SPLIT, int SUMS>
@@ -679,6 +690,29 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, EPI == SM_EPI_QKV_WATTN ? 1
   if constexpr (NORM == NORM_LN) {
 #pragma unroll
     for (int j = 0; j < NT; ++j) csum_v[NORM == NORM_LN ? j : 0] = *(const f32x4_t*)(p.w_col_sum + ncol[j]);
+  }
+  if constexpr (EPI == SM_EPI_QKV_F32) {   // (the arithmetic of small_wattn_epilogue; C is fp32, W is not fp8)
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      float row_scale = 1.0f;
+      if constexpr (NORM != NORM_NONE) {
+        row_scale = rstd[NORM != NORM_NONE ? i : 0];
+      } else if (p.a_row_sumsq) {
+        const float* parts = p.a_row_sumsq + (int64_t)mrow[i] * CS_SUMSQ_PARTS;
+        const f32x4_t s0 = *(const f32x4_t*)parts, s1 = *(const f32x4_t*)(parts + 4);
+        const float ss = ((s0[0] + s0[1]) + (s0[2] + s0[3])) + ((s1[0] + s1[1]) + (s1[2] + s1[3]));
+        row_scale = rsqrtf(ss / (float)p.K + p.norm_eps);
+      }
+#pragma unroll
+      for (int j = 0; j < NT; ++j) {
+        const bf16x4_t bias_b = __builtin_bit_cast(bf16x4_t, bias_w[j]);
+        f32x4_t x;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) x[r] = __builtin_fmaf(acc[i][j][r], row_scale, bf2f(bias_b[r]));
+        if (mok[i]) *(f32x4_t*)((float*)p.C + (int64_t)mrow[i] * p.ldc + col[j]) = x;
+      }
+    }
+    return;
   }
   bf16_t* const pC = (bf16_t*)p.C;
   float oss[SUMS != SUMS_NONE ? MT : 1], osm[SUMS == SUMS_BOTH ? MT : 1];

@@ -301,7 +301,12 @@ void qkv_window_attn_(const Tensor& out, const Tensor& x, const Tensor& w_packed
     args.w_scale = (const float*)w_scale->data_ptr();
   }
   set_prefetch(args, get(prefetch), x.device());
-  check_status(cs_qkv_window_attn(&args, (const float*)cos_sin.data_ptr(), (float)scale, (int32_t)heads, (int32_t)d, current_stream()),
+  // (a workspace of the allocator's: its memory is handed on in the order of the current stream)
+  const int64_t windows = win_start ? win_start->numel() - 1 : M / WATTN_WINDOW;
+  const int32_t need = cs_qkv_window_attn_workspace((int32_t)M, (int32_t)windows, (int32_t)heads, (int32_t)K, w_scale ? 1 : 0);
+  const Tensor workspace = need ? at::empty({need}, x.options().dtype(at::kByte)) : Tensor();
+  check_status(cs_qkv_window_attn_ws(&args, (const float*)cos_sin.data_ptr(), (float)scale, (int32_t)heads, (int32_t)d,
+                                     need ? workspace.data_ptr() : nullptr, need, current_stream()),
                "cs_qkv_window_attn");
 }
 

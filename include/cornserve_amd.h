@@ -326,6 +326,14 @@ int cs_attn_varlen_keys_rotated(const void* q, const void* k, const void* v, int
 int cs_qkv_window_attn(const CsGemmArgs* gemm, const float* cos_sin, float scale, int32_t heads, int32_t head_dim,
                        void* stream);
 
+/* The same with a workspace (16-byte aligned device memory that nothing else uses until the call's work has run): a few windows
+ * then run as two launches, the projection over the whole chip and the attention of its fp32 values.  Same bits.
+ * cs_qkv_window_attn_workspace (host routine): the bytes it takes for `rows` rows of A in `windows` windows, 0 where one
+ * launch is the faster form; a workspace that is smaller is CS_ERR_INVALID_ARG, NULL means one launch.                 */
+int cs_qkv_window_attn_workspace(int32_t rows, int32_t windows, int32_t heads, int32_t K, int32_t w_fp8);
+int cs_qkv_window_attn_ws(const CsGemmArgs* gemm, const float* cos_sin, float scale, int32_t heads, int32_t head_dim,
+                          void* workspace, int64_t workspace_bytes, void* stream);
+
 /* Host routine: expand cu_seqlens_host[n_seg+1] into query-block work items of at most block_q rows
  * (block_q = cs_attn_block_q(max_seqlen)).  Writes n_work items of 4 int32 into work_host.      */
 int cs_attn_block_q(int32_t max_seqlen);

@@ -734,6 +734,52 @@ def test_qkv_window_attn_few_windows_equal_many(ops, dev, windows, heads, ragged
     assert torch.equal(got, want)
 
 
+@pytest.mark.parametrize("form,rows", [("inline", 4), ("plain", 128), ("array", 132), ("inline", 256), ("inline", 260), ("array", 512),
+                                       ("plain", 508), ("inline", 516), ("fp8", 128)])
+def test_qkv_window_attn_two_launches_equal_one(ops, dev, form, rows):
+    """The projection and the attention as two launches over a workspace: the bits of the one launch, at the edges of the
+    projection's tile forms and of the rule (16 heads: 512 rows, no fp8 weights), with a hint that both launches read."""
+    import ctypes
+
+    from cornserve_amd import lib
+
+    dll = lib.load()
+    heads, d, K = 16, 80, 1280
+    last = rows % 64 or 64
+    counts = [64] * ((rows - last) // 64) + ([last - 4, 4] if last > 4 else [last])
+    cu = torch.tensor([0, *torch.tensor(counts).cumsum(0).tolist()], dtype=torch.int32, device=dev)
+    x, w, b = rnd((rows, K), 1.0, 131, dev), rnd((3 * heads * d, K), 0.05, 132, dev), rnd((3 * heads * d,), 0.02, 133, dev)
+    cos = torch.rand((rows, d), generator=torch.Generator().manual_seed(rows)).to(dev)
+    args = lib.CsGemmArgs()
+    sc = (w.float().abs().amax(1) / 448.0).contiguous()
+    if form == "fp8":
+        wp, bp, sp = ops.pack_qkv_window_attn((w.float() / sc[:, None]).to(torch.float8_e4m3fn), b, heads, w_scale=sc)
+        args.w_fp8, args.w_scale = 1, sp.data_ptr()
+    else:
+        wp, bp = ops.pack_qkv_window_attn(w, b, heads)
+    ss, hint = ops.row_sumsq(x), torch.zeros(24 << 20, dtype=torch.uint8, device=dev)
+    args.A, args.lda, args.W, args.ldw, args.bias, args.ldc = x.data_ptr(), K, wp.data_ptr(), K, bp.data_ptr(), heads * d
+    args.M, args.N, args.K, args.norm_eps = rows, heads * 256, K, 1e-6
+    args.attn_win_start, args.attn_n_win = cu.data_ptr(), len(counts)
+    args.a_norm_inline, args.a_row_sumsq = int(form == "inline"), ss.data_ptr() if form == "array" else None
+    args.prefetch, args.prefetch_bytes = hint.data_ptr(), hint.numel()
+    need = dll.cs_qkv_window_attn_workspace(rows, len(counts), heads, K, args.w_fp8)
+    assert need == (0 if rows > 512 or form == "fp8" else rows * heads * 256 * 4)
+    work = torch.full((max(need, 16) + 4096,), 255, dtype=torch.uint8, device=dev)
+    got = []
+    for ptr, size in ((None, 0), (work.data_ptr(), max(need, 16))):
+        out = torch.full((rows + 8, heads * d), 7.0, dtype=torch.bfloat16, device=dev)
+        args.C = out.data_ptr()
+        call = lambda p, n: dll.cs_qkv_window_attn_ws(ctypes.byref(args), cos.data_ptr(), d**-0.5, heads, d, p, n, 0)
+        assert call(ptr, size) == 0
+        torch.cuda.synchronize()
+        assert (out[rows:] == 7.0).all()
+        got.append(out)
+    assert torch.equal(*got) and (work[max(need, 16):] == 255).all()
+    if need:   # refused before anything is launched
+        assert call(work.data_ptr(), need - 1) != 0 and call(work.data_ptr() + 4, need) != 0
+
+
 def test_gemm_prefetch_hint_leaves_the_result_alone(ops, dev):
     """A launch with few tiles and a `prefetch` tensor starts extra workgroups that only read that tensor: the product
     has the bits it has without the hint, whatever the hinted size (odd, shorter than one 16-byte piece, many MB), on
