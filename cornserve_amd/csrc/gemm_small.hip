@@ -152,7 +152,8 @@ int cs_gemm_small_workgroups(const CsGemmArgs& a) {
 
 // One workgroup per window and head while the chip holds them all at once: 24 to 26 us up to 16 windows of 16 heads (inline norm,
 // weights from HBM; 21 to 23 without norm), where a big tile (four windows) takes 32 to 35 us whatever the count; with a second
-// round (24 windows: 39 us) it is the slower.
+// round (24 windows: 39 us) it is the slower.  (The first 512 rows of bf16 weights go to two launches where there is a workspace, see
+// below.)
 bool cs_qkv_window_attn_few(int64_t windows, int heads, int K) { return K % 128 == 0 && windows * heads <= 256; }
 
 // Of these the ones that two launches over a workspace serve better (gemm_small_qkv_wattn.hip): while the projection's tiles are

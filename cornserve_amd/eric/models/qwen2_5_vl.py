@@ -316,9 +316,9 @@ class Qwen2_5_VisionTransformer(QwenVisionBase):
         routes agree within the parity tolerance, not bit for bit; since the route depends on the item alone, an item's
         embedding is the same bits whatever it is batched with (setting the attribute to False afterwards selects the
         separate kernels for every item).  `fuse_min_rows` > 0 is a deployment knob that gives this up for latency: a
-        batch with fewer one-launch rows than that takes the separate kernels throughout, whose GEMM spreads over more
-        compute units than a workgroup per window and head (96 patches 1.52 against 1.80 ms; 1024 3.08 against 2.95, 2048 4.23
-        against 4.25, 3072 5.40 against 5.00: only the smallest batches gain).
+        batch with fewer one-launch rows than that takes the separate kernels throughout (nothing to gain since a few
+        windows take their projection over the whole chip: 96 patches 1.52 against 1.51 ms, 256 1.85 against 1.85, 576 2.68
+        against 2.64, 1024 3.06 against 2.94).
 
         `split_residual`: carry the residual stream (:175,177) with 16 significant bits -- the bf16 tensor every
         kernel reads plus a byte plane with the next 8 mantissa bits, joined and re-split inside the two residual GEMMs
