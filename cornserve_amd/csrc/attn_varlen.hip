@@ -96,9 +96,13 @@ CS_DEVICE void score_tile(f32x16_t (&sacc)[2], const char* k_tile, const bf16x8_
 // wave sees a score more than LAZY_LOG2 (in log2 units) above it.  P then ranges up to 2^LAZY_LOG2 instead of 1,
 // which fp32 accumulation and bf16's exponent range do not care about, the final division by the denominator
 // (built from the same P) cancels the reference, and the rescale of O -- DT*16 multiplies and an exponential per
-// tile -- runs only in the first tiles of a segment.  m_run starts at -inf, so the first tile always sets it to
-// its own maximum.  With L_FROM_MFMA the denominator is not summed here (see attn_full_kernel).
+// tile -- runs only in the first tiles of a segment.  The whole wave is raised, each query to its own maximum so far: the
+// nearer the reference is to a query's largest scores, the less their P is rounded (scores of standard deviation 9, largest
+// weights near 1: error against 64 bits 1.63e-3 at d = 80 and 1.71e-3 at d = 64, where raising only the queries that ask for
+// it gives 1.66e-3 and 1.86e-3).  m_run starts at -inf, so the first tile always sets it to its own maximum.  With
+// L_FROM_MFMA the denominator is not summed here (see attn_full_kernel).
 // FIRST_TILE: the caller knows that nothing has been accumulated yet (O = 0, m_run = -inf): no rescale to consider.
+constexpr float LAZY_LOG2 = 6.0f;
 template <int DT, bool L_FROM_MFMA, bool FIRST_TILE = false>
 CS_DEVICE void softmax_tile(const f32x16_t (&sacc)[2], bf16x8_t (&pf)[2][2], f32x16_t (&oacc)[DT], float& m_run,
                             float& l_run, float sl2) {
@@ -108,7 +112,6 @@ CS_DEVICE void softmax_tile(const f32x16_t (&sacc)[2], bf16x8_t (&pf)[2][2], f32
 #pragma unroll
     for (int r = 0; r < 16; ++r) mx = fmaxf(mx, sacc[kt][r]);
   mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-  constexpr float LAZY_LOG2 = 6.0f;
   float alpha = 1.0f;
   if constexpr (FIRST_TILE) {
     m_run = mx;
@@ -163,18 +166,8 @@ CS_DEVICE void write_output(const f32x16_t (&oacc)[DT], float l_run, bf16_t* oro
     }
 }
 
-// ---- softmax of the long-segment kernels, half a key tile (32 keys) at a time, and per query.  The reference maximum m of a query
-//      is that of its segment's first tile, and P = exp2((s - m) * scale - shift).  With the shift, a score has to exceed m by
-//      2^(shift + 1) before P reaches 2; until then m stays.  Whether it happened shows in the packed words themselves -- P >= 2
-//      is the top exponent bit of a bf16 -- so the usual half tile needs no maximum, no exchange between lanes and no
-//      comparison in front of its exponentials: 4 word-wise ORs instead of 9 instructions and an LDS round trip (a NaN has
-//      the bit set as well and takes the slow way, where fmaxf leaves m alone).  The slow way raises m for exactly the
-//      queries that exceeded it, so that a query's bits depend on its own scores only, whichever queries share its wave.
-//      The shift cancels in the division by the denominator; segments of one tile cannot exceed their maximum and use none,
-//      which gives them the bits of attn_kernel.
-constexpr float P_SHIFT_LOG2 = 8.0f;
-constexpr uint32_t P_TWO_BIT = 0x40004000u;   // set in a bf16 pair iff one of two non-negative values is >= 2 (or NaN)
-
+// ---- softmax_tile in the pieces that the pipeline of attn_full_direct_kernel works on, half a key tile (32 keys) at a time: the
+//      same operations on a query's values in the same order, so that a query has the same bits in every kernel.
 CS_DEVICE float row_max(const f32x16_t& s) {
   float mx = s[0];
 #pragma unroll
@@ -186,53 +179,6 @@ CS_DEVICE float pair_max(float v) {
   const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, v), __builtin_bit_cast(uint32_t, v), false, false);
   const uint32_t lower = r[0], upper = r[1];   // (named: a bit cast of a vector element takes the vector's first)
   return fmaxf(__builtin_bit_cast(float, lower), __builtin_bit_cast(float, upper));
-}
-// P of one half tile as operands of the second product (two bf16 per word); the OR of their words.  SUM: adds P to the lane's
-// running sum.
-template <bool SUM>
-CS_DEVICE uint32_t exp_half(const f32x16_t& s, i32x4_t (&p)[2], float sl2, float mb, float& l_run) {
-  uint32_t any = 0;
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const float a = __builtin_amdgcn_exp2f(__builtin_fmaf(s[2 * i], sl2, -mb));
-    const float b = __builtin_amdgcn_exp2f(__builtin_fmaf(s[2 * i + 1], sl2, -mb));
-    if constexpr (SUM) {
-      l_run += a;
-      l_run += b;
-    }
-    bf16x2_t w;
-    w[0] = f2bf(a);
-    w[1] = f2bf(b);
-    const uint32_t word = __builtin_bit_cast(uint32_t, w);
-    p[i >> 2][i & 3] = (int)word;
-    any |= word;
-  }
-  return any;
-}
-// The slow way: m raised where a query exceeded it, O and the sum rescaled, P computed again.
-template <int DT, bool SUM>
-CS_DEVICE void raise_reference(const f32x16_t& s, i32x4_t (&p)[2], f32x16_t (&oacc)[DT], float& m_run, float& mb, float& l_run, float sl2,
-                               float shift) {
-  const float mx = pair_max(row_max(s));
-  const bool up = __builtin_fmaf(mx, sl2, -mb) >= 1.0f;
-  const float alpha = up ? __builtin_amdgcn_exp2f((m_run - mx) * sl2) : 1.0f;
-#pragma unroll
-  for (int t = 0; t < DT; ++t)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) oacc[t][r] *= alpha;
-  if constexpr (SUM) l_run *= alpha;
-  m_run = up ? mx : m_run;
-  mb = __builtin_fmaf(m_run, sl2, shift);
-  exp_half<SUM>(s, p, sl2, mb, l_run);
-}
-// exp_half, and raise_reference if any lane of the wave asks for it (l_run of before the half tile is what is rescaled)
-template <int DT, bool SUM>
-CS_DEVICE void softmax_half(const f32x16_t& s, i32x4_t (&p)[2], f32x16_t (&oacc)[DT], float& m_run, float& mb, float& l_run, float sl2,
-                            float shift) {
-  float l_new = l_run;
-  const uint32_t any = exp_half<SUM>(s, p, sl2, mb, l_new);
-  if (__any((any & P_TWO_BIT) != 0)) raise_reference<DT, SUM>(s, p, oacc, m_run, mb, l_run, sl2, shift);
-  else l_run = l_new;
 }
 
 template <int D, int NWAVES, bool ROPE, int HPW>
@@ -659,9 +605,9 @@ __global__ __launch_bounds__(256, 2) void attn_full_kernel(const AttnArgs a) {
   for (int t = 0; t < DT; ++t)
 #pragma unroll
     for (int r = 0; r < 16; ++r) oacc[t][r] = 0.f;
-  float m_run = 0.f, mb = 0.f, l_run = 0.f;
+  float m_run = -INFINITY, l_run = 0.f;
   const bool wave_active = wave * 32 < nq;
-  const float sl2 = a.scale_log2e, shift = seg_len > BKV ? P_SHIFT_LOG2 : 0.0f;
+  const float sl2 = a.scale_log2e;
 
   int buf = 0;
   for (int kv0 = 0; kv0 < seg_len; kv0 += BKV, buf ^= 1) {
@@ -672,21 +618,17 @@ __global__ __launch_bounds__(256, 2) void attn_full_kernel(const AttnArgs a) {
       const char* kd = k_buf(buf);
       const char* vd = v_buf(buf);
       f32x16_t sacc[2];
+      bf16x8_t pf[2][2];
       score_tile<KS, RS>(sacc, kd, qf, nvalid, fr, hf);
-      if (kv0 == 0) {
-        m_run = pair_max(fmaxf(row_max(sacc[0]), row_max(sacc[1])));
-        mb = __builtin_fmaf(m_run, sl2, shift);
-      }
+      softmax_tile<DT, L_FROM_MFMA>(sacc, pf, oacc, m_run, l_run, sl2);
 #pragma unroll
-      for (int kt = 0; kt < 2; ++kt) {
-        i32x4_t pf[2];
-        softmax_half<DT, !L_FROM_MFMA>(sacc[kt], pf, oacc, m_run, mb, l_run, sl2, shift);
+      for (int t = 0; t < DT; ++t) {
 #pragma unroll
-        for (int t = 0; t < DT; ++t)
+        for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
           for (int kk = 0; kk < 2; ++kk) {
             const bf16x8_t vf = read_vt_frag(vd, t, kt * 2 + kk, lane);
-            oacc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, __builtin_bit_cast(bf16x8_t, pf[kk]), oacc[t], 0, 0, 0);
+            oacc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, pf[kt][kk], oacc[t], 0, 0, 0);
           }
       }
     }
@@ -694,29 +636,33 @@ __global__ __launch_bounds__(256, 2) void attn_full_kernel(const AttnArgs a) {
     __syncthreads();
   }
 
-  if constexpr (!L_FROM_MFMA) l_run += __shfl_xor(l_run, 32, 64);
   const int qi = wave * 32 + fr;
   write_output<D, DT, L_FROM_MFMA>(oacc, l_run, a.out + (int64_t)(q0 + min(qi, nq - 1)) * a.ldo + hoff, qi < nq, hf);
 }
 
 // Full attention without rotary on the keys (SigLIP; the Qwen families after cs_rope_qk): a software pipeline over half tiles of
-// 32 keys.  One step issues the matrix instructions of two different half tiles -- P.V of the previous one and the scores of the
-// next one -- while the vector unit works on the softmax of the one between them.  Nothing in a step waits for a result of the
-// same step, so the matrix cores run under the softmax of the SAME wave: with the three phases one after the other, three waves
-// per SIMD took 1,370 clocks of a SIMD per wave and 64-key tile (704 of them matrix instructions), two waves of this kernel take
-// 960 to 1,080.  How the instructions of a step interleave is laid down with scheduling groups; two waves per SIMD (two
-// workgroups per CU) use what a wave leaves free.  V fragments live in two register sets, the next step's being read during
-// this one; K fragments are read at the start of their own step, whose first matrix instructions are those of P.V (two
-// register sets for K as well: the same time, and head dim 96 spills).
-//   16 heads, back to back, before -> after, d = 72: 4 x 4096 rows 411 -> 365 us, 4096 rows 124 -> 102, 3300 + 1196 + 1024 + 720 rows
-//   125 -> 100, 7 x 729 rows 38.0 -> 36.4, 2 x 729 rows 19.8 -> 15.4; d = 80: 8 x 1024 rows 75 -> 68, 1024 rows 24.0 -> 17.8, 1380 + 816
-//   rows 43 -> 29, 4888 rows 230 -> 172, 16 segments of 432 to 9000 rows 2918 -> 2025, 16 x 1008 rows 138 -> 131; d = 64: 2 x 1500 rows 43.1 ->
-//   40.4; d = 96: 55.4 -> 52.0 us.
-// What bounds it now is power: under it the shader clock falls from 1.9 to 1.4 .. 1.7 GHz, and a build without the LDS reads runs as many
-// clocks at a higher clock rate.  Also measured: 64 query rows per wave and one wave per SIMD (half the LDS reads, but a lone wave
-// issues an instruction every five clocks: 2,630 clocks per 64 rows and tile against 1,930), eight waves around one K/V stream
-// (the same time within 3 %; 7 x 729 rows 41 us), and dims 64 .. 79 of O^T in 16x16 blocks (a sixth less V read and multiplied,
-// eight lane swaps more: no faster).
+// 32 keys.  One step issues the matrix instructions of two different half tiles -- P.V of the previous one and the scores of one
+// of the next tile -- while the vector unit works on the softmax of the one between them.  Nothing in a step waits for a matrix
+// result of the same step, so the matrix cores run under the softmax of the SAME wave: with the three phases one after the
+// other, three waves per SIMD took 1,370 clocks of a SIMD per wave and 64-key tile, 704 of them matrix instructions.  The
+// arithmetic is softmax_tile's, bit for bit: scores run a whole tile ahead, because a tile's reference maximum is that of all its 64
+// keys, and a half tile's scores stay in their registers until the products of the same half of the next tile overwrite them
+// (the exponents are taken out in phase 1, P.V; those products are phase 2).  How the instructions of a phase interleave is
+// laid down with scheduling groups; two waves per SIMD (two workgroups per CU) use what a wave leaves free.  V fragments live
+// in two register sets, the next step's being read during this one; K fragments are read at the start of their own step.
+//   16 heads, back to back, one phase after the other -> this kernel, d = 72: 4 x 4096 rows 370 -> 354 us, 4096 rows 105 -> 94,
+//   3300 + 1196 + 1024 + 720 rows 146 -> 86, 7 x 729 rows 34.1 -> 34.4, 2 x 729 rows 18.6 -> 14.9; d = 80: 8 x 1024 rows 59.3 -> 60.4, 1024
+//   rows 22.4 -> 17.4, 1380 + 816 rows 38.6 -> 26.4, 4888 rows 205 -> 162, 9000 + 5000 + 3000 + 1000 + 432 rows 719 -> 640, 16 x 1008 rows 113 ->
+//   117; d = 64: 2 x 1500 rows 37.7 -> 32.9; d = 96: 46.9 -> 42.7 us.  (A launch that fills the chip with equal segments gains
+//   nothing; 4 to 12 instead of 8 exponentials in phase 1 are the same within 3 %.)
+// A reference that is the first tile's maximum plus a margin, whose overrun shows in the packed words, needs no maximum of a tile:
+// 3 to 5 % faster, but P is rounded elsewhere and less exactly (wide scores, d = 80: error against 64 bits 1.67e-3 instead of 1.63e-3,
+// d = 64: 1.97e-3 instead of 1.71e-3).
+// What bounds it is power: the shader clock falls from 1.9 to 1.4 .. 1.7 GHz under such a pipeline, and a build without the LDS reads
+// ran as many clocks at a higher clock rate.  Also measured: 64 query rows per wave and one wave per SIMD (half the LDS reads,
+// but a lone wave issues an instruction every five clocks: 2,630 clocks per 64 rows and tile against 1,930), eight waves around
+// one K/V stream (the same time within 3 %; 7 x 729 rows 41 us), and dims 64 .. 79 of O^T in 16x16 blocks (a sixth less V read and
+// multiplied, eight lane swaps more: no faster).
 //
 // K and V tiles go global -> LDS directly (buffer_load ... lds: no staging registers, no LDS store instructions, no
 // address arithmetic per tile) into a ring of three tile buffers, requested two tiles ahead.  A direct load fixes the LDS
@@ -917,9 +863,8 @@ __global__ __launch_bounds__(256, 2) void attn_full_direct_kernel(const AttnArgs
   for (int t = 0; t < DT; ++t)
 #pragma unroll
     for (int r = 0; r < 16; ++r) oacc[t][r] = 0.f;
-  float m_run = 0.f, mb = 0.f, l_run = 0.f;
-  const bool wave_active = wave * 32 < nq;
-  const float sl2 = a.scale_log2e, shift = n_tiles > 1 ? P_SHIFT_LOG2 : 0.0f;
+  float mb = 0.f, l_run = 0.f;
+  const float sl2 = a.scale_log2e;
   const int sg = lane & 15;
   const int k_lane = fr * RS + hf * 16;
   const int v_lane = (4 * hf + (sg >> 2)) * V_RS + (16 * ((lane >> 4) & 1) + 4 * (sg & 3)) * 2;   // see read_vt_frag
@@ -958,38 +903,77 @@ __global__ __launch_bounds__(256, 2) void attn_full_direct_kernel(const AttnArgs
     for (int r = 0; r < 16; ++r)
       if (8 * (r >> 2) + (r & 3) >= left) s[r] = -INFINITY;
   };
-  // One step: O += V^T.P of p_in and vf, s_out = scores of half k_half of the tile in buffer k_b, p_out = softmax of s_in; meanwhile
-  // the V fragments of the next step are read (half v_half of the tile in buffer v_b).
-  auto step = [&](const f32x16_t& s_in, i32x4_t (&p_out)[2], f32x16_t& s_out, const i32x4_t (&p_in)[2],
-                  const bf16x8_t (&vf)[DT][2], int k_b, int k_half, bf16x8_t (&vf_next)[DT][2], int v_b, int v_half) {
-    bf16x8_t kf[KS];
-    read_k(kf, k_b, k_half);
-    read_v(vf_next, v_b, v_half);
-    pv(p_in, vf);
-    scores(s_out, kf);
-    float l_new = l_run;
-    const uint32_t any = exp_half<!L_FROM_MFMA>(s_in, p_out, sl2, mb, l_new);
-    // per matrix instruction two LDS reads, its share of the plain vector instructions (16 multiply-adds, 8 conversions, 4 ORs, the
-    // sums, a few addresses) and two exponentials
-    constexpr int N_MFMA = KS + 2 * DT, N_VALU = (L_FROM_MFMA ? 32 : 48) / N_MFMA + (L_FROM_MFMA ? 1 : 0);
+  // One step: O += V^T.P of p_in and vf (phase 1), then s_io, a half tile's scores, becomes those of half `half` of the tile in buffer k_b
+  // (phase 2); p_out = exponentials of what s_io held, a part of them in either phase.  Meanwhile the V fragments of the next
+  // step are read (half `half` of the tile in buffer v_b), and the maximum of s_max is taken, which `vote` gets between the phases.
+  constexpr int EXP_1 = 8;   // exponentials of phase 1
+  auto exponents = [&](float (&e)[16], const f32x16_t& s) {
 #pragma unroll
-    for (int i = 0; i < N_MFMA; ++i) {
+    for (int r = 0; r < 16; ++r) e[r] = __builtin_fmaf(s[r], sl2, -mb);
+#pragma unroll
+    for (int r = 0; r < EXP_1; ++r) e[r] = __builtin_amdgcn_exp2f(e[r]);
+  };
+  auto step = [&](f32x16_t& s_io, i32x4_t (&p_out)[2], const i32x4_t (&p_in)[2], const bf16x8_t (&vf)[DT][2], bf16x8_t (&vf_next)[DT][2],
+                  int k_b, int v_b, int half, const f32x16_t& s_max, float& psum, auto vote) {
+    bf16x8_t kf[KS];
+    float e[16];
+    read_k(kf, k_b, half);
+    read_v(vf_next, v_b, half);
+    pv(p_in, vf);
+    float mx = row_max(s_max);
+    asm volatile("" : "+v"(mx));   // (here and below: what is used behind a branch is not moved there, out of the overlap)
+    exponents(e, s_io);
+#pragma unroll
+    for (int i = 0; i < 2 * DT; ++i) {
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
-      __builtin_amdgcn_sched_group_barrier(0x002, N_VALU, 0);
-      __builtin_amdgcn_sched_group_barrier(0x400, 2, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, (KS + 4 * DT + 2 * DT - 1) / (2 * DT), 0);
+      __builtin_amdgcn_sched_group_barrier(0x002, 28 / (2 * DT), 0);
+      __builtin_amdgcn_sched_group_barrier(0x400, (EXP_1 + 2 * DT - 1) / (2 * DT), 0);
     }
-    if (__any((any & P_TWO_BIT) != 0)) raise_reference<DT, !L_FROM_MFMA>(s_in, p_out, oacc, m_run, mb, l_run, sl2, shift);
-    else l_run = l_new;
+    vote(e, mx);
+    __builtin_amdgcn_sched_barrier(0);
+    scores(s_io, kf);
+#pragma unroll
+    for (int r = EXP_1; r < 16; ++r) e[r] = __builtin_amdgcn_exp2f(e[r]);
+    if constexpr (!L_FROM_MFMA) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) psum += e[r];
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      bf16x2_t w;
+      w[0] = f2bf(e[2 * i]);
+      w[1] = f2bf(e[2 * i + 1]);
+      p_out[i >> 2][i & 3] = __builtin_bit_cast(int, w);
+    }
+#pragma unroll
+    for (int i = 0; i < KS; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x400, (16 - EXP_1 + KS - 1) / KS, 0);
+      __builtin_amdgcn_sched_group_barrier(0x002, L_FROM_MFMA ? 2 : 5, 0);
+    }
+    asm volatile("" : "+v"(p_out[0]), "+v"(p_out[1]));
   };
 
-  f32x16_t s0, s1;
+  // The next tile of the ring: tile t+1 has landed; every wave has read what it needs of tile t-1 (t == 0: of the Q tile), whose buffer
+  // takes tile t+2.
+  auto next_tile = [&](int t, int b) {
+    sync_all();
+    if (t == 0) init_padding(2);   // (first read in iteration 1, behind its barrier)
+    if (t + 2 < n_tiles) issue_tile(t + 2, b);
+  };
+  if (wave * 32 >= nq) {   // a wave without queries: its share of the loads and the barriers
+    for (int t = 0, b = 2; t < n_tiles; ++t, b = b == 2 ? 0 : b + 1) next_tile(t, b);
+    return;
+  }
+
+  f32x16_t s0, s1;   // scores of both halves of a tile
   bf16x8_t vfa[DT][2], vfb[DT][2];
   i32x4_t p0[2], p1[2];
 #pragma unroll
   for (int t = 0; t < DT; ++t) vfa[t][0] = vfa[t][1] = zero8;
   p1[0] = p1[1] = i32x4_t{0, 0, 0, 0};   // the first step multiplies zeros
-  if (wave_active) {
+  {
     bf16x8_t kfa[KS], kfb[KS];
     read_k(kfa, 0, 0);
     read_k(kfb, 0, 1);
@@ -999,30 +983,49 @@ __global__ __launch_bounds__(256, 2) void attn_full_direct_kernel(const AttnArgs
       mask(s0, seg_len, 0);
       mask(s1, seg_len, 1);
     }
-    m_run = pair_max(fmaxf(row_max(s0), row_max(s1)));
-    mb = __builtin_fmaf(m_run, sl2, shift);
   }
+  float mx_first = row_max(s0);   // maximum of the tile's first half (this lane's keys)
+  // (a query without a score that is a number keeps -inf, as softmax_tile leaves it)
+  float m_run = fmaxf(pair_max(fmaxf(mx_first, row_max(s1))), -INFINITY);
+  mb = m_run * sl2;
   int b0 = 0, b1 = 1, b2 = 2;   // buffers of tiles t, t+1, t+2
   for (int t = 0; t < n_tiles; ++t) {
-    sync_all();   // tile t+1 has landed; every wave has read what it needs of tile t-1 (t == 0: of the Q tile), whose buffer is free
-    if (t == 0) init_padding(2);   // (read two barriers from here at the earliest)
-    if (t + 2 < n_tiles) issue_tile(t + 2, b2);
-    if (wave_active) {
-      const int left = seg_len - t * BKV;
-      step(s0, p0, s1, p1, vfa, b0, 1, vfb, b0, 0);   // scores: second half of t; P.V: second half of t-1; softmax: first half of t
-      if (left < BKV) mask(s1, left, 1);
-      // (behind the last tile, the scores of whatever the next buffer holds are computed and not used)
-      step(s1, p1, s0, p0, vfb, b1, 0, vfa, b0, 1);   // scores: first half of t+1; P.V: first half of t; softmax: second half of t
-      if (left > BKV && left < 2 * BKV) mask(s0, left - BKV, 0);
+    next_tile(t, b2);
+    const int left = seg_len - (t + 1) * BKV;   // keys of the tiles behind this one
+    float psum = 0.f, alpha = 1.0f;
+    // P.V: second half of t-1; softmax: first half of t; scores: first half of t+1
+    // (behind the last tile, the scores of whatever the next buffer holds are computed and not used)
+    step(s0, p0, p1, vfa, vfb, b1, b0, 0, s1, psum, [&](float (&e)[16], float mx_second) {
+#pragma unroll
+      for (int r = 0; r < EXP_1; ++r) asm volatile("" : "+v"(e[r]));
+      const float mx = pair_max(fmaxf(mx_first, mx_second));
+      if (__any((mx - m_run) * sl2 > LAZY_LOG2)) {   // (the whole wave: softmax_tile)
+        const float m_new = fmaxf(m_run, mx);
+        alpha = __builtin_amdgcn_exp2f((m_run - m_new) * sl2);
+#pragma unroll
+        for (int d = 0; d < DT; ++d)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) oacc[d][r] *= alpha;
+        m_run = m_new;
+        mb = m_run * sl2;
+        exponents(e, s0);
+      }
+    });
+    if (left > 0 && left < BKV) mask(s0, left, 0);
+    // P.V: first half of t; softmax: second half of t; scores: second half of t+1
+    step(s1, p1, p0, vfb, vfa, b1, b0, 1, s0, psum, [&](float (&)[16], float mx) { mx_first = mx; });
+    if (left > 0 && left < BKV) mask(s1, left, 1);
+    if constexpr (!L_FROM_MFMA) {
+      psum += __shfl_xor(psum, 32, 64);
+      l_run = __builtin_fmaf(l_run, alpha, psum);
     }
     const int bt = b0;
     b0 = b1;
     b1 = b2;
     b2 = bt;
   }
-  if (wave_active) pv(p1, vfa);
+  pv(p1, vfa);
 
-  if constexpr (!L_FROM_MFMA) l_run += __shfl_xor(l_run, 32, 64);
   const int qi = wave * 32 + fr;
   write_output<D, DT, L_FROM_MFMA>(oacc, l_run, a.out + (int64_t)(q0 + min(qi, nq - 1)) * a.ldo + hoff, qi < nq, hf);
 }

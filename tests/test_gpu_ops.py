@@ -1251,6 +1251,33 @@ def test_attention_short_segment_same_bits_in_either_kernel(ops, dev, d, rotary)
     assert torch.equal(both[:104], short)
 
 
+@pytest.mark.parametrize("d,route", [(64, "plain"), (64, "keys"), (64, "table"), (72, "plain"), (80, "plain"), (80, "keys"), (80, "table"),
+                                     (96, "plain"), (96, "keys"), (96, "table")])
+def test_attention_long_segments_have_the_bits_of_one_tile_after_the_other(ops, dev, d, route):
+    """The long-segment kernels -- the pipeline over half tiles, without rotary and with rotated keys, and the kernel that
+    rotates while it stages -- compute what the 64-row kernel computes when it walks the same segments tile by tile (handed a
+    work list of 64-row query blocks): same reference maxima, same roundings of P, same order of every sum.  Scores wide
+    enough that references rise in later tiles."""
+    nh, lens = 4, [65, 128, 31, 193, 700, 64, 1030]
+    cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    L, H = int(cu[-1]), nh * d
+    for amp in (1.0, 3.0):
+        g = torch.Generator().manual_seed(61)
+        qkv = (torch.randn((L, 3 * H), generator=g) * amp).bfloat16().to(dev)
+        ang = torch.rand((L, d // 2), generator=g) * 6.0
+        cs = None if route == "plain" else torch.cat([ang.cos(), ang.sin()], dim=1).float().contiguous().to(dev)
+        q, k, v = qkv[:, :H], qkv[:, H:2 * H], qkv[:, 2 * H:]
+        items = [(b, e, r, min(64, e - r)) for b, e in zip(cu[:-1].tolist(), cu[1:].tolist()) for r in range(b, e, 64)]
+        blocks = ops.AttnPlan(torch.tensor(items, dtype=torch.int32, device=dev), len(items), 64)
+        want = ops.attn_varlen(q, k, v, blocks, nh, d, d**-0.5, cs)
+        plan = ops.attn_plan(cu, dev)
+        if route == "keys":
+            got = ops.attn_varlen_rotary_(qkv.clone(), plan, nh, d, d**-0.5, cs)
+        else:
+            got = ops.attn_varlen(q, k, v, plan, nh, d, d**-0.5, cs)
+        assert torch.equal(got, want), amp
+
+
 @pytest.mark.parametrize("d,rotary", [(64, False), (64, True), (72, False), (80, False), (80, True), (96, False), (96, True)])
 def test_attention_segment_lengths_around_tiles_and_query_blocks(ops, dev, d, rotary):
     """The long-segment kernels at the edges of half tiles (32 keys), tiles (64) and query blocks (128), in one batch and in
@@ -1280,7 +1307,8 @@ def test_attention_segment_lengths_around_tiles_and_query_blocks(ops, dev, d, ro
 @pytest.mark.parametrize("d", [72, 80, 96])
 def test_attention_query_is_independent_of_its_neighbours(ops, dev, d):
     """Raising the reference maximum of one query (its largest scores sit in the last tile and exceed the first tile's by far
-    more than 2^9) must not touch the bits of the queries that share its wave; infinite and NaN queries stay their own."""
+    more than 2^9) must not touch the bits of any query outside its wave; the 32 queries of a wave raise theirs together, so
+    those that share it stay within the bar of `base`.  Infinite and NaN queries stay their own."""
     nh, L = 2, 300
     H = nh * d
     g = torch.Generator().manual_seed(33)
@@ -1289,14 +1317,16 @@ def test_attention_query_is_independent_of_its_neighbours(ops, dev, d):
     qkv = qkv.bfloat16().to(dev)
     plan = ops.attn_plan(np.array([0, L], np.int32), dev)
     run = lambda x: ops.attn_varlen(x[:, :H], x[:, H:2 * H], x[:, 2 * H:], plan, nh, d, d**-0.5)   # noqa: E731
-    base = run(qkv)
-    close(base, attn_ref(qkv, [0, L], nh, d), 2**-6, f"raised late d={d}")
+    base, ref = run(qkv), attn_ref(qkv, [0, L], nh, d)
+    close(base, ref, 2**-6, f"raised late d={d}")
+    wave = torch.arange(L) // 32 == 37 // 32
+    shares = wave & (torch.arange(L) != 37)
     for value in (40.0, float("inf"), float("nan")):
         x = qkv.clone()
         x[37, :H] = x[37, :H] * value
-        out = run(x)
-        keep = torch.arange(L, device=dev) != 37
-        assert torch.equal(out[keep], base[keep]), value
+        out = run(x).cpu()
+        assert torch.equal(out[~wave], base.cpu()[~wave]), value
+        close(out[shares], ref[shares], 2**-6, f"d={d}, beside a query times {value}")
         assert bool(torch.isfinite(out[37].float()).all()) == (value == 40.0)
 
 
