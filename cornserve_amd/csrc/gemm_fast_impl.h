@@ -297,15 +297,18 @@ __global__ __launch_bounds__(64 * NW) void gemm_fast_kernel(const CsGemmArgs p) 
   };
   const __amdgpu_buffer_rsrc_t rsrc_a = __builtin_amdgcn_make_buffer_rsrc((void*)p.A, 0, -1, 0x00020000);
   const __amdgpu_buffer_rsrc_t rsrc_w = __builtin_amdgcn_make_buffer_rsrc((void*)p.W, 0, -1, 0x00020000);
-  // Descriptors of what the epilogue's fast form reads and writes, each as long as its matrix: what a lane past the last row would
-  // load is zero and what it would store is dropped, so row tails need no guards (a row past the last one starts at or behind
-  // the end whatever its column).  A lane past the last column of its row takes an offset behind every end instead (OUTSIDE).
+  // Descriptors of what the epilogue's fast form reads and writes, each ending with its matrix's last element, so that row tails need
+  // no guards: a row of C past the last one starts at or behind the end whatever its column (p.fast_epilogue: ldc is at least
+  // the width), and what a lane would store there is dropped; residual rows past the last one read zeros, or -- where rows share
+  // memory, down to one row for all (ldr = 0) -- elements that nobody uses.  A lane past the last column of its row takes an
+  // offset behind every end instead (OUTSIDE) to store, and reads the next row's elements or zeros.
   constexpr uint32_t OUTSIDE = 0xFFFF0000u;   // (with room for an immediate; p.fast_epilogue: every matrix ends below it)
   auto rsrc_of = [&](const void* base, int64_t bytes) { return __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, (int)(uint32_t)bytes, 0x00020000); };
-  const __amdgpu_buffer_rsrc_t rsrc_c = rsrc_of(p.C, (int64_t)p.M * p.ldc * 2);
-  const __amdgpu_buffer_rsrc_t rsrc_clo = rsrc_of(p.c_lo, (int64_t)p.M * p.ldc);
-  const __amdgpu_buffer_rsrc_t rsrc_res = rsrc_of(p.residual, (int64_t)p.M * p.ldr * 2);
-  const __amdgpu_buffer_rsrc_t rsrc_reslo = rsrc_of(p.residual_lo, (int64_t)p.M * p.ldr);
+  const int64_t c_len = (int64_t)(p.M - 1) * p.ldc + (EPI == CS_EPI_SWIGLU ? p.N / 2 : p.N), res_len = (int64_t)(p.M - 1) * p.ldr + p.N;
+  const __amdgpu_buffer_rsrc_t rsrc_c = rsrc_of(p.C, c_len * 2);
+  const __amdgpu_buffer_rsrc_t rsrc_clo = rsrc_of(p.c_lo, c_len);
+  const __amdgpu_buffer_rsrc_t rsrc_res = rsrc_of(p.residual, res_len * 2);
+  const __amdgpu_buffer_rsrc_t rsrc_reslo = rsrc_of(p.residual_lo, res_len);
   const __amdgpu_buffer_rsrc_t rsrc_scale = rsrc_of(p.w_scale, (int64_t)p.N * 4);
   const __amdgpu_buffer_rsrc_t rsrc_bias = rsrc_of(p.bias, (int64_t)p.N * 2);
   const __amdgpu_buffer_rsrc_t rsrc_asumsq = rsrc_of(p.a_row_sumsq, (int64_t)p.M * (CS_SUMSQ_PARTS * 4));
@@ -1394,9 +1397,12 @@ int launch(const CsGemmArgs& a, hipStream_t stream) {
   p.tiles_m = (p.M + BM - 1) / BM;
   p.tiles_n = (p.N + BN - 1) / BN;
   // The epilogue's fast form addresses C, the residual and their byte planes with 32-bit byte offsets from the
-  // matrix bases, and takes output row m for accumulator row m.
+  // matrix bases, and takes output row m for accumulator row m.  (Output rows that share memory -- one row may have any ldc --
+  // take the general form, whose guards do not need a row to end before the next begins.)
   const int64_t lim = 0xFFFF0000ll, rows = (int64_t)p.tiles_m * BM;   // (rows past the last one have offsets too)
-  p.fast_epilogue = !p.c_rows && !((uintptr_t)p.w_scale & 15) && (rows + 1) * p.ldc * 2 < lim && (!p.residual || (rows + 1) * p.ldr * 2 < lim);
+  const int64_t width = EPI == CS_EPI_SWIGLU ? p.N / 2 : p.N;
+  p.fast_epilogue = !p.c_rows && !((uintptr_t)p.w_scale & 15) && p.ldc >= width && (rows + 1) * p.ldc * 2 < lim &&
+                    (!p.residual || (p.ldr >= 0 && (rows + 1) * p.ldr * 2 < lim));
   constexpr int lds = RingShape<BM, BN, W_FP8>::BYTES +
                       (residual_piece_through_ring<BM, BN, WAVES_M, WAVES_N, EPI, W_FP8, FUSE, SPLIT_RES>() ? NW * 1024 : 0);
   static bool attr_set = false;

@@ -556,6 +556,80 @@ def test_every_big_tile_form_gives_the_same_bits(ops, dev, M, N, K, fp8):
             close(want[0][:M, :N][:64], lin_ref(a[:64], w, b), 2**-7, f"{M}x{N}x{K}")
 
 
+def _big_form(name):
+    """The launcher of one big tile form, for calls that must not depend on the choice of forms."""
+    import ctypes
+
+    from cornserve_amd import lib
+
+    base = f"cs_gemm_fast_tile_{name}"
+    run = getattr(ctypes.CDLL(str(lib.LIB_PATH)), f"_Z{len(base)}{base}RK10CsGemmArgsP12ihipStream_t")
+    run.argtypes, run.restype = [ctypes.POINTER(lib.CsGemmArgs), ctypes.c_void_p], ctypes.c_int
+    return run
+
+
+# A residual whose rows share memory (one row broadcast; rows that overlap) is the residual that a copy of it would be, in every
+# kernel and form: ring-fed and direct epilogues, whole tiles and both edges, the few-row kernel (K a multiple of 128, 200 rows)
+# and the general one (K = 80).
+@pytest.mark.parametrize("M,N,K", [(200, 1280, 1280), (512, 640, 192), (1345, 1288, 192), (6145, 1152, 256), (300, 264, 80)])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_gemm_residual_rows_that_share_memory(ops, dev, M, N, K, fp8):
+    import ctypes
+
+    from cornserve_amd import lib
+
+    a, w, b = rnd((M, K), 1.0, 211, dev), rnd((N, K), 0.05, 212, dev), rnd((N,), 0.02, 213, dev)
+    sc = (w.float().abs().amax(1) / 448.0).contiguous() if fp8 else None
+    wq = (w.float() / sc[:, None]).to(torch.float8_e4m3fn) if fp8 else w
+    buf = rnd(((M - 1) * N + N,), 4.0, 214, dev)
+    buf_lo = torch.randint(0, 256, buf.shape, generator=torch.Generator().manual_seed(215), dtype=torch.uint8).to(dev)
+    base = lin_ref(a[-3:], wq.float() * sc[:, None] if fp8 else w, b)
+    for ld in (0, 8, N - 8):
+        res, lo = buf.as_strided((M, N), (ld, 1)), buf_lo.as_strided((M, N), (ld, 1))
+        for split in ((False, True) if K % 64 == 0 else (False,)):
+            got = []
+            for r, l in ((res, lo), (res.contiguous(), lo.contiguous())):
+                kw = {"residual_lo": l, "out": torch.full((M, N), 3.0, dtype=torch.bfloat16, device=dev),
+                      "out_lo": torch.zeros((M, N), dtype=torch.uint8, device=dev)} if split else {}
+                out = ops.gemm(a, wq, b, w_scale=sc, epilogue=ops.EPI_RESIDUAL, residual=r, **kw)
+                got.append((out, kw.get("out_lo")))
+            assert torch.equal(got[0][0], got[1][0]), (ld, split)
+            assert not split or torch.equal(got[0][1], got[1][1]), ld
+            if not split:   # against fp32: the last rows and columns
+                close(got[0][0][-3:], _epilogue_ref(ops, ops.EPI_RESIDUAL, base, res[-3:]), 2**-7, f"ldr {ld}")
+            for name in BIG_FORMS if K >= 192 else ():
+                g = lib.CsGemmArgs()
+                out, out_lo = torch.full((M, N), 3.0, dtype=torch.bfloat16, device=dev), torch.zeros((M, N), dtype=torch.uint8, device=dev)
+                g.A, g.W, g.C, g.M, g.N, g.K, g.lda, g.ldw, g.ldc = a.data_ptr(), wq.data_ptr(), out.data_ptr(), M, N, K, K, K, N
+                g.bias, g.epilogue, g.residual, g.ldr = b.data_ptr(), ops.EPI_RESIDUAL, res.data_ptr(), ld
+                if fp8:
+                    g.w_fp8, g.w_scale = 1, sc.data_ptr()
+                if split:
+                    g.c_lo, g.residual_lo = out_lo.data_ptr(), lo.data_ptr()
+                assert _big_form(name)(ctypes.byref(g), torch.cuda.current_stream().cuda_stream) == 0, name
+                assert torch.equal(out, got[1][0]), (name, ld, split)
+                assert not split or torch.equal(out_lo, got[1][1]), (name, ld)
+
+
+@pytest.mark.parametrize("epi", ["EPI_BIAS", "EPI_SWIGLU", "EPI_RESIDUAL"])
+def test_gemm_single_row_with_any_output_pitch(ops, dev, epi):
+    """The pitch of a one-row output says nothing (torch leaves any number there); 8 is less than the row."""
+    import ctypes
+
+    from cornserve_amd import lib
+
+    N, K, epi = 200, 192, getattr(ops, epi)
+    a, w, b, res = rnd((1, K), 1.0, 221, dev), rnd((N, K), 0.05, 222, dev), rnd((N,), 0.02, 223, dev), rnd((1, N), 1.0, 224, dev)
+    want = ops.gemm(a, w, b, epilogue=epi, residual=res if epi == ops.EPI_RESIDUAL else None)
+    for name in BIG_FORMS:
+        g = lib.CsGemmArgs()
+        out = torch.full((2, N), 3.0, dtype=torch.bfloat16, device=dev)
+        g.A, g.W, g.C, g.M, g.N, g.K, g.lda, g.ldw, g.ldc = a.data_ptr(), w.data_ptr(), out.data_ptr(), 1, N, K, K, K, 8
+        g.bias, g.epilogue, g.residual, g.ldr = b.data_ptr(), epi, res.data_ptr(), 8
+        assert _big_form(name)(ctypes.byref(g), torch.cuda.current_stream().cuda_stream) == 0, name
+        assert torch.equal(out[0, : want.shape[1]], want[0]) and bool((out[0, want.shape[1]:] == 3).all()) and bool((out[1] == 3).all()), name
+
+
 # The few-row kernel (K a multiple of 128) at shapes of the encoders: an output has the bits it has as a row of a product with
 # many rows, with the norms folded inline or from arrays, and the row sums of its output are the big tiles'.  (Inline norms
 # always run here; of the rest, (1, 64, 256) compares the few-row kernel with itself and (2700, 1280, 1280) the big tiles.
