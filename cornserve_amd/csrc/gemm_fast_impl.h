@@ -165,7 +165,17 @@ constexpr bool residual_piece_through_ring() {
   return SPLIT_RES && EPI == CS_EPI_RESIDUAL && NT % 2 == 0 && !RingShape<BM, BN, W_FP8>::FIVE_UNITS &&
          (WAVES_N == 1 || FUSE == 0) && MT >= 2 && MT <= 4 && FUSE != FUSE_NORM_A && FUSE != FUSE_LN_A;
 }
+// ... in tiles at an edge of the matrix too (but for the form whose scales leave no registers for the offsets that takes).
 template <int BM, int BN, int WAVES_M, int WAVES_N, int EPI, bool W_FP8, int FUSE, bool SPLIT_RES>
+constexpr bool ring_takes_edges() {
+  return residual_piece_through_ring<BM, BN, WAVES_M, WAVES_N, EPI, W_FP8, FUSE, SPLIT_RES>() &&
+         !(W_FP8 && (BM / WAVES_M / 16) * (BN / WAVES_N / 16) >= 40);
+}
+// EDGES: some tile may reach past the last row or column.  Only those products have an instance without: the edge offsets of the
+// piece, in the tail of the K loop, cost every tile, edge or not; elsewhere an edge is one uniform branch a tile.  With -> without,
+// 128x160 tiles: 2048 x 1280 x 1280 16.7 -> 16.4 us, fp8 weights 21.6 -> 20.9, 4096 x 1280 x 1280 with row sums 21.0 -> 19.8; 256x160:
+// 8192 x 1280 x 3456 62.4 -> 61.3.
+template <int BM, int BN, int WAVES_M, int WAVES_N, int EPI, bool W_FP8, int FUSE, bool SPLIT_RES, bool EDGES>
 __global__ __launch_bounds__(64 * NW) void gemm_fast_kernel(const CsGemmArgs p) {
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   static_assert(WAVES_M * WAVES_N == NW, "four waves, one per SIMD");
@@ -479,10 +489,9 @@ __global__ __launch_bounds__(64 * NW) void gemm_fast_kernel(const CsGemmArgs p) 
     // fp8 weights: the columns' scales, in row block 0's slot behind everything that passes through it
     constexpr int SCALE_OFF = MT <= 3 ? ROW_BYTES : ROW_BYTES + ROW_LO_BYTES;
     static_assert(!PRE || !W_FP8 || (SCALE_OFF + NW * 1024 <= STAGE && BN * 4 <= 1024), "the scales fit row block 0's slot");
-    const bool m_edge = m0 + BM > p.M, n_edge = n0 + BN > p.N;
-    // (a 16-byte chunk of the byte plane that straddles the last column is left to the other form; so are the edge tiles of the
-    // form whose scales leave no registers for them)
-    constexpr bool PRE_EDGE = PRE && !(W_FP8 && MT * NT >= 40);
+    const bool m_edge = EDGES && m0 + BM > p.M, n_edge = EDGES && n0 + BN > p.N;
+    // (a 16-byte chunk of the byte plane that straddles the last column is left to the other form)
+    constexpr bool PRE_EDGE = EDGES && ring_takes_edges<BM, BN, WAVES_M, WAVES_N, EPI, W_FP8, FUSE, SPLIT_RES>();
     const bool pre_on = PRE && p.fast_epilogue && !has_next && !(n_edge && p.N % 16) && (PRE_EDGE || !(m_edge || n_edge));
     // lane-only byte offsets of the direct loads (the tile and the row block go into the scalar offset)
     uint32_t pre_hi_v = 0, pre_lo_v[PRE ? LO_LD : 1] = {}, pre_bias_v = 0, pre_scale_v = 0;
@@ -1391,22 +1400,12 @@ __global__ __launch_bounds__(64 * NW) void gemm_fast_kernel(const CsGemmArgs p) 
   }
 }
 
-template <int BM, int BN, int WAVES_M, int WAVES_N, int EPI, bool W_FP8, int FUSE = 0, bool SPLIT_RES = false>
-int launch(const CsGemmArgs& a, hipStream_t stream) {
-  CsGemmArgs p = a;
-  p.tiles_m = (p.M + BM - 1) / BM;
-  p.tiles_n = (p.N + BN - 1) / BN;
-  // The epilogue's fast form addresses C, the residual and their byte planes with 32-bit byte offsets from the
-  // matrix bases, and takes output row m for accumulator row m.  (Output rows that share memory -- one row may have any ldc --
-  // take the general form, whose guards do not need a row to end before the next begins.)
-  const int64_t lim = 0xFFFF0000ll, rows = (int64_t)p.tiles_m * BM;   // (rows past the last one have offsets too)
-  const int64_t width = EPI == CS_EPI_SWIGLU ? p.N / 2 : p.N;
-  p.fast_epilogue = !p.c_rows && !((uintptr_t)p.w_scale & 15) && p.ldc >= width && (rows + 1) * p.ldc * 2 < lim &&
-                    (!p.residual || (p.ldr >= 0 && (rows + 1) * p.ldr * 2 < lim));
+template <int BM, int BN, int WAVES_M, int WAVES_N, int EPI, bool W_FP8, int FUSE, bool SPLIT_RES, bool EDGES>
+int launch_kernel(CsGemmArgs& p, hipStream_t stream) {
   constexpr int lds = RingShape<BM, BN, W_FP8>::BYTES +
                       (residual_piece_through_ring<BM, BN, WAVES_M, WAVES_N, EPI, W_FP8, FUSE, SPLIT_RES>() ? NW * 1024 : 0);
   static bool attr_set = false;
-  auto kern = gemm_fast_kernel<BM, BN, WAVES_M, WAVES_N, EPI, W_FP8, FUSE, SPLIT_RES>;
+  auto kern = gemm_fast_kernel<BM, BN, WAVES_M, WAVES_N, EPI, W_FP8, FUSE, SPLIT_RES, EDGES>;
   if (!attr_set) {
     if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
       return CS_ERR_LAUNCH;
@@ -1420,6 +1419,24 @@ int launch(const CsGemmArgs& a, hipStream_t stream) {
   else p.prefetch = nullptr;
   hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * NW), lds, stream, p);
   return cs_launch_status();
+}
+
+template <int BM, int BN, int WAVES_M, int WAVES_N, int EPI, bool W_FP8, int FUSE = 0, bool SPLIT_RES = false>
+int launch(const CsGemmArgs& a, hipStream_t stream) {
+  CsGemmArgs p = a;
+  p.tiles_m = (p.M + BM - 1) / BM;
+  p.tiles_n = (p.N + BN - 1) / BN;
+  // The epilogue's fast form addresses C, the residual and their byte planes with 32-bit byte offsets from the
+  // matrix bases, and takes output row m for accumulator row m.  (Output rows that share memory -- one row may have any ldc --
+  // take the general form, whose guards do not need a row to end before the next begins.)
+  const int64_t lim = 0xFFFF0000ll, rows = (int64_t)p.tiles_m * BM;   // (rows past the last one have offsets too)
+  const int64_t width = EPI == CS_EPI_SWIGLU ? p.N / 2 : p.N;
+  p.fast_epilogue = !p.c_rows && !((uintptr_t)p.w_scale & 15) && p.ldc >= width && (rows + 1) * p.ldc * 2 < lim &&
+                    (!p.residual || (p.ldr >= 0 && (rows + 1) * p.ldr * 2 < lim));
+  if constexpr (ring_takes_edges<BM, BN, WAVES_M, WAVES_N, EPI, W_FP8, FUSE, SPLIT_RES>()) {
+    if (p.M % BM == 0 && p.N % BN == 0) return launch_kernel<BM, BN, WAVES_M, WAVES_N, EPI, W_FP8, FUSE, SPLIT_RES, false>(p, stream);
+  }
+  return launch_kernel<BM, BN, WAVES_M, WAVES_N, EPI, W_FP8, FUSE, SPLIT_RES, true>(p, stream);
 }
 
 template <int BM, int BN, int WAVES_M, int WAVES_N, bool W_FP8>

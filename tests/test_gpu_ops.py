@@ -481,8 +481,9 @@ BIG_FORMS = ("256x256", "256x160", "256x128", "224x192", "192x192", "192x160", "
 
 # Every big tile form, called by itself, on the same products: which form a launch takes must change no bit.  Whole tiles of no
 # form, of some and of most; one tile, one round and several tiles a workgroup; 3, 4, 6 and 18 K tiles; row tails of 1 row and of
-# one less than a tile; column tails of 8, 32 and 96 columns.
-@pytest.mark.parametrize("M,N,K", [(1, 200, 192), (447, 1152, 256), (449, 1288, 192), (1344, 960, 384), (5103, 1152, 1152), (6145, 1280, 192),
+# one less than a tile; column tails of 8, 32 and 96 columns; whole tiles of every ring-fed form, one and several a workgroup (768
+# and 12288 x 960).
+@pytest.mark.parametrize("M,N,K", [(768, 960, 192), (12288, 960, 192), (1, 200, 192), (447, 1152, 256), (449, 1288, 192), (1344, 960, 384), (5103, 1152, 1152), (6145, 1280, 192),
                                    (16500, 320, 192)])
 @pytest.mark.parametrize("fp8", [False, True])
 def test_every_big_tile_form_gives_the_same_bits(ops, dev, M, N, K, fp8):
