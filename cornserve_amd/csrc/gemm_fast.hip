@@ -1,5 +1,6 @@
 // Fast-path bf16 MFMA GEMM for gfx950: choice of the tile form.  The kernel itself is in gemm_fast_impl.h; each tile
 // form is built in its own translation unit (gemm_fast_t*.hip).
+#include <math.h>
 #include <stdlib.h>
 
 #include "gemm_common.h"
@@ -41,15 +42,16 @@ struct BigForm {
   int (*run)(const CsGemmArgs&, hipStream_t);
 };
 constexpr float LAUNCH_US = 3.0f;
+constexpr float NONE = INFINITY;   // not built: no launch may be costed with it (takes() below)
 const BigForm FORMS[] = {
-    {256, 256, {5.7f, 6.1f, 11.8f, 0.f, 18.9f, 21.3f, 0.99f, 0.38f}, {6.5f, 6.0f, 28.8f, 0.f, 20.2f, 18.9f, 1.08f, 0.29f}, cs_gemm_fast_tile_256x256},
-    {256, 160, {4.2f, 4.4f, 8.4f, 6.5f, 12.1f, 12.9f, 0.61f, 0.30f}, {5.0f, 4.6f, 18.2f, 0.f, 11.9f, 12.3f, 0.85f, 0.19f}, cs_gemm_fast_tile_256x160},
-    {256, 128, {2.9f, 3.6f, 6.3f, 5.4f, 9.1f, 8.6f, 0.55f, 0.25f}, {3.7f, 3.3f, 14.4f, 0.f, 10.5f, 8.9f, 0.59f, 0.20f}, cs_gemm_fast_tile_256x128},
-    {224, 192, {4.4f, 4.7f, 8.6f, 7.0f, 14.5f, 13.9f, 0.67f, 0.28f}, {4.7f, 4.4f, 18.7f, 0.f, 17.4f, 13.5f, 0.75f, 0.22f}, cs_gemm_fast_tile_224x192},
-    {192, 192, {3.7f, 4.2f, 7.5f, 6.1f, 11.1f, 10.1f, 0.62f, 0.23f}, {4.1f, 3.8f, 15.0f, 0.f, 14.1f, 10.0f, 0.68f, 0.19f}, cs_gemm_fast_tile_192x192},
-    {192, 160, {3.1f, 3.5f, 6.5f, 4.9f, 9.1f, 9.7f, 0.52f, 0.22f}, {3.6f, 3.0f, 11.2f, 0.f, 9.3f, 9.4f, 0.73f, 0.14f}, cs_gemm_fast_tile_192x160},
-    {128, 192, {1.5f, 2.3f, 4.3f, 3.1f, 6.7f, 5.7f, 0.48f, 0.19f}, {3.1f, 2.8f, 9.1f, 0.f, 9.9f, 6.5f, 0.56f, 0.12f}, cs_gemm_fast_tile_128x192},
-    {128, 160, {1.3f, 2.0f, 3.9f, 2.7f, 6.1f, 5.9f, 0.41f, 0.20f}, {0.f, 0.f, 0.f, 0.f, 7.3f, 7.2f, 0.57f, 0.09f}, cs_gemm_fast_tile_128x160},
+    {256, 256, {5.7f, 6.1f, 11.8f, NONE, 18.9f, 21.3f, 0.99f, 0.38f}, {6.5f, 6.0f, 28.8f, NONE, 20.2f, 18.9f, 1.08f, 0.29f}, cs_gemm_fast_tile_256x256},
+    {256, 160, {4.2f, 4.4f, 8.4f, 6.5f, 12.1f, 12.9f, 0.61f, 0.30f}, {5.0f, 4.6f, 18.2f, NONE, 11.9f, 12.3f, 0.85f, 0.19f}, cs_gemm_fast_tile_256x160},
+    {256, 128, {2.9f, 3.6f, 6.3f, 5.4f, 9.1f, 8.6f, 0.55f, 0.25f}, {3.7f, 3.3f, 14.4f, NONE, 10.5f, 8.9f, 0.59f, 0.20f}, cs_gemm_fast_tile_256x128},
+    {224, 192, {4.4f, 4.7f, 8.6f, 7.0f, 14.5f, 13.9f, 0.67f, 0.28f}, {4.7f, 4.4f, 18.7f, NONE, 17.4f, 13.5f, 0.75f, 0.22f}, cs_gemm_fast_tile_224x192},
+    {192, 192, {3.7f, 4.2f, 7.5f, 6.1f, 11.1f, 10.1f, 0.62f, 0.23f}, {4.1f, 3.8f, 15.0f, NONE, 14.1f, 10.0f, 0.68f, 0.19f}, cs_gemm_fast_tile_192x192},
+    {192, 160, {3.1f, 3.5f, 6.5f, 4.9f, 9.1f, 9.7f, 0.52f, 0.22f}, {3.6f, 3.0f, 11.2f, NONE, 9.3f, 9.4f, 0.73f, 0.14f}, cs_gemm_fast_tile_192x160},
+    {128, 192, {1.5f, 2.3f, 4.3f, 3.1f, 6.7f, 5.7f, 0.48f, 0.19f}, {3.1f, 2.8f, 9.1f, NONE, 9.9f, 6.5f, 0.56f, 0.12f}, cs_gemm_fast_tile_128x192},
+    {128, 160, {1.3f, 2.0f, 3.9f, 2.7f, 6.1f, 5.9f, 0.41f, 0.20f}, {NONE, NONE, NONE, NONE, 7.3f, 7.2f, 0.57f, 0.09f}, cs_gemm_fast_tile_128x160},
 };
 
 int64_t tiles_of(const BigForm& f, int M, int N) { return (int64_t)(((uint32_t)M + f.bm - 1) / (uint32_t)f.bm) * (((uint32_t)N + f.bn - 1) / (uint32_t)f.bn); }
@@ -160,16 +162,23 @@ int cs_gemm_fast(const CsGemmArgs& a, hipStream_t stream, bool* handled) {
 }
 
 // For the few-row kernel's choice: the time of a launch as a share of what the best of 256x256, 256x128 (SwiGLU), and 256x160 or, for at
-// most 128 tiles of it, 128x160 would take; and the tiles of its (last) launch.
+// most 128 tiles of it, 128x160 would take, of those that take the launch; and the tiles of its (last) launch.  1 where 128x160 is the
+// one to compare with and is not built (fp8 weights, but for residual products): compared with 256x160 instead, GELU products of
+// 256 and 352 fp8 rows x 4352 x 1152 went to the big tiles, 17.7 us where few-row tiles take 10.7.
 double cs_gemm_fast_saves(const CsGemmArgs& a, int64_t* tiles) {
   const Plan p = plan_of(a);
   *tiles = tiles_of(*p.form, a.M, a.N - p.lead_cols);
+  const int narrow_rows = (int64_t)((a.M + 255) / 256) * ((a.N + 159) / 160) <= 128 ? 128 : 256;
   double of = 0;
   for (const BigForm& f : FORMS) {
-    const bool narrow = f.bn == 160 && f.bm == ((int64_t)((a.M + 255) / 256) * ((a.N + 159) / 160) <= 128 ? 128 : 256);
-    const bool one = narrow || (!a.c_row_sumsq && f.bm == 256 && (f.bn == 256 || (f.bn == 128 && a.epilogue == CS_EPI_SWIGLU)));
+    const bool narrow = f.bn == 160 && f.bm == narrow_rows;
+    if (!takes(f, a)) {
+      if (narrow) return 1.0;
+      continue;
+    }
+    if (!narrow && !(f.bm == 256 && (f.bn == 256 || (f.bn == 128 && a.epilogue == CS_EPI_SWIGLU)))) continue;
     const double t = form_us(f, a, a.N);
-    if (one && (of == 0 || t < of)) of = t;
+    if (of == 0 || t < of) of = t;
   }
   return p.us < of ? p.us / of : 1.0;
 }
