@@ -129,6 +129,17 @@ extern "C" int cs_gemm_few_row_workgroups(const CsGemmArgs* args) {
   return args && !args->conv_patch && direct_shape(*args) ? cs_gemm_small_workgroups(*args) : 0;
 }
 
+extern "C" int cs_gemm_big_form(const CsGemmArgs* args, int32_t plan[3]) {
+  if (!args || !plan) return CS_ERR_INVALID_ARG;
+  plan[0] = plan[1] = plan[2] = 0;
+  if (args->conv_patch || args->a_norm_inline || !direct_shape(*args) || cs_gemm_small_workgroups(*args)) return CS_OK;
+  const Plan p = plan_of(*args);
+  plan[0] = p.form->bm;
+  plan[1] = p.form->bn;
+  plan[2] = p.lead_cols;
+  return CS_OK;
+}
+
 // Called by cs_gemm after argument validation.  Sets *handled when this path took the problem.
 int cs_gemm_fast(const CsGemmArgs& a, hipStream_t stream, bool* handled) {
   *handled = false;

@@ -159,6 +159,11 @@ int cs_gemm(const CsGemmArgs* args, void* stream);
  * that read the prefetch hint), 0 if another kernel does.  Nothing is read through the pointers.                        */
 int cs_gemm_few_row_workgroups(const CsGemmArgs* args);
 
+/* Host routine: the big tile form that cs_gemm takes for these arguments, into plan[0] x plan[1] (rows x columns of a tile); of
+ * two launches that split the columns it is the second's, and plan[2] counts the leading columns that the first, of 256x256
+ * tiles, covers (0: one launch).  Zeros if another kernel takes them.  Nothing is read through the pointers.             */
+int cs_gemm_big_form(const CsGemmArgs* args, int32_t plan[3]);
+
 /* Host routine: 1 if a folded-norm launch of M rows, N weight rows and width K is faster with a_norm_inline than with row
  * sums read from arrays (few rows), 0 if not or if the shape has no inline form.  window_attn = 1: the same question for
  * cs_qkv_window_attn with M = 64 * windows and N = 256 * heads.                                                      */
