@@ -27,12 +27,13 @@ using csgemm::BK;
 // alone, SwiGLU, another activation, a folded LayerNorm; residual products: the workgroup's last tile, whose residual piece came
 // through the ring, and the tiles before it.  Fitted to 27 products of the encoders at up to 34 row counts from 1100 to 20000, every
 // form that takes them, weights from HBM (about 3,700 launches; root mean square error 2 to 3 % with fp8 weights, 8 to 10 % with
-// bf16 ones, most of it common to all forms of a product).  A launch is as long as its rounds, and a round as long as a tile of
-// its form however few of the 256 compute units have one, so what counts is a form whose tiles fill whole rounds: 6240 rows x 3456
-// (folded LayerNorm) are 550 tiles of 256x160 in three rounds, 58.6 us, and 504 of 224x192 in two, 45.2 us.  Chosen by this table,
-// launches take 1.010 of the time of the best form on average (residual products from 2500 rows on, the others from 1000); with
-// five forms (256x256, 256x160 and its 128-row half, 256x128 and 128x192 behind whole rounds of 256x256) and tile area as the
-// cost they took 1.062.
+// bf16 ones, most of it common to all forms of a product), before edge tiles of residual products took the fast epilogue (0 to 7 us
+// less than their entries say, in every form).  A launch is as long as its rounds, and a round as long as a tile of its form however
+// few of the 256 compute units have one, so what counts is a form whose tiles fill whole rounds: 6240 rows x 3456 (folded
+// LayerNorm) are 550 tiles of 256x160 in three rounds, 62.8 us, and 504 of 224x192 in two, 49.2 us.  Chosen by this table, launches
+// take 1.009 of the time of the best form on average (33 products at 24 to 34 row counts on the present kernels; residual
+// products from 2500 rows on, the others from 1000; the worst 1.10); with five forms (256x256, 256x160 and its 128-row half, 256x128
+// and 128x192 behind whole rounds of 256x256) and tile area as the cost they took 1.062.
 struct FormUs {
   float bias, swiglu, act, ln, res, res_more, stage, flow;
 };
@@ -44,13 +45,13 @@ struct BigForm {
 constexpr float LAUNCH_US = 3.0f;
 constexpr float NONE = INFINITY;   // not built: no launch may be costed with it (takes() below)
 const BigForm FORMS[] = {
-    {256, 256, {5.7f, 6.1f, 11.8f, NONE, 18.9f, 21.3f, 0.99f, 0.38f}, {6.5f, 6.0f, 28.8f, NONE, 20.2f, 18.9f, 1.08f, 0.29f}, cs_gemm_fast_tile_256x256},
-    {256, 160, {4.2f, 4.4f, 8.4f, 6.5f, 12.1f, 12.9f, 0.61f, 0.30f}, {5.0f, 4.6f, 18.2f, NONE, 11.9f, 12.3f, 0.85f, 0.19f}, cs_gemm_fast_tile_256x160},
-    {256, 128, {2.9f, 3.6f, 6.3f, 5.4f, 9.1f, 8.6f, 0.55f, 0.25f}, {3.7f, 3.3f, 14.4f, NONE, 10.5f, 8.9f, 0.59f, 0.20f}, cs_gemm_fast_tile_256x128},
-    {224, 192, {4.4f, 4.7f, 8.6f, 7.0f, 14.5f, 13.9f, 0.67f, 0.28f}, {4.7f, 4.4f, 18.7f, NONE, 17.4f, 13.5f, 0.75f, 0.22f}, cs_gemm_fast_tile_224x192},
-    {192, 192, {3.7f, 4.2f, 7.5f, 6.1f, 11.1f, 10.1f, 0.62f, 0.23f}, {4.1f, 3.8f, 15.0f, NONE, 14.1f, 10.0f, 0.68f, 0.19f}, cs_gemm_fast_tile_192x192},
-    {192, 160, {3.1f, 3.5f, 6.5f, 4.9f, 9.1f, 9.7f, 0.52f, 0.22f}, {3.6f, 3.0f, 11.2f, NONE, 9.3f, 9.4f, 0.73f, 0.14f}, cs_gemm_fast_tile_192x160},
-    {128, 192, {1.5f, 2.3f, 4.3f, 3.1f, 6.7f, 5.7f, 0.48f, 0.19f}, {3.1f, 2.8f, 9.1f, NONE, 9.9f, 6.5f, 0.56f, 0.12f}, cs_gemm_fast_tile_128x192},
+    {256, 256, {5.7f, 6.1f, 11.8f, NONE, 18.9f, 21.3f, 0.99f, 0.38f}, {6.5f, 6.0f, 8.6f, NONE, 20.2f, 18.9f, 1.08f, 0.29f}, cs_gemm_fast_tile_256x256},
+    {256, 160, {4.2f, 4.4f, 8.4f, 6.5f, 12.1f, 12.9f, 0.61f, 0.30f}, {5.0f, 4.6f, 6.4f, NONE, 11.9f, 12.3f, 0.85f, 0.19f}, cs_gemm_fast_tile_256x160},
+    {256, 128, {2.9f, 3.6f, 6.3f, 5.4f, 9.1f, 8.6f, 0.55f, 0.25f}, {3.7f, 3.3f, 4.7f, NONE, 10.5f, 8.9f, 0.59f, 0.20f}, cs_gemm_fast_tile_256x128},
+    {224, 192, {4.4f, 4.7f, 8.6f, 7.0f, 14.5f, 13.9f, 0.67f, 0.28f}, {4.7f, 4.4f, 6.2f, NONE, 17.4f, 13.5f, 0.75f, 0.22f}, cs_gemm_fast_tile_224x192},
+    {192, 192, {3.7f, 4.2f, 7.5f, 6.1f, 11.1f, 10.1f, 0.62f, 0.23f}, {4.1f, 3.8f, 5.0f, NONE, 14.1f, 10.0f, 0.68f, 0.19f}, cs_gemm_fast_tile_192x192},
+    {192, 160, {3.1f, 3.5f, 6.5f, 4.9f, 9.1f, 9.7f, 0.52f, 0.22f}, {3.6f, 3.0f, 4.5f, NONE, 9.3f, 9.4f, 0.73f, 0.14f}, cs_gemm_fast_tile_192x160},
+    {128, 192, {1.5f, 2.3f, 4.3f, 3.1f, 6.7f, 5.7f, 0.48f, 0.19f}, {3.1f, 2.8f, 3.7f, NONE, 9.9f, 6.5f, 0.56f, 0.12f}, cs_gemm_fast_tile_128x192},
     {128, 160, {1.3f, 2.0f, 3.9f, 2.7f, 6.1f, 5.9f, 0.41f, 0.20f}, {NONE, NONE, NONE, NONE, 7.3f, 7.2f, 0.57f, 0.09f}, cs_gemm_fast_tile_128x160},
 };
 

@@ -181,6 +181,22 @@ def test_few_row_kernel_takes_launches_of_at_most_two_rounds():
     assert groups(96, 1280, 1216) == groups(8192, 1280, 1280) == 0                   # K % 128; many rows
 
 
+def test_fp8_activation_products_take_the_forms_that_are_fast_with_them():
+    """GELU products with fp8 weights, whose times are their own column of the table of forms: 1458 rows x 4352 x 1152 21.4 us in
+    256x128 tiles (23.9 in the next form), 10000 rows 104.5 in 256x256 (109.6 in 192x192), 7290 rows x 5120 x 1280 93.8 in 256x256 tiles
+    over 4352 columns and 128x192 over the rest (109.6 in 192x160)."""
+    def plan(M, N, K, epilogue):
+        a = _gemm_args(M, N, K, epilogue=epilogue)
+        a.w_fp8, a.w_scale = 1, 1 << 20
+        form = (ctypes.c_int32 * 3)()
+        assert lib.load().cs_gemm_big_form(ctypes.byref(a), form) == 0
+        return tuple(form)
+
+    assert plan(1458, 4352, 1152, lib.EPI_GELU_TANH) == (256, 128, 0)
+    assert plan(10000, 4352, 1152, lib.EPI_GELU_TANH) == (256, 256, 0)
+    assert plan(7290, 5120, 1280, lib.EPI_QUICK_GELU) == (128, 192, 4352)
+
+
 def test_few_row_launches_read_their_prefetch_hint():
     """A launch of at most 192 tiles starts workgroups on idle compute units that read the hint: up to 128, none without a
     hint or time.  Where a few-row form of nearly the big form's time is too full for that and the big form is not, the big
