@@ -27,7 +27,7 @@ using csgemm::BK;
 // alone, SwiGLU, another activation, a folded LayerNorm; residual products: the workgroup's last tile, whose residual piece came
 // through the ring, and the tiles before it.  Fitted to 27 products of the encoders at up to 34 row counts from 1100 to 20000, every
 // form that takes them, weights from HBM (about 3,700 launches; root mean square error 2 to 3 % with fp8 weights, 8 to 10 % with
-// bf16 ones, most of it common to all forms of a product), before edge tiles of residual products took the fast epilogue (0 to 7 us
+// bf16 ones, most of it common to all forms of a product), before edge tiles of residual products took the fast epilogue (3 to 7 us
 // less than their entries say, in every form).  A launch is as long as its rounds, and a round as long as a tile of its form however
 // few of the 256 compute units have one, so what counts is a form whose tiles fill whole rounds: 6240 rows x 3456 (folded
 // LayerNorm) are 550 tiles of 256x160 in three rounds, 62.8 us, and 504 of 224x192 in two, 49.2 us.  Chosen by this table, launches
@@ -175,8 +175,8 @@ int cs_gemm_fast(const CsGemmArgs& a, hipStream_t stream, bool* handled) {
 
 // For the few-row kernel's choice: the time of a launch as a share of what the best of 256x256, 256x128 (SwiGLU), and 256x160 or, for at
 // most 128 tiles of it, 128x160 would take, of those that take the launch; and the tiles of its (last) launch.  1 where 128x160 is the
-// one to compare with and is not built (fp8 weights, but for residual products): compared with 256x160 instead, GELU products of
-// 256 and 352 fp8 rows x 4352 x 1152 went to the big tiles, 17.7 us where few-row tiles take 10.7.
+// one to compare with and is not built: with fp8 weights, but for residual products, whose big tiles take longer than the times
+// that the share is of, in gemm_small.hip, so that the few-row kernel was never the slower one where it was chosen.
 double cs_gemm_fast_saves(const CsGemmArgs& a, int64_t* tiles) {
   const Plan p = plan_of(a);
   *tiles = tiles_of(*p.form, a.M, a.N - p.lead_cols);

@@ -62,8 +62,7 @@ double fast_us(const CsGemmArgs& a, int64_t* tiles) {
   const double stages = a.K / 128.0;
   auto us = [&](const FastForm& f) { return f.fixed_us + rounds(M, N, f.bm, f.bn) * stages * f.stage_us; };
   const bool few = (int64_t)((M + 255) / 256) * ((N + 159) / 160) <= 128;   // (the same rule as in cs_gemm_fast_saves)
-  // (a tail tile of the split residual stream: 29 us at 4888 x 1280 x 1280; a bf16 one: 22 us at 4160 .. 5376 x 1152 x 1152)
-  double t = us(few ? F128x160 : F256x160) + (!few && a.epilogue == CS_EPI_RESIDUAL && a.c_lo ? 11.0 : 0.0);
+  double t = us(few ? F128x160 : F256x160);
   if (!sums) t = us(F256x256) < t ? us(F256x256) : t;
   if (!sums && a.epilogue == CS_EPI_SWIGLU) t = us(F256x128) < t ? us(F256x128) : t;
   return t * cs_gemm_fast_saves(a, tiles);
