@@ -650,14 +650,14 @@ __global__ __launch_bounds__(256, 2) void attn_full_kernel(const AttnArgs a) {
 // (the exponents are taken out in phase 1, P.V; those products are phase 2).  How the instructions of a phase interleave is
 // laid down with scheduling groups; two waves per SIMD (two workgroups per CU) use what a wave leaves free.  V fragments live
 // in two register sets, the next step's being read during this one; K fragments are read at the start of their own step.
-//   16 heads, back to back, one phase after the other -> this kernel, d = 72: 4 x 4096 rows 370 -> 354 us, 4096 rows 105 -> 94,
-//   3300 + 1196 + 1024 + 720 rows 146 -> 86, 7 x 729 rows 34.1 -> 34.4, 2 x 729 rows 18.6 -> 14.9; d = 80: 8 x 1024 rows 59.3 -> 60.4, 1024
-//   rows 22.4 -> 17.4, 1380 + 816 rows 38.6 -> 26.4, 4888 rows 205 -> 162, 9000 + 5000 + 3000 + 1000 + 432 rows 719 -> 640, 16 x 1008 rows 113 ->
-//   117; d = 64: 2 x 1500 rows 37.7 -> 32.9; d = 96: 46.9 -> 42.7 us.  (A launch that fills the chip with equal segments gains
-//   nothing; 4 to 12 instead of 8 exponentials in phase 1 are the same within 3 %.)
+//   16 heads, back to back, one phase after the other -> this kernel, d = 72: 4 x 4096 rows 376 -> 356 us, 4096 rows 105 -> 94,
+//   3300 + 1196 + 1024 + 720 rows 142 -> 85, 7 x 729 rows 33.5 -> 33.5, 2 x 729 rows 18.5 -> 14.4; d = 80: 8 x 1024 rows 59.5 -> 60.6, 1024
+//   rows 22.4 -> 17.1, 1380 + 816 rows 38.9 -> 26.1, 4888 rows 206 -> 160, 9000 + 5000 + 3000 + 1000 + 432 rows 725 -> 643, 16 x 1008 rows 113 ->
+//   117; d = 64: 2 x 1500 rows 37.5 -> 31.4; d = 96: 46.8 -> 40.9 us.  (A launch that fills the chip with equal segments gains
+//   nothing; 6 to 12 instead of 4 exponentials in phase 1 take the same to 3 % longer.)
 // A reference that is the first tile's maximum plus a margin, whose overrun shows in the packed words, needs no maximum of a tile:
-// 3 to 5 % faster, but P is rounded elsewhere and less exactly (wide scores, d = 80: error against 64 bits 1.67e-3 instead of 1.63e-3,
-// d = 64: 1.97e-3 instead of 1.71e-3).
+// 2 to 4 % faster at d = 72 and 80, but P is rounded elsewhere and less exactly (wide scores, d = 80: error against 64 bits 1.67e-3
+// instead of 1.63e-3, d = 64: 1.97e-3 instead of 1.71e-3).
 // What bounds it is power: the shader clock falls from 1.9 to 1.4 .. 1.7 GHz under such a pipeline, and a build without the LDS reads
 // ran as many clocks at a higher clock rate.  Also measured: 64 query rows per wave and one wave per SIMD (half the LDS reads,
 // but a lone wave issues an instruction every five clocks: 2,630 clocks per 64 rows and tile against 1,930), eight waves around
@@ -906,7 +906,7 @@ __global__ __launch_bounds__(256, 2) void attn_full_direct_kernel(const AttnArgs
   // One step: O += V^T.P of p_in and vf (phase 1), then s_io, a half tile's scores, becomes those of half `half` of the tile in buffer k_b
   // (phase 2); p_out = exponentials of what s_io held, a part of them in either phase.  Meanwhile the V fragments of the next
   // step are read (half `half` of the tile in buffer v_b), and the maximum of s_max is taken, which `vote` gets between the phases.
-  constexpr int EXP_1 = 8;   // exponentials of phase 1
+  constexpr int EXP_1 = 4;   // exponentials of phase 1
   auto exponents = [&](float (&e)[16], const f32x16_t& s) {
 #pragma unroll
     for (int r = 0; r < 16; ++r) e[r] = __builtin_fmaf(s[r], sl2, -mb);
@@ -998,9 +998,9 @@ __global__ __launch_bounds__(256, 2) void attn_full_direct_kernel(const AttnArgs
     step(s0, p0, p1, vfa, vfb, b1, b0, 0, s1, psum, [&](float (&e)[16], float mx_second) {
 #pragma unroll
       for (int r = 0; r < EXP_1; ++r) asm volatile("" : "+v"(e[r]));
-      const float mx = pair_max(fmaxf(mx_first, mx_second));
+      const float mx = fmaxf(mx_first, mx_second);   // (of this lane's keys: the other lane of the query votes as well)
       if (__any((mx - m_run) * sl2 > LAZY_LOG2)) {   // (the whole wave: softmax_tile)
-        const float m_new = fmaxf(m_run, mx);
+        const float m_new = fmaxf(m_run, pair_max(mx));
         alpha = __builtin_amdgcn_exp2f((m_run - m_new) * sl2);
 #pragma unroll
         for (int d = 0; d < DT; ++d)
