@@ -157,7 +157,8 @@ struct RingShape {
 // folded into W, its bias into the GEMM bias, and w_col_sum[n] = sum_k W'[n,k] carries the mean term).
 constexpr int FUSE_NORM_A = 1, FUSE_SUMSQ_C = 2, FUSE_LN_A = 3, FUSE_STATS_C = 4;
 // The forms whose epilogue takes its residual piece through the LDS ring (see the kernel): residual epilogue on the split
-// stream, one wave spanning the tile's columns.  They use 4 KB of LDS behind the ring.  With fp8 weights as well:
+// stream, two to four row blocks a wave, one wave (without row sums also two) across the tile's columns.  They use 4 KB of LDS
+// behind the ring.  With fp8 weights as well:
 // 16128 rows x 1280 columns, mean of K = 1280 and 3456, 121.0 -> 110.5 us.
 template <int BM, int BN, int WAVES_M, int WAVES_N, int EPI, bool W_FP8, int FUSE, bool SPLIT_RES>
 constexpr bool residual_piece_through_ring() {
@@ -463,14 +464,14 @@ __global__ __launch_bounds__(64 * NW) void gemm_fast_kernel(const CsGemmArgs p) 
     const int vb_next = vb + gridDim.x;
     const bool has_next = vb_next < ntiles;
     int m0_next = 0, n0_next = 0;
-    // ---- Residual GEMMs on the split 16-bit stream (the 160-column forms: one wave spans the tile's columns).  Their
-    //      epilogue reads a [rows x 160] piece of the residual stream, three bytes per value, that nothing has touched
+    // ---- Residual GEMMs on the split 16-bit stream (the ring-fed forms; a wave has WTN of the tile's columns).  Their
+    //      epilogue reads a tile-sized piece of the residual stream, three bytes per value, that nothing has touched
     //      since the previous encoder block, and with one wave per SIMD nothing hides that latency.  The last output
     //      tile of a workgroup requests no further K tiles, so the slots of the ring fall free one by one in its last
     //      iterations, and the piece is requested straight into them with the same direct-to-LDS loads as the operands
     //      (no registers), per row block of 16 rows: NP loads of the bf16 plane (every lane fetches the 16 bytes of each
     //      pair of pieces it will need, so it reads back its own bytes) and LO_LD loads of the byte plane (the row
-    //      block's [16][BN] bytes as one run of 16-byte chunks; 4-byte loads would cost the memory pipeline as much per
+    //      block's [16][WTN] bytes as one run of 16-byte chunks; 4-byte loads would cost the memory pipeline as much per
     //      load as 16-byte ones).  A wave reads back only what it requested itself, so no barrier is involved.  The
     //      memory pipeline takes about two clocks per cache line a load touches, whoever waits for it, so the loads
     //      are spread: row block 0 (and the bias, into the 4 KB behind the ring) over the second half of the
@@ -983,7 +984,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_fast_kernel(const CsGemmArgs p) 
         constexpr int i = decltype(i_c)::value;
         if constexpr (i > 0) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * NP + (i + 1 < MT ? ROW_LD : 0)) : "memory");
         // (a wave's chunk of a direct load is 64 lanes x 16 bytes; the bf16 plane: every lane reads back what it
-        // requested; the byte plane: rows of BN bytes, one after the other)
+        // requested; the byte plane: rows of WTN bytes, one after the other)
         const char* const hi_src = smem + hi_base_of(i) + (wave * NP) * 1024 + lane_e * 16;
         const char* const lo_src = smem + lo_base_of(i) + (wave * LO_LD) * 1024 + fa * WTN + kq * (4 * G);
         const uint32_t off = (row0 + 16 * i) * (uint32_t)p.ldc + n_lane;   // in elements
@@ -1446,8 +1447,8 @@ int dispatch_epi_w(const CsGemmArgs& a, hipStream_t s) {
     if (a.a_row_sum) {   // LayerNorm in front of this GEMM
       if (!a.a_row_sumsq || !a.w_col_sum || a.pos || a.c_row_sumsq || a.c_row_sum) return CS_ERR_UNSUPPORTED;
       // (the per-column sums take 4 registers per piece on top of the bias: with the 64 pieces of a 256x256 tile's
-      // wave the epilogue no longer fits the architectural registers, so that tile is not built; cs_gemm_fast
-      // sends these launches to the 256x160 tile)
+      // wave the epilogue no longer fits the architectural registers, so that tile is not built; every other
+      // form takes these launches)
       if constexpr (BM == 256 && BN == 256) return CS_ERR_UNSUPPORTED;
       else switch (a.epilogue) {
         case CS_EPI_BIAS: return launch<BM, BN, WAVES_M, WAVES_N, CS_EPI_BIAS, false, FUSE_LN_A>(a, s);

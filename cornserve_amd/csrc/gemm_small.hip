@@ -164,8 +164,8 @@ bool cs_qkv_window_attn_two_pays(int64_t rows, int64_t windows, int heads, int K
   return !w_fp8 && cs_qkv_window_attn_few(windows, heads, K) && (rows + 63) / 64 * (heads * 2) <= 256;
 }
 
-// (Compared with the big forms of any epilogue, also where a folded LayerNorm has the 160-column ones alone, so it says no too
-// early rather than too late: passes with the rule | both | neither inline, Qwen3-VL 256 patches 1.95 | 1.94 | 2.68 ms, 576 2.62 |
+// (Compared with the big forms as a SwiGLU launch would take them, a folded LayerNorm's among others 256x256, which it does not
+// have, so it says no too early rather than too late: passes with the rule | both | neither inline, Qwen3-VL 256 patches 1.95 | 1.94 | 2.68 ms, 576 2.62 |
 // 2.54 | 2.87, 896 3.17 | 2.94 | 3.17, 1280 4.03 | 4.59 | 4.03; Qwen2.5-VL 256 2.12 | 2.12 | 2.59, 432 2.57 | 2.42 | 2.61, 576 2.78 |
 // 2.74 | 2.76, 896 2.95 | 3.24 | 2.93, 1280 3.89 | 4.60 | 3.88.)
 extern "C" int cs_gemm_norm_inline_pays(int32_t M, int32_t N, int32_t K, int32_t window_attn) {

@@ -163,7 +163,8 @@ def _num_tower_layers(config: Any) -> int:
 
 class LlavaOneVisionEncoder(SiglipEncoderBase):
     def __init__(self, config: Any, fold_norm: bool = False) -> None:
-        """`fold_norm`: see Gemma3VisionEncoder (the same tower): off by default."""
+        """`fold_norm`: see Gemma3VisionEncoder (the same tower): off by default (one 768x1152 image 6.00 ms folded, 6.04
+        apart; a video of 16 frames 12.45 and 12.17)."""
         super().__init__()
         self.config = config
         self.vision_tower = SiglipVisionModel(config.vision_config, num_hidden_layers_override=_num_tower_layers(config),

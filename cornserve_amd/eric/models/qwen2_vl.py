@@ -71,9 +71,10 @@ class Qwen2VisionTransformer(QwenVisionBase):
     def __init__(self, config: Any, weight_format: str = "bf16", fold_norm: bool = False) -> None:
         """`fold_norm`: norm1 / norm2 of every block are applied inside the GEMM that follows them (see
         Qwen2_5_VisionTransformer; here the norms are LayerNorms: the residual GEMMs also emit the row sums).
-        Off by default: the folded LayerNorm GEMM exists in 160-column tiles only (and, for few rows, with inline norms,
-        which this class does not ask for), which costs the wide QKV and fc1 projections about what the norm kernels take
-        (measured: 12.10 against 12.25 ms per 8192 patches, 4.14 against 4.05 per 1024)."""
+        Off by default: folded products have every tile form but 256x256 and no few-row one (but for inline norms, which
+        this class does not ask for), their producers 160-column tiles only, which costs about what the norm kernels take
+        (measured, folded against apart: 12.21 and 12.31 ms for 8192 patches, 5.16 and 5.34 for 1380 + 816, 3.94 and 3.86 for
+        1024)."""
         super().__init__()
         vc = config.vision_config if hasattr(config, "vision_config") else config
         if weight_format not in ("bf16", "fp8_e4m3"):
