@@ -152,7 +152,8 @@ typedef struct CsGemmArgs {
 } CsGemmArgs;
 #define CS_SUMSQ_PARTS 8
 
-/* Constraints: K % 8 == 0 (16 with fp8), lda/ldw % 8 == 0, N % 4 == 0, A and W 16-byte aligned. */
+/* Constraints: K % 8 == 0 (16 with fp8), lda/ldw % 8 == 0, N % 4 == 0, A and W 16-byte aligned.  Rows of the residual may share
+ * memory (ldr = 0 broadcasts one); rows of C may not (ldc is at least their width, unless M = 1). */
 int cs_gemm(const CsGemmArgs* args, void* stream);
 
 /* Host routine: how many workgroups cs_gemm starts for these arguments if the few-row kernel takes them (one a tile, and those
