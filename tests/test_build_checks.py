@@ -77,3 +77,26 @@ def test_an_object_whose_source_fails_the_check_does_not_survive(tmp_path, monke
         with pytest.raises(RuntimeError, match="accumulation registers"):
             build.build_library(force=force)
         assert not (out / "a.o").exists() and not linked
+
+
+@pytest.mark.parametrize("listing,passes", [(_CLEAN, True), (_SPILL, False)])
+def test_the_check_reads_the_listing_of_the_compilation_itself(tmp_path, monkeypatch, listing, passes):
+    """One compilation gives object and listing; the object appears when the listing has passed, and nothing else stays."""
+    commands = []
+
+    def run(cmd):
+        commands.append(cmd)
+        target = Path(cmd[cmd.index("-o") + 1])
+        target.write_text("object")
+        (target.parent / f"a-hip-amdgcn-amd-amdhsa-{build.ARCH}.s").write_text(listing)
+
+    monkeypatch.setattr(build, "OBJ_DIR", tmp_path)
+    monkeypatch.setattr(build, "_run", run)
+    obj = tmp_path / "a.o"
+    if passes:
+        build._compile_checked("hipcc", tmp_path / "a.hip", obj)
+    else:
+        with pytest.raises(RuntimeError, match="accumulation registers"):
+            build._compile_checked("hipcc", tmp_path / "a.hip", obj)
+    assert obj.exists() == passes and len(commands) == 1 and "-save-temps=obj" in commands[0]
+    assert [p.name for p in tmp_path.iterdir()] == ["a.o"] * passes
