@@ -460,14 +460,20 @@ __global__ __launch_bounds__(64 * NW) void gemm_fast_kernel(const CsGemmArgs p) 
   if constexpr (!RING5)
     static_for<PB>([&](auto n) { direct_load(2, a_base_of(2, ring), w_base_of(2, ring), ic<PB_FIRST + decltype(n)::value>{}); });
 
-  for (;;) {  // persistent loop over this workgroup's output tiles (vb, vb + gridDim.x, ...)
+  // A persistent loop over this workgroup's output tiles (vb, vb + gridDim.x, ...), but for the ring-fed forms, which have one tile
+  // a workgroup: only a workgroup's last tile leaves the ring to its residual piece, and a tile that does not spends 4 to 6 us
+  // more in its epilogue, while starting a workgroup and filling its ring again costs 2.2 us.  Persistent -> a workgroup per tile,
+  // row sums, 1280 columns, K = 1280 / 3456: 9000 rows 46.3 / 86.2 -> 44.1 / 84.1 us, 16384 rows 59.7 / 123.0 -> 56.3 / 121.9, 58648
+  // rows 280 / 518 -> 266 / 508; fp8 weights, 16128 rows 71.3 / 134.9 -> 66.6 / 131.2.
+  constexpr bool PRE = residual_piece_through_ring<BM, BN, WAVES_M, WAVES_N, EPI, W_FP8, FUSE, SPLIT_RES>();
+  for (;;) {
     const int vb_next = vb + gridDim.x;
-    const bool has_next = vb_next < ntiles;
+    const bool has_next = !PRE && vb_next < ntiles;
     int m0_next = 0, n0_next = 0;
     // ---- Residual GEMMs on the split 16-bit stream (the ring-fed forms; a wave has WTN of the tile's columns).  Their
     //      epilogue reads a tile-sized piece of the residual stream, three bytes per value, that nothing has touched
-    //      since the previous encoder block, and with one wave per SIMD nothing hides that latency.  The last output
-    //      tile of a workgroup requests no further K tiles, so the slots of the ring fall free one by one in its last
+    //      since the previous encoder block, and with one wave per SIMD nothing hides that latency.  The output
+    //      tile of such a workgroup, its only one, is followed by no further K tiles, so the slots of the ring fall free one by one in its last
     //      iterations, and the piece is requested straight into them with the same direct-to-LDS loads as the operands
     //      (no registers), per row block of 16 rows: NP loads of the bf16 plane (every lane fetches the 16 bytes of each
     //      pair of pieces it will need, so it reads back its own bytes) and LO_LD loads of the byte plane (the row
@@ -478,7 +484,6 @@ __global__ __launch_bounds__(64 * NW) void gemm_fast_kernel(const CsGemmArgs p) 
     //      third-last K iteration and the first half of the second-last, row block 1 over the two half-iterations
     //      after that; row blocks 2 and 3 are requested during the epilogue itself, while row blocks 0 and 1 are
     //      worked on.
-    constexpr bool PRE = residual_piece_through_ring<BM, BN, WAVES_M, WAVES_N, EPI, W_FP8, FUSE, SPLIT_RES>();
     constexpr int NP = NT / 2;                          // pairs of pieces: 16 bytes of the bf16 plane per lane
     constexpr int LO_CHUNKS = 16 * WTN / 16;            // 16-byte chunks of a row block's byte plane (the wave's columns)
     constexpr int LO_LD = (LO_CHUNKS + 63) / 64;        // ... and the loads that move them
@@ -493,7 +498,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_fast_kernel(const CsGemmArgs p) 
     const bool m_edge = EDGES && m0 + BM > p.M, n_edge = EDGES && n0 + BN > p.N;
     // (a 16-byte chunk of the byte plane that straddles the last column is left to the other form)
     constexpr bool PRE_EDGE = EDGES && ring_takes_edges<BM, BN, WAVES_M, WAVES_N, EPI, W_FP8, FUSE, SPLIT_RES>();
-    const bool pre_on = PRE && p.fast_epilogue && !has_next && !(n_edge && p.N % 16) && (PRE_EDGE || !(m_edge || n_edge));
+    const bool pre_on = PRE && p.fast_epilogue && !(n_edge && p.N % 16) && (PRE_EDGE || !(m_edge || n_edge));
     // lane-only byte offsets of the direct loads (the tile and the row block go into the scalar offset)
     uint32_t pre_hi_v = 0, pre_lo_v[PRE ? LO_LD : 1] = {}, pre_bias_v = 0, pre_scale_v = 0;
     int pre_sbase = 0;   // element offset of the wave's first row and the tile's first column in the residual matrix
@@ -632,7 +637,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_fast_kernel(const CsGemmArgs p) 
           if constexpr (CUR_B) ld();
           else if (has_next) ld();
         }
-        // the residual piece of the workgroup's last tile: first loads of row block 0 (third-last iteration) / row
+        // the residual piece: first loads of row block 0 (third-last iteration) / row
         // block 1 (second-last) into the slot that the barrier has just freed (the tile requests no K tile any more)
         if constexpr (PRE && (TAIL == 3 || TAIL == 2)) {
           constexpr int COUNT = TAIL == 3 ? PRE_N0A : PRE_N1A, EVERY = NMFMA / COUNT;
@@ -1414,7 +1419,8 @@ int launch_kernel(CsGemmArgs& p, hipStream_t stream) {
   }
   const int tiles = p.tiles_m * p.tiles_n;
   // One resident workgroup per CU (LDS-bound); with more tiles than CUs the kernel is persistent.
-  int grid = tiles <= 256 ? tiles : 256;
+  // (but a workgroup per tile where the residual piece passes through the ring: see the kernel's tile loop)
+  int grid = tiles <= 256 || residual_piece_through_ring<BM, BN, WAVES_M, WAVES_N, EPI, W_FP8, FUSE, SPLIT_RES>() ? tiles : 256;
   // few tiles and a prefetch hint: the idle compute units read the hinted bytes (see the kernel)
   if (p.prefetch && p.prefetch_bytes >= 16 && tiles <= 192) grid = tiles + (256 - tiles < 128 ? 256 - tiles : 128);
   else p.prefetch = nullptr;
