@@ -138,6 +138,11 @@ int cs_gemm_small(const CsGemmArgs& a, hipStream_t stream, bool* handled) {
   return f->run(p, stream);
 }
 
+double cs_gemm_small_us(const CsGemmArgs& a) {
+  double us;
+  return few_row_form(a, &us) ? us : 0;
+}
+
 // Workgroups of such a launch, 0 if the big tiles take it.
 int cs_gemm_small_workgroups(const CsGemmArgs& a) {
   double us;

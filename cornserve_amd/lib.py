@@ -78,6 +78,7 @@ _SIGNATURES: dict[str, list] = {
     "cs_gemm": [POINTER(CsGemmArgs), c_void_p],
     "cs_gemm_few_row_workgroups": [POINTER(CsGemmArgs)],
     "cs_gemm_big_form": [POINTER(CsGemmArgs), c_void_p],
+    "cs_gemm_lead_rows": [POINTER(CsGemmArgs)],
     "cs_gemm_norm_inline_pays": [c_int32, c_int32, c_int32, c_int32],
     "cs_gemm_rmsnorm_noalloc": [POINTER(CsGemmArgs), c_void_p],
     "cs_qkv_window_attn": [POINTER(CsGemmArgs), c_void_p, c_float, c_int32, c_int32, c_void_p],

@@ -165,6 +165,10 @@ int cs_gemm_few_row_workgroups(const CsGemmArgs* args);
  * tiles, covers (0: one launch).  Zeros if another kernel takes them.  Nothing is read through the pointers.             */
 int cs_gemm_big_form(const CsGemmArgs* args, int32_t plan[3]);
 
+/* Host routine: of two launches that split the rows, how many leading rows the first covers, in the form that cs_gemm_big_form
+ * names (whole rounds of its tiles); 0 for any other call.  Nothing is read through the pointers.                          */
+int cs_gemm_lead_rows(const CsGemmArgs* args);
+
 /* Host routine: 1 if a folded-norm launch of M rows, N weight rows and width K is faster with a_norm_inline than with row
  * sums read from arrays (few rows), 0 if not or if the shape has no inline form.  window_attn = 1: the same question for
  * cs_qkv_window_attn with M = 64 * windows and N = 256 * heads.                                                      */

@@ -632,6 +632,58 @@ def test_gemm_column_split_gives_the_bits_of_one_launch(ops, dev, M, N, K, fp8):
         assert all(torch.equal(x, y) for r in results[1:] for x, y in zip(r, results[0])), (epi, kind, list(plan))
 
 
+# Two launches over a row split -- whole rounds of one form's tiles over the leading rows, another form or the few-row kernel over the
+# rest -- give the bits of one form over all rows: the shift of every operand, row sums, scattered rows, tails of 2 to 4208 rows.
+# That the shapes are split is asserted.
+@pytest.mark.parametrize("M,N,K,epi,kind,lead", [
+    (8200, 1280, 256, "EPI_RESIDUAL", "sums", 6144), (9001, 1280, 192, "EPI_RESIDUAL", "sums", 6144), (12400, 1152, 320, "EPI_RESIDUAL", "stats", 8192),
+    (12400, 1280, 320, "EPI_RESIDUAL", "split", 8192), (12400, 1152, 320, "EPI_RESIDUAL", "plain", 8192), (8300, 5120, 5120, "EPI_SWIGLU", "norm", 6400),
+    (13060, 5120, 1280, "EPI_QUICK_GELU", "", 13056), (13060, 3840, 1280, "EPI_BIAS", "fp8", 13056), (9730, 5120, 5120, "EPI_BIAS", "rows", 9728),
+    (9730, 2560, 640, "EPI_RESIDUAL", "fp8", 8192),
+])
+def test_gemm_row_split_gives_the_bits_of_one_launch(ops, dev, M, N, K, epi, kind, lead):
+    import ctypes
+
+    from cornserve_amd import lib
+
+    epi = getattr(ops, epi)
+    a, w, b, res = rnd((M, K), 1.0, 241, dev), rnd((N, K), 0.05, 242, dev), rnd((N,), 0.02, 243, dev), rnd((M, N), 1.0, 244, dev)
+    lo = torch.randint(0, 256, (M, N), generator=torch.Generator().manual_seed(245), dtype=torch.uint8).to(dev)
+    rows = torch.randperm(M, generator=torch.Generator().manual_seed(246)).int().to(dev)
+    sc = (w.float().abs().amax(1) / 448.0).contiguous()
+    wq = (w.float() / sc[:, None]).to(torch.float8_e4m3fn).view(torch.uint8) if kind == "fp8" else w
+    ss = (a.float() ** 2).view(M, ops.SUMSQ_PARTS, -1).sum(2).contiguous()
+    width = N // 2 if epi == ops.EPI_SWIGLU else N
+    results = []
+    for run in (lib.load().cs_gemm, _big_form("192x160"), lib.load().cs_gemm):
+        out = torch.full((M + 2, width + 16), 7.0, dtype=torch.bfloat16, device=dev)
+        out_lo = torch.full((M + 2, width + 16), 9, dtype=torch.uint8, device=dev)
+        osum = torch.full((2, M + 1, ops.SUMSQ_PARTS), 5.0, device=dev)
+        g = lib.CsGemmArgs()
+        g.A, g.W, g.C, g.M, g.N, g.K, g.lda, g.ldw, g.ldc, g.epilogue = a.data_ptr(), wq.data_ptr(), out.data_ptr(), M, N, K, K, K, width + 16, epi
+        g.bias = b.data_ptr()
+        if kind == "fp8":
+            g.w_fp8, g.w_scale = 1, sc.data_ptr()
+        if epi == ops.EPI_RESIDUAL:
+            g.residual, g.ldr = res.data_ptr(), N
+        if kind in ("sums", "stats", "split"):
+            g.c_lo, g.residual_lo = out_lo.data_ptr(), lo.data_ptr()
+        if kind in ("sums", "stats"):
+            g.c_row_sumsq = osum[0].data_ptr()
+        if kind == "stats":
+            g.c_row_sum = osum[1].data_ptr()
+        if kind == "norm":
+            g.a_row_sumsq, g.norm_eps = ss.data_ptr(), 1e-6
+        if kind == "rows":
+            g.c_rows = rows.data_ptr()
+        assert lib.load().cs_gemm_lead_rows(ctypes.byref(g)) == lead
+        assert run(ctypes.byref(g), torch.cuda.current_stream().cuda_stream) == 0
+        assert bool((out[M:] == 7).all()) and bool((out[:, width:] == 7).all()) and bool((osum[:, M:] == 5).all())
+        assert bool((out_lo[M:] == 9).all()) and bool((out_lo[:, width:] == 9).all())
+        results.append((out, out_lo, osum))
+    assert all(torch.equal(x, y) for r in results[1:] for x, y in zip(r, results[0]))
+
+
 # A residual whose rows share memory (one row broadcast; rows that overlap) is the residual that a copy of it would be, in every
 # kernel and form: ring-fed and direct epilogues, whole tiles and both edges, the few-row kernel (K a multiple of 128, 200 rows)
 # and the general one (K = 80).
