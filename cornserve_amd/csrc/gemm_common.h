@@ -13,11 +13,12 @@ inline bool inline_norm_width(int K) { return K % 128 == 0 && K <= 160 * CS_SUMS
 // what fits the launch's own time.  Whole passes without hint -> with this rule (without the 4 us): Qwen2.5-VL 96 patches 1.81 ->
 // 1.80 (1.83) ms, 1280 3.88 -> 3.69 (3.68); Qwen2-VL 64 patches 1.74 -> 1.72 (1.89), 1936 6.06 -> 5.99 (5.99); Qwen3-VL 1280 4.09 ->
 // 3.96 (3.77).  Beyond 192 tiles the few idle compute units cost more than they bring (200 tiles, Qwen2.5-VL 1600 patches: 4.19
-// -> 4.26), as in the big tiles' launches.
+// -> 4.26), as in the big tiles' launches; there the few-row kernel's computing workgroups read a share each behind their last K stage
+// (hint_rows_of in gemm_small_impl.h), up to 32 MB: one image of 1024 patches 2.92 -> 2.79 ms, 1600 4.15 -> 4.00.
 constexpr int HINT_MAX_TILES = 192;
 inline int hint_workgroups(int tiles) { return tiles > HINT_MAX_TILES ? 0 : 256 - tiles < 128 ? 256 - tiles : 128; }
 inline void fit_hint(CsGemmArgs& a, int tiles, double us) {
-  const int64_t room = us > 4.0 ? (int64_t)(hint_workgroups(tiles) * 8192.0 * (us - 4.0)) : 0;
+  const int64_t room = tiles > HINT_MAX_TILES ? (int64_t)32 << 20 : us > 4.0 ? (int64_t)(hint_workgroups(tiles) * 8192.0 * (us - 4.0)) : 0;
   if (!a.prefetch || a.prefetch_bytes < 16 || room < 16) {
     a.prefetch = nullptr;
     a.prefetch_bytes = 0;

@@ -7,8 +7,8 @@
 // flight at once.  What bounds it is the LDS: per stage of 128 k it takes in (BM + BN) x 256 bytes and hands out
 // waves x (MT + NT) x 4 KB of fragments, and time per stage follows that sum at about 270 KB a microsecond and compute
 // unit (128 bytes a clock) in the GEMM's tile forms; the rest of a launch is 4 to 5 us of launch, first loads and epilogue.
-// (That gives the window attention form, one wave a SIMD, 13 us.  It takes 14.6 with weights in the caches, 19.7 with the inline
-// norm, and 4 to 8 more with its 10 MB of weights from HBM.)
+// (The window attention form, one wave a SIMD, takes 17 us with weights in the caches, 8 of them launch, first loads and the
+// attention; 21 with the inline norm, 23 with its 10 MB of weights from HBM.)
 // Measured on an MI355X with weights that no cache holds: 1280 columns, K = 3456: 96 rows 34.3 -> 8.7 us (32x32 tiles),
 // 1024 rows 38 -> 20 us (64x80); K = 1280: 96 rows 19 -> 6 us, 1024 rows 19 -> 11 us.  The big tiles are the faster ones from
 // about 2000 rows on at K = 1280, from 3100 (128x128 tiles until then) at K = 3456 to 5120: the choice is in gemm_small.hip.
@@ -142,6 +142,11 @@ struct SmallShape {
   static constexpr int SUMS_BYTES = SUMS == SUMS_NONE ? 0 : BM * 16 * SUMS;
   static constexpr int LDS = STAGES * STAGE + NORM_BYTES + SUMS_BYTES;
   static_assert(LDS <= 160 * 1024, "the ring fits the LDS");
+  static constexpr int64_t NLD_OF(int waves) { return KS * (BM / 8) / waves + (KS * (BN * W_ROW / 1024) + waves - 1) / waves; }   // direct loads per wave and stage
+  // A prefetch hint behind the last stage (see hint_rows_of): rows of one segment, as wide as a stage's step, per stage
+  // (not in 128x128 tiles, with their launches of 20 us and more: the branch to it costs 0.8 % of them)
+  static constexpr bool RING_HINT = !W_FP8 && BM * BN < 128 * 128;
+  static constexpr int HINT_SEG = KS * 128, HINT_STAGES = KS == 2 ? STAGES - 1 : STAGES - 2, HINT_PITCH = HINT_STAGES * HINT_SEG;
 };
 
 // What follows the projection in a window (see small_wattn_epilogue), 16 queries a wave: `qk(f)` is fragment f (0 .. 4 q, 5 .. 9
@@ -248,49 +253,22 @@ CS_DEVICE void window_attention(const CsGemmArgs& p, const char* vt, char* ks, F
 // What changes hands goes through LDS (the ring is free by now): q and k in fp32 with norm and bias applied (a rotary
 // pair's halves sit in different fragments), v rounded and transposed, then the rotated keys.  Every operation on a value
 // is the one of the big tile's epilogue (gemm_fast_impl.h), in its order.
-template <int MT, int NT, bool W_FP8, int NORM>
-CS_DEVICE void small_wattn_epilogue(const CsGemmArgs& p, char* smem, const f32x4_t (&acc)[MT][NT],
-                                    const float (&rstd_in)[NORM != NORM_NONE ? MT : 1], const int (&mrow)[MT], int m0, int n0, int cnt, int wave, int lane) {
+template <int MT, int NT, bool W_FP8>
+CS_DEVICE void small_wattn_epilogue(const CsGemmArgs& p, char* smem, const f32x4_t (&acc)[MT][NT], const float (&rstd)[MT], const u32x2_t (&bias_w)[NT],
+                                    const float (&co)[10], const float (&si)[10], int m0, int n0, int cnt, int wave, int lane) {
   static_assert(MT == 4 && NT == 4, "all four row blocks, four fragments per wave");
-  constexpr int HD = 80, HALF = 40, X_BYTES = 4 * 10 * 1024, VT_ROW = 144, VT_BYTES = HD * VT_ROW;
+  constexpr int HD = 80, X_BYTES = 4 * 10 * 1024, VT_ROW = 144, VT_BYTES = HD * VT_ROW;
   const int lr = lane & 15, kq = lane >> 4;
   char* const xs = smem;                              // [row block][fragment 0..9][lane]: 4 fp32
   char* const vt = smem + X_BYTES;                    // [head dim][key]: bf16, 144-byte rows
   char* const ks = smem + X_BYTES + VT_BYTES;         // [row block][part 0, 1: 16 bytes, part 2: 8 bytes][lane]
-  // per-row scale of the folded RMSNorm: rows 16 i + lr of the window
-  float rstd[MT];
-#pragma unroll
-  for (int i = 0; i < MT; ++i) {
-    rstd[i] = 1.0f;
-    if constexpr (NORM != NORM_NONE) {
-      rstd[i] = rstd_in[NORM != NORM_NONE ? i : 0];
-    } else if (p.a_row_sumsq) {
-      const float* parts = p.a_row_sumsq + (int64_t)mrow[i] * CS_SUMSQ_PARTS;
-      const f32x4_t s0 = *(const f32x4_t*)parts, s1 = *(const f32x4_t*)(parts + 4);
-      const float ss = ((s0[0] + s0[1]) + (s0[2] + s0[3])) + ((s1[0] + s1[1]) + (s1[2] + s1[3]));
-      rstd[i] = rsqrtf(ss / (float)p.K + p.norm_eps);
-    }
-  }
-  // the rotary table's rows of this wave's queries
-  float co[10], si[10];
-  {
-    const float* cs = p.attn_cos_sin + (int64_t)(m0 + min(16 * wave + lr, cnt - 1)) * HD + 10 * kq;
-#pragma unroll
-    for (int t = 0; t < 10; t += 2) {
-      const f32x2_t c2 = *(const f32x2_t*)(cs + t), s2 = *(const f32x2_t*)(cs + HALF + t);
-      co[t] = c2[0];
-      co[t + 1] = c2[1];
-      si[t] = s2[0];
-      si[t + 1] = s2[1];
-    }
-  }
   __syncthreads();   // (nobody reads operands from the ring any more)
 #pragma unroll
   for (int j = 0; j < NT; ++j) {
     const int J = 4 * wave + j;
     if (J >= 15) break;
     const int ch = n0 + (J / 2) * 32 + 8 * kq + (J % 2) * 4;
-    const bf16x4_t bias_b = *(const bf16x4_t*)((const bf16_t*)p.bias + ch);
+    const bf16x4_t bias_b = __builtin_bit_cast(bf16x4_t, bias_w[j]);
     f32x4_t wsc = {1.f, 1.f, 1.f, 1.f};
     if constexpr (W_FP8) wsc = *(const f32x4_t*)(p.w_scale + ch);
 #pragma unroll
@@ -313,7 +291,7 @@ CS_DEVICE void small_wattn_epilogue(const CsGemmArgs& p, char* smem, const f32x4
 }
 
 template <int BM, int BN, int WAVES_M, int WAVES_N, int KS, int STAGES, int EPI, bool W_FP8, int NORM, bool SPLIT, int SUMS>
-__global__ __launch_bounds__(64 * WAVES_M * WAVES_N, EPI == SM_EPI_QKV_WATTN ? 1 : 2) void gemm_small_kernel(const CsGemmArgs p) {
+__global__ __launch_bounds__(64 * WAVES_M * WAVES_N, EPI == SM_EPI_QKV_WATTN ? 1 : 2) void gemm_small_kernel(const CsGemmArgs p, const int hint_rows) {
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   using Shape = SmallShape<BM, BN, KS, STAGES, W_FP8, NORM, SUMS>;
   constexpr bool WATTN = EPI == SM_EPI_QKV_WATTN;
@@ -405,9 +383,29 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, EPI == SM_EPI_QKV_WATTN ? 1
   const uint32_t bias_mask = p.bias ? 0xFFFFFFFFu : 0u, lo_mask = p.residual_lo ? 0xFFFFFFFFu : 0u;
   u32x2_t add_hi[ADDEND ? MT : 1][ADDEND ? NT : 1];
   uint32_t add_lo[SPLIT ? MT : 1][SPLIT ? NT : 1];
-  if constexpr (!WATTN) {
 #pragma unroll
-    for (int j = 0; j < NT; ++j) bias_w[j] = *(const u32x2_t*)(bias_src + ncol[j]);
+  for (int j = 0; j < NT; ++j) bias_w[j] = *(const u32x2_t*)(bias_src + ncol[j]);
+  // WATTN: the rotary table's rows of this wave's queries, and the row sums of the folded RMSNorm (from arrays) of the window's rows
+  float co[WATTN ? 10 : 1], si[WATTN ? 10 : 1];
+  f32x4_t row_parts[WATTN && NORM == NORM_NONE ? MT : 1][2] = {};
+  if constexpr (WATTN) {
+    const float* cs = p.attn_cos_sin + (int64_t)(m0 + min(16 * wave + fa, cnt - 1)) * 80 + 10 * kq;
+#pragma unroll
+    for (int t = 0; t < 10; t += 2) {
+      const f32x2_t c2 = *(const f32x2_t*)(cs + t), s2 = *(const f32x2_t*)(cs + 40 + t);
+      co[WATTN ? t : 0] = c2[0];
+      co[WATTN ? t + 1 : 0] = c2[1];
+      si[WATTN ? t : 0] = s2[0];
+      si[WATTN ? t + 1 : 0] = s2[1];
+    }
+    if constexpr (NORM == NORM_NONE) {
+#pragma unroll
+      for (int i = 0; i < MT; ++i) {   // (without a norm the table's rows stand in for them)
+        const float* parts = p.a_row_sumsq ? p.a_row_sumsq + (int64_t)mrow[i] * CS_SUMSQ_PARTS : p.attn_cos_sin + (int64_t)mrow[i] * 80;
+        row_parts[WATTN && NORM == NORM_NONE ? i : 0][0] = *(const f32x4_t*)parts;
+        row_parts[WATTN && NORM == NORM_NONE ? i : 0][1] = *(const f32x4_t*)(parts + 4);
+      }
+    }
   }
   if constexpr (ADDEND) {
 #pragma unroll
@@ -453,9 +451,9 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, EPI == SM_EPI_QKV_WATTN ? 1
     }
     w_dst[j] = KS * A_SUB + sub * W_SUB + blk * 1024;
   }
-  const __amdgpu_buffer_rsrc_t rsrc_a =
+  __amdgpu_buffer_rsrc_t rsrc_a =
       __builtin_amdgcn_make_buffer_rsrc((void*)p.A, 0, (int)(uint32_t)(((int64_t)(p.M - 1) * p.lda + p.K) * 2), 0x00020000);
-  const __amdgpu_buffer_rsrc_t rsrc_w = __builtin_amdgcn_make_buffer_rsrc(
+  __amdgpu_buffer_rsrc_t rsrc_w = __builtin_amdgcn_make_buffer_rsrc(
       (void*)p.W, 0, (int)(uint32_t)(((int64_t)(p.N - 1) * p.ldw + p.K) * (W_FP8 ? 1 : 2)), 0x00020000);
   // (the device-only builtin with nothing template-dependent around it: else the host pass drops the kernel)
   auto load_a = [&](char* lds_dst, uint32_t off, int soff) {
@@ -465,9 +463,9 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, EPI == SM_EPI_QKV_WATTN ? 1
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_w, (sm_lds_void_t*)lds_dst, 16, off, soff, 0, 0);
   };
   // direct loads FROM .. TO - 1 of a stage (the activation rows first)
-  auto issue = [&](int stage, int slot, auto from_c, auto to_c) {
+  auto issue = [&](int stage, int slot_off, auto from_c, auto to_c) {
     constexpr int FROM = decltype(from_c)::value, TO = decltype(to_c)::value;
-    char* const base = smem + slot * STAGE;
+    char* const base = smem + slot_off;
 #pragma unroll
     for (int n = FROM; n < TO; ++n) {
       if (n < A_LD) load_a(base + a_dst[n < A_LD ? n : 0], a_src[n < A_LD ? n : 0], stage * (KS * 128));
@@ -496,40 +494,59 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, EPI == SM_EPI_QKV_WATTN ? 1
   float ss[NORM != NORM_NONE ? NORM_MT : 1], sm[NORM == NORM_LN ? NORM_MT : 1];
   const int norm_row = WATTN ? wave * 16 + fa : wm * WTM + fa;
   bf16x8_t xn[2][2];
-  int steps = 0, part = 0;
+  int phase = 0, part = 0;
   float* const parts_ss = (float*)(smem + STAGES * STAGE);
   float* const parts_sm = parts_ss + BM * CS_SUMSQ_PARTS * 4;
-  auto close_part = [&]() {
-    if constexpr (NORM != NORM_NONE) {
+  // A K tile is two k-steps, a part five: of five K tiles the third closes a part after its first k-step, the fifth after its second.
+  // The tile only sets the chains aside (`ss0`); they are stored behind it, where no branch cuts an iteration's schedule (WATTN, 16
+  // windows, weights from HBM: 24.9 -> 23.3 us).
+  constexpr int NS = NORM != NORM_NONE ? NORM_MT : 1, NM = NORM == NORM_LN ? NORM_MT : 1;
+  float ss0[NS], sm0[NM];
+  auto store_part = [&](bool aside) {
 #pragma unroll
-      for (int i = 0; i < NORM_MT; ++i) {
-        // (the waves that share a tile row write the same values)
-        const int at = (part * BM + norm_row + 16 * i) * 4 + kq;
-        parts_ss[at] = ss[i];
-        ss[i] = 0.f;
-        if constexpr (NORM == NORM_LN) {
-          parts_sm[at] = sm[i];
-          sm[i] = 0.f;
-        }
+    for (int i = 0; i < NS; ++i) {
+      // (the waves that share a tile row write the same values)
+      const int at = (part * BM + norm_row + 16 * i) * 4 + kq;
+      parts_ss[at] = aside ? ss0[i] : ss[i];
+      ss[i] = aside ? ss[i] : 0.f;
+      if constexpr (NORM == NORM_LN) {
+        parts_sm[at] = aside ? sm0[i < NM ? i : 0] : sm[i < NM ? i : 0];
+        sm[i < NM ? i : 0] = aside ? sm[i < NM ? i : 0] : 0.f;
       }
-      ++part;
-      steps = 0;
+    }
+    ++part;
+  };
+  auto end_of_step = [&](int step) {
+    if (step == 0) {
+#pragma unroll
+      for (int i = 0; i < NS; ++i) {
+        ss0[i] = ss[i];
+        ss[i] = phase == 2 ? 0.f : ss[i];
+      }
+#pragma unroll
+      for (int i = 0; i < NM; ++i) {
+        sm0[i] = sm[i];
+        sm[i] = phase == 2 ? 0.f : sm[i];
+      }
     }
   };
-  if constexpr (NORM != NORM_NONE) {
-#pragma unroll
-    for (int i = 0; i < NORM_MT; ++i) {
-      ss[i] = 0.f;
-      if constexpr (NORM == NORM_LN) sm[i] = 0.f;
+  auto end_of_tile = [&]() {
+    if constexpr (NORM != NORM_NONE) {
+      if (phase == 2 || phase == 4) store_part(phase == 2);
+      phase = phase == 4 ? 0 : phase + 1;
     }
-  }
+  };
+#pragma unroll
+  for (int i = 0; i < NS; ++i) ss[i] = 0.f;
+#pragma unroll
+  for (int i = 0; i < NM; ++i) sm[i] = 0.f;
 
   // ---- operand fragments of one K tile, two sets: one is read while the matrix cores work on the other
   bf16x8_t xf[2][2][MT], wf[2][W_FP8 ? 1 : 2][W_FP8 ? 1 : NT];
   i32x2_t wraw[2][W_FP8 ? 2 : 1][W_FP8 ? NT : 1];
-  auto read_tile = [&](int slot, auto sub_c, auto set_c) {   // K tile `sub` of the slot's stage into fragment set `set`
+  auto read_tile = [&](int slot_off, auto sub_c, auto set_c) {   // K tile `sub` of the slot's stage into fragment set `set`
     constexpr int SUB = decltype(sub_c)::value, SET = decltype(set_c)::value;
-    const char* const base = smem + slot * STAGE;
+    const char* const base = smem + slot_off;
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
       const char* const a_tile = base + SUB * A_SUB + x_off[s];
@@ -570,7 +587,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, EPI == SM_EPI_QKV_WATTN ? 1
             if constexpr (NORM == NORM_LN) sm[i] = sm_dot2(x[q], SM_ONE_PAIR, sm[i]);
           }
         }
-        if (++steps == 5) close_part();
+        end_of_step(s);
       }
     }
   };
@@ -582,14 +599,37 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, EPI == SM_EPI_QKV_WATTN ? 1
   auto wait_landed = [&](int later) {   // at most the loads of the `later` stages requested after the needed one remain
     small_wait<NLD>(later, std::make_integer_sequence<int, STAGES>{});
   };
+  // Slots by their byte offset in the ring: of stage kt - 1, kt and kt + 1
+  int prev = (STAGES - 1) * STAGE, slot = 0, next = STAGE;
+  auto turn = [&]() {
+    prev = slot;
+    slot = next;
+    next = next == (STAGES - 1) * STAGE ? 0 : next + STAGE;
+  };
+  // With a share of the prefetch hint the ring runs on into it behind the last stage (see hint_rows_of): the loads' sources move.
+  // The slots of the ring are free by then, and nobody reads what arrives.
+  const bool reads_hint = Shape::RING_HINT && hint_rows > 0 && nst >= STAGES;
+  auto switch_to_hint = [&]() {
+    if constexpr (Shape::RING_HINT) {
+      const int first = (int)blockIdx.x * hint_rows, rows = min(max((int)((uint32_t)p.prefetch_bytes / Shape::HINT_PITCH) - first, 0), hint_rows);
+      const char* const base = (const char*)p.prefetch + (int64_t)first * Shape::HINT_PITCH - nst * Shape::HINT_SEG;
+      rsrc_a = rsrc_w = __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, rows * Shape::HINT_PITCH, 0x00020000);
+      constexpr int LANES = Shape::HINT_SEG / 16;   // ... to a segment
+      const uint32_t lane_off = (lane / LANES) * Shape::HINT_PITCH + (lane % LANES) * 16;
 #pragma unroll
-  for (int s = 0; s < STAGES; ++s)
-    if (s < nst) issue(s, s, C0, CEND);
-  wait_landed(min(STAGES, nst) - 1);
+      for (int n = 0; n < NLD; ++n) {
+        const uint32_t off = lane_off + (wave * NLD + n) * (64 / LANES * Shape::HINT_PITCH);
+        if (n < A_LD) a_src[n < A_LD ? n : 0] = off;
+        else w_src[n < A_LD ? 0 : n - A_LD] = off;
+      }
+    }
+  };
   int kt = 0;
-  read_tile(0, C0, C0);
-  // STEADY iterations have a stage to request (and, but for the first one, the rest of an earlier one), so that no branch
-  // interrupts their schedule; `slot` is a constant where the loop is unrolled over the ring.
+  // STEADY iterations have a stage to request and no branch that would interrupt their schedule.  Their loop is rolled: a launch of
+  // few rows runs through some ten iterations, and unrolled over the ring each of them fetches its instructions for the first
+  // time (256 rows x 1280 x 1280 7.1 -> 6.6 us).  Only the smallest tiles, whose iterations are a handful of MFMAs, save more
+  // with the slots' addresses as constants where the loop is long (96 rows x 1280 x 3456 8.1 us rolled, 7.7).
+  constexpr bool UNROLLED = BM == 32 && BN <= 64;
   constexpr std::true_type T{};
   constexpr std::false_type F{};
   if constexpr (KS == 2) {
@@ -597,72 +637,93 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, EPI == SM_EPI_QKV_WATTN ? 1
     // tile 1 is read.  The barrier in the middle says that stage kt + 1 has landed for every wave and that nobody reads
     // stage kt's slot any more.  Second half: tile 1 is multiplied while tile 0 of stage kt + 1 is read.  Stage kt + STAGES
     // goes into the freed slot, half of its loads in this half and half in the next.
-    auto iteration = [&](auto steady_c, auto first_c, int slot) {
-      constexpr bool STEADY = decltype(steady_c)::value, FIRST = decltype(first_c)::value;
-      const int prev = slot == 0 ? STAGES - 1 : slot - 1, next = slot == STAGES - 1 ? 0 : slot + 1;
+    small_for([&](auto s_c) {
+      constexpr int S = decltype(s_c)::value;
+      if (S < nst) issue(S, S * STAGE, C0, std::integral_constant<int, S < STAGES - 1 ? NLD : NLD / 2>{});
+    }, std::make_integer_sequence<int, STAGES>{});
+    if (nst >= STAGES) sm_wait_barrier<(STAGES - 2) * NLD + NLD / 2>();
+    else wait_landed(nst - 1);
+    read_tile(0, C0, C0);
+    auto iteration = [&](auto steady_c) {
+      constexpr bool STEADY = decltype(steady_c)::value;
       read_tile(slot, C1, C1);
-      if constexpr (!FIRST) {
-        if (STEADY || kt + STAGES - 1 < nst) issue(kt + STAGES - 1, prev, CMID, CEND);
-      }
+      if (STEADY || kt + STAGES - 1 < nst) issue(kt + STAGES - 1, prev, CMID, CEND);
       multiply(C0);
       if constexpr (STEADY) {
-        small_schedule<2 * (MT + NT), FIRST ? 0 : NLD - NLD / 2, 2 * MT * NT>();
+        small_schedule<2 * (MT + NT), NLD - NLD / 2, 2 * MT * NT>();
+        end_of_tile();
+        if (Shape::RING_HINT && kt + STAGES == nst) switch_to_hint();
         sm_wait_barrier<(STAGES - 2) * NLD>();
         read_tile(next, C0, C0);
         issue(kt + STAGES, slot, C0, CMID);
-      } else if (kt + 1 < nst) {
-        wait_landed(min(STAGES - 2, nst - kt - 2));
-        if (kt + STAGES < nst) issue(kt + STAGES, slot, C0, CMID);
-        read_tile(next, C0, C0);
+      } else {
+        end_of_tile();
+        if (kt + 1 < nst) {
+          wait_landed(min(STAGES - 2, nst - kt - 2));
+          read_tile(next, C0, C0);
+        }
       }
       multiply(C1);
       if constexpr (STEADY) small_schedule<2 * (MT + NT), NLD / 2, 2 * MT * NT>();
+      end_of_tile();
       ++kt;
+      turn();
     };
-    if (STAGES < nst) {
-      iteration(T, T, 0);
-      while (kt + 2 * STAGES <= nst)
-        small_for([&](auto n) { iteration(T, F, (decltype(n)::value + 1) % STAGES); }, std::make_integer_sequence<int, STAGES>{});
-    } else {
-      iteration(F, T, 0);
-    }
-    for (int slot = 1 % STAGES; kt < nst; slot = slot == STAGES - 1 ? 0 : slot + 1) iteration(F, F, slot);
+    const int steady = reads_hint ? nst - 1 : nst - STAGES;
+    if (UNROLLED && steady >= 2 * STAGES)
+      while (kt + STAGES <= steady) small_for([&](auto) { iteration(T); }, std::make_integer_sequence<int, STAGES>{});
+    while (kt < steady) iteration(T);
+    while (kt < nst) iteration(F);
   } else {
     // One K tile per stage (tiles so large that a stage of two would leave a ring of two): the fragments of tile kt are in
-    // registers at the top of iteration kt, the barrier frees its slot for tile kt + STAGES.
-    static_assert(KS == 2 || STAGES % 2 == 0, "the fragment set alternates with the slot");
-    auto iteration = [&](auto steady_c, auto set_c, int slot) {
+    // registers at the top of iteration kt, the barrier frees its slot for tile kt + STAGES.  K is a multiple of 128, so
+    // the tiles go in pairs, one for each fragment set.
+    small_for([&](auto s_c) {
+      constexpr int S = decltype(s_c)::value;
+      if (S < nst) issue(S, S * STAGE, C0, CEND);
+    }, std::make_integer_sequence<int, STAGES>{});
+    wait_landed(min(STAGES, nst) - 1);
+    read_tile(0, C0, C0);
+    auto iteration = [&](auto steady_c, auto set_c) {
       constexpr bool STEADY = decltype(steady_c)::value;
       constexpr std::integral_constant<int, 1 - decltype(set_c)::value> OTHER{};
-      const int next = slot == STAGES - 1 ? 0 : slot + 1;
       if constexpr (STEADY) {
+        if (Shape::RING_HINT && kt + STAGES == nst) switch_to_hint();
         sm_wait_barrier<(STAGES - 2) * NLD>();
         read_tile(next, C0, OTHER);
         issue(kt + STAGES, slot, C0, CEND);
       } else if (kt + 1 < nst) {
-        wait_landed(min(STAGES - 2, nst - kt - 2));
-        if (kt + STAGES < nst) issue(kt + STAGES, slot, C0, CEND);
+        // (behind a hint, whose loads are not waited for, the needed stage was requested before them)
+        if (reads_hint) sm_wait_barrier<(STAGES - 2) * NLD>();
+        else wait_landed(min(STAGES - 2, nst - kt - 2));
+        if (!reads_hint && kt + STAGES < nst) issue(kt + STAGES, slot, C0, CEND);
         read_tile(next, C0, OTHER);
       }
       multiply(set_c);
       if constexpr (STEADY) small_schedule<2 * (MT + NT + (WATTN && NORM != NORM_NONE ? 1 : 0)), NLD, 2 * MT * NT>();
+      end_of_tile();
       ++kt;
+      turn();
     };
-    while (kt + 2 * STAGES <= nst)
-      small_for([&](auto n) { iteration(T, std::integral_constant<int, decltype(n)::value % 2>{}, decltype(n)::value); },
-                std::make_integer_sequence<int, STAGES>{});
-    for (int slot = 0; kt < nst;) {   // (here kt is a multiple of STAGES, so the slot starts at 0 and set 0)
-      iteration(F, C0, slot);
-      slot = slot == STAGES - 1 ? 0 : slot + 1;
-      if (kt < nst) iteration(F, C1, slot);
-      slot = slot == STAGES - 1 ? 0 : slot + 1;
+    const int steady = reads_hint ? nst - 2 : nst - STAGES - 1;   // (the last of an odd count goes with the others)
+    while (kt < steady) {
+      iteration(T, C0);
+      iteration(T, C1);
+    }
+    while (kt < nst) {
+      iteration(F, C0);
+      if (kt < nst) iteration(F, C1);
     }
   }
 
+  // (the LDS that loads in flight write must stay this workgroup's; without a hint nobody waits here for the stores)
+  auto end_of_hint = [&]() {
+    if (reads_hint) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  };
   // ---- epilogue
   float rstd[NORM != NORM_NONE ? MT : 1], nmean_rstd[NORM == NORM_LN ? MT : 1];
   if constexpr (NORM != NORM_NONE) {
-    if (steps) close_part();
+    if ((2 * nst * KS) % 5) store_part(false);   // (the last part is narrower)
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // (this wave's own values: no barrier)
     if constexpr (WATTN) __syncthreads();                // (each row block's are another wave's)
 #pragma unroll
@@ -679,7 +740,22 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, EPI == SM_EPI_QKV_WATTN ? 1
     }
   }
   if constexpr (WATTN) {
-    small_wattn_epilogue<MT, NT, W_FP8, NORM>(p, smem, acc, rstd, mrow, m0, n0, cnt, wave, lane);
+    float row_scale[MT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      row_scale[i] = 1.0f;
+      if constexpr (NORM != NORM_NONE) {
+        row_scale[i] = rstd[NORM != NORM_NONE ? i : 0];
+      } else if (p.a_row_sumsq) {
+        const f32x4_t s0 = row_parts[NORM == NORM_NONE ? i : 0][0], s1 = row_parts[NORM == NORM_NONE ? i : 0][1];
+        const float total = ((s0[0] + s0[1]) + (s0[2] + s0[3])) + ((s1[0] + s1[1]) + (s1[2] + s1[3]));
+        row_scale[i] = rsqrtf(total / (float)p.K + p.norm_eps);
+      }
+    }
+    // (in the two slots that the hint's last loads, which may be in flight, do not go to: the last two stages', neighbours because
+    // their number is even)
+    small_wattn_epilogue<MT, NT, W_FP8>(p, smem + (W_FP8 ? 0 : (nst - 2) % STAGES * STAGE), acc, row_scale, bias_w, co, si, m0, n0, cnt, wave, lane);
+    end_of_hint();
     return;
   }
   f32x4_t scale_v[W_FP8 ? NT : 1], csum_v[NORM == NORM_LN ? NT : 1];   // (all loads ahead of the first store)
@@ -712,6 +788,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, EPI == SM_EPI_QKV_WATTN ? 1
         if (mok[i]) *(f32x4_t*)((float*)p.C + (int64_t)mrow[i] * p.ldc + col[j]) = x;
       }
     }
+    end_of_hint();
     return;
   }
   bf16_t* const pC = (bf16_t*)p.C;
@@ -825,6 +902,18 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, EPI == SM_EPI_QKV_WATTN ? 1
       }
     }
   }
+  end_of_hint();
+}
+
+// A launch with a tile for every compute unit has nobody idle to read its hint, but nothing to request in its last STAGES - 1
+// iterations and its epilogue either: its workgroups read a share each with the ring's own loads, into slots that are free by then.
+// The hint is cut into rows of HINT_STAGES segments; a lane's row and place in it are fixed, and the stages walk along the row.
+// Returns the rows of a workgroup, at most what its loads cover; what is left of the hint is not read.
+template <class Shape, int WAVES>
+int hint_rows_of(int64_t bytes, int tiles) {
+  if (!Shape::RING_HINT) return 0;
+  const int64_t share = (bytes / Shape::HINT_PITCH + tiles - 1) / tiles, most = WAVES * Shape::NLD_OF(WAVES) * (1024 / Shape::HINT_SEG);
+  return (int)(share < most ? share : most);
 }
 
 template <int BM, int BN, int WAVES_M, int WAVES_N, int KS, int STAGES, int EPI, bool W_FP8, int NORM, bool SPLIT, int SUMS = SUMS_NONE>
@@ -843,8 +932,9 @@ int launch_small(const CsGemmArgs& a, hipStream_t stream) {
     if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess) return CS_ERR_LAUNCH;
     attr_set = true;
   }
-  const int tiles = p.tiles_m * p.tiles_n;   // (a hint that is still there is one to be read)
-  hipLaunchKernelGGL(kern, dim3(tiles + (p.prefetch ? hint_workgroups(tiles) : 0)), dim3(64 * WAVES_M * WAVES_N), lds, stream, p);
+  const int tiles = p.tiles_m * p.tiles_n, extra = p.prefetch ? hint_workgroups(tiles) : 0;   // (a hint that is still there is one to be read)
+  const int hint_rows = p.prefetch && !extra ? hint_rows_of<SmallShape<BM, BN, KS, STAGES, W_FP8, NORM, SUMS>, WAVES_M * WAVES_N>(p.prefetch_bytes, tiles) : 0;
+  hipLaunchKernelGGL(kern, dim3(tiles + extra), dim3(64 * WAVES_M * WAVES_N), lds, stream, p, hint_rows);
   return cs_launch_status();
 }
 

@@ -136,7 +136,8 @@ typedef struct CsGemmArgs {
    * (such a launch is bound by operand latency, not by arithmetic).  Results are not affected; the hint is ignored
    * by launches that fill the chip and by the general kernel.  NULL / 0: no hint.  A prefetching workgroup moves
    * about 8 KB per microsecond and the launch ends when its last workgroup does.  The few-row kernel reads of the hint,
-   * from its start, what fits the launch's own time.  The big tiles read all of it: hint what the idle compute units
+   * from its start, what fits the launch's own time; with more than 192 tiles its computing workgroups read up to 32 MB of it behind
+   * their last K stage (bf16 W).  The big tiles read all of it: hint what the idle compute units
    * (256 minus the launch's tiles, at most 128) can read in that time -- 9 MB behind a 64-tile launch of 20 K tiles costs
    * nothing, 18 MB behind a 192-tile one doubles its duration.                                                        */
   const void* prefetch;

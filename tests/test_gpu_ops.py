@@ -1035,6 +1035,52 @@ def test_few_row_launches_with_a_prefetch_hint_keep_their_bits(ops, dev):
 
 
 @pytest.mark.parametrize("M,N,K", [
+    (1024, 1280, 1280), (1024, 1280, 3456),          # 64x80, with row sums 32x160
+    (1024, 1280, 256), (224, 1120, 256), (224, 1120, 1024),   # as many K stages as the ring has slots, fewer, more (64x80; 32x32)
+    (250, 1696, 1280), (500, 1760, 1280), (500, 3456, 1152), (2048, 1696, 1280), (400, 6912, 1280),   # 32x64 ... 128x128, two rounds
+])
+def test_full_few_row_launches_read_their_hint_with_the_ring(ops, dev, M, N, K):
+    """A launch of more than 192 tiles has nobody idle to read its hint: the ring runs on into it behind the last K stage.  Same bits
+    without a hint and with hints from less than a row of it to more than all workgroups read."""
+    hints = [torch.zeros(n, dtype=torch.uint8, device=dev) for n in (16, 1 << 10, 1000016, 40 << 20)]
+    a, w, b = rnd((M, K), 1.0, 131, dev), rnd((N, K), 0.05, 132, dev), rnd((N,), 0.02, 133, dev)
+    res, lo = rnd((M, N), 1.0, 134, dev), torch.zeros((M, N), dtype=torch.uint8, device=dev)
+    colsum = w.float().sum(1)
+
+    def forms(hint):
+        out_lo = torch.empty_like(lo)
+        kw = {"epilogue": ops.EPI_RESIDUAL, "residual": res, "residual_lo": lo, "out_lo": out_lo, "prefetch": hint}
+        got = [ops.gemm(a, w, b, **kw), out_lo.clone(), ops.gemm(a, w, b, epilogue=ops.EPI_GELU_TANH, prefetch=hint)]
+        if N <= 160 * ops.SUMSQ_PARTS:
+            ss, sm = torch.zeros((M, ops.SUMSQ_PARTS), device=dev), torch.zeros((M, ops.SUMSQ_PARTS), device=dev)
+            got += [ops.gemm(a, w, b, c_row_sumsq=ss, c_row_sum=sm, **kw), ss, sm]
+        if K <= 1280:
+            got += [ops.gemm(a, w, b, epilogue=ops.EPI_SWIGLU, norm_inline=True, norm_eps=1e-6, prefetch=hint),
+                    ops.gemm(a, w, b, norm_inline=True, w_col_sum=colsum, norm_eps=1e-6, prefetch=hint)]
+        return got
+
+    plain = forms(None)
+    for h in hints:
+        assert all(torch.equal(x, y) for x, y in zip(forms(h), plain, strict=True)), h.numel()
+
+
+@pytest.mark.parametrize("windows,K,form", [(16, 1280, "inline"), (16, 1280, "plain"), (13, 1152, "array"), (16, 256, "inline"), (14, 384, "plain")])
+def test_full_few_window_launches_read_their_hint_with_the_ring(ops, dev, windows, K, form):
+    """The same for a workgroup per window and head (13 x 16 and more of them), whose attention works in the slots that the hint
+    leaves alone: a last window of 4 rows, K of a multiple of four K tiles and of an odd multiple of two."""
+    heads, d = 16, 80
+    M = windows * 64 - 60
+    win_start = torch.tensor([64 * i for i in range(windows)] + [M], dtype=torch.int32, device=dev)
+    x, cos = rnd((M, K), 1.0, 135, dev), torch.rand((M, d), generator=torch.Generator().manual_seed(1)).to(dev)
+    wp, bp = ops.pack_qkv_window_attn(rnd((3 * heads * d, K), 0.05, 136, dev), rnd((3 * heads * d,), 0.02, 137, dev), heads)
+    kw = {"inline": {"norm_inline": True, "norm_eps": 1e-6}, "array": {"a_row_sumsq": ops.row_sumsq(x), "norm_eps": 1e-6}, "plain": {}}[form]
+    run = lambda h: ops.qkv_window_attn(x, wp, bp, cos, heads, d**-0.5, win_start=win_start, prefetch=h, **kw)  # noqa: E731
+    plain = run(None)
+    for n in (16, 1 << 10, 1000016, 40 << 20):
+        assert torch.equal(run(torch.zeros(n, dtype=torch.uint8, device=dev)), plain), n
+
+
+@pytest.mark.parametrize("M,N,K", [
     (8192, 3072, 192),    # 256x128 (128x192 with an activation): three-stage ring with byte-wide W tiles, 3 K tiles
     (8192, 2304, 256),    # 224x192, 128x192 with a residual or an activation
     (1000, 1280, 320),    # 128x192; 128x160 with a residual
