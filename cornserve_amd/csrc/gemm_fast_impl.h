@@ -176,11 +176,26 @@ constexpr bool ring_takes_edges() {
 // piece, in the tail of the K loop, cost every tile, edge or not; elsewhere an edge is one uniform branch a tile.  With -> without,
 // 128x160 tiles: 2048 x 1280 x 1280 16.7 -> 16.4 us, fp8 weights 21.6 -> 20.9, 4096 x 1280 x 1280 with row sums 21.0 -> 19.8; 256x160:
 // 8192 x 1280 x 3456 62.4 -> 61.3.
+// Full launches read their prefetch hint (CsGemmArgs.prefetch) with the ring, but for the products whose residual piece needs it then
+// and the window blocks, which have no registers left.  Weights that come from HBM cost a launch of 4096 rows 2 to 10 us (1152 x 4352:
+// 42.7 us with them in the caches, 49.5 without, 53 in a pass); SigLIP's qkv and fc1 products hint those behind them: one 896x896
+// image 6.93 -> 6.66 ms, one 768x1152 image in tiles 6.02 -> 5.76.  At most HINT_MAX_BYTES, which travel in the last iterations.
+constexpr int HINT_PITCH = 3 * 128;
+constexpr int64_t HINT_MAX_BYTES = 16 << 20;
+template <int BM, int BN, int WAVES_M, int WAVES_N, int EPI, bool W_FP8, int FUSE, bool SPLIT_RES>
+constexpr bool ring_reads_hint() {
+  return EPI != CS_EPI_QKV_WATTN && EPI != CS_EPI_QKV_WATTN_RAGGED &&
+         !residual_piece_through_ring<BM, BN, WAVES_M, WAVES_N, EPI, W_FP8, FUSE, SPLIT_RES>();
+}
+CS_DEVICE __amdgpu_buffer_rsrc_t hint_descriptor(const char* base, int bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, bytes, 0x00020000);
+}
 template <int BM, int BN, int WAVES_M, int WAVES_N, int EPI, bool W_FP8, int FUSE, bool SPLIT_RES, bool EDGES>
-__global__ __launch_bounds__(64 * NW) void gemm_fast_kernel(const CsGemmArgs p) {
+__global__ __launch_bounds__(64 * NW) void gemm_fast_kernel(const CsGemmArgs p, const int hint_rows) {
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   static_assert(WAVES_M * WAVES_N == NW, "four waves, one per SIMD");
   using Ring = RingShape<BM, BN, W_FP8>;
+  constexpr bool RING_HINT = ring_reads_hint<BM, BN, WAVES_M, WAVES_N, EPI, W_FP8, FUSE, SPLIT_RES>();
   constexpr bool WATTN = EPI == CS_EPI_QKV_WATTN || EPI == CS_EPI_QKV_WATTN_RAGGED, RAGGED = EPI == CS_EPI_QKV_WATTN_RAGGED;
   constexpr int A_BYTES = Ring::A_BYTES, W_BYTES = Ring::W_BYTES;
   constexpr bool RING5 = Ring::FIVE_UNITS;
@@ -306,8 +321,8 @@ __global__ __launch_bounds__(64 * NW) void gemm_fast_kernel(const CsGemmArgs p) 
       }
     }
   };
-  const __amdgpu_buffer_rsrc_t rsrc_a = __builtin_amdgcn_make_buffer_rsrc((void*)p.A, 0, -1, 0x00020000);
-  const __amdgpu_buffer_rsrc_t rsrc_w = __builtin_amdgcn_make_buffer_rsrc((void*)p.W, 0, -1, 0x00020000);
+  __amdgpu_buffer_rsrc_t rsrc_a = __builtin_amdgcn_make_buffer_rsrc((void*)p.A, 0, -1, 0x00020000);
+  __amdgpu_buffer_rsrc_t rsrc_w = __builtin_amdgcn_make_buffer_rsrc((void*)p.W, 0, -1, 0x00020000);
   // Descriptors of what the epilogue's fast form reads and writes, each ending with its matrix's last element, so that row tails need
   // no guards: a row of C past the last one starts at or behind the end whatever its column (p.fast_epilogue: ldc is at least
   // the width), and what a lane would store there is dropped; residual rows past the last one read zeros, or -- where rows share
@@ -469,6 +484,10 @@ __global__ __launch_bounds__(64 * NW) void gemm_fast_kernel(const CsGemmArgs p) 
   for (;;) {
     const int vb_next = vb + gridDim.x;
     const bool has_next = !PRE && vb_next < ntiles;
+    // Behind a workgroup's last tile the ring runs on into its share of the prefetch hint (hint_rows_of): rows of HINT_PITCH bytes, of
+    // which K tile t of "the next tile" is bytes 128 t .. + 127, eight lanes to a row.  Nobody reads what arrives.
+    const bool reads_hint = RING_HINT && !has_next && hint_rows > 0;
+    const bool more = has_next || reads_hint;   // (whether the last iterations have something to request)
     int m0_next = 0, n0_next = 0;
     // ---- Residual GEMMs on the split 16-bit stream (the ring-fed forms; a wave has WTN of the tile's columns).  Their
     //      epilogue reads a tile-sized piece of the residual stream, three bytes per value, that nothing has touched
@@ -592,6 +611,19 @@ __global__ __launch_bounds__(64 * NW) void gemm_fast_kernel(const CsGemmArgs p) 
           tile_origin(vb_next, m0_next, n0_next);
           setup_sources(m0_next, n0_next);
         }
+        if constexpr (RING_HINT) {
+          if (reads_hint) {
+            const int first = (int)blockIdx.x * hint_rows, rows = min(max((int)((uint32_t)p.prefetch_bytes / HINT_PITCH) - first, 0), hint_rows);
+            rsrc_a = rsrc_w = hint_descriptor((const char*)p.prefetch + (int64_t)first * HINT_PITCH, rows * HINT_PITCH);
+            int lane_s = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+            asm volatile("" : "+v"(lane_s));
+            const uint32_t off = (uint32_t)((wave * (W_FP8 ? A_LD : NLD) * 8 + (lane_s >> 3)) * HINT_PITCH + (lane_s & 7) * 16);
+#pragma unroll
+            for (int j = 0; j < A_LD; ++j) a_src[j] = off + j * (8 * HINT_PITCH);
+#pragma unroll
+            for (int j = 0; j < W_LD; ++j) w_src[j] = W_FP8 ? OUTSIDE : off + (A_LD + j) * (8 * HINT_PITCH);
+          }
+        }
       };
       if constexpr (SWITCH_BEFORE_A) switch_sources();
       __builtin_amdgcn_sched_barrier(0);
@@ -602,7 +634,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_fast_kernel(const CsGemmArgs p) 
         if constexpr (N < EA * PA && N % EA == EA - 1) {
           auto ld = [&]() { direct_load(k_a, a_base_of(AHEAD_A, ring), w_base_of(AHEAD_A, ring), ic<PA_FIRST + N / EA>{}); };
           if constexpr (CUR_A) ld();
-          else if (has_next) ld();
+          else if (more) ld();
         }
         // the rest of row block 0 (second-last iteration) / row block 1 (last): their slot was the current one an
         // iteration ago
@@ -617,7 +649,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_fast_kernel(const CsGemmArgs p) 
       // outstanding, and this wave has received its last fragments of K tile kt.
       if constexpr (TAIL == 1) {
         __builtin_amdgcn_s_waitcnt(WAITCNT_LGKM0);  // nothing more is read from LDS for this output tile
-      } else if (!CUR_A && !has_next) {
+      } else if (!CUR_A && !more) {
         // nothing was requested after K tile kt+1 -- except row block 0 of the residual piece, which may stay in flight
         if (PRE && pre_on) __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(PRE ? PRE_N0 : 0));
         else __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(0));
@@ -635,7 +667,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_fast_kernel(const CsGemmArgs p) 
         if constexpr (N < EB * PB && N % EB == EB - 1) {
           auto ld = [&]() { direct_load(k_b, a_base_of(AHEAD_B, ring), w_base_of(AHEAD_B, ring), ic<PB_FIRST + N / EB>{}); };
           if constexpr (CUR_B) ld();
-          else if (has_next) ld();
+          else if (more) ld();
         }
         // the residual piece: first loads of row block 0 (third-last iteration) / row
         // block 1 (second-last) into the slot that the barrier has just freed (the tile requests no K tile any more)
@@ -1404,6 +1436,8 @@ __global__ __launch_bounds__(64 * NW) void gemm_fast_kernel(const CsGemmArgs p) 
     m0 = m0_next;
     n0 = n0_next;
   }
+  // (the LDS that loads in flight write must stay this workgroup's)
+  if (RING_HINT && hint_rows > 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
 
 template <int BM, int BN, int WAVES_M, int WAVES_N, int EPI, bool W_FP8, int FUSE, bool SPLIT_RES, bool EDGES>
@@ -1421,10 +1455,21 @@ int launch_kernel(CsGemmArgs& p, hipStream_t stream) {
   // One resident workgroup per CU (LDS-bound); with more tiles than CUs the kernel is persistent.
   // (but a workgroup per tile where the residual piece passes through the ring: see the kernel's tile loop)
   int grid = tiles <= 256 || residual_piece_through_ring<BM, BN, WAVES_M, WAVES_N, EPI, W_FP8, FUSE, SPLIT_RES>() ? tiles : 256;
-  // few tiles and a prefetch hint: the idle compute units read the hinted bytes (see the kernel)
-  if (p.prefetch && p.prefetch_bytes >= 16 && tiles <= 192) grid = tiles + (256 - tiles < 128 ? 256 - tiles : 128);
-  else p.prefetch = nullptr;
-  hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * NW), lds, stream, p);
+  // a prefetch hint: with few tiles the idle compute units read it, else the workgroups behind their last tile (see the kernel), of
+  // a hint as much as travels in its last iterations
+  int hint_rows = 0;
+  if (!p.prefetch || p.prefetch_bytes < 16) {
+    p.prefetch = nullptr;
+  } else if (tiles <= 192) {
+    grid = tiles + (256 - tiles < 128 ? 256 - tiles : 128);
+  } else if (ring_reads_hint<BM, BN, WAVES_M, WAVES_N, EPI, W_FP8, FUSE, SPLIT_RES>()) {
+    // rows that a workgroup's loads cover (with fp8 weights those of the activations: the others' rows are half as wide)
+    constexpr int most = (BM / 8 + (W_FP8 ? 0 : (BN / 8 + NW - 1) / NW * NW)) * 8;
+    if (p.prefetch_bytes > HINT_MAX_BYTES) p.prefetch_bytes = HINT_MAX_BYTES;
+    hint_rows = (int)((p.prefetch_bytes / HINT_PITCH + grid - 1) / grid);
+    if (hint_rows > most) hint_rows = most;
+  }
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * NW), lds, stream, p, hint_rows);
   return cs_launch_status();
 }
 

@@ -156,6 +156,8 @@ class SiglipEncoderBase(EricModel):
     `_init_tower(fold_norm)`."""
     # the residual stream (siglip.py:178,188) is carried with 16 significant bits, as in Qwen2_5_VisionTransformer
     split_residual: bool = True
+    # batches of at most this many rows pass weight-prefetch hints (12288 rows: 18.6 -> 18.65 ms with them)
+    prefetch_rows = 8192
 
     def _init_tower(self, fold_norm: bool) -> None:
         vc = self.config.vision_config
@@ -220,6 +222,10 @@ class SiglipEncoderBase(EricModel):
                 w, b, cs = fold_layernorm(lyr.mlp.fc1.weight, lyr.mlp.fc1.bias, *entry["ln2"])
                 # pad AFTER folding: the pad rows stay exactly zero (weight, bias and column sum)
                 entry["fc1"], entry["fc1_colsum"] = (pad_rows(w), pad_rows(b)), pad_rows(cs)
+            # one buffer for the weights of the two products behind the attention: the qkv product hints both at once
+            entry["hint"] = torch.cat([entry["out"][0], entry["fc1"][0]])
+            entry["out"] = (entry["hint"][:H], entry["out"][1])
+            entry["fc1"] = (entry["hint"][H:], entry["fc1"][1])
             layers.append(entry)
         return {"pe_w": pe_w, "pe_b": vm.embeddings.patch_embedding.bias, "kp": kp, "ip": ip,
                 "pos": vm.embeddings.position_embedding.weight, "layers": layers,
@@ -274,21 +280,24 @@ class SiglipEncoderBase(EricModel):
             sm = torch.zeros_like(ss)
             ops.row_stats(x, ss, sm, chunk_order=True)
             stats_out.update(c_row_sumsq=ss, c_row_sum=sm)
+        # weights that nothing has touched since the previous pass come from HBM: a launch in front has them read (CsGemmArgs.prefetch)
+        hint = M <= self.prefetch_rows
         for lyr in pk["layers"]:
+            pf_qkv, pf_fc1 = (lyr["hint"], lyr["fc2"][0]) if hint else (None, None)
             if fold:
                 ops.gemm(x, lyr["qkv_w"], lyr["qkv_b"], out=qkv, a_row_sumsq=ss, a_row_sum=sm,
-                         w_col_sum=lyr["qkv_colsum"], norm_eps=eps)
+                         w_col_sum=lyr["qkv_colsum"], norm_eps=eps, prefetch=pf_qkv)
             else:
                 ops.layernorm(x, *lyr["ln1"], eps, out=n)
-                ops.gemm(n, lyr["qkv_w"], lyr["qkv_b"], out=qkv)
+                ops.gemm(n, lyr["qkv_w"], lyr["qkv_b"], out=qkv, prefetch=pf_qkv)
             ops.attn_varlen(qkv[:, :H], qkv[:, H : 2 * H], qkv[:, 2 * H :], plan, nh, d, d**-0.5, out=att)
             ops.gemm(att, *lyr["out"], epilogue=ops.EPI_RESIDUAL, residual=x, out=x, **stats_out)
             if fold:
                 ops.gemm(x, *lyr["fc1"], epilogue=epi, out=hmid, a_row_sumsq=ss, a_row_sum=sm,
-                         w_col_sum=lyr["fc1_colsum"], norm_eps=eps)
+                         w_col_sum=lyr["fc1_colsum"], norm_eps=eps, prefetch=pf_fc1)
             else:
                 ops.layernorm(x, *lyr["ln2"], eps, out=n)
-                ops.gemm(n, *lyr["fc1"], epilogue=epi, out=hmid)
+                ops.gemm(n, *lyr["fc1"], epilogue=epi, out=hmid, prefetch=pf_fc1)
             ops.gemm(hmid, *lyr["fc2"], epilogue=ops.EPI_RESIDUAL, residual=x, out=x, **stats_out)
         if pk["post"] is None:
             return x.view(B, tokens, H)

@@ -116,9 +116,13 @@ class QwenVisionBase(EricModel):
     `forward_device`, `chunk_shape` and the attributes patch_size, temporal_patch_size, spatial_merge_size,
     in_channels, weight_format and patch_embed."""
 
-    # Batches of at most this many patches pass the GEMM launches a weight-prefetch hint (0: never): such launches
-    # leave compute units idle, and those read the weights a later launch of the block needs into the last-level cache.
-    prefetch_rows = 6144
+    # Batches of at most this many patches pass the GEMM launches a weight-prefetch hint (0: never): idle compute units, or the ring of
+    # a full launch behind its last tile, read the weights a later launch of the block needs into the last-level cache.  Beyond it
+    # nothing is gained (12288 patches of Qwen2-VL 24.2 -> 24.35 ms with hints).
+    prefetch_rows = 8192
+    # Up to this many rows (192 tiles of 128x160) the output projection has the last MLP weights read; beyond it the product in front
+    # of the last one does.
+    proj_hint_rows = 3072
 
     # what the checkpoint's image processor normalises with (preprocessor_config.json): CLIP statistics for
     # Qwen2-VL and Qwen2.5-VL; subclasses override
@@ -557,12 +561,10 @@ class Qwen2_5_VisionTransformer(QwenVisionBase):
 
         # rows [0, fused_rows) belong to the items whose window blocks run as one launch, the rest to the others
         xf = x[:fused_rows]
-        # A batch of few rows leaves compute units idle in the N = hidden GEMMs, and what bounds those launches is
-        # the latency of weights that nothing has touched since the previous forward pass: the one-launch window block
-        # has its idle units read the gate|up weights, the attention-output projection the down-projection's, the
-        # down-projection the next block's qkv weights.  (A launch of more than 192 tiles reads none: those of 1024 rows have
-        # 224 to 256 small ones; one of the few-row kernel reads what fits its own time.  3072 patches 5.39 -> 5.02 ms, 1280
-        # 3.87 -> 3.57, 96 1.82 -> 1.80, 1024 the same.)
+        # What bounds a launch of few rows is the latency of weights that nothing has touched since the previous forward pass: the
+        # one-launch window block reads the gate|up weights, the attention-output projection (from `proj_hint_rows` on, gate|up) the
+        # down-projection's, the down-projection the next block's qkv and projection weights.  (3072 patches 5.39 -> 5.02 ms, 1280
+        # 3.87 -> 3.57, 1024 2.92 -> 2.75, 4096 6.04 -> 5.82.)
         hint = L <= self.prefetch_rows
 
         def next_qkv(i: int) -> torch.Tensor | None:
@@ -580,6 +582,7 @@ class Qwen2_5_VisionTransformer(QwenVisionBase):
             pf_qkv = b["gu"]["w"] if hint else None   # (from the one-launch window block only: the plain QKV GEMM of a
             # small batch leaves too few compute units idle to read 18 MB in its own time -- measured slower)
             pf_proj = b["down"]["w"] if hint else None
+            pf_gu = b["down"]["w"] if hint and L > self.proj_hint_rows else None
             pf_down = next_qkv(i) if hint else None
             if not full and fused_rows:
                 wp, bp, *sp = b["qkv_wattn"]      # (a third entry with fp8 weights: their scales)
@@ -612,7 +615,7 @@ class Qwen2_5_VisionTransformer(QwenVisionBase):
                 self._g(att, b["proj"], epilogue=ops.EPI_RESIDUAL, residual=x, out=x, c_row_sumsq=None if inline_mlp else ss,
                         prefetch=pf_proj, **res)
                 mark("gemm_gate_up")
-                self._g(x, b["gu"], epilogue=ops.EPI_SWIGLU, out=hmid, **norm(inline_mlp, slice(0, R)))
+                self._g(x, b["gu"], epilogue=ops.EPI_SWIGLU, out=hmid, prefetch=pf_gu, **norm(inline_mlp, slice(0, R)))
                 mark("gemm_down")
                 self._g(hmid, b["down"], epilogue=ops.EPI_RESIDUAL, residual=x, out=x,
                         c_row_sumsq=ss if attn_reads_sums(i + 1) else None, prefetch=pf_down, **res)

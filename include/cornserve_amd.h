@@ -129,17 +129,17 @@ typedef struct CsGemmArgs {
   /* cs_qkv_window_attn only, set by the caller: windows of fewer than 64 rows (see there); NULL / 0 otherwise         */
   const int32_t* attn_win_start;
   int32_t attn_n_win;
-  /* Optional hint for launches that leave compute units idle (at most 192 tiles of the direct-to-LDS kernels, cs_gemm and
-   * cs_qkv_window_attn alike): prefetch_bytes bytes at prefetch (16-byte aligned) -- typically the weights of the NEXT
-   * launch, which no kernel has touched since the previous forward pass -- are read once by up to 128 workgroups
-   * started next to the computing ones, so that they sit in the last-level cache when the next launch asks for them
-   * (such a launch is bound by operand latency, not by arithmetic).  Results are not affected; the hint is ignored
-   * by launches that fill the chip and by the general kernel.  NULL / 0: no hint.  A prefetching workgroup moves
-   * about 8 KB per microsecond and the launch ends when its last workgroup does.  The few-row kernel reads of the hint,
-   * from its start, what fits the launch's own time; with more than 192 tiles its computing workgroups read up to 32 MB of it behind
-   * their last K stage (bf16 W).  The big tiles read all of it: hint what the idle compute units
-   * (256 minus the launch's tiles, at most 128) can read in that time -- 9 MB behind a 64-tile launch of 20 K tiles costs
-   * nothing, 18 MB behind a 192-tile one doubles its duration.                                                        */
+  /* Optional hint (direct-to-LDS kernels, cs_gemm and cs_qkv_window_attn alike): prefetch_bytes bytes at prefetch (16-byte
+   * aligned) -- typically the weights of the NEXT launch, which no kernel has touched since the previous forward pass -- are
+   * read once, so that they sit in the last-level cache when the next launch asks for them (such a launch is bound by operand
+   * latency, not by arithmetic).  Results are not affected; the general kernel ignores the hint.  NULL / 0: no hint.
+   * With at most 192 tiles up to 128 workgroups are started for it next to the computing ones, on idle compute units.  A
+   * prefetching workgroup moves about 8 KB per microsecond and the launch ends when its last workgroup does.  The few-row
+   * kernel reads of the hint, from its start, what fits the launch's own time.  The big tiles read all of it: hint what the
+   * idle compute units (256 minus the launch's tiles, at most 128) can read in that time -- 9 MB behind a 64-tile launch of 20
+   * K tiles costs nothing, 18 MB behind a 192-tile one doubles its duration.
+   * With more tiles the computing workgroups read a share each behind their last K tile: the few-row kernel up to 32 MB
+   * (bf16 W; not in 128x128 tiles), the big tiles up to 16 MB (not ring-fed residual products or cs_qkv_window_attn).      */
   const void* prefetch;
   int64_t prefetch_bytes;
   /* Folded norm without the row-sum arrays: with a_norm_inline = 1 the sums over the rows of A are taken inside the

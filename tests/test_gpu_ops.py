@@ -684,6 +684,56 @@ def test_gemm_row_split_gives_the_bits_of_one_launch(ops, dev, M, N, K, epi, kin
     assert all(torch.equal(x, y) for r in results[1:] for x, y in zip(r, results[0]))
 
 
+# A launch of more than 192 tiles reads its hint with the ring behind every workgroup's last tile (ring-fed residual products and the
+# general epilogue's launches leave it alone): the bits of the launch without a hint, in every form, with one tile a workgroup and
+# several, at edges, with hints from less than a row of it to more than all workgroups read.
+@pytest.mark.parametrize("M,N,K", [(4096, 3456, 192), (4097, 3464, 256), (7290, 5120, 320)])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_full_launches_read_their_hint_with_the_ring(ops, dev, M, N, K, fp8):
+    import ctypes
+
+    from cornserve_amd import lib
+
+    a, w, b = rnd((M, K), 1.0, 251, dev), rnd((N, K), 0.05, 252, dev), rnd((N,), 0.02, 253, dev)
+    res, lo = rnd((M, N), 1.0, 254, dev), torch.zeros((M, N), dtype=torch.uint8, device=dev)
+    sc = (w.float().abs().amax(1) / 448.0).contiguous()
+    wq = (w.float() / sc[:, None]).to(torch.float8_e4m3fn).view(torch.uint8) if fp8 else w
+    ss, sm = torch.empty((M, ops.SUMSQ_PARTS), device=dev), torch.empty((M, ops.SUMSQ_PARTS), device=dev)
+    ops.row_stats(a, ss, sm)
+    csum = w.float().sum(1)
+    hints = [torch.zeros(n, dtype=torch.uint8, device=dev) for n in (16, 1 << 10, 1000016, 40 << 20)]
+    cases = [(ops.EPI_BIAS, ""), (ops.EPI_SWIGLU, ""), (ops.EPI_GELU_TANH, ""), (ops.EPI_RESIDUAL, ""), (ops.EPI_RESIDUAL, "split")]
+    if not fp8:
+        cases += [(ops.EPI_BIAS, "rms"), (ops.EPI_SWIGLU, "rms"), (ops.EPI_BIAS, "ln"), (ops.EPI_QUICK_GELU, "ln")]
+    runs = {name: _big_form(name) for name in BIG_FORMS}
+    for epi, kind in cases:
+        for name, run in runs.items():
+            want = None
+            for h in (None, *hints):
+                out, out_lo = torch.empty((M, N // 2 if epi == ops.EPI_SWIGLU else N), dtype=torch.bfloat16, device=dev), torch.zeros_like(lo)
+                g = lib.CsGemmArgs()
+                g.A, g.W, g.C, g.bias, g.M, g.N, g.K, g.lda, g.ldw, g.ldc, g.epilogue = (
+                    a.data_ptr(), wq.data_ptr(), out.data_ptr(), b.data_ptr(), M, N, K, K, K, out.shape[1], epi)
+                if fp8:
+                    g.w_fp8, g.w_scale = 1, sc.data_ptr()
+                if epi == ops.EPI_RESIDUAL:
+                    g.residual, g.ldr = res.data_ptr(), N
+                if kind == "split":
+                    g.c_lo, g.residual_lo = out_lo.data_ptr(), lo.data_ptr()
+                if kind in ("rms", "ln"):
+                    g.a_row_sumsq, g.norm_eps = ss.data_ptr(), 1e-6
+                if kind == "ln":
+                    g.a_row_sum, g.w_col_sum = sm.data_ptr(), csum.data_ptr()
+                if h is not None:
+                    g.prefetch, g.prefetch_bytes = h.data_ptr(), h.numel()
+                status = run(ctypes.byref(g), torch.cuda.current_stream().cuda_stream)
+                assert status in (0, 2), (name, epi, kind, status)
+                if status:
+                    break
+                want = want or (out, out_lo)
+                assert torch.equal(out, want[0]) and torch.equal(out_lo, want[1]), (name, epi, kind, h.numel())
+
+
 # A residual whose rows share memory (one row broadcast; rows that overlap) is the residual that a copy of it would be, in every
 # kernel and form: ring-fed and direct epilogues, whole tiles and both edges, the few-row kernel (K a multiple of 128, 200 rows)
 # and the general one (K = 80).
