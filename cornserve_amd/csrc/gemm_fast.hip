@@ -158,9 +158,12 @@ Plan plan_of(const CsGemmArgs& a) {
       const double lead_us = form_us(f, part_of(a, 0, lead, 0, a.N), a.N);
       if (lead_us >= split.us) continue;
       const CsGemmArgs rest = part_of(a, lead, a.M - lead, 0, a.N);
-      double t = FEW_ROW_TAIL * cs_gemm_small_us(rest);
-      const BigForm* form = nullptr;
-      if (t == 0) form = best_form(rest, a.N, &t);
+      double t, few = FEW_ROW_TAIL * cs_gemm_small_us(rest);
+      const BigForm* form = best_form(rest, a.N, &t);
+      if (few > 0 && few < t) {
+        t = few;
+        form = nullptr;
+      }
       t += lead_us + (tight(f) ? 0.0 : ROW_SPLIT_US);
       if (t < (split.lead_cols ? 0.97 : 1.0) * split.us) split = {form, 0, t, lead, &f};
     }

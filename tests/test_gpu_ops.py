@@ -974,6 +974,38 @@ def test_qkv_window_attn_few_windows_equal_many(ops, dev, windows, heads, ragged
     assert torch.equal(got, want)
 
 
+@pytest.mark.parametrize("windows,more,heads,ragged,form", [(65, 81, 16, False, "array"), (80, 81, 16, True, "array"), (144, 145, 16, False, "plain"),
+                                                            (68, 81, 16, True, "fp8"), (345, 426, 3, True, "plain")])
+def test_qkv_window_attn_windows_behind_the_last_round(ops, dev, windows, more, heads, ragged, form):
+    """Windows behind the last whole round of big tiles, few enough for a workgroup per window and head, take a second launch: the
+    bits of a launch of a few windows more, which are too many for that."""
+    K, d = 1280, 80
+    g = torch.Generator().manual_seed(windows)
+    counts = torch.randint(1, 17, (more,), generator=g) * 4 if ragged else torch.full((more,), 64)
+    cu = torch.cat([torch.zeros(1, dtype=torch.int64), counts.cumsum(0)]).int().to(dev)
+    M, rows = int(counts.sum()), int(counts[:windows].sum())
+    x, w, b = rnd((M, K), 1.0, 141, dev), rnd((3 * heads * d, K), 0.05, 142, dev), rnd((3 * heads * d,), 0.02, 143, dev)
+    cos = torch.rand((M, d), generator=g).to(dev)
+    kw = {"norm_eps": 1e-6} if form == "array" else {}
+    if form == "fp8":
+        sc = (w.float().abs().amax(1) / 448.0).contiguous()
+        wp, bp, sp = ops.pack_qkv_window_attn((w.float() / sc[:, None]).to(torch.float8_e4m3fn), b, heads, w_scale=sc)
+        kw["w_scale"] = sp
+    else:
+        wp, bp = ops.pack_qkv_window_attn(w, b, heads)
+    ss = ops.row_sumsq(x)
+
+    def run(n, m):
+        sums = {"a_row_sumsq": ss[:m]} if form == "array" else {}
+        out = torch.full((M + 1, heads * d), 7.0, dtype=torch.bfloat16, device=dev)
+        ops.qkv_window_attn(x[:m], wp, bp, cos[:m], heads, d**-0.5, out=out[:m], win_start=cu[: n + 1].contiguous() if ragged else None,
+                            prefetch=torch.zeros(1 << 20, dtype=torch.uint8, device=dev), **kw, **sums)
+        assert bool((out[m:] == 7).all())
+        return out[:rows]
+
+    assert torch.equal(run(windows, rows), run(more, M))
+
+
 @pytest.mark.parametrize("form,rows", [("inline", 4), ("plain", 128), ("array", 132), ("inline", 256), ("inline", 260), ("array", 512),
                                        ("plain", 508), ("inline", 516), ("fp8", 128)])
 def test_qkv_window_attn_two_launches_equal_one(ops, dev, form, rows):
