@@ -154,15 +154,15 @@ int cs_gemm_small_workgroups(const CsGemmArgs& a) {
   return tiles + (p.prefetch ? csgemm::hint_workgroups(tiles) : 0);
 }
 
-// One workgroup per window and head while the chip holds them all at once: 24 to 26 us up to 16 windows of 16 heads (inline norm,
-// weights from HBM; 21 to 23 without norm), where a big tile (four windows) takes 32 to 35 us whatever the count; with a second
+// One workgroup per window and head while the chip holds them all at once: 23 to 25 us up to 16 windows of 16 heads (inline norm,
+// weights from HBM; 21 to 24 without norm), where a big tile (four windows) takes 32 to 35 us whatever the count; with a second
 // round (24 windows: 39 us) it is the slower.  (The first 512 rows of bf16 weights go to two launches where there is a workspace, see
 // below.)
 bool cs_qkv_window_attn_few(int64_t windows, int heads, int K) { return K % 128 == 0 && windows * heads <= 256; }
 
 // Of these the ones that two launches over a workspace serve better (gemm_small_qkv_wattn.hip): while the projection's tiles are
-// one round.  One launch | two, 16 heads, K = 1280, weights from HBM, inline norm: 96 rows 25.4 | 15.7 us, 256 25.4 | 17.7, 320
-// 25.3 | 21.1, 512 25.1 | 22.6 (64x128 tiles from 257 rows on); whole passes of Qwen2.5-VL, 256 patches 2.10 | 1.86 ms, 576 2.71 |
+// one round.  One launch | two, 16 heads, K = 1280, weights from HBM, inline norm: 128 rows 24.8 | 16.0 us, 256 24.0 | 18.0, 320
+// 23.7 | 21.3, 512 23.5 | 23.0 (64x128 tiles from 257 rows on); when one launch took 25.1 to 25.4, whole passes of Qwen2.5-VL, 256 patches 2.10 | 1.86 ms, 576 2.71 |
 // 2.66.  Not with fp8 weights, half the bytes: 96 rows 14.8 | 12.9 us, 192 14.8 | 14.8, and at up to 128 rows, where it would be
 // faster, a pass lasts as long as the host takes to launch it (1.87 | 1.90 ms).
 bool cs_qkv_window_attn_two_pays(int64_t rows, int64_t windows, int heads, int K, bool w_fp8) {

@@ -66,11 +66,11 @@ int launch_projection(const CsGemmArgs& p, int bm, int bn, hipStream_t stream) {
 
 }  // namespace
 
-// The same in two launches over a workspace of rows x a.N floats.  With one workgroup per window and head a launch lasts 24 to 26
+// The same in two launches over a workspace of rows x a.N floats.  With one workgroup per window and head a launch lasts 23 to 25
 // us however few they are: each of them has 800 KB of operands to take in, and most of the chip is idle.  Here the projection
 // runs in few-row tiles, whose columns fill the chip, and the kernel above does the rest; the values between are fp32 (the
-// rotary takes unrounded ones) and every one is computed by the same operations, so the bits are the same.  96 rows 25.4 -> 15.7
-// us, 256 25.4 -> 17.7; an image of 96 patches through the encoder 1.77 -> 1.49 ms.
+// rotary takes unrounded ones) and every one is computed by the same operations, so the bits are the same.  128 rows 24.8 -> 16.0
+// us, 256 24.0 -> 18.0; an image of 96 patches through the encoder 1.77 -> 1.49 ms.
 int cs_qkv_window_attn_two(const CsGemmArgs& a, int rows, int windows, float* x, hipStream_t stream) {
   CsGemmArgs p = a;
   p.M = rows;

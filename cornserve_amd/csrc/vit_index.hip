@@ -23,8 +23,8 @@ struct ItemMeta {  // matches the int32[8] record documented in cornserve_amd.h
 };
 
 // Bound by the sines and cosines, 80 of them a patch with heads of 80: a lane computes the four of one frequency (with one thread
-// per patch an image of 1024 patches, four workgroups, took 15.6 us: a chain of 80 calls).  96 patches 10.4 -> 4.5 us, 1024 15.6 ->
-// 6.1, 58648 40 -> 19.
+// per patch an image of 1024 patches, four workgroups, took 15.5 us: a chain of 80 calls).  96 patches 10.2 -> 4.7 us, 1024 15.5 ->
+// 5.0, 58648 42 -> 20.
 constexpr int INDEX_LANES = 32, INDEX_PATCHES = 8;   // lanes of a patch, patches of a workgroup
 __global__ __launch_bounds__(INDEX_LANES * INDEX_PATCHES) void vit_index_kernel(const ItemMeta* __restrict__ meta, int merge, int win,
                                                         const float* __restrict__ inv_freq, int rot_dim,
