@@ -53,6 +53,7 @@
 #include <utility>
 
 #include "gemm_common.h"
+#include "hint_ring.h"
 
 namespace {
 
@@ -179,8 +180,9 @@ constexpr bool ring_takes_edges() {
 // Full launches read their prefetch hint (CsGemmArgs.prefetch) with the ring, but for the products whose residual piece needs it then
 // and the window blocks, which have no registers left.  Weights that come from HBM cost a launch of 4096 rows 2 to 10 us (1152 x 4352:
 // 42.7 us with them in the caches, 49.5 without, 53 in a pass); SigLIP's qkv and fc1 products hint those behind them: one 896x896
-// image 6.93 -> 6.66 ms, one 768x1152 image in tiles 6.02 -> 5.76.  At most HINT_MAX_BYTES, which travel in the last iterations.
-constexpr int HINT_PITCH = 3 * 128;
+// image 6.93 -> 6.66 ms, one 768x1152 image in tiles 6.02 -> 5.76.  At most HINT_MAX_BYTES, which travel in the last iterations, and
+every byte of a workgroup's share (hint_ring.h).  While the share's rows had a third segment, of which the five-unit ring requests nothing and
+the three-stage one half: one 896x896 image 7.00 -> 6.91 ms, five 384x384 tiles 4.72 -> 4.62, Qwen2-VL 3136 patches 7.82 -> 7.74.
 constexpr int64_t HINT_MAX_BYTES = 16 << 20;
 template <int BM, int BN, int WAVES_M, int WAVES_N, int EPI, bool W_FP8, int FUSE, bool SPLIT_RES>
 constexpr bool ring_reads_hint() {
@@ -452,11 +454,10 @@ __global__ __launch_bounds__(64 * NW) void gemm_fast_kernel(const CsGemmArgs p, 
   // Five-unit ring: A(kt+2) in the first half, W(kt+2) in the second (same K tile, AHEAD_B == AHEAD_A).
   // Three-stage ring: the second portion of K tile kt+2 in the first half, the first portion of K tile kt+3
   // in the second half.
-  constexpr int PA = RING5 ? A_LD : NLD - NLD / 2;  // loads issued in a first half
-  constexpr int PB = NLD - PA;                       // loads issued in a second half
-  constexpr int PA_FIRST = RING5 ? 0 : PB;           // index of the first load of the first-half portion
-  constexpr int PB_FIRST = RING5 ? A_LD : 0;
-  constexpr int AHEAD_A = 2, AHEAD_B = RING5 ? 2 : 3;
+  constexpr cshint::BigRing LOADS = {A_LD, W_LD, RING5};
+  constexpr int PA = LOADS.pa(), PB = LOADS.pb();                           // loads issued in a first half, in a second half
+  constexpr int PA_FIRST = LOADS.pa_first(), PB_FIRST = LOADS.pb_first();   // ... the first of them
+  constexpr int AHEAD_A = LOADS.ahead_a(), AHEAD_B = LOADS.ahead_b();
   constexpr int EA = NMFMA / PA, EB = NMFMA / PB;    // MFMAs per direct load in each half
   static_assert(EA >= 1 && EB >= 1, "one slot after an MFMA per direct load");
   // Loads outstanding by design at the two wait points: everything issued after the K tile that is needed.
@@ -484,7 +485,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_fast_kernel(const CsGemmArgs p, 
   for (;;) {
     const int vb_next = vb + gridDim.x;
     const bool has_next = !PRE && vb_next < ntiles;
-    // Behind a workgroup's last tile the ring runs on into its share of the prefetch hint (hint_rows_of): rows of HINT_PITCH bytes, of
+    // Behind a workgroup's last tile the ring runs on into its share of the prefetch hint (hint_ring.h): rows of BIG_PITCH bytes, of
     // which K tile t of "the next tile" is bytes 128 t .. + 127, eight lanes to a row.  Nobody reads what arrives.
     const bool reads_hint = RING_HINT && !has_next && hint_rows > 0;
     const bool more = has_next || reads_hint;   // (whether the last iterations have something to request)
@@ -613,15 +614,14 @@ __global__ __launch_bounds__(64 * NW) void gemm_fast_kernel(const CsGemmArgs p, 
         }
         if constexpr (RING_HINT) {
           if (reads_hint) {
-            const int first = (int)blockIdx.x * hint_rows, rows = min(max((int)((uint32_t)p.prefetch_bytes / HINT_PITCH) - first, 0), hint_rows);
-            rsrc_a = rsrc_w = hint_descriptor((const char*)p.prefetch + (int64_t)first * HINT_PITCH, rows * HINT_PITCH);
+            const cshint::Share share = cshint::share_of((uint32_t)p.prefetch_bytes, cshint::BIG_PITCH, hint_rows, (int)blockIdx.x);
+            rsrc_a = rsrc_w = hint_descriptor((const char*)p.prefetch + (int64_t)share.first * cshint::BIG_PITCH, share.rows * cshint::BIG_PITCH);
             int lane_s = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
             asm volatile("" : "+v"(lane_s));
-            const uint32_t off = (uint32_t)((wave * (W_FP8 ? A_LD : NLD) * 8 + (lane_s >> 3)) * HINT_PITCH + (lane_s & 7) * 16);
 #pragma unroll
-            for (int j = 0; j < A_LD; ++j) a_src[j] = off + j * (8 * HINT_PITCH);
+            for (int j = 0; j < A_LD; ++j) a_src[j] = cshint::big_offset(LOADS, W_FP8, wave, j, lane_s);
 #pragma unroll
-            for (int j = 0; j < W_LD; ++j) w_src[j] = W_FP8 ? OUTSIDE : off + (A_LD + j) * (8 * HINT_PITCH);
+            for (int j = 0; j < W_LD; ++j) w_src[j] = W_FP8 ? OUTSIDE : cshint::big_offset(LOADS, W_FP8, wave, A_LD + j, lane_s);
           }
         }
       };
@@ -667,7 +667,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_fast_kernel(const CsGemmArgs p, 
         if constexpr (N < EB * PB && N % EB == EB - 1) {
           auto ld = [&]() { direct_load(k_b, a_base_of(AHEAD_B, ring), w_base_of(AHEAD_B, ring), ic<PB_FIRST + N / EB>{}); };
           if constexpr (CUR_B) ld();
-          else if (more) ld();
+          else if (AHEAD_B - TAIL < cshint::BIG_SEGMENTS ? more : has_next) ld();
         }
         // the residual piece: first loads of row block 0 (third-last iteration) / row
         // block 1 (second-last) into the slot that the barrier has just freed (the tile requests no K tile any more)
@@ -1463,11 +1463,9 @@ int launch_kernel(CsGemmArgs& p, hipStream_t stream) {
   } else if (tiles <= 192) {
     grid = tiles + (256 - tiles < 128 ? 256 - tiles : 128);
   } else if (ring_reads_hint<BM, BN, WAVES_M, WAVES_N, EPI, W_FP8, FUSE, SPLIT_RES>()) {
-    // rows that a workgroup's loads cover (with fp8 weights those of the activations: the others' rows are half as wide)
-    constexpr int most = (BM / 8 + (W_FP8 ? 0 : (BN / 8 + NW - 1) / NW * NW)) * 8;
+    constexpr cshint::BigRing loads = {BM / 8 / NW, (BN / (W_FP8 ? 16 : 8) + NW - 1) / NW, RingShape<BM, BN, W_FP8>::FIVE_UNITS};
     if (p.prefetch_bytes > HINT_MAX_BYTES) p.prefetch_bytes = HINT_MAX_BYTES;
-    hint_rows = (int)((p.prefetch_bytes / HINT_PITCH + grid - 1) / grid);
-    if (hint_rows > most) hint_rows = most;
+    hint_rows = cshint::rows_of(p.prefetch_bytes, cshint::BIG_PITCH, grid, cshint::big_rows(loads, W_FP8));
   }
   hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * NW), lds, stream, p, hint_rows);
   return cs_launch_status();

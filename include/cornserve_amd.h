@@ -139,7 +139,8 @@ typedef struct CsGemmArgs {
    * idle compute units (256 minus the launch's tiles, at most 128) can read in that time -- 9 MB behind a 64-tile launch of 20
    * K tiles costs nothing, 18 MB behind a 192-tile one doubles its duration.
    * With more tiles the computing workgroups read a share each behind their last K tile: the few-row kernel up to 32 MB
-   * (bf16 W; not in 128x128 tiles), the big tiles up to 16 MB (not ring-fed residual products or cs_qkv_window_attn).      */
+   * (bf16 W; not in 128x128 tiles), the big tiles up to 16 MB (fp8 W: 64 KB for each row of the tile form, 8 MB with 128; not
+   * ring-fed residual products or cs_qkv_window_attn), both from the hint's start and but for less than a KB at its end.   */
   const void* prefetch;
   int64_t prefetch_bytes;
   /* Folded norm without the row-sum arrays: with a_norm_inline = 1 the sums over the rows of A are taken inside the
