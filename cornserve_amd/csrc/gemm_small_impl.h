@@ -29,6 +29,7 @@
 #include <utility>
 
 #include "gemm_common.h"
+#include "hint_ring.h"
 
 namespace {
 
@@ -142,11 +143,11 @@ struct SmallShape {
   static constexpr int SUMS_BYTES = SUMS == SUMS_NONE ? 0 : BM * 16 * SUMS;
   static constexpr int LDS = STAGES * STAGE + NORM_BYTES + SUMS_BYTES;
   static_assert(LDS <= 160 * 1024, "the ring fits the LDS");
-  static constexpr int64_t NLD_OF(int waves) { return KS * (BM / 8) / waves + (KS * (BN * W_ROW / 1024) + waves - 1) / waves; }   // direct loads per wave and stage
+  static constexpr int NLD_OF(int waves) { return KS * (BM / 8) / waves + (KS * (BN * W_ROW / 1024) + waves - 1) / waves; }   // direct loads per wave and stage
   // A prefetch hint behind the last stage (see hint_rows_of): rows of one segment, as wide as a stage's step, per stage
   // (not in 128x128 tiles, with their launches of 20 us and more: the branch to it costs 0.8 % of them)
   static constexpr bool RING_HINT = !W_FP8 && BM * BN < 128 * 128;
-  static constexpr int HINT_SEG = KS * 128, HINT_STAGES = KS == 2 ? STAGES - 1 : STAGES - 2, HINT_PITCH = HINT_STAGES * HINT_SEG;
+  static constexpr int HINT_SEG = cshint::small_segment(KS), HINT_PITCH = cshint::small_segments(KS, STAGES) * HINT_SEG;
 };
 
 // What follows the projection in a window (see small_wattn_epilogue), 16 queries a wave: `qk(f)` is fragment f (0 .. 4 q, 5 .. 9
@@ -611,14 +612,12 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, EPI == SM_EPI_QKV_WATTN ? 1
   const bool reads_hint = Shape::RING_HINT && hint_rows > 0 && nst >= STAGES;
   auto switch_to_hint = [&]() {
     if constexpr (Shape::RING_HINT) {
-      const int first = (int)blockIdx.x * hint_rows, rows = min(max((int)((uint32_t)p.prefetch_bytes / Shape::HINT_PITCH) - first, 0), hint_rows);
-      const char* const base = (const char*)p.prefetch + (int64_t)first * Shape::HINT_PITCH - nst * Shape::HINT_SEG;
-      rsrc_a = rsrc_w = __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, rows * Shape::HINT_PITCH, 0x00020000);
-      constexpr int LANES = Shape::HINT_SEG / 16;   // ... to a segment
-      const uint32_t lane_off = (lane / LANES) * Shape::HINT_PITCH + (lane % LANES) * 16;
+      const cshint::Share share = cshint::share_of((uint32_t)p.prefetch_bytes, Shape::HINT_PITCH, hint_rows, (int)blockIdx.x);
+      const char* const base = (const char*)p.prefetch + (int64_t)share.first * Shape::HINT_PITCH - nst * Shape::HINT_SEG;
+      rsrc_a = rsrc_w = __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, share.rows * Shape::HINT_PITCH, 0x00020000);
 #pragma unroll
       for (int n = 0; n < NLD; ++n) {
-        const uint32_t off = lane_off + (wave * NLD + n) * (64 / LANES * Shape::HINT_PITCH);
+        const uint32_t off = cshint::small_offset(KS, STAGES, NLD, wave, n, lane);
         if (n < A_LD) a_src[n < A_LD ? n : 0] = off;
         else w_src[n < A_LD ? 0 : n - A_LD] = off;
       }
@@ -647,7 +646,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, EPI == SM_EPI_QKV_WATTN ? 1
     auto iteration = [&](auto steady_c) {
       constexpr bool STEADY = decltype(steady_c)::value;
       read_tile(slot, C1, C1);
-      if (STEADY || kt + STAGES - 1 < nst) issue(kt + STAGES - 1, prev, CMID, CEND);
+      if (STEADY || cshint::small_second_half(kt, STAGES, nst, reads_hint)) issue(kt + STAGES - 1, prev, CMID, CEND);
       multiply(C0);
       if constexpr (STEADY) {
         small_schedule<2 * (MT + NT), NLD - NLD / 2, 2 * MT * NT>();
@@ -669,7 +668,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, EPI == SM_EPI_QKV_WATTN ? 1
       ++kt;
       turn();
     };
-    const int steady = reads_hint ? nst - 1 : nst - STAGES;
+    const int steady = cshint::small_steady(KS, STAGES, nst, reads_hint);
     if (UNROLLED && steady >= 2 * STAGES)
       while (kt + STAGES <= steady) small_for([&](auto) { iteration(T); }, std::make_integer_sequence<int, STAGES>{});
     while (kt < steady) iteration(T);
@@ -705,7 +704,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, EPI == SM_EPI_QKV_WATTN ? 1
       ++kt;
       turn();
     };
-    const int steady = reads_hint ? nst - 2 : nst - STAGES - 1;   // (the last of an odd count goes with the others)
+    const int steady = cshint::small_steady(KS, STAGES, nst, reads_hint);   // (the last of an odd count goes with the others)
     while (kt < steady) {
       iteration(T, C0);
       iteration(T, C1);
@@ -906,14 +905,22 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, EPI == SM_EPI_QKV_WATTN ? 1
 }
 
 // A launch with a tile for every compute unit has nobody idle to read its hint, but nothing to request in its last STAGES - 1
-// iterations and its epilogue either: its workgroups read a share each with the ring's own loads, into slots that are free by then.
-// The hint is cut into rows of HINT_STAGES segments; a lane's row and place in it are fixed, and the stages walk along the row.
-// Returns the rows of a workgroup, at most what its loads cover; what is left of the hint is not read.
+// iterations and its epilogue either: its workgroups read a share each with the ring's own loads, into slots that are free by then
+// (hint_ring.h).  Returns the rows of a workgroup, at most what its loads cover; what is left of the hint is not read.
 template <class Shape, int WAVES>
 int hint_rows_of(int64_t bytes, int tiles) {
   if (!Shape::RING_HINT) return 0;
-  const int64_t share = (bytes / Shape::HINT_PITCH + tiles - 1) / tiles, most = WAVES * Shape::NLD_OF(WAVES) * (1024 / Shape::HINT_SEG);
-  return (int)(share < most ? share : most);
+  return cshint::rows_of(bytes, Shape::HINT_PITCH, tiles, cshint::small_rows(Shape::HINT_SEG / 128, WAVES, Shape::NLD_OF(WAVES)));
+}
+
+// Bytes of a hint of `bytes` that a launch of so many tiles leaves at its end: none with idle workgroups, else what the shares do not
+// reach (less than a row is not worth another launch's while).
+template <class Shape, int WAVES>
+int64_t hint_left_of(int64_t bytes, int tiles) {
+  if (hint_workgroups(tiles)) return 0;
+  if (!Shape::RING_HINT) return bytes;
+  const int64_t left = bytes - cshint::bytes_of(bytes, Shape::HINT_PITCH, tiles, cshint::small_rows(Shape::HINT_SEG / 128, WAVES, Shape::NLD_OF(WAVES)));
+  return left < Shape::HINT_PITCH ? 0 : left;
 }
 
 template <int BM, int BN, int WAVES_M, int WAVES_N, int KS, int STAGES, int EPI, bool W_FP8, int NORM, bool SPLIT, int SUMS = SUMS_NONE>

@@ -63,6 +63,12 @@ int launch_projection(const CsGemmArgs& p, int bm, int bn, hipStream_t stream) {
   if (bn == 64) return launch_small<64, 64, 4, 2, 2, 4, SM_EPI_QKV_F32, false, NORM, false>(p, stream);
   return launch_small<64, 128, 4, 2, 2, 3, SM_EPI_QKV_F32, false, NORM, false>(p, stream);
 }
+// ... and of the hint that it has, the bytes that this launch leaves
+int64_t projection_leaves(int64_t hint, int tiles, int bm, int bn) {
+  if (bm == 32) return hint_left_of<SmallShape<32, 64, 2, 6, false, NORM_NONE, SUMS_NONE>, 4>(hint, tiles);
+  if (bn == 64) return hint_left_of<SmallShape<64, 64, 2, 4, false, NORM_NONE, SUMS_NONE>, 8>(hint, tiles);
+  return hint_left_of<SmallShape<64, 128, 2, 3, false, NORM_NONE, SUMS_NONE>, 8>(hint, tiles);
+}
 
 }  // namespace
 
@@ -85,7 +91,7 @@ int cs_qkv_window_attn_two(const CsGemmArgs& a, int rows, int windows, float* x,
   // (the hint's rest)
   CsGemmArgs q = a;
   if (a.prefetch && p.prefetch) {
-    const int64_t done = p.prefetch_bytes & ~(int64_t)15;
+    const int64_t done = (p.prefetch_bytes - projection_leaves(p.prefetch_bytes, tiles_of(bm, bn), bm, bn)) & ~(int64_t)15;
     q.prefetch = (const char*)a.prefetch + done;
     q.prefetch_bytes = a.prefetch_bytes - done;
   }

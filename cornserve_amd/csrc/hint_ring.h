@@ -15,6 +15,10 @@ constexpr int rows_of(int64_t bytes, int pitch, int workgroups, int most) {
   const int64_t share = (bytes / pitch + workgroups - 1) / workgroups;
   return (int)(share < most ? share : most);
 }
+constexpr int64_t bytes_of(int64_t bytes, int pitch, int workgroups, int most) {   // what all of them read, from the hint's start
+  const int64_t whole = bytes / pitch, reach = (int64_t)workgroups * most;
+  return (whole < reach ? whole : reach) * pitch;
+}
 constexpr Share share_of(uint32_t bytes, int pitch, int hint_rows, int workgroup) {
   const int first = workgroup * hint_rows, left = (int)(bytes / (uint32_t)pitch) - first;
   return {first, left < 0 ? 0 : left < hint_rows ? left : hint_rows};
@@ -42,6 +46,22 @@ constexpr int big_loads(const BigRing& r, bool w_fp8) { return w_fp8 ? r.a_ld : 
 constexpr int big_rows(const BigRing& r, bool w_fp8) { return 4 * big_loads(r, w_fp8) * 8; }
 constexpr uint32_t big_offset(const BigRing& r, bool w_fp8, int wave, int load, int lane) {   // eight lanes to a segment
   return (uint32_t)(((wave * big_loads(r, w_fp8) + load) * 8 + (lane >> 3)) * BIG_PITCH + (lane & 7) * 16);
+}
+
+// ---- The few-row kernel (gemm_small_impl.h): a ring of `stages` slots, `ks` K tiles of 64 to a stage, `nst` stages of the matrix.  ks 1:
+// iteration kt requests stage kt + stages whole, but for the last two (K tiles go in pairs), which request nothing.  ks 2: its loads'
+// first half behind the barrier of iteration kt, the second half at the top of iteration kt + 1; the last iteration, which has no
+// barrier, completes a stage of the hint.
+constexpr int small_segment(int ks) { return ks * 128; }
+constexpr int small_segments(int ks, int stages) { return ks == 2 ? stages - 1 : stages - 2; }
+constexpr int small_steady(int ks, int stages, int nst, bool hint) {   // iterations that begin a stage
+  return ks == 2 ? (hint ? nst - 1 : nst - stages) : (hint ? nst - 2 : nst - stages - 1);
+}
+// (ks 2) whether iteration kt requests the second half of stage kt + stages - 1
+constexpr bool small_second_half(int kt, int stages, int nst, bool hint) { return hint || kt + stages - 1 < nst; }
+constexpr int small_rows(int ks, int waves, int nld) { return waves * nld * (1024 / small_segment(ks)); }
+constexpr uint32_t small_offset(int ks, int stages, int nld, int wave, int load, int lane) {   // a segment is 8 ks lanes
+  return (uint32_t)((lane / (8 * ks) + (wave * nld + load) * (8 / ks)) * (small_segments(ks, stages) * small_segment(ks)) + lane % (8 * ks) * 16);
 }
 
 }  // namespace cshint

@@ -38,8 +38,7 @@ void check(const char* what, int64_t bytes, int workgroups, int waves, int segme
         }
       });
   }
-  const int64_t want = bytes / pitch * pitch, reach = (int64_t)workgroups * most * pitch;
-  if (covered != (want < reach ? want : reach)) { printf("%s, %ld bytes: %ld in shares\n", what, (long)bytes, (long)covered); exit(1); }
+  if (covered != bytes_of(bytes, pitch, workgroups, most)) { printf("%s, %ld bytes: %ld in shares\n", what, (long)bytes, (long)covered); exit(1); }
   for (int64_t i = 0; i < bytes; ++i)
     if (times[i] != (i < covered)) { printf("%s, %ld bytes: byte %ld is read %d times\n", what, (long)bytes, (long)i, times[i]); exit(1); }
 }
@@ -73,8 +72,45 @@ int main() {
 }
 """
 
+# a few-row launch's iterations in order, with the sources moved behind the top of iteration nst - stages
+_FEW_ROWS = r"""
+int main() {
+  const int forms[][5] = {{32, 32, 4, 2, 8}, {32, 64, 4, 2, 6}, {64, 64, 8, 2, 4}, {64, 80, 4, 2, 4}, {64, 128, 8, 2, 3}, {32, 160, 4, 2, 3},
+                          {64, 160, 8, 1, 4}, {64, 240, 4, 1, 4}};
+  for (auto& f : forms) {
+    const int bm = f[0], bn = f[1], waves = f[2], ks = f[3], stages = f[4];
+    const int nld = ks * (bm / 8) / waves + (ks * (bn / 8) + waves - 1) / waves;
+    for (int nst : {stages, stages + 2}) {
+      if (ks == 1 && nst % 2) continue;
+      auto requests = [&](auto&& read) {
+        for (int kt = 0; kt < nst; ++kt) {
+          const bool steady = kt < small_steady(ks, stages, nst, true);
+          auto loads = [&](int stage, int from, int to) {
+            if (stage < nst) return;
+            if (stage - nst >= small_segments(ks, stages)) { printf("stage %d of %d\n", stage, nst); exit(1); }
+            for (int n = from; n < to; ++n) read(stage - nst, n);
+          };
+          if (ks == 2) {
+            if (steady || small_second_half(kt, stages, nst, true)) loads(kt + stages - 1, nld / 2, nld);
+            if (steady) loads(kt + stages, 0, nld / 2);
+          } else if (steady) {
+            loads(kt + stages, 0, nld);
+          }
+        }
+      };
+      char what[64];
+      snprintf(what, sizeof what, "%dx%d, %d stages", bm, bn, nst);
+      for (int64_t bytes : {16l, 1000l, 768l * 193, 1000016l, 20l << 20})
+        for (int workgroups : {193, 256, 480})
+          check(what, bytes, workgroups, waves, small_segment(ks), small_segments(ks, stages), small_rows(ks, waves, nld), requests,
+                [&](int wave, int load, int lane) { return small_offset(ks, stages, nld, wave, load, lane); });
+    }
+  }
+}
+"""
 
-@pytest.mark.parametrize("kernel,main", [pytest.param("big", _BIG, id="big tiles")])
+
+@pytest.mark.parametrize("kernel,main", [pytest.param("big", _BIG, id="big tiles"), pytest.param("few", _FEW_ROWS, id="few rows")])
 def test_the_ring_reads_every_byte_of_its_share_once(tmp_path, kernel, main):
     gxx = shutil.which("g++")
     if gxx is None:
