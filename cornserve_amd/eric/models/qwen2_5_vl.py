@@ -564,7 +564,8 @@ class Qwen2_5_VisionTransformer(QwenVisionBase):
         # What bounds a launch of few rows is the latency of weights that nothing has touched since the previous forward pass: the
         # one-launch window block reads the gate|up weights, the attention-output projection (from `proj_hint_rows` on, gate|up) the
         # down-projection's, the down-projection the next block's qkv and projection weights.  (3072 patches 5.39 -> 5.02 ms, 1280
-        # 3.87 -> 3.57, 1024 2.92 -> 2.75, 4096 6.04 -> 5.82.)
+        # 3.87 -> 3.57, 1024 2.92 -> 2.75, 4096 6.04 -> 5.82; the hint at gate|up alone, unfolded norms: 3136 5.30 -> 5.22, 4096 6.23 -> 6.01,
+        # 4224 6.99 -> 6.78, 5776 8.62 -> 8.57, the same from 6840 on; with fp8 weights, half the bytes, 0.998 to 1.001 throughout.)
         hint = L <= self.prefetch_rows
 
         def next_qkv(i: int) -> torch.Tensor | None:
@@ -624,7 +625,7 @@ class Qwen2_5_VisionTransformer(QwenVisionBase):
                 mark("norm")
                 ops.rmsnorm(x, b["n2"], eps, out=n)
                 mark("gemm_gate_up")
-                self._g(n, b["gu"], epilogue=ops.EPI_SWIGLU, out=hmid)
+                self._g(n, b["gu"], epilogue=ops.EPI_SWIGLU, out=hmid, prefetch=pf_gu)
                 mark("gemm_down")
                 self._g(hmid, b["down"], epilogue=ops.EPI_RESIDUAL, residual=x, out=x, prefetch=pf_down, **res)
 

@@ -296,6 +296,36 @@ def test_qwen_batch_items_are_independent(dev):
         assert all(torch.equal(a, b) for a, b in zip(hinted, plain)), kw
 
 
+def mlp_hints(model, batch, last: str, monkeypatch) -> list[list[tuple[int, int]]]:
+    """Per block, the [N, K] of the products whose launch has the block's last MLP weights read, in order."""
+    from cornserve_amd import ops
+
+    seen, gemm = [], ops.gemm
+
+    def recorded(a, w, *args, prefetch=None, **kw):
+        seen.append((tuple(w.shape), 0 if prefetch is None else prefetch.data_ptr()))
+        return gemm(a, w, *args, prefetch=prefetch, **kw)
+
+    monkeypatch.setattr(ops, "gemm", recorded)
+    model(Modality.IMAGE, "", batch)
+    monkeypatch.undo()
+    return [[shape for shape, at in seen if at == b[last]["w"].data_ptr()] for b in model._ensure_packed()["blocks"]]
+
+
+@pytest.mark.parametrize("family,kw", [("2.5", {}), ("2.5", {"fold_norm": False}), ("2.5", {"weight_format": "fp8_e4m3"})])
+def test_last_mlp_weights_are_hinted_by_the_first_mlp_product_beyond_proj_hint_rows(dev, family, kw, monkeypatch):
+    px, grid = synth.qwen_inputs([(1, 16, 16)], seed=4)
+    model, last, first = build_qwen(dev, 2, (1,), seed=4, **kw)[0], "down", "gu"
+    batch = {"pixel_values": px, "image_grid_thw": grid}
+    blocks = model._ensure_packed()["blocks"]
+    model.proj_hint_rows = 255
+    assert all(tuple(b[first]["w"].shape) in hints for b, hints in zip(blocks, mlp_hints(model, batch, last, monkeypatch)))
+    model.proj_hint_rows = 256
+    assert mlp_hints(model, batch, last, monkeypatch) == [[tuple(b["proj"]["w"].shape)] for b in blocks]
+    model.prefetch_rows = 255
+    assert mlp_hints(model, batch, last, monkeypatch) == [[], []]
+
+
 @pytest.mark.parametrize("family", ["2.5", "2.5, unfused windows", "2.5, full attention first", "2, folded", "3", "gemma, folded"])
 @pytest.mark.parametrize("few", [True, False])
 def test_the_first_statistics_are_summed_in_chunk_order(dev, monkeypatch, family, few):
