@@ -121,7 +121,8 @@ class QwenVisionBase(EricModel):
     # nothing is gained (12288 patches of Qwen2-VL 24.2 -> 24.35 ms with hints).
     prefetch_rows = 8192
     # Up to this many rows (192 tiles of 128x160) the output projection has the last MLP weights read; beyond it the product in front
-    # of the last one does.
+    # of the last one does, and the projection does not, also where its launch has 176 to 192 tiles again (4097 to 4608 rows; with both
+    # reading them 0.997 to 1.003).
     proj_hint_rows = 3072
 
     # what the checkpoint's image processor normalises with (preprocessor_config.json): CLIP statistics for
@@ -185,6 +186,12 @@ class QwenVisionBase(EricModel):
             w, b, *s = ops.unpack_qkv_window_attn(wp, bp, self.num_heads, w_scale=sp[0] if sp else None)
             block["qkv"] = {"w": w, "b": b, "s": s[0] if s else None}
         return block["qkv"]
+
+    def _last_mlp_hint(self, rows: int, w: torch.Tensor) -> tuple[torch.Tensor | None, torch.Tensor | None]:
+        """Which launch of a block has its last MLP weights `w` read: (the output projection's hint, the first MLP product's)."""
+        if rows > self.prefetch_rows:
+            return None, None
+        return (w, None) if rows <= self.proj_hint_rows else (None, w)
 
     def patchify_frames(self, frames: list[torch.Tensor], arithmetic: str = "fused",
                         pixel_budgets: list | None = None) -> tuple[torch.Tensor, np.ndarray]:
@@ -582,8 +589,7 @@ class Qwen2_5_VisionTransformer(QwenVisionBase):
             full = i in self.fullatt_block_indexes
             pf_qkv = b["gu"]["w"] if hint else None   # (from the one-launch window block only: the plain QKV GEMM of a
             # small batch leaves too few compute units idle to read 18 MB in its own time -- measured slower)
-            pf_proj = b["down"]["w"] if hint else None
-            pf_gu = b["down"]["w"] if hint and L > self.proj_hint_rows else None
+            pf_proj, pf_gu = self._last_mlp_hint(L, b["down"]["w"])
             pf_down = next_qkv(i) if hint else None
             if not full and fused_rows:
                 wp, bp, *sp = b["qkv_wattn"]      # (a third entry with fp8 weights: their scales)

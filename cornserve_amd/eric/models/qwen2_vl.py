@@ -185,10 +185,10 @@ class Qwen2VisionTransformer(QwenVisionBase):
         for i, b in enumerate(pk["blocks"]):
             after = pk["blocks"][i + 1]["qkv"] if i + 1 < len(pk["blocks"]) else pk["m1"]
             after_proj = pk["blocks"][i + 1]["proj"]["w"] if i + 1 < len(pk["blocks"]) else None
-            pf_qkv, pf_proj, pf_fc1, pf_fc2 = ((b["fc1"]["w"], b["fc2"]["w"], after["w"], after_proj) if hint
-                                               else (None, None, None, None))
-            if hint and L > self.proj_hint_rows:
-                pf_fc1 = b["fc2"]["w"]
+            pf_qkv, pf_fc2 = (b["fc1"]["w"], after_proj) if hint else (None, None)
+            pf_proj, pf_fc1 = self._last_mlp_hint(L, b["fc2"]["w"])
+            if pf_proj is not None:
+                pf_fc1 = after["w"]
             if fold:
                 mark("gemm_qkv")
                 ops.gemm(x, b["qkv"]["w"], b["qkv"]["b"], out=qkv, prefetch=pf_qkv, **stats_in(b["qkv"]))

@@ -312,14 +312,19 @@ def mlp_hints(model, batch, last: str, monkeypatch) -> list[list[tuple[int, int]
     return [[shape for shape, at in seen if at == b[last]["w"].data_ptr()] for b in model._ensure_packed()["blocks"]]
 
 
-@pytest.mark.parametrize("family,kw", [("2.5", {}), ("2.5", {"fold_norm": False}), ("2.5", {"weight_format": "fp8_e4m3"})])
+@pytest.mark.parametrize("family,kw", [("2.5", {}), ("2.5", {"fold_norm": False}), ("2.5", {"weight_format": "fp8_e4m3"}),
+                                       ("2", {}), ("2", {"fold_norm": True}), ("3", {}), ("3", {"fold_norm": False})])
 def test_last_mlp_weights_are_hinted_by_the_first_mlp_product_beyond_proj_hint_rows(dev, family, kw, monkeypatch):
-    px, grid = synth.qwen_inputs([(1, 16, 16)], seed=4)
-    model, last, first = build_qwen(dev, 2, (1,), seed=4, **kw)[0], "down", "gu"
+    px, grid = (synth.qwen3_inputs if family == "3" else synth.qwen_inputs)([(1, 16, 16)], seed=4)
+    if family == "2.5":
+        model, last, first = build_qwen(dev, 2, (1,), seed=4, **kw)[0], "down", "gu"
+    else:
+        model = (build_qwen2(dev, 2, seed=4, **kw) if family == "2" else build_qwen3(dev, 2, (0,), 1024, seed=4, **kw))[0]
+        last, first = "fc2", "fc1"
     batch = {"pixel_values": px, "image_grid_thw": grid}
     blocks = model._ensure_packed()["blocks"]
     model.proj_hint_rows = 255
-    assert all(tuple(b[first]["w"].shape) in hints for b, hints in zip(blocks, mlp_hints(model, batch, last, monkeypatch)))
+    assert mlp_hints(model, batch, last, monkeypatch) == [[tuple(b[first]["w"].shape)] for b in blocks]
     model.proj_hint_rows = 256
     assert mlp_hints(model, batch, last, monkeypatch) == [[tuple(b["proj"]["w"].shape)] for b in blocks]
     model.prefetch_rows = 255
