@@ -181,8 +181,8 @@ constexpr bool ring_takes_edges() {
 // and the window blocks, which have no registers left.  Weights that come from HBM cost a launch of 4096 rows 2 to 10 us (1152 x 4352:
 // 42.7 us with them in the caches, 49.5 without, 53 in a pass); SigLIP's qkv and fc1 products hint those behind them: one 896x896
 // image 6.93 -> 6.66 ms, one 768x1152 image in tiles 6.02 -> 5.76.  At most HINT_MAX_BYTES, which travel in the last iterations, and
-every byte of a workgroup's share (hint_ring.h).  While the share's rows had a third segment, of which the five-unit ring requests nothing and
-the three-stage one half: one 896x896 image 7.00 -> 6.91 ms, five 384x384 tiles 4.72 -> 4.62, Qwen2-VL 3136 patches 7.82 -> 7.74.
+// every byte of a workgroup's share (hint_ring.h).  While the share's rows had a third segment, of which the five-unit ring requests nothing and
+// the three-stage one half: one 896x896 image 7.00 -> 6.91 ms, five 384x384 tiles 4.72 -> 4.62, Qwen2-VL 3136 patches 7.82 -> 7.74.
 constexpr int64_t HINT_MAX_BYTES = 16 << 20;
 template <int BM, int BN, int WAVES_M, int WAVES_N, int EPI, bool W_FP8, int FUSE, bool SPLIT_RES>
 constexpr bool ring_reads_hint() {
