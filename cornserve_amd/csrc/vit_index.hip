@@ -14,6 +14,8 @@
 //   (permute(0,1,3,2,4) then boolean compaction, :372-379).  Empty pad windows contribute nothing.
 #include <math.h>
 
+#include <algorithm>
+
 #include "common.h"
 
 namespace {
@@ -24,8 +26,12 @@ struct ItemMeta {  // matches the int32[8] record documented in cornserve_amd.h
 
 // Bound by the sines and cosines, 80 of them a patch with heads of 80: a lane computes the four of one frequency (with one thread
 // per patch an image of 1024 patches, four workgroups, took 15.5 us: a chain of 80 calls).  96 patches 10.2 -> 4.7 us, 1024 15.5 ->
-// 5.0, 58648 42 -> 20.
-constexpr int INDEX_LANES = 32, INDEX_PATCHES = 8;   // lanes of a patch, patches of a workgroup
+// 5.0, 58648 42 -> 20.  Every item has as many workgroups as the largest could use, up to one for 256 of its patches or, if that is more,
+// INDEX_CHIP among all items, and a workgroup goes on to further patches.  With one for every 8 patches an image of 58560 patches beside
+// 100, 1000 and 10000 small ones took 169, 1558 and 15380 us, nearly all of it workgroups with nothing to do (now 33, 54 and 518), and
+// an item of more than 2^27 patches had more threads than a launch can have: most of its rows were left unwritten.
+constexpr int INDEX_LANES = 32, INDEX_PATCHES = 8;   // lanes of a patch, patches of a workgroup at a time
+constexpr int INDEX_CHIP = 16384;
 __global__ __launch_bounds__(INDEX_LANES * INDEX_PATCHES) void vit_index_kernel(const ItemMeta* __restrict__ meta, int merge, int win,
                                                         const float* __restrict__ inv_freq, int rot_dim,
                                                         int32_t* __restrict__ window_index,
@@ -37,43 +43,44 @@ __global__ __launch_bounds__(INDEX_LANES * INDEX_PATCHES) void vit_index_kernel(
   const int mm = merge * merge;
   const int frame_units = it.gh * it.gw;
   const int n_patches = it.t * frame_units * mm;
-  const int pl = blockIdx.x * INDEX_PATCHES + threadIdx.x / INDEX_LANES;  // patch within the item, ORIGINAL order
   const int lane = threadIdx.x % INDEX_LANES;
-  if (pl >= n_patches) return;
-  const int ul = pl / mm, s = pl - ul * mm;
-  const int f = ul / frame_units;
-  const int rem = ul - f * frame_units;
-  const int r = rem / it.gw, c = rem - r * it.gw;
-  const int wr = r / win, wc = c / win;
-  const int rh = min(win, it.gh - wr * win);
-  const int cw = min(win, it.gw - wc * win);
-  const int pos = wr * win * it.gw + rh * wc * win + (r - wr * win) * cw + (c - wc * win);
-  const int u = it.unit_base + ul;                     // original unit id
-  const int up = it.unit_base + f * frame_units + pos;  // window-order unit id
-  if (s == 0 && lane == 0) {
-    if (window_index) window_index[up] = u;
-    if (reverse_index) reverse_index[u] = up;
-  }
-  const int h = r * merge + s / merge;
-  const int w = c * merge + s % merge;
-  const int64_t row_orig = (int64_t)u * mm + s;
-  const int64_t row_win = (int64_t)up * mm + s;
-  // (the caller's patch matrix may hold the items in another order than they are processed in)
-  if (src_rows && lane == 0) src_rows[row_win] = (int32_t)((int64_t)(it.src_unit_base + ul) * mm + s);
-  if (pos_ids && lane == 0) {
-    pos_ids[row_orig * 2 + 0] = h;
-    pos_ids[row_orig * 2 + 1] = w;
-  }
-  if (cos_sin) {
-    const int half = rot_dim / 2;
-    float* out = cos_sin + row_win * (2 * rot_dim);
-    for (int j = lane; j < half; j += INDEX_LANES) {
-      const float fr = inv_freq[j];
-      const float ah = (float)h * fr, aw = (float)w * fr;
-      out[j] = cosf(ah);
-      out[half + j] = cosf(aw);
-      out[rot_dim + j] = sinf(ah);
-      out[rot_dim + half + j] = sinf(aw);
+  for (int64_t patch = (int64_t)blockIdx.x * INDEX_PATCHES + threadIdx.x / INDEX_LANES; patch < n_patches; patch += (int64_t)gridDim.x * INDEX_PATCHES) {
+    const int pl = (int)patch;   // within the item, ORIGINAL order
+    const int ul = pl / mm, s = pl - ul * mm;
+    const int f = ul / frame_units;
+    const int rem = ul - f * frame_units;
+    const int r = rem / it.gw, c = rem - r * it.gw;
+    const int wr = r / win, wc = c / win;
+    const int rh = min(win, it.gh - wr * win);
+    const int cw = min(win, it.gw - wc * win);
+    const int pos = wr * win * it.gw + rh * wc * win + (r - wr * win) * cw + (c - wc * win);
+    const int u = it.unit_base + ul;                     // original unit id
+    const int up = it.unit_base + f * frame_units + pos;  // window-order unit id
+    if (s == 0 && lane == 0) {
+      if (window_index) window_index[up] = u;
+      if (reverse_index) reverse_index[u] = up;
+    }
+    const int h = r * merge + s / merge;
+    const int w = c * merge + s % merge;
+    const int64_t row_orig = (int64_t)u * mm + s;
+    const int64_t row_win = (int64_t)up * mm + s;
+    // (the caller's patch matrix may hold the items in another order than they are processed in)
+    if (src_rows && lane == 0) src_rows[row_win] = (int32_t)((int64_t)(it.src_unit_base + ul) * mm + s);
+    if (pos_ids && lane == 0) {
+      pos_ids[row_orig * 2 + 0] = h;
+      pos_ids[row_orig * 2 + 1] = w;
+    }
+    if (cos_sin) {
+      const int half = rot_dim / 2;
+      float* out = cos_sin + row_win * (2 * rot_dim);
+      for (int j = lane; j < half; j += INDEX_LANES) {
+        const float fr = inv_freq[j];
+        const float ah = (float)h * fr, aw = (float)w * fr;
+        out[j] = cosf(ah);
+        out[half + j] = cosf(aw);
+        out[rot_dim + j] = sinf(ah);
+        out[rot_dim + half + j] = sinf(aw);
+      }
     }
   }
 }
@@ -300,7 +307,8 @@ extern "C" int cs_vit_index(const int32_t* item_meta, int32_t n_items, int32_t m
   if (n_items == 0 || max_units_per_item == 0) return CS_OK;
   if (n_items > 65535) return CS_ERR_TOO_LARGE;
   const int64_t max_patches = (int64_t)max_units_per_item * merge * merge;
-  const dim3 grid((unsigned)((max_patches + INDEX_PATCHES - 1) / INDEX_PATCHES), n_items), block(INDEX_LANES * INDEX_PATCHES);
+  const int64_t most = std::max<int64_t>((max_patches + 255) / 256, INDEX_CHIP / n_items);
+  const dim3 grid((unsigned)std::min<int64_t>((max_patches + INDEX_PATCHES - 1) / INDEX_PATCHES, most), n_items), block(INDEX_LANES * INDEX_PATCHES);
   hipLaunchKernelGGL(vit_index_kernel, grid, block, 0, stream, (const ItemMeta*)item_meta, merge, win, inv_freq,
                      rot_dim, window_index, reverse_index, src_rows, pos_ids, cos_sin);
   return cs_launch_status();

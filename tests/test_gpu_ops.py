@@ -70,6 +70,37 @@ def test_vit_index_bit_exact(ops, dev, golden_dir):
         assert (ix.cos_sin.cpu() - ref).abs().max().item() <= 2e-6, name  # fp32 cos/sin, angles < 100 rad
 
 
+@pytest.mark.parametrize("grids", [[(1, 180, 200)] + [(1, 2, 4)] * 300, [(2, 62, 66), (1, 2, 2)] * 24])
+def test_vit_index_workgroups_go_on_to_further_patches(ops, dev, grids):
+    """An item that is much larger than its share of the launch (one beside 300 small ones: 141 workgroups for 36000 patches)."""
+    inv_freq = (1.0 / (10000.0 ** (torch.arange(0, 40, 2, dtype=torch.float) / 40))).to(dev)
+    sl = ops.vit_seqlens_host(np.array(grids, np.int64), 2, 4)
+    meta = torch.from_numpy(sl.item_meta).to(dev)
+    ix = ops.vit_index(meta, sl.total_patches, sl.max_units_per_item, 2, 4, inv_freq, want_pos_ids=True)
+    wi, pos = vi.get_window_index(grids)[0], vi.rot_pos_ids(grids)
+    assert np.array_equal(ix.window_index.cpu().numpy(), wi) and np.array_equal(ix.reverse_index.cpu().numpy(), np.argsort(wi))
+    assert np.array_equal(ix.pos_ids.cpu().numpy(), pos)
+    assert np.array_equal(ix.src_rows.cpu().numpy(), (wi[:, None] * 4 + np.arange(4)[None, :]).reshape(-1))
+    for i in (0, 1, len(grids) - 1):   # an item alone has a workgroup for every eight patches: the same rows
+        one = ops.vit_seqlens_host(np.array(grids[i : i + 1], np.int64), 2, 4)
+        alone = ops.vit_index(torch.from_numpy(one.item_meta).to(dev), one.total_patches, one.max_units_per_item, 2, 4, inv_freq)
+        first = sum(t * h * w for t, h, w in grids[:i])
+        assert torch.equal(alone.cos_sin, ix.cos_sin[first : first + one.total_patches]), i
+
+
+def test_vit_index_of_more_patches_than_a_launch_has_threads(ops, dev):
+    """One item of 134 million patches (32 lanes each are more than 2^32), its window index alone."""
+    from cornserve_amd import lib
+
+    side = 5794
+    meta = torch.tensor([[1, side, side, 0, 1, 1, 0, 0]], dtype=torch.int32, device=dev)
+    index = torch.full((side * side + 1,), -1, dtype=torch.int32, device=dev)
+    st = lib.load().cs_vit_index(meta.data_ptr(), 1, side * side, 2, 1 << 20, None, 0, index.data_ptr(), None, None, None, None,
+                                 torch.cuda.current_stream().cuda_stream)
+    assert st == 0 and index[-1].item() == -1
+    assert torch.equal(index[:-1], torch.arange(side * side, dtype=torch.int32, device=dev))
+
+
 def test_row_gather_bit_exact(ops, dev):
     x = rnd((1000, 1280), dev=dev)
     rows = torch.randperm(1000, generator=torch.Generator().manual_seed(0)).int().to(dev)
