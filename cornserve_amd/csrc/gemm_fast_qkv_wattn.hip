@@ -25,7 +25,24 @@ int big_tiles(CsGemmArgs a, bool ragged, hipStream_t stream) {
   return launch<256, 256, 4, 1, CS_EPI_QKV_WATTN, false, 0>(a, stream);
 }
 
+// Windows behind the last whole round of big tiles (256 workgroups of four windows and a head) cost a round of their own; few enough
+// for a workgroup per window and head go to a second launch, which finds the weights in the caches.  Weights from HBM, K = 1280, whole
+// rounds | with the windows that are split | with one more, in one launch again.  bf16 and folded norm: 16 heads 64 windows 42 us | 65 to 80
+// 56 to 59 | 81 67, 128 76 | 144 94 | 145 104; 32 heads 32 43 | 33 to 40 57 to 60 | 41 69; 10 100 42 | 125 57 | 126 68; 8 128 40 | 160 59 |
+// 161 66; 4 256 40 | 320 58 | 321 66; 2 512 40 | 640 57 | 641 66; 3 340 41 | 425 57 | 426 64.  fp8: 16 heads 64 46 | 80 59 | 81 74; 8 128 41 | 160
+// 60 | 161 75; 3 340 42 | 425 59 | 426 73; 24 heads, K = 1920, 40 61 | 50 77 | 51 101.  K = 640, 8 heads: 128 25 | 160 39 | 161 43.
+// Returns the windows of the first launch, 0 for one launch.
+int64_t lead_windows(int64_t windows, int heads, int K) {
+  if (cs_qkv_window_attn_few(windows, heads, K)) return 0;
+  const int64_t round = 256 / heads * 4, rest = round ? windows % round : 0;
+  return rest && rest < windows && cs_qkv_window_attn_few(rest, heads, K) ? windows - rest : 0;
+}
+
 }  // namespace
+
+extern "C" int cs_qkv_window_attn_lead_windows(int32_t windows, int32_t heads, int32_t K) {
+  return windows < 1 || heads < 1 || K < 1 ? 0 : (int)lead_windows(windows, heads, K);
+}
 
 extern "C" int cs_qkv_window_attn_workspace(int32_t rows, int32_t windows, int32_t heads, int32_t K, int32_t w_fp8) {
   if (rows < 1 || windows < 1 || heads < 1 || K < 1 || !cs_qkv_window_attn_two_pays(rows, windows, heads, K, w_fp8 != 0)) return 0;
@@ -80,12 +97,8 @@ extern "C" int cs_qkv_window_attn_ws(const CsGemmArgs* gemm, const float* cos_si
     return cs_qkv_window_attn_small(a, rows, stream);
   }
   if (a.a_norm_inline) return CS_ERR_UNSUPPORTED;
-  // Windows behind the last whole round of big tiles cost a round of their own; few enough for a workgroup per window and head go
-  // to a second launch, which finds the weights in the caches: 16 heads, 65 to 80 windows
-  // 71.5 -> 62 us (64 windows 43.5), 140 111.5 -> 102.
-  const int64_t windows = ragged ? a.attn_n_win : a.M / 64, round = 256 / heads * 4, rest = round ? windows % round : 0;
-  if (rest && rest < windows && cs_qkv_window_attn_few(rest, heads, a.K)) {
-    const int64_t lead = windows - rest;
+  const int64_t windows = ragged ? a.attn_n_win : a.M / 64, lead = lead_windows(windows, heads, a.K), rest = windows - lead;
+  if (lead) {
     CsGemmArgs first = a, second = a;
     first.prefetch = nullptr;
     first.prefetch_bytes = 0;

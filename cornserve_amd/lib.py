@@ -82,6 +82,7 @@ _SIGNATURES: dict[str, list] = {
     "cs_gemm_norm_inline_pays": [c_int32, c_int32, c_int32, c_int32],
     "cs_gemm_rmsnorm_noalloc": [POINTER(CsGemmArgs), c_void_p],
     "cs_qkv_window_attn": [POINTER(CsGemmArgs), c_void_p, c_float, c_int32, c_int32, c_void_p],
+    "cs_qkv_window_attn_lead_windows": [c_int32, c_int32, c_int32],
     "cs_qkv_window_attn_workspace": [c_int32, c_int32, c_int32, c_int32, c_int32],
     "cs_qkv_window_attn_ws": [POINTER(CsGemmArgs), c_void_p, c_float, c_int32, c_int32, c_void_p, c_int64, c_void_p],
     "cs_row_sumsq": [c_void_p, c_int64, c_int32, c_int32, c_void_p, c_void_p],

@@ -338,6 +338,10 @@ int cs_attn_varlen_keys_rotated(const void* q, const void* k, const void* v, int
 int cs_qkv_window_attn(const CsGemmArgs* gemm, const float* cos_sin, float scale, int32_t heads, int32_t head_dim,
                        void* stream);
 
+/* Host routine: of a call whose last windows take a second launch (same bits), how many windows the first covers; 0 for any
+ * other call.                                                                                                            */
+int cs_qkv_window_attn_lead_windows(int32_t windows, int32_t heads, int32_t K);
+
 /* The same with a workspace (16-byte aligned device memory that nothing else uses until the call's work has run): a few windows
  * then run as two launches, the projection over the whole chip and the attention of its fp32 values.  Same bits.
  * cs_qkv_window_attn_workspace (host routine): the bytes it takes for `rows` rows of A in `windows` windows, 0 where one

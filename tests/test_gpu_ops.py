@@ -715,8 +715,8 @@ def test_gemm_row_split_gives_the_bits_of_one_launch(ops, dev, M, N, K, epi, kin
     assert all(torch.equal(x, y) for r in results[1:] for x, y in zip(r, results[0]))
 
 
-# A launch of more than 192 tiles reads its hint with the ring behind every workgroup's last tile (ring-fed residual products and the
-# general epilogue's launches leave it alone): the bits of the launch without a hint, in every form, with one tile a workgroup and
+# A launch of more than 192 tiles reads its hint with the ring behind every workgroup's last tile (ring-fed residual products
+# leave it alone): the bits of the launch without a hint, in every form that is built, with one tile a workgroup and
 # several, at edges, with hints from less than a row of it to more than all workgroups read.
 @pytest.mark.parametrize("M,N,K", [(4096, 3456, 192), (4097, 3464, 256), (7290, 5120, 320)])
 @pytest.mark.parametrize("fp8", [False, True])
@@ -758,8 +758,10 @@ def test_full_launches_read_their_hint_with_the_ring(ops, dev, M, N, K, fp8):
                 if h is not None:
                     g.prefetch, g.prefetch_bytes = h.data_ptr(), h.numel()
                 status = run(ctypes.byref(g), torch.cuda.current_stream().cuda_stream)
-                assert status in (0, 2), (name, epi, kind, status)
-                if status:
+                # (not built: a folded LayerNorm in 256x256, and of 128x160 with fp8 weights all but the residual products)
+                built = not (kind == "ln" and name == "256x256") and not (fp8 and name == "128x160" and epi != ops.EPI_RESIDUAL)
+                assert status == (0 if built else lib.CS_ERR_UNSUPPORTED), (name, epi, kind, status)
+                if not built:
                     break
                 want = want or (out, out_lo)
                 assert torch.equal(out, want[0]) and torch.equal(out_lo, want[1]), (name, epi, kind, h.numel())
@@ -1010,7 +1012,11 @@ def test_qkv_window_attn_few_windows_equal_many(ops, dev, windows, heads, ragged
 def test_qkv_window_attn_windows_behind_the_last_round(ops, dev, windows, more, heads, ragged, form):
     """Windows behind the last whole round of big tiles, few enough for a workgroup per window and head, take a second launch: the
     bits of a launch of a few windows more, which are too many for that."""
+    from cornserve_amd import lib
+
     K, d = 1280, 80
+    lead = lib.load().cs_qkv_window_attn_lead_windows
+    assert lead(windows, heads, K) == windows - windows % (256 // heads * 4) > 0 and lead(more, heads, K) == 0
     g = torch.Generator().manual_seed(windows)
     counts = torch.randint(1, 17, (more,), generator=g) * 4 if ragged else torch.full((more,), 64)
     cu = torch.cat([torch.zeros(1, dtype=torch.int64), counts.cumsum(0)]).int().to(dev)
