@@ -222,7 +222,7 @@ int cs_gemm_fast(const CsGemmArgs& a, hipStream_t stream, bool* handled) {
   const Plan plan = plan_of(a);
   if (plan.lead_rows) {
     CsGemmArgs lead = part_of(a, 0, plan.lead_rows, 0, a.N);
-    lead.prefetch = nullptr;  // the tail launch is the one with idle compute units
+    lead.prefetch = nullptr;  // (the hint stays with the tail, whose few tiles leave compute units idle; the lead could read it with its ring)
     const CsGemmArgs rest = part_of(a, plan.lead_rows, a.M - plan.lead_rows, 0, a.N);
     const int st = plan.lead->run(lead, stream);
     if (st != CS_OK) return st;

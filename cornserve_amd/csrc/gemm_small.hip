@@ -92,14 +92,17 @@ const Form* best_form(const Form (&forms)[COUNT], const CsGemmArgs& a, double* u
 
 int tiles_of(const Form& f, const CsGemmArgs& a) { return ((a.M + f.bm - 1) / f.bm) * ((a.N + f.bn - 1) / f.bn); }
 
-// Whether a launch has too many tiles to read its hint where the big form would read it.  The launch that the hint is for then
+// Whether a launch has too many tiles for idle compute units to read its hint, where the big form has some.  Of 128x128 tiles nobody
+// reads it then, and the launch that the hint is for
 // finds its weights cold (2700 rows of Qwen2-VL: projection 24 us instead of 17), so such a launch goes to the few-row kernel only
 // if it is 15 % faster there.  Passes with few-row tiles and the hint unread -> with the big form: Qwen2-VL 2700 patches (fc2: 220
 // tiles of 128x128 or 176 of 128x160; 43 and 49 us by the table) 7.51 -> 7.31 ms, 3024 8.17 -> 7.93.  One image of 1024 rows has
 // 256 small tiles that are 30 to 50 % faster, and keeps them.  Not so with row sums, where it goes either way (Qwen2.5-VL 1600
 // patches 4.17 -> 4.14, 1764 4.22 -> 4.34, 1936 4.27 -> 4.13) and the few-row forms stay; nor with fp8 weights, where the big form
 // is slower by more than that (2700 patches 5.78 -> 6.06).  A hint that the big form has no time for either, as that for the
-// merger's 52 MB, would only make its launch longer.
+// merger's 52 MB, would only make its launch longer.  Smaller tiles read it with the ring, and the line is the same for them: a product
+// and the one that its hint of 4 MB is for, K = 2048, both with weights from HBM, 128x160 | 64x80 for the first: 2048 rows x 1152 36.7 | 39.1 us,
+// 1280 x 1920 35.6 | 38.9, 832 x 2560 31.0 | 34.4, 1664 x 1280 35.7 | 35.7 (of the encoders' products only those of 128x128 tiles come this near).
 constexpr double HINT_WORTH = 0.15;
 bool loses_hint(const Form& f, const CsGemmArgs& a, double big_us, int64_t big_tiles) {
   if (!a.prefetch || a.prefetch_bytes < 16 || a.w_fp8 || a.c_row_sumsq || tiles_of(f, a) <= csgemm::HINT_MAX_TILES) return false;
