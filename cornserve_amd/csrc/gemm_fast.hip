@@ -119,7 +119,7 @@ CsGemmArgs part_of(const CsGemmArgs& a, int m0, int rows, int n0, int cols) {
 // How a launch is made: `form` alone (lead_cols == lead_rows == 0); 256x256 tiles over the first lead_cols columns, which fill
 // whole rounds or nearly, and `form` over the rest in a launch of its own; or `lead` over the first lead_rows rows likewise and,
 // over the others, the few-row kernel (form == nullptr) or `form`.
-constexpr float ROW_SPLIT_US = 3.0f, FEW_ROW_TAIL = 1.33f;
+constexpr float ROW_SPLIT_US = 3.0f;
 struct Plan {
   const BigForm* form;
   int lead_cols;
@@ -143,11 +143,16 @@ Plan plan_of(const CsGemmArgs& a) {
   }
   // Rows behind the last whole round of a form's tiles cost a round of their own, however few they are; in a second launch they take
   // the form that suits so many rows.  One launch -> two, row sums, K = 1280 / 3456: 8800 rows x 1280 48.1 / 85.0 -> 43.1 / 76.8 us,
-  // 20480 87.4 / 177.5 -> 74.7 / 165.8, 58648 280 / 518 -> 259 / 480; fp8 SwiGLU 17000 rows x 6912 x 1280 258 -> 236; GELU 12393 rows
+  // 20480 87.4 / 177.5 -> 74.7 / 165.8, 58648 266 / 508 -> 259 / 480; fp8 SwiGLU 17000 rows x 6912 x 1280 258 -> 236; GELU 12393 rows
   // x 4352 x 1152 121.2 -> 115.6.  ROW_SPLIT_US on top of both launches' estimates, but for residual products led by 160-column
   // tiles, whose times are the surest: without it 5400 rows x 6912 x 1280 (87.9 -> 90.0), 6240 x 4352 x 1152 (62.8 -> 65.1) and the fp8
-  // residual product 19200 x 1280 x 1280 (77.6 -> 80.2) are split too.  FEW_ROW_TAIL: what the few-row kernel takes
-  // longer than its table says where K is long (9800 x 1152 x 4352: 90.1 -> 94.3).  (A position addend counts rows from the matrix's first.)
+  // residual product 19200 x 1280 x 1280 (77.6 -> 80.2) are split too.  (A position addend counts rows from the matrix's first.)
+  // Over 960 launches (15 products, 64 row counts each from 2700 to 28000, one launch in every form and two in every pair of forms timed)
+  // the choice takes 1.006 of the best of them in the mean, 1.04 at 95 %, 1.11 at worst; without row splits 1.013, 1.07 and 1.26.  With 0 us
+  // for ROW_SPLIT_US 1.005, with 3 us for all products 1.008.  A few-row tail counts what its own table says: at 1.33 of that, which one shape
+  // asks for (9792 x 1152 x 4352, 91.9 us so, 93.6 now), 27 launches are planned otherwise and 23 of them are slower: 27184 rows x 1280 x 5120
+  // 317 -> 365 us, fp8 SwiGLU 7252 x 6912 x 1280 109 -> 122, row sums 25504 x 1280 x 1280 100 -> 104.  (A row split has to promise 3 % more
+  // than a column split: a choice, no measurement.  Without it 11 of these launches are planned otherwise, all 2 to 10 % faster.)
   const auto tight = [&](const BigForm& f) { return a.epilogue == CS_EPI_RESIDUAL && f.bn == 160; };
   if (!a.pos) {
     for (const BigForm& f : FORMS) {
@@ -158,7 +163,8 @@ Plan plan_of(const CsGemmArgs& a) {
       const double lead_us = form_us(f, part_of(a, 0, lead, 0, a.N), a.N);
       if (lead_us >= split.us) continue;
       const CsGemmArgs rest = part_of(a, lead, a.M - lead, 0, a.N);
-      double t, few = FEW_ROW_TAIL * cs_gemm_small_us(rest);
+      double t;
+      const double few = cs_gemm_small_us(rest);
       const BigForm* form = best_form(rest, a.N, &t);
       if (few > 0 && few < t) {
         t = few;

@@ -671,6 +671,8 @@ def test_gemm_column_split_gives_the_bits_of_one_launch(ops, dev, M, N, K, fp8):
     (12400, 1280, 320, "EPI_RESIDUAL", "split", 8192), (12400, 1152, 320, "EPI_RESIDUAL", "plain", 8192), (8300, 5120, 5120, "EPI_SWIGLU", "norm", 6400),
     (13060, 5120, 1280, "EPI_QUICK_GELU", "", 13056), (13060, 3840, 1280, "EPI_BIAS", "fp8", 13056), (9730, 5120, 5120, "EPI_BIAS", "rows", 9728),
     (9730, 2560, 640, "EPI_RESIDUAL", "fp8", 8192),
+    (7252, 6912, 1280, "EPI_SWIGLU", "fp8", 7168), (16492, 1280, 1280, "EPI_RESIDUAL", "fp8", 16384),
+    (25504, 1280, 1280, "EPI_RESIDUAL", "sums", 24576),
 ])
 def test_gemm_row_split_gives_the_bits_of_one_launch(ops, dev, M, N, K, epi, kind, lead):
     import ctypes
